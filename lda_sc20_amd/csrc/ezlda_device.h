@@ -26,6 +26,7 @@ struct DevState {
     // tokens, word-major (token id = word rank, doc order, position)
     uint32_t *word_off = nullptr;   // V+1
     uint16_t *z = nullptr;          // N
+    uint32_t *doc_tok = nullptr;    // N: token id of each doc-major position (resident corpora)
     // tokens by doc slot: doc q (docs by descending length) owns slots
     // [soff[q], soff[q+1]), its tokens grouped by word rank, then position
     uint32_t *soff = nullptr;       // D+1
@@ -77,6 +78,9 @@ hipError_t launch_topk(const DevState &s, hipStream_t st);
 // per-token pair, which the sampler does not need).
 hipError_t launch_build_dt(const DevState &s, hipStream_t st, bool n_dk2 = false);
 hipError_t launch_z_to_doc(const DevState &s, hipStream_t st);
+// Topics of the doc-major positions [b, b + n) into out (device or pinned
+// host memory, 16-byte aligned); b is a multiple of 8.
+hipError_t launch_topics_out(const DevState &s, uint32_t b, uint32_t n, uint16_t *out, hipStream_t st);
 // Sampler stages (mode bits): the items of head words, of tail words, and
 // the max-topic shortcut alone (tokens it accepts get their top topic; the
 // others keep theirs for a later full draw).  A token's draw depends only on

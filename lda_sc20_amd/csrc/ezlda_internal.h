@@ -47,6 +47,10 @@ struct ezlda_ctx {
     std::vector<uint32_t> soff;      // D+1: slots of doc q
     std::vector<uint32_t> slot_tok;  // N: slot -> token id
     std::vector<uint32_t> row_off;   // D: DT row offset of doc q (the runs carry it)
+    // readback of the topics (ezlda_get_topics): pinned slots, one a host
+    // thread, with the event of each slot's last kernel
+    uint16_t *read_buf = nullptr;
+    std::vector<hipEvent_t> read_ev;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     int n_xcd = 1;      // XCDs of the device (round-robin workgroup dispatch)

@@ -447,6 +447,35 @@ hipError_t launch_z_to_doc(const DevState &s, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Topics in the corpus' own (doc-major) order, straight into pinned host
+// memory: eight positions a lane, one 16-byte store.  Bound by the gathers (a
+// 2-byte read of z fills a line) and then by the copy out of the pinned pieces:
+// 3.8 ms for 49.5M tokens with its host side; the host loop it replaced (one
+// thread, a random read a token) took 188 ms.
+__global__ void __launch_bounds__(256) k_topics_out(uint32_t b, uint32_t n, const uint32_t *__restrict__ doc_tok,
+                                                    const uint16_t *__restrict__ z, uint16_t *__restrict__ out) {
+    const uint32_t i = (blockIdx.x * 256u + threadIdx.x) * 8u;
+    if (i >= n) return;
+    const uint32_t *dt = doc_tok + b + i;
+    if (i + 8u <= n) {
+        const uint4 p = *reinterpret_cast<const uint4 *>(dt), q = *reinterpret_cast<const uint4 *>(dt + 4);
+        const uint32_t t[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+        uint32_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = z[t[u]];
+        *reinterpret_cast<uint4 *>(out + i) =
+            make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+    } else {
+        for (uint32_t u = 0; i + u < n; ++u) out[i + u] = z[dt[u]];
+    }
+}
+
+hipError_t launch_topics_out(const DevState &s, uint32_t b, uint32_t n, uint16_t *out, hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_topics_out, dim3((n + 2047u) / 2048u), dim3(256), 0, st, b, n, s.doc_tok, s.z, out);
+    return hipGetLastError();
+}
+
 // --------------------------------------------------- DT rows and aux
 // DT_Update_Kernel (utility.cu:79-284), on the doc-major copy of z: doc q
 // (docs in descending length order) owns slots [soff[q], soff[q+1]), its

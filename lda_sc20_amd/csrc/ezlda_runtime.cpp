@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cstdio>
 #include <cmath>
 #include <cstring>
@@ -12,6 +13,7 @@
 #include <new>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -46,6 +48,12 @@ void parallel_for(int64_t n, F f) {
     }
     for (auto &x : th) x.join();
 }
+
+// Topics of one readback slot (a multiple of 8), and slots at most: the copy
+// out of a slot (with the page faults of a fresh destination) is slower than
+// the link that fills it, so several threads share it.
+constexpr uint32_t kReadTokens = 1u << 19;
+constexpr uint32_t kReadSlots = 8;
 
 // DT rows: 16-bit entries for K <= kCompactK (the oracle's ORC_COMPACT_K),
 // tb = max(10, ceil(log2 K)) topic bits, counts in pieces of at most
@@ -211,6 +219,10 @@ void free_device(ezlda_ctx *c) {
     c->dev_bytes = 0;
     c->layout_bytes = 0;
     c->s = ez::DevState{};
+    if (c->read_buf) (void)hipHostFree(c->read_buf);
+    c->read_buf = nullptr;
+    for (hipEvent_t e : c->read_ev) (void)hipEventDestroy(e);
+    c->read_ev.clear();
     for (EzChunk &ch : c->chunks)
         if (ch.img) (void)hipHostFree(ch.img);
     c->chunks.clear();
@@ -241,6 +253,21 @@ int lupload(ezlda_ctx *c, T **p, const std::vector<T> &v) {
     int r = ldalloc(c, p, v.size());
     if (r) return r;
     if (!v.empty()) EZ_TRY_HIP(c, hipMemcpy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+    return EZLDA_OK;
+}
+
+int alloc_readback(ezlda_ctx *c, uint32_t N) {
+    const uint32_t slots = std::min<uint32_t>((uint32_t)std::min<int>(host_threads(), (int)kReadSlots),
+                                              (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens));
+    if (!slots) return EZLDA_OK;
+    EZ_TRY_HIP(c, hipHostMalloc((void **)&c->read_buf, (size_t)slots * std::min(N, kReadTokens) * sizeof(uint16_t),
+                                hipHostMallocDefault));
+    c->read_ev.reserve(slots);
+    for (uint32_t i = 0; i < slots; ++i) {
+        hipEvent_t e = nullptr;
+        EZ_TRY_HIP(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        c->read_ev.push_back(e);
+    }
     return EZLDA_OK;
 }
 
@@ -1036,6 +1063,8 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
     int r = 0;
     if ((r = upload(c, &s.word_off, c->word_off))) return r;
     if ((r = upload(c, &s.z, z))) return r;
+    if ((r = upload(c, &s.doc_tok, c->doc_tok))) return r;
+    if ((r = alloc_readback(c, N))) return r;
     if ((r = upload(c, &s.soff, c->soff))) return r;
     if ((r = upload(c, &s.slot_wrd, slot_wrd))) return r;
     if ((r = upload(c, &s.slot_tok, c->slot_tok))) return r;
@@ -1577,20 +1606,67 @@ int ezlda_loglik_noalloc(ezlda_ctx *c, double *ll) try {
     return ezc::exception_status(c);
 }
 
+namespace {
+
+// The topics in doc-major order: pieces of kReadTokens are gathered on the
+// device into the pinned slots and copied out by one thread a slot (the
+// caller's is the first; pieces are taken from a shared counter, so a thread
+// that could not be started leaves its pieces to the others).
+int read_topics(ezlda_ctx *c, uint16_t *zout) {
+    const uint32_t N = c->s.N, n_pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
+    int dev = 0;
+    EZ_TRY_HIP(c, hipGetDevice(&dev));
+    std::atomic<uint32_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    auto work = [&](size_t slot) {
+        if (slot) {  // another thread: the context's device is not its current one
+            const hipError_t e = hipSetDevice(dev);
+            if (e != hipSuccess) {
+                failed = (int)e;
+                return;
+            }
+        }
+        for (uint32_t i = next++; i < n_pieces && failed == (int)hipSuccess; i = next++) {
+            const uint32_t b = i * kReadTokens, n = std::min(kReadTokens, N - b);
+            uint16_t *buf = c->read_buf + slot * kReadTokens;
+            hipError_t e = ez::launch_topics_out(c->s, b, n, buf, c->st);
+            if (e == hipSuccess) e = hipEventRecord(c->read_ev[slot], c->st);
+            if (e == hipSuccess) e = hipEventSynchronize(c->read_ev[slot]);
+            if (e != hipSuccess) {
+                failed = (int)e;
+                return;
+            }
+            std::memcpy(zout + b, buf, (size_t)n * sizeof(uint16_t));
+        }
+    };
+    std::vector<std::thread> th;
+    th.reserve(c->read_ev.size());
+    try {
+        for (size_t k = 1; k < c->read_ev.size(); ++k) th.emplace_back(work, k);
+    } catch (const std::system_error &) {
+    }
+    if (N) work(0);
+    for (auto &x : th) x.join();
+    if (failed != (int)hipSuccess)
+        return fail(c, EZLDA_EHIP, std::string("reading the topics: ") + hipGetErrorString((hipError_t)failed.load()));
+    return EZLDA_OK;
+}
+
+}  // namespace
+
 int ezlda_get_topics(ezlda_ctx *c, uint16_t *zout) try {
     if (int r = need_loaded(c)) return r;
     if (is_chunked(c)) {  // from the chunk images (z by doc slot)
-        for (size_t i = 0; i < c->doc_tok.size(); ++i) {
-            const uint32_t p = c->tok_slot_g[c->doc_tok[i]];
-            const EzChunk &ch = c->chunks[chunk_of_slot(c, p)];
-            zout[i] = reinterpret_cast<const uint16_t *>(ch.img + 2 * (size_t)ch.N)[p - ch.slot0];
-        }
+        parallel_for((int64_t)c->doc_tok.size(), [&](int64_t b, int64_t e, int) {
+            for (int64_t i = b; i < e; ++i) {
+                const uint32_t p = c->tok_slot_g[c->doc_tok[i]];
+                const EzChunk &ch = c->chunks[chunk_of_slot(c, p)];
+                zout[i] = reinterpret_cast<const uint16_t *>(ch.img + 2 * (size_t)ch.N)[p - ch.slot0];
+            }
+        });
         return EZLDA_OK;
     }
-    std::vector<uint16_t> z(c->s.N);
-    EZ_TRY_HIP(c, hipMemcpy(z.data(), c->s.z, z.size() * sizeof(uint16_t), hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < z.size(); ++i) zout[i] = z[c->doc_tok[i]];
-    return EZLDA_OK;
+    return read_topics(c, zout);
 } catch (...) {
     return ezc::exception_status(c);
 }
