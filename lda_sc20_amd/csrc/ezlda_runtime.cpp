@@ -34,10 +34,12 @@ int host_threads() {
     return (int)n;
 }
 
+// f(begin, end, thread) over parts of [0, n); `work` is what n stands for
+// where it isn't n itself (items of many tokens).
 template <class F>
-void parallel_for(int64_t n, F f) {
+void parallel_for(int64_t n, F f, int64_t work = 0) {
     const int T = host_threads();
-    if (n < 65536 || T == 1) {
+    if (std::max(n, work) < 65536 || T == 1) {
         f(0, n, 0);
         return;
     }
@@ -280,23 +282,45 @@ int need_loaded(ezlda_ctx *c) {
 // Sampler work items (word, first token, end token).  Head words: the doc
 // order (by length) is cut into T tiles of equal head-token work, T = n_xcd * 2^a chosen so one
 // tile's DT rows fit in an XCD's L2; XCD x owns tiles [x*T/n_xcd, ...).  A
-// head word gets one item per group of tiles (finer for frequent words, so
-// an item keeps >= kMinItemTokens tokens); each XCD's items are sorted by
-// (tile, word) and the lists are interleaved so that workgroup 8j+x, which
+// head word gets one item per group of tiles (finer for frequent words, over
+// several XCDs' tiles for words of few tokens, so that an item keeps
+// >= kMinItemTokens tokens if its word has them); each XCD's items are sorted
+// by (tile, word) and the lists are interleaved so that workgroup 8j+x, which
 // round-robin dispatch sends to XCD x, is XCD x's j-th item.  Short lists
 // are padded with empty items (word 0xFFFFFFFF).  Tail words follow, one
-// item per word.  Items longer than token_segment are split.  The order of
+// item per word.  Items of more than token_segment tokens, or of more than
+// `cap` cost (cost[q] a token of doc q), are split.  The order of
 // items changes which workgroup draws a token, never the draw.
-std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uint32_t> &word_off,
-                                      const std::vector<uint32_t> &tok_rank, const std::vector<uint32_t> &soff,
-                                      const std::vector<uint32_t> &slot_wrd, int VD, int K, int n_xcd,
-                                      int *tiles_used) {
+std::vector<uint4> cut_sample_items(const ezlda_args &a, const std::vector<uint32_t> &word_off,
+                                    const std::vector<uint32_t> &tok_rank, const std::vector<uint32_t> &soff,
+                                    const std::vector<uint32_t> &slot_wrd, int VD, int K, int n_xcd,
+                                    const std::vector<uint32_t> &cost, uint64_t cap, int *tiles_used) {
     const uint32_t SEG = (uint32_t)a.token_segment;
     const int V = (int)word_off.size() - 1;
     const int D = (int)soff.size() - 1;
     std::vector<uint4> out;
+    const bool by_cost = D > 0 && (uint64_t)SEG * cost[0] > cap;  // docs come longest first
     auto push_split = [&](std::vector<uint4> &v, uint32_t w, uint32_t b, uint32_t e) {
-        for (uint32_t x = b; x < e; x += SEG) v.push_back(make_uint4(w, x, std::min(x + SEG, e), 0u));
+        if (!by_cost) {
+            for (uint32_t x = b; x < e; x += SEG) v.push_back(make_uint4(w, x, std::min(x + SEG, e), 0u));
+            return;
+        }
+        uint32_t x = b;
+        while (x < e) {
+            uint32_t y = x;
+            uint64_t c = 0;
+            // in steps of 64 tokens, each at its first (longest) document's
+            // cost, then to the end of a document, so that no run of a word's
+            // tokens in one is split
+            while (y < e && y - x < SEG && (c < cap || y - x < (uint32_t)a.block_dim)) {
+                const uint32_t m = std::min(64u, std::min(e - y, SEG - (y - x)));
+                c += (uint64_t)m * cost[tok_rank[y]];
+                y += m;
+            }
+            while (y < e && y - x < SEG && tok_rank[y] == tok_rank[y - 1]) ++y;
+            v.push_back(make_uint4(w, x, y, 0u));
+            x = y;
+        }
     };
     int T = 0;
     uint64_t head_tokens = word_off[VD];
@@ -337,11 +361,14 @@ std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uin
             if (n == 0) continue;
             int g = per_xcd;  // tiles per item: the coarsest that still splits per XCD
             while (g > 1 && (uint64_t)n * (uint64_t)g / (uint64_t)T >= 2ull * kMinItemTokens) g /= 2;
+            while (g < T && (uint64_t)n * (uint64_t)g / (uint64_t)T < kMinItemTokens) g = std::min(T, 2 * g);
             for (int t = 0; t < T; t += g) {
                 const uint32_t d0 = tile_doc[t], d1 = tile_doc[std::min(T, t + g)];
                 const uint32_t lo = (uint32_t)(std::lower_bound(tok_rank.begin() + b, tok_rank.begin() + e, d0) - tok_rank.begin());
                 const uint32_t hi = (uint32_t)(std::lower_bound(tok_rank.begin() + b, tok_rank.begin() + e, d1) - tok_rank.begin());
-                if (hi > lo) lists[t / per_xcd].push_back({(uint32_t)t, (uint32_t)w, lo, hi});
+                // an item over several XCDs' tiles belongs to none of them: dealt by word
+                const int x = g > per_xcd ? (t / per_xcd + w) % n_xcd : t / per_xcd;
+                if (hi > lo) lists[x].push_back({(uint32_t)t, (uint32_t)w, lo, hi});
             }
         }
         std::vector<std::vector<uint4>> split(n_xcd);
@@ -359,6 +386,41 @@ std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uin
     }
     for (int w = VD; w < V; ++w) push_split(out, (uint32_t)w, word_off[w], word_off[w + 1]);
     if (tiles_used) *tiles_used = T;
+    return out;
+}
+
+// The items of a layout.  A persistent sampler ends when its longest item
+// does, and a word's items come longest documents first, so an item's cost
+// (in row entries: its tokens' rows, at most min(n_d, K) entries each, and
+// kRunCost for the latencies of a run's loads) is capped at half of one
+// workgroup's share of the whole sweep; but an item is worth staging phi for
+// only from some size on.  Measured, sampler ms a sweep with the items of at
+// most token_segment tokens cut per XCD / with these: 8.9M tokens of heavy-
+// tailed documents at K = 2048 6.91 / 2.80, 9M tokens of short documents at
+// K = 4096 (20,011 dense words) 2.35 / 0.90, 1M tokens at K = 64 0.214 /
+// 0.169, 1.7M tokens at K = 300 0.360 / 0.207, 49.5M tokens at K = 1024 (where
+// the cap does not bind) 3.01 / 3.01.  Caps of a quarter or an eighth of the
+// share: K = 300 0.231 / 0.254, heavy-tailed 2.82 / 3.21.
+std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uint32_t> &word_off,
+                                      const std::vector<uint32_t> &tok_rank, const std::vector<uint32_t> &soff,
+                                      const std::vector<uint32_t> &slot_wrd, int VD, int K, int n_xcd,
+                                      int *tiles_used) {
+    const uint32_t kRunCost = 96;
+    const int D = (int)soff.size() - 1;
+    const uint64_t n_wg = (uint64_t)(a.grid_dim > 0 ? a.grid_dim : (a.block_dim == 64 ? 16 : 8) * device_cus());
+    std::vector<uint32_t> cost(D);
+    uint64_t total = 0;
+    for (int q = 0; q < D; ++q) {
+        const uint32_t n = soff[q + 1] - soff[q];
+        cost[q] = kRunCost + std::min<uint32_t>(n, (uint32_t)K);
+        total += (uint64_t)n * cost[q];
+    }
+    const uint64_t least = (uint64_t)a.block_dim * (256u + (uint64_t)K / 8u);
+    std::vector<uint4> out = cut_sample_items(a, word_off, tok_rank, soff, slot_wrd, VD, K, n_xcd, cost,
+                                              std::max(least, total / (2 * n_wg)), tiles_used);
+    // the cap never costs a corpus the allocation-free log-likelihood
+    if (out.size() > ez::kLLScratchItems)
+        out = cut_sample_items(a, word_off, tok_rank, soff, slot_wrd, VD, K, n_xcd, cost, UINT64_MAX, tiles_used);
     return out;
 }
 
@@ -389,7 +451,7 @@ std::vector<uint4> build_runs(std::vector<uint4> &items, const std::vector<uint3
             if (items[i].x != 0xFFFFFFFFu) for_runs(items[i], [&](uint32_t, uint32_t) { ++k; });
             cnt[i + 1] = k;
         }
-    });
+    }, (int64_t)tok_doc.size());
     for (int64_t i = 0; i < n; ++i) cnt[i + 1] += cnt[i];
     std::vector<uint4> runs(cnt[n]);
     parallel_for(n, [&](int64_t b, int64_t e, int) {
@@ -402,7 +464,7 @@ std::vector<uint4> build_runs(std::vector<uint4> &items, const std::vector<uint3
                              [](const uint4 &x, const uint4 &y) { return x.w > y.w; });
             it = make_uint4(it.x, (uint32_t)cnt[i], (uint32_t)cnt[i + 1], 0u);
         }
-    });
+    }, (int64_t)tok_doc.size());
     return runs;
 }
 
