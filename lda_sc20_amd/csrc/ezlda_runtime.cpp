@@ -310,14 +310,19 @@ std::vector<uint4> cut_sample_items(const ezlda_args &a, const std::vector<uint3
             uint32_t y = x;
             uint64_t c = 0;
             // in steps of 64 tokens, each at its first (longest) document's
-            // cost, then to the end of a document, so that no run of a word's
-            // tokens in one is split
+            // cost, then to the end of a run (run_cap tokens from a document's
+            // first): the runs are those of the whole word
             while (y < e && y - x < SEG && (c < cap || y - x < (uint32_t)a.block_dim)) {
                 const uint32_t m = std::min(64u, std::min(e - y, SEG - (y - x)));
                 c += (uint64_t)m * cost[tok_rank[y]];
                 y += m;
             }
-            while (y < e && y - x < SEG && tok_rank[y] == tok_rank[y - 1]) ++y;
+            if (y < e && y - x < SEG && tok_rank[y] == tok_rank[y - 1]) {
+                const uint32_t q = tok_rank[y];
+                const uint32_t first = (uint32_t)(std::lower_bound(tok_rank.begin() + b, tok_rank.begin() + y, q) -
+                                                  tok_rank.begin());
+                while (y < e && y - x < SEG && tok_rank[y] == q && (y - first) % (uint32_t)a.run_cap) ++y;
+            }
             v.push_back(make_uint4(w, x, y, 0u));
             x = y;
         }
