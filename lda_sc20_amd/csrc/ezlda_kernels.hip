@@ -812,14 +812,24 @@ __device__ __forceinline__ RowBlock load_block(const uint4 *__restrict__ p) {
     return r;
 }
 
+// The sampler's phi table in LDS, for compact rows, holds phi * 2^24: an
+// entry's count, moved to the low bits of its half-word, is a subnormal f16 of
+// value count * 2^-24, so one v_fma_mix_f32 takes it as it is and the products
+// (hence the rounded sums) are those of count * phi.  Both scalings are exact.
+static constexpr float kPhiUp = 16777216.0f, kPhiDown = 5.9604644775390625e-08f;
+
 // The two compact entries of a dword (low half first) decoded together: both
 // counts by one packed 16-bit shift, both topics by one mask (tm2 = the topic
 // mask in each half), each phi address (topic * 4) by one shift that reads
 // its half of the word (SDWA word select; the compiler forms it for the high
-// half by itself, the low half is written out).
+// half by itself, the low half is written out).  With the sum that is three
+// VALU operations an entry (four with a conversion of each count); the scan
+// keeps the VALU busy 66% of the cycles on the 49.5M-token corpus at K = 1024
+// and 85% on rows of up to 2,700 entries (2.96 -> 2.92 and 2.81 -> 2.63 ms).
 typedef unsigned short ez_us2 __attribute__((ext_vector_type(2)));
+typedef _Float16 ez_h2 __attribute__((ext_vector_type(2)));
 struct C16x2 {
-    float c0, c1;
+    _Float16 c0, c1;  // count * 2^-24
     uint32_t a0, a1;
 };
 __device__ __forceinline__ uint32_t lo16_times4(uint32_t t) {
@@ -831,9 +841,12 @@ __device__ __forceinline__ uint32_t lo16_times4(uint32_t t) {
 }
 __device__ __forceinline__ C16x2 c16_x2(uint32_t w, uint32_t tb, uint32_t tm2) {
     const ez_us2 c = __builtin_bit_cast(ez_us2, w) >> (ez_us2)((unsigned short)tb);
+    const ez_h2 h = __builtin_bit_cast(ez_h2, c);
     const uint32_t t = w & tm2;
-    return C16x2{(float)c.x, (float)c.y, lo16_times4(t), (t >> 16) << 2};
+    return C16x2{h.x, h.y, lo16_times4(t), (t >> 16) << 2};
 }
+// s + count * phi in one rounding (v_fma_mix_f32)
+__device__ __forceinline__ float fma_count(_Float16 c, float phi, float s) { return __builtin_fmaf((float)c, phi, s); }
 __device__ __forceinline__ float phi_a(uint32_t a) { return *(lds_cfloat *)a; }
 
 // The entries of one 16-byte load, in order.
@@ -845,8 +858,8 @@ __device__ __forceinline__ float sum_u4(const uint4 &e, float s, uint32_t tb) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const C16x2 d = c16_x2(w[q], tb, tm2);
-            s = __builtin_fmaf(d.c0, phi_a(d.a0), s);
-            s = __builtin_fmaf(d.c1, phi_a(d.a1), s);
+            s = fma_count(d.c0, phi_a(d.a0), s);
+            s = fma_count(d.c1, phi_a(d.a1), s);
         }
     } else {
         s = __builtin_fmaf(dt_count(e.x), phi_at0(e.x), s);
@@ -869,15 +882,12 @@ __device__ __forceinline__ float sum_block(const RowBlock &r, float s, uint32_t 
     return s;
 }
 
-// S-bucket search over n consecutive 16-byte loads of a row (issued
-// together) from running sum `run`: the first entry whose running sum
-// exceeds t2 (running sums never decrease).
+// S-bucket search over n consecutive 16-byte pieces of a row from running
+// sum `run`: the first entry whose running sum exceeds t2 (running sums never
+// decrease).
 template <bool COMPACT, int N>
-__device__ __forceinline__ void search_u4(const uint4 *__restrict__ p, float &run, float t2, uint32_t tb,
-                                          uint32_t &newz, bool &found) {
-    uint4 blk[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) blk[i] = p[i];
+__device__ __forceinline__ void search_u4(const uint4 (&blk)[N], float &run, float t2, uint32_t tb, uint32_t &newz,
+                                          bool &found) {
 #pragma unroll
     for (int gi = 0; gi < N; ++gi) {
         const uint4 e = blk[gi];
@@ -887,8 +897,8 @@ __device__ __forceinline__ void search_u4(const uint4 *__restrict__ p, float &ru
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const C16x2 d = c16_x2(w[q], tb, tm2);
-                const float ra = __builtin_fmaf(d.c0, phi_a(d.a0), run);
-                const float rb = __builtin_fmaf(d.c1, phi_a(d.a1), ra);
+                const float ra = fma_count(d.c0, phi_a(d.a0), run);
+                const float rb = fma_count(d.c1, phi_a(d.a1), ra);
                 if (!found && ra > t2) {
                     newz = d.a0 >> 2;
                     found = true;
@@ -956,6 +966,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
     const float alpha = A.alpha, beta = A.beta;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
     constexpr bool qtab = QTAB;  // K <= EZ_Q_TABLE_MAX_K
+    constexpr float up = COMPACT ? kPhiUp : 1.0f, down = COMPACT ? kPhiDown : 1.0f;
     float *phi = smf;                         // NS*64
     float *qs = phi + NS * 64;                // NS*64 when qtab: running sums inside each slab
     float *qt = qs + (qtab ? NS * 64 : 0);    // NS: slab totals
@@ -969,23 +980,23 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
 
     if (w < A.VD) {
         const int32_t *row = A.wt_head + (size_t)w * K;
-        for (int k = tid; k < NS * 64; k += blockDim.x) phi[k] = k < K ? ((float)row[k] + beta) * A.inv[k] : 0.0f;
+        for (int k = tid; k < NS * 64; k += blockDim.x) phi[k] = k < K ? ((float)row[k] + beta) * A.inv[k] * up : 0.0f;
     } else {
-        for (int k = tid; k < NS * 64; k += blockDim.x) phi[k] = k < K ? beta * A.inv[k] : 0.0f;
+        for (int k = tid; k < NS * 64; k += blockDim.x) phi[k] = k < K ? beta * A.inv[k] * up : 0.0f;
         __syncthreads();
         const int tw = w - A.VD;
         const uint32_t b = A.tail_off[tw], n = A.tail_nnz[tw];
         for (uint32_t i = tid; i < n; i += blockDim.x) {
             const uint32_t e = A.wt_tail[b + i];
             const uint32_t k = e & 0xFFFFu;
-            phi[k] = ((float)(e >> 16) + beta) * A.inv[k];
+            phi[k] = ((float)(e >> 16) + beta) * A.inv[k] * up;
         }
     }
     __syncthreads();
     if (tid == 0) {
-        f123[0] = phi[tp.x];
-        f123[1] = tp.y != kNone ? phi[tp.y] : 0.0f;
-        f123[2] = tp.z != kNone ? phi[tp.z] : 0.0f;
+        f123[0] = phi[tp.x] * down;
+        f123[1] = tp.y != kNone ? phi[tp.y] * down : 0.0f;
+        f123[2] = tp.z != kNone ? phi[tp.z] * down : 0.0f;
         phi[tp.x] = 0.0f;
     }
     __syncthreads();
@@ -1002,13 +1013,13 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
         float run = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            run = run + alpha * v[i].x;
+            run = run + alpha * (v[i].x * down);
             v[i].x = run;
-            run = run + alpha * v[i].y;
+            run = run + alpha * (v[i].y * down);
             v[i].y = run;
-            run = run + alpha * v[i].z;
+            run = run + alpha * (v[i].z * down);
             v[i].z = run;
-            run = run + alpha * v[i].w;
+            run = run + alpha * (v[i].w * down);
             v[i].w = run;
         }
         if (qtab) {
@@ -1144,20 +1155,23 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
             if (j >= (uint32_t)UK) u = ez_u24(ez_philox_x0(A.seed, t + sg.w, sweep, EZ_TAG_SAMPLE));
             const float target = u * total;
             uint32_t newz = k1;
-            if (target < P1) {
-                newz = k1;
-            } else if (target < Aa) {
-                const float t2 = target - P1;
-                int bs = -1;
+            // P1 below, S up to Aa, Q above.  The S bucket's loads are issued
+            // before the Q lanes search their running sums in LDS, which hides
+            // part of their latency.
+            const bool in_s = target >= P1 && target < Aa;
+            const float t2s = target - P1;
+            int bs = -1;
+            float run = 0.0f;
+            constexpr int NH = kHalfCp && COMPACT ? kBlkU4 / 2 : kBlkU4;  // loads of one search
+            uint4 blk[NH];
+            if (in_s) {
 #pragma unroll
                 for (int b = kCP - 1; b >= 0; --b)
-                    if (cp[b] > t2) bs = b;
-                float run = 0.0f;
-                bool found = false;
+                    if (cp[b] > t2s) bs = b;
                 if (bs >= 0) {
                     // the checkpointed block that holds the target: from the
                     // running sum before it, or with kHalfCp from the one in
-                    // its middle, at most half the block's loads
+                    // its middle, half the block's loads
                     float mid = ch[0];
 #pragma unroll
                     for (int b = 0; b < kCP - 1; ++b)
@@ -1165,35 +1179,17 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                             run = cp[b];
                             mid = ch[b + 1];
                         }
-                    const uint4 *bp = rp + kBlkU4 * (uint32_t)bs;
-                    if (kHalfCp && COMPACT) {
-                        if (mid > t2) {
-                            search_u4<COMPACT, kBlkU4 / 2>(bp, run, t2, tb, newz, found);
-                        } else {
-                            run = mid;
-                            search_u4<COMPACT, kBlkU4 / 2>(bp + kBlkU4 / 2, run, t2, tb, newz, found);
-                        }
-                    } else {
-                        search_u4<COMPACT, kBlkU4>(bp, run, t2, tb, newz, found);
+                    uint32_t at = kBlkU4 * (uint32_t)bs;
+                    if (NH < kBlkU4 && !(mid > t2s)) {
+                        run = mid;
+                        at += NH;
                     }
-                } else if (nb > (uint32_t)kCP) {
-                    // past the checkpoints: the remaining blocks in order
-                    run = cp[kCP - 1];
-                    for (uint32_t gb = kCP; gb < nb && !found; ++gb)
-                        search_u4<COMPACT, kBlkU4>(rp + kBlkU4 * gb, run, t2, tb, newz, found);
+#pragma unroll
+                    for (int i = 0; i < NH; ++i) blk[i] = rp[at + i];
                 }
-                if (!found) {  // rounding left every running sum at or below t2
-                    if (COMPACT) {
-                        const uint16_t *rr = reinterpret_cast<const uint16_t *>(A.dt) + di.x;
-                        for (uint32_t i = 0; i < nnz; ++i)
-                            if (c16_count(rr[i], tb) > 0.0f && phi_c16(rr[i], tb) > 0.0f) newz = c16_topic(rr[i], tb);
-                    } else {
-                        const uint32_t *rr = A.dt + di.x;
-                        for (uint32_t i = 0; i < nnz; ++i)
-                            if (dt_count(rr[i]) > 0.0f && phi_at0(rr[i]) > 0.0f) newz = dt_topic(rr[i]);
-                    }
-                }
-            } else {
+            }
+            asm volatile("" ::: "memory");  // the loads stay above the Q search
+            if (!(target < Aa)) {
                 const float t2 = target - Aa;
                 int lo = 0, hi = NS;  // first slab whose running sum exceeds t2
                 while (lo < hi) {
@@ -1233,7 +1229,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
 #pragma unroll
                             for (int c = 0; c < 4; ++c) {
                                 const int k = k0 + 4 * (i4 + u) + c;
-                                run = run + alpha * x[c];
+                                run = run + alpha * (x[c] * down);
                                 if (lo == ke && k < ke && run > t3) lo = k;
                             }
                         }
@@ -1242,10 +1238,32 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                         newz = (uint32_t)lo;
                     } else {
                         for (int k = ke - 1; k >= k0; --k)
-                            if (alpha * phi[k] > 0.0f) {
+                            if (alpha * (phi[k] * down) > 0.0f) {
                                 newz = (uint32_t)k;
                                 break;
                             }
+                    }
+                }
+            }
+            if (in_s) {
+                bool found = false;
+                if (bs >= 0) {
+                    search_u4<COMPACT, NH>(blk, run, t2s, tb, newz, found);
+                } else if (nb > (uint32_t)kCP) {
+                    // past the checkpoints: the remaining blocks in order
+                    run = cp[kCP - 1];
+                    for (uint32_t gb = kCP; gb < nb && !found; ++gb)
+                        search_u4<COMPACT, kBlkU4>(load_block(rp + kBlkU4 * gb).e, run, t2s, tb, newz, found);
+                }
+                if (!found) {  // rounding left every running sum at or below t2
+                    if (COMPACT) {
+                        const uint16_t *rr = reinterpret_cast<const uint16_t *>(A.dt) + di.x;
+                        for (uint32_t i = 0; i < nnz; ++i)
+                            if (c16_count(rr[i], tb) > 0.0f && phi_c16(rr[i], tb) > 0.0f) newz = c16_topic(rr[i], tb);
+                    } else {
+                        const uint32_t *rr = A.dt + di.x;
+                        for (uint32_t i = 0; i < nnz; ++i)
+                            if (dt_count(rr[i]) > 0.0f && phi_at0(rr[i]) > 0.0f) newz = dt_topic(rr[i]);
                     }
                 }
             }
@@ -1270,20 +1288,21 @@ __global__ void __launch_bounds__(1024) k_sample(const SampleArgs A) {
     uint32_t &s_item = *reinterpret_cast<uint32_t *>(f123 + 3);
     const uint32_t sweep = A.counters[0];
     uint32_t n_full = 0, n_scanned = 0;
-    if (A.n_queues == 0) {
-        sample_item<SHORTCUT, COMPACT, QTAB>(A, blockIdx.x, smf, f123, sweep, n_full, n_scanned);
-    } else {
-        const uint32_t nq = A.n_queues, x0 = blockIdx.x % nq;
-        for (uint32_t h = 0; h < nq; ++h) {
-            const uint32_t q = (x0 + h) % nq;
-            while (true) {
+    const bool own = A.n_queues == 0;  // one item a workgroup
+    const uint32_t nq = own ? 1u : A.n_queues, x0 = blockIdx.x % nq;
+    for (uint32_t h = 0; h < nq; ++h) {
+        const uint32_t q = (x0 + h) % nq;
+        while (true) {
+            uint64_t item = blockIdx.x;
+            if (!own) {
                 __syncthreads();  // the previous item is done with s_item and LDS
                 if (threadIdx.x == 0) s_item = atomicAdd(&A.queue[q * kQueueStride], 1u);
                 __syncthreads();
-                const uint64_t item = (uint64_t)q + (uint64_t)s_item * nq;
-                if (item >= A.n_items) break;
-                sample_item<SHORTCUT, COMPACT, QTAB>(A, (uint32_t)item, smf, f123, sweep, n_full, n_scanned);
+                item = (uint64_t)q + (uint64_t)s_item * nq;
             }
+            if (item >= A.n_items) break;
+            sample_item<SHORTCUT, COMPACT, QTAB>(A, (uint32_t)item, smf, f123, sweep, n_full, n_scanned);
+            if (own) break;
         }
     }
     // per-wavefront totals of the counters

@@ -32,8 +32,9 @@ EZ_HD uint32_t ez_mulhi32(uint32_t a, uint32_t b) {
 EZ_HD ez_u4 ez_philox4x32_10(ez_u4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
-        const uint32_t lo0 = 0xD2511F53u * c.x, hi0 = ez_mulhi32(0xD2511F53u, c.x);
-        const uint32_t lo1 = 0xCD9E8D57u * c.z, hi1 = ez_mulhi32(0xCD9E8D57u, c.z);
+        const uint64_t p0 = (uint64_t)0xD2511F53u * c.x, p1 = (uint64_t)0xCD9E8D57u * c.z;
+        const uint32_t lo0 = (uint32_t)p0, hi0 = (uint32_t)(p0 >> 32);
+        const uint32_t lo1 = (uint32_t)p1, hi1 = (uint32_t)(p1 >> 32);
         ez_u4 n;
         n.x = hi1 ^ c.y ^ k0;
         n.y = lo1;
