@@ -781,12 +781,22 @@ __global__ void __launch_bounds__(256) k_dt_sort(int q0, int q1, int VD, uint32_
 }
 
 // ------------------------------------------------------------- sampler
-// Checkpoints of the S running sum kept per lane (one per block of kBlkU4
-// 16-byte loads, i.e. 4*kBlkU4 DT entries, and with kHalfCp, in 16-bit rows,
-// one more in the middle of each block, so the S-bucket search re-reads half a
-// block: 6.09 -> 5.98 ms a sweep on the 99M-token corpus at K = 1024; with
-// 32-bit rows it cost 1.5 ms of 63.6 at K = 10000, so they search whole blocks).
-static constexpr int kCP = EZ_SAMPLE_CP;
+// Checkpoints of the S running sum kept per lane: one per block of kBlkU4
+// 16-byte loads (4 * kBlkU4 entries of 32 bits, 8 * kBlkU4 of 16) for the
+// first CP blocks, and with kHalfCp, in 16-bit rows, one more in the middle of
+// each, so the S-bucket search re-reads half a block (6.09 -> 5.98 ms a sweep
+// on the 99M-token corpus at K = 1024; with 32-bit rows it cost 1.5 ms of 63.6
+// at K = 10000, so they search whole blocks).  A wavefront with a longer row
+// keeps CF more, m blocks apart (m the same for its lanes), so the search
+// past the first CP reads at most m blocks again: walking them from the
+// CP-th took most of the sampler on heavy-tailed documents (8.9M tokens of
+// up to 20,000 a document at K = 2048: 2.63 -> 1.67 ms a sweep with 8 + 8,
+// 1.72 with 9 + 6, 1.78 with 12 + 4; 49.5M tokens at K = 1024 2.92 -> 2.90
+// with 12 + 4, 2.92 with 9 + 6).  The counts are what fits 128 registers.
+template <bool COMPACT, bool QTAB>
+struct Checkpoints {
+    static constexpr int CP = !QTAB && COMPACT ? 8 : EZ_SAMPLE_CP, CF = !QTAB && COMPACT ? 8 : 4;
+};
 static constexpr int kBlkU4 = EZ_SAMPLE_BLK;
 #ifndef EZ_SAMPLE_HALF_CP
 #define EZ_SAMPLE_HALF_CP 1
@@ -966,6 +976,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
     const float alpha = A.alpha, beta = A.beta;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
     constexpr bool qtab = QTAB;  // K <= EZ_Q_TABLE_MAX_K
+    constexpr int CP = Checkpoints<COMPACT, QTAB>::CP, CF = Checkpoints<COMPACT, QTAB>::CF;
     constexpr float up = COMPACT ? kPhiUp : 1.0f, down = COMPACT ? kPhiDown : 1.0f;
     float *phi = smf;                         // NS*64
     float *qs = phi + NS * 64;                // NS*64 when qtab: running sums inside each slab
@@ -1119,15 +1130,15 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
         n_full += (uint32_t)__popc(need);
         n_scanned += nnz;
         // S: one FMA per entry, left to right; cp[b] = running sum at the
-        // end of block b (the first kCP blocks), so the S-bucket search
+        // end of block b (the first CP blocks), so the S-bucket search
         // re-reads one block instead of the row up to the target
         // Block b + 1 is loaded before block b is summed (only by lanes
         // whose row has it, so a wavefront stops loading at its longest row).
-        float cp[kCP], ch[kCP];  // running sum at the end / the middle of block b
+        float cp[CP], ch[CP];  // running sum at the end / the middle of block b
         float S = 0.0f;
         RowBlock cur = load_block(rp);
 #pragma unroll
-        for (int b = 0; b < kCP; ++b) {
+        for (int b = 0; b < CP; ++b) {
             RowBlock nxt;
             if ((uint32_t)b + 1u < nb) nxt = load_block(rp + kBlkU4 * (b + 1));
             ch[b] = S;
@@ -1135,12 +1146,23 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
             cp[b] = S;
             cur = nxt;
         }
-        for (uint32_t b = kCP; b < nb; ++b) {
-            RowBlock nxt;
-            if (b + 1u < nb) nxt = load_block(rp + kBlkU4 * (b + 1u));
-            float unused;
-            S = sum_block<COMPACT>(cur, S, tb, unused);
-            cur = nxt;
+        // past them, CF more checkpoints m blocks apart
+        float cf[CF];
+#pragma unroll
+        for (int i = 0; i < CF; ++i) cf[i] = 0.0f;
+        uint32_t m = 0;
+        while (__ballot(nb > (uint32_t)(CP + CF * m))) ++m;
+        for (uint32_t i = 0, b = CP; m != 0 && i < (uint32_t)CF; ++i) {
+            for (const uint32_t e = b + m; b < e; ++b) {
+                RowBlock nxt;
+                if (b + 1u < nb) nxt = load_block(rp + kBlkU4 * (b + 1u));
+                float unused;
+                if (b < nb) S = sum_block<COMPACT>(cur, S, tb, unused);
+                cur = nxt;
+            }
+#pragma unroll
+            for (int q = 0; q < CF; ++q)
+                if (i == (uint32_t)q) cf[q] = S;
         }
         const float Aa = P1 + S;
         const float total = Aa + Q;
@@ -1166,7 +1188,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
             uint4 blk[NH];
             if (in_s) {
 #pragma unroll
-                for (int b = kCP - 1; b >= 0; --b)
+                for (int b = CP - 1; b >= 0; --b)
                     if (cp[b] > t2s) bs = b;
                 if (bs >= 0) {
                     // the checkpointed block that holds the target: from the
@@ -1174,7 +1196,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                     // its middle, half the block's loads
                     float mid = ch[0];
 #pragma unroll
-                    for (int b = 0; b < kCP - 1; ++b)
+                    for (int b = 0; b < CP - 1; ++b)
                         if (b + 1 == bs) {
                             run = cp[b];
                             mid = ch[b + 1];
@@ -1249,10 +1271,18 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                 bool found = false;
                 if (bs >= 0) {
                     search_u4<COMPACT, NH>(blk, run, t2s, tb, newz, found);
-                } else if (nb > (uint32_t)kCP) {
-                    // past the checkpoints: the remaining blocks in order
-                    run = cp[kCP - 1];
-                    for (uint32_t gb = kCP; gb < nb && !found; ++gb)
+                } else if (nb > (uint32_t)CP) {
+                    // past them: the blocks of the far checkpoint that holds
+                    // the target, in order
+                    uint32_t g0 = CP;
+                    run = cp[CP - 1];
+#pragma unroll
+                    for (int i = 0; i < CF - 1; ++i)
+                        if (!(cf[i] > t2s)) {
+                            g0 = CP + m * (uint32_t)(i + 1);
+                            run = cf[i];
+                        }
+                    for (uint32_t gb = g0; gb < nb && !found; ++gb)
                         search_u4<COMPACT, kBlkU4>(load_block(rp + kBlkU4 * gb).e, run, t2s, tb, newz, found);
                 }
                 if (!found) {  // rounding left every running sum at or below t2
