@@ -319,51 +319,80 @@ __device__ __forceinline__ void top3_insert(Top3 &t, float v, uint32_t k) {
     }
 }
 
-// Topics by beta * inv[k] (the value of a topic a word has no count of),
-// largest first, ties to the lower topic.  A workgroup of four wavefronts
-// ranks 64 topics: lane i's topic is compared with a quarter of all topics
-// by each wavefront, and the four counts are added in LDS.
-__global__ void __launch_bounds__(256) k_zero_order(const float *__restrict__ inv, int K, float beta,
-                                                    uint32_t *__restrict__ zero_order) {
-    extern __shared__ float sv[];  // K values, then 64 ranks
-    uint32_t *rank = reinterpret_cast<uint32_t *>(sv + K);
-    for (int k = threadIdx.x; k < K; k += blockDim.x) sv[k] = ((float)0u + beta) * inv[k];
+// inv, and the topics by beta * inv[k] (the value of a topic a word has no
+// count of), largest first, ties to the lower topic.  A workgroup of 16
+// wavefronts ranks 64 topics: it computes every topic's value into LDS, lane
+// i's topic is compared with a sixteenth of them by each wavefront (four
+// values a read, all lanes the same address), and the counts are added in
+// LDS.  Topics before the workgroup's own win ties, later ones lose them, so
+// only its own 64 need the tie test.  Bound by its K^2 compares: 20 -> 5.7 us at
+// K = 1024, 176 -> 19 us at K = 10000 (four wavefronts, a scalar read and the
+// tie test for each, inv from a launch before it).
+__global__ void __launch_bounds__(1024) k_inv_order(const int32_t *__restrict__ nk, int K, float vbeta, float beta,
+                                                    float *__restrict__ inv, uint32_t *__restrict__ zero_order) {
+    extern __shared__ float sv[];  // K values padded to whole groups of 4, then 64 ranks
+    const int KG = (K + 3) >> 2;
+    uint32_t *rank = reinterpret_cast<uint32_t *>(sv + 4 * KG);
+    const int own = (int)blockIdx.x * 64;
+    for (int k = threadIdx.x; k < 4 * KG; k += blockDim.x) {
+        float v = -1.0f;  // padding: below every value
+        if (k < K) {
+            const float iv = 1.0f / ((float)nk[k] + vbeta);
+            v = beta * iv;
+            if (k >= own && k < own + 64) inv[k] = iv;
+        }
+        sv[k] = v;
+    }
     if (threadIdx.x < 64) rank[threadIdx.x] = 0;
     __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int k = blockIdx.x * 64 + lane;
-    const int q = (K + 3) >> 2, j0 = wv * q, j1 = min(K, j0 + q);
-    if (k < K) {
-        const float v = sv[k];
-        uint32_t r = 0;
-        for (int j = j0; j < j1; ++j) r += better(sv[j], (uint32_t)j, v, (uint32_t)k) ? 1u : 0u;
-        atomicAdd(&rank[lane], r);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+    const int k = own + lane;
+    const float v = k < K ? sv[k] : 0.0f;
+    const float4 *s4 = reinterpret_cast<const float4 *>(sv);
+    const int q = (KG + nwv - 1) / nwv, g0 = wv * q, g1 = min(KG, g0 + q);
+    const int o0 = own >> 2, o1 = o0 + 16;  // the workgroup's own groups
+    uint32_t r = 0;
+#pragma unroll 4
+    for (int g = g0; g < min(g1, o0); ++g) {
+        const float4 x = s4[g];
+        r += (x.x >= v) + (x.y >= v) + (x.z >= v) + (x.w >= v);
     }
+    for (int g = max(g0, o0); g < min(g1, o1); ++g) {
+        const float4 x = s4[g];
+        const float y[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) r += better(y[c], (uint32_t)(4 * g + c), v, (uint32_t)k) ? 1u : 0u;
+    }
+#pragma unroll 4
+    for (int g = max(g0, o1); g < g1; ++g) {
+        const float4 x = s4[g];
+        r += (x.x > v) + (x.y > v) + (x.z > v) + (x.w > v);
+    }
+    if (k < K) atomicAdd(&rank[lane], r);
     __syncthreads();
     if (wv == 0 && k < K) zero_order[rank[lane]] = (uint32_t)k;
 }
 
 // Per word the three largest phi_wk, ties to the lower topic
 // (MaxTopicDense/Sparse_Update_Kernel, utility.cu:305-678, :679-1062).  One
-// wavefront per word; a tail word's counts are scattered into a 16-bit LDS
-// row first.  Per-lane lists are merged with a butterfly; the order is total,
-// so the merge order does not matter.
-// Words [w0, w1) of one launch.  Only tail words use the LDS count table:
-// a launch with w0 < VD and no LDS (w1 <= VD) runs head words at full
-// occupancy; a launch that reaches tail words has the table.
-__global__ void k_word_top(int w0, int w1, int VD, int K, float beta, const int32_t *__restrict__ wt_head,
+// wavefront per word; a tail word's topics are marked in a bitmap in LDS (K
+// bits, so it leaves the occupancy alone at every K: with a table of 16-bit
+// counts, 20 KB a wavefront at K = 10000, 30,000 words took 104 us, in two
+// launches, 59 with the bitmap).  The order is total, so the order in which
+// the lanes' lists are merged does not matter.
+__global__ void k_word_top(int V, int VD, int K, float beta, const int32_t *__restrict__ wt_head,
                            const uint32_t *__restrict__ tail_off, const uint32_t *__restrict__ wt_tail,
                            const uint32_t *__restrict__ tail_nnz, const float *__restrict__ inv,
                            const uint32_t *__restrict__ zero_order, ushort4 *__restrict__ wtop) {
     extern __shared__ uint32_t sh[];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-    const int KH = (K + 1) >> 1;
-    uint32_t *h = sh + wv * KH;
-    if (w1 > VD) {
-        for (int k = lane; k < KH; k += 64) h[k] = 0;
+    const int NW = (K + 31) >> 5;
+    uint32_t *bm = sh + wv * NW;
+    if (V > VD) {
+        for (int k = lane; k < NW; k += 64) bm[k] = 0;
         wave_lds_sync();
     }
-    for (int w = w0 + blockIdx.x * nwv + wv; w < w1; w += gridDim.x * nwv) {
+    for (int w = blockIdx.x * nwv + wv; w < V; w += gridDim.x * nwv) {
         Top3 t{-1.f, -1.f, -1.f, kNone, kNone, kNone};
         if (w < VD) {
             // four loads of the row and of inv in flight per lane
@@ -390,7 +419,7 @@ __global__ void k_word_top(int w0, int w1, int VD, int K, float beta, const int3
             for (uint32_t i = lane; i < n; i += 64) {
                 const uint32_t e = wt_tail[b + i];
                 const uint32_t k = e & 0xFFFFu;
-                atomicAdd(&h[k >> 1], (e >> 16) << ((k & 1u) << 4));
+                atomicOr(&bm[k >> 5], 1u << (k & 31u));
                 top3_insert(t, ((float)(e >> 16) + beta) * inv[k], k);
             }
             wave_lds_sync();
@@ -398,14 +427,14 @@ __global__ void k_word_top(int w0, int w1, int VD, int K, float beta, const int3
             for (int j0 = 0; j0 < K && got < 3u; j0 += 64) {
                 const int j = j0 + lane;
                 const uint32_t k = j < K ? zero_order[j] : 0u;
-                const bool free_k = j < K && h16_get(h, k) == 0u;
+                const bool free_k = j < K && !((bm[k >> 5] >> (k & 31u)) & 1u);
                 const uint64_t m = __ballot(free_k);
                 if (free_k && got + (uint32_t)__popcll(m & lanemask_lt(lane)) < 3u)
                     top3_insert(t, ((float)0u + beta) * inv[k], k);
                 got += (uint32_t)__popcll(m);
             }
             wave_lds_sync();
-            for (uint32_t i = lane; i < n; i += 64) h[(wt_tail[b + i] & 0xFFFFu) >> 1] = 0;
+            for (uint32_t i = lane; i < n; i += 64) bm[(wt_tail[b + i] & 0xFFFFu) >> 5] = 0;
             wave_lds_sync();
         }
         // the wavefront's best three: three max-reductions of the lanes'
@@ -2234,24 +2263,16 @@ hipError_t launch_topic_hist(const DevState &s, hipStream_t st) {
 }
 
 hipError_t launch_topk(const DevState &s, hipStream_t st) {
-    hipLaunchKernelGGL(k_inv, dim3(grid_for(s.K, 256, 1 << 16)), dim3(256), 0, st, s.nk, s.K, s.vbeta, s.inv);
     if (s.V > s.VD)
-        hipLaunchKernelGGL(k_zero_order, dim3(grid_for(s.K, 64, 1 << 16)), dim3(256),
-                           (size_t)s.K * sizeof(float) + 64 * sizeof(uint32_t), st, s.inv, s.K, s.beta, s.zero_order);
-    // head words need no LDS: where the tail words' count tables limit the
-    // wavefronts per CU, they get a launch of their own at full occupancy
-    const bool split = s.VD > 0 && s.V > s.VD && (size_t)s.lds_cu / wave_hist_bytes(s.K) < 16;
-    const int w_tail = split || s.V == s.VD ? s.VD : 0;  // first word of the LDS launch
-    if (w_tail > 0) {
-        const WaveGrid g = wave_grid(s, (size_t)w_tail, 0, 1 << 16);
-        hipLaunchKernelGGL(k_word_top, dim3(g.grid), dim3(64 * g.nwv), 0, st, 0, w_tail, s.VD, s.K, s.beta,
-                           s.wt_head, s.tail_off, s.wt_tail, s.tail_nnz, s.inv, s.zero_order, s.wtop);
-    }
-    if (s.V > w_tail) {
-        const WaveGrid g = wave_grid(s, (size_t)(s.V - w_tail), wave_hist_bytes(s.K), 1 << 16);
-        hipLaunchKernelGGL(k_word_top, dim3(g.grid), dim3(64 * g.nwv), g.nwv * wave_hist_bytes(s.K), st, w_tail, s.V,
-                           s.VD, s.K, s.beta, s.wt_head, s.tail_off, s.wt_tail, s.tail_nnz, s.inv, s.zero_order,
-                           s.wtop);
+        hipLaunchKernelGGL(k_inv_order, dim3(grid_for(s.K, 64, 1 << 16)), dim3(1024),
+                           ((size_t)((s.K + 3) & ~3) + 64) * sizeof(float), st, s.nk, s.K, s.vbeta, s.beta, s.inv,
+                           s.zero_order);
+    else
+        hipLaunchKernelGGL(k_inv, dim3(grid_for(s.K, 256, 1 << 16)), dim3(256), 0, st, s.nk, s.K, s.vbeta, s.inv);
+    if (s.V > 0) {
+        const size_t lds = s.V > s.VD ? 4 * (size_t)((s.K + 31) >> 5) * sizeof(uint32_t) : 0;
+        hipLaunchKernelGGL(k_word_top, dim3(grid_for((size_t)s.V, 4, 1 << 16)), dim3(256), lds, st, s.V, s.VD, s.K,
+                           s.beta, s.wt_head, s.tail_off, s.wt_tail, s.tail_nnz, s.inv, s.zero_order, s.wtop);
     }
     return hipGetLastError();
 }

@@ -1,0 +1,72 @@
+"""GPU: kernels at the sizes where their tiles end, against the CPU oracle
+(integers and topics bit for bit)."""
+import numpy as np
+import pytest
+
+from conftest import make_corpus
+from lda_sc20_amd import ezlda
+from oracle import binding as ob
+
+pytestmark = pytest.mark.gpu
+
+BETA = 0.01
+
+
+def _pair(off, words, V, K, seed=21, z0=None, **kw):
+    ctx = ezlda.Context(K=K, alpha=50.0 / K, beta=BETA, seed=seed, **kw)
+    ctx.load(ezlda.Corpus(V, off, words), z0=z0)
+    return ctx, ob.Oracle(K, float(np.float32(50.0 / K)), BETA, seed, V, off, words, z0=z0)
+
+
+# groups of 4 values, workgroups of 64 topics, a bitmap word of 32 topics
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 31, 32, 33, 63, 64, 65, 127, 129, 255, 257, 1023, 1025, 4099, 16383])
+def test_top3_of_sparse_words(K):
+    off, words = make_corpus(K, 60, 90, 50, zipf=1.2)
+    for z0 in (None, np.zeros(len(words), np.uint16), (np.arange(len(words)) % min(K, 3)).astype(np.uint16)):
+        # many topics without a token: equal values, ordered by topic
+        ctx, orc = _pair(off, words, 90, K, z0=z0, dense_words=5)
+        for x in (ctx, orc):
+            x.build_wt()
+            x.topk()
+        assert np.array_equal(ctx.get_inv().view(np.uint32), orc.get_inv().view(np.uint32))
+        assert np.array_equal(ctx.get_top(), orc.get_top())
+        ctx.close()
+
+
+# readback pieces: below, at and past a piece (2^19 topics) and a lane's eight
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 2047, 2049, (1 << 19) - 1, (1 << 19), (1 << 19) + 1, (1 << 20) + 11])
+def test_topics_are_read_back_in_the_corpus_order(n):
+    rng = np.random.default_rng(n)
+    cuts = np.sort(rng.choice(np.arange(1, n), min(n - 1, max(1, n // 60)), replace=False)) if n > 1 else []
+    off = np.concatenate([[0], cuts, [n]]).astype(np.int64)
+    words = rng.integers(0, 300, n).astype(np.int32)
+    z = rng.integers(0, 9, n).astype(np.uint16)
+    ctx = ezlda.Context(K=9, alpha=0.5, beta=BETA, seed=1)
+    ctx.load(ezlda.Corpus(300, off, words), z0=z)
+    assert np.array_equal(ctx.get_topics(), z)
+    ctx.close()
+
+
+# items cut by cost: documents of up to 5,000 tokens holding a word hundreds of
+# times, rows of more than a block per checkpoint (16- and 32-bit), and
+# corpora of fewer items than workgroups; the run cap does not change a draw
+@pytest.mark.parametrize("K,D,lens,kw", [
+    (700, 24, (4000, 5000), {}),
+    (1500, 24, (4000, 5000), {"run_cap": 7}),
+    (2048, 40, (300, 5000), {"run_cap": 3, "grid_dim": 24}),
+    (4096, 30, (1500, 5000), {"dense_words": 4, "grid_dim": 16}),
+    (9000, 24, (2000, 5000), {"grid_dim": 16}),
+    (20, 300, (1, 90), {}),
+])
+def test_sweeps_of_long_documents(K, D, lens, kw):
+    rng = np.random.default_rng(K)
+    n = rng.integers(lens[0], lens[1], D)
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int64)
+    words = np.minimum(rng.geometric(0.02, int(off[-1])) - 1, 399).astype(np.int32)
+    ctx, orc = _pair(off, words, 400, K, **kw)
+    for s in range(2):
+        ctx.sweep(1)
+        orc.sweep(1)
+        assert np.array_equal(ctx.get_topics(), orc.get_topics()), s
+    assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
+    ctx.close()
