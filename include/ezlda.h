@@ -358,9 +358,9 @@ int ezlda_server_wait(ezlda_server *srv, uint32_t request_id, uint16_t *z_out, i
 int ezlda_server_drain(ezlda_server *srv);
 int ezlda_server_get_stats(ezlda_server *srv, ezlda_server_stats *stats);
 int ezlda_server_reset_stats(ezlda_server *srv);
-/* The plain path: one document per kernel launch (one workgroup runs all of
- * its sweeps, its row in LDS), synchronous, on its own stream; same results
- * as the server.  Calls on one server are serialized. */
+/* The plain path: one document alone, one kernel launch per sweep,
+ * synchronous, on its own stream; same results as the server.  Calls on one
+ * server are serialized. */
 int ezlda_foldin_plain(ezlda_server *srv, uint32_t request_id, const int32_t *words, int32_t n, uint16_t *z_out,
                        int32_t *counts_out);
 

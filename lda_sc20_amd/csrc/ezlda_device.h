@@ -119,7 +119,8 @@ struct FoldinBatch {
     uint32_t *wcount = nullptr;     // V: tokens per word in the step
     uint32_t *wcursor = nullptr;    // V: bucket cursors
     uint32_t *bsum = nullptr;       // 3 x ceil(V / 1024): per-block big-word tokens, big items, other tokens
-    uint32_t *tokw = nullptr;       // resident tokens: slot << 16 | position, by word (big words first)
+    uint32_t *tokw = nullptr;       // resident tokens: slot << 16 | position, by word (big words first); or the
+                                    // workgroups of a step that is not bucketed: slot << 16 | part
     uint4 *items = nullptr;         // foldin_max_items(V, tokens) big items: (word, first, end, 0)
     uint32_t *ctr = nullptr;        // big items, big-word tokens, other tokens, 0
     uint16_t *zout = nullptr;       // finishing documents' topics, packed
@@ -130,17 +131,23 @@ uint32_t foldin_max_items(int V, uint32_t max_tokens);
 // Copies admitted documents (source offset, pool offset, tokens, 0) from an
 // upload buffer into the word pool.
 hipError_t launch_foldin_admit(const uint4 *adm, int nadm, const uint32_t *src, uint32_t *wpool, hipStream_t st);
-// One fold-in sweep of every slot (request id, pool offset (a multiple of 8),
-// tokens, sweep); fin[j] = (output index or ~0, topic offset) for the
-// documents that finish with this sweep; ntok = their tokens.  nslots <=
-// 65535 documents of <= 65535 tokens.
-// The plain path: every sweep of one document (n tokens, word ranks) in one
-// launch of one workgroup; z receives its n topics.
+// The plain path: every sweep of one document (n tokens, word ranks), one
+// launch a sweep; z receives its n topics, z2 (n values) the ones in between.
 hipError_t launch_foldin_doc(const uint32_t *words, uint32_t n, uint32_t rid, int sweeps, int K, float alpha,
                              const float *phi, const float *qs, const float *qacc, uint64_t seed, uint16_t *z,
-                             hipStream_t st);
-hipError_t launch_foldin_step(const FoldinBatch &fb, const uint4 *slots, const uint2 *fin, int nslots, uint32_t ntok,
-                              int V, int K, float alpha, const float *phi, const float *qs, const float *qacc,
+                             uint16_t *z2, hipStream_t st);
+// One fold-in sweep of every slot (request id, pool offset (a multiple of 8),
+// tokens, sweep); fin[j] = (output index or ~0, topic offset) for the
+// documents that finish with this sweep (any_fin: there are some); ntok = the
+// slots' tokens, max_n of the longest.  nslots <= 65535 documents of <= 65535
+// tokens.
+// A step of ntok tokens that is drawn without bucketing them by word runs in
+// workgroups of foldin_few_group(ntok) tokens of a slot (0: it is bucketed):
+// goff[j] is then the first of slot j's workgroups, ngroups their number.
+uint32_t foldin_few_group(uint32_t ntok);
+hipError_t launch_foldin_step(const FoldinBatch &fb, const uint4 *slots, const uint2 *fin, const uint32_t *goff,
+                              uint32_t ngroups, int nslots, uint32_t ntok, uint32_t max_n, bool any_fin, int V, int K,
+                              float alpha, const float *phi, const float *qs, const float *qacc,
                               const uint32_t *wpool, uint16_t *zpool, uint64_t seed, hipStream_t st);
 
 // Bytes of dynamic LDS the sampler needs for K topics and block size bd.

@@ -13,8 +13,7 @@
 // after `sweeps` sweeps; its pool range and slot are reused.  Draws are keyed
 // by (seed, request id, token, sweep), never by slot or position, so a result
 // is the same alone and in any mix.  ezlda_foldin_plain, the comparison
-// path, runs one document per launch (all of its sweeps in one workgroup) on
-// its own stream.
+// path, runs one document alone (one launch a sweep) on its own stream.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -97,7 +96,7 @@ struct ezlda_server {
     uint32_t budget_tokens = 0, pool_tokens = 0, up_cap = 0;
     StepRec rec[2];     // two steps in flight: host buffers and finishing documents
     int64_t retiring = 0;  // documents done on the device, results not yet published
-    // plain path: one document's words (ranks) and topics
+    // plain path: one document's words (ranks) and topics (two buffers)
     uint32_t *pw = nullptr;
     uint16_t *pz = nullptr;
     hipStream_t st = nullptr, pst = nullptr;
@@ -218,14 +217,15 @@ bool ensure_pinned(T **p, size_t *cap, size_t need) {
 }
 
 // Upload buffer layout for ns slots and na admitted documents:
-// [slots: ns uint4][fin: ns uint2][pad to 16][adm: na uint4][words]
+// [slots: ns uint4][fin: ns uint2][goff: ns u32][pad to 16][adm: na uint4][words]
 struct UpLayout {
-    size_t fin, adm, words, end;
+    size_t fin, goff, adm, words, end;
 };
 UpLayout up_layout(size_t ns, size_t na, size_t nw) {
     UpLayout l;
     l.fin = ns * sizeof(uint4);
-    l.adm = align16(l.fin + ns * sizeof(uint2));
+    l.goff = l.fin + ns * sizeof(uint2);
+    l.adm = align16(l.goff + ns * sizeof(uint32_t));
     l.words = l.adm + na * sizeof(uint4);
     l.end = l.words + nw * sizeof(uint32_t);
     return l;
@@ -286,7 +286,7 @@ void worker_main(ezlda_server *s) {
         StepRec &R = s->rec[cur], &P = s->rec[cur ^ 1];
         adm.clear();
         adm_rec.clear();
-        uint32_t up_words = 0, ns = 0, nfin = 0, zsum = 0, ntok = 0;
+        uint32_t up_words = 0, ns = 0, nfin = 0, zsum = 0, ntok = 0, max_n = 0, ngroups = 0;
         UpLayout L{};
         {
             std::unique_lock<std::mutex> lk(s->mu);
@@ -334,6 +334,7 @@ void worker_main(ezlda_server *s) {
                     Slot &x = s->slots[si];
                     hs[j] = make_uint4(x.rid, x.off, x.n, x.sweep);
                     ntok += x.n;
+                    max_n = std::max(max_n, x.n);
                     if (++x.sweep == (uint32_t)s->sweeps) {
                         Finishing f;
                         f.rid = x.rid;
@@ -349,6 +350,14 @@ void worker_main(ezlda_server *s) {
                         s->free_slots.push_back(si);
                     } else {
                         hf[j] = make_uint2(0xFFFFFFFFu, 0u);
+                    }
+                }
+                // places of the slots' workgroups where the step needs no buckets
+                if (const uint32_t group = ez::foldin_few_group(ntok)) {
+                    uint32_t *hg = (uint32_t *)(R.up_h + L.goff);
+                    for (uint32_t j = 0; j < ns; ++j) {
+                        hg[j] = ngroups;
+                        ngroups += (hs[j].z + group - 1) / group;
                     }
                 }
                 if (nfin) {
@@ -373,8 +382,9 @@ void worker_main(ezlda_server *s) {
                 e = ez::launch_foldin_admit((const uint4 *)(s->up_d + L.adm), (int)adm_rec.size(),
                                             (const uint32_t *)(s->up_d + L.words), s->wpool, s->st);
             if (e == hipSuccess)
-                e = ez::launch_foldin_step(s->fb, (const uint4 *)s->up_d, (const uint2 *)(s->up_d + L.fin), (int)ns,
-                                           ntok, s->V, s->K, s->alpha, s->phi, s->qs, s->qacc, s->wpool, s->zpool,
+                e = ez::launch_foldin_step(s->fb, (const uint4 *)s->up_d, (const uint2 *)(s->up_d + L.fin),
+                                           (const uint32_t *)(s->up_d + L.goff), ngroups, (int)ns,
+                                           ntok, max_n, nfin > 0, s->V, s->K, s->alpha, s->phi, s->qs, s->qacc, s->wpool, s->zpool,
                                            s->seed, s->st);
             if (e == hipSuccess && zsum)
                 e = hipMemcpyAsync(R.z_h, s->fb.zout, (size_t)zsum * sizeof(uint16_t), hipMemcpyDeviceToHost, s->st);
@@ -445,7 +455,7 @@ ezlda_server *ezlda_server_create(ezlda_ctx *ctx, const ezlda_server_args *a) tr
          salloc(s, &s->wpool, s->pool_tokens) == EZLDA_OK && salloc(s, &s->zpool, s->pool_tokens) == EZLDA_OK &&
          salloc(s, &s->up_d, s->up_bytes) == EZLDA_OK &&
          alloc_batch(s, &s->fb, s->pool_tokens, s->max_slots, 8 * cus) &&
-         salloc(s, &s->pw, 65536) == EZLDA_OK && salloc(s, &s->pz, 65536) == EZLDA_OK;
+         salloc(s, &s->pw, 65536) == EZLDA_OK && salloc(s, &s->pz, 2 * 65536) == EZLDA_OK;
     for (StepRec &R : s->rec)
         ok = ok && hipHostMalloc((void **)&R.up_h, s->up_bytes, hipHostMallocDefault) == hipSuccess &&
              hipEventCreateWithFlags(&R.ev, hipEventDisableTiming) == hipSuccess;
@@ -653,10 +663,10 @@ int ezlda_foldin_plain(ezlda_server *s, uint32_t request_id, const int32_t *word
         r[i] = (uint32_t)s->rank_of[words[i]];
     }
     std::lock_guard<std::mutex> lk(s->plain_mu);
-    // one document, one launch: every sweep runs inside k_fi_doc
+    // one document alone on the plain path's stream, one launch a sweep
     if (n) SV_HIP(s, hipMemcpyAsync(s->pw, r.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, s->pst));
     SV_HIP(s, ez::launch_foldin_doc(s->pw, (uint32_t)n, request_id, s->sweeps, s->K, s->alpha, s->phi, s->qs, s->qacc,
-                                    s->seed, s->pz, s->pst));
+                                    s->seed, s->pz, s->pz + 65536, s->pst));
     std::vector<uint16_t> z((size_t)n);
     if (n) SV_HIP(s, hipMemcpyAsync(z.data(), s->pz, n * sizeof(uint16_t), hipMemcpyDeviceToHost, s->pst));
     SV_HIP(s, hipStreamSynchronize(s->pst));

@@ -1587,9 +1587,12 @@ __device__ __forceinline__ void for_doc_tokens(const T *__restrict__ p, uint32_t
 // Rows of the resident documents (one workgroup per slot): topics drawn from
 // the init stream on sweep 0, a 16-bit LDS histogram, a row of topic | count
 // << 16 in ascending topic order, zero padded to a multiple of kFB.
+// With `group` tokens a workgroup set, also lists the workgroups of k_fi_few:
+// slot << 16 | part, from the slot's place in goff.
 __global__ void __launch_bounds__(256) k_fi_rows(const uint4 *__restrict__ slots, int nslots, int K, uint64_t seed,
                                                  uint16_t *__restrict__ zpool, uint32_t *__restrict__ rows,
-                                                 uint32_t *__restrict__ row_nnz) {
+                                                 uint32_t *__restrict__ row_nnz, uint32_t group,
+                                                 const uint32_t *__restrict__ goff, uint32_t *__restrict__ groups) {
     extern __shared__ uint32_t shr[];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, bd = blockDim.x;
     const int KH = (K + 1) >> 1;
@@ -1600,6 +1603,8 @@ __global__ void __launch_bounds__(256) k_fi_rows(const uint4 *__restrict__ slots
         const uint4 sl = slots[j];
         const uint32_t rid = sl.x, off = sl.y, n = sl.z, sweep = sl.w;
         uint16_t *z = zpool + off;
+        if (group)
+            for (uint32_t p = tid; p * group < n; p += bd) groups[goff[j] + p] = ((uint32_t)j << 16) | p;
         if (sweep == 0) {
             for (uint32_t i = tid; i < n; i += bd)
                 z[i] = (uint16_t)(ez_philox_x0(seed, ((uint64_t)rid << 32) | i, 0u, EZ_TAG_FOLDIN_INIT) % (uint32_t)K);
@@ -1834,6 +1839,29 @@ __device__ __forceinline__ int first_above(const float *q, int k0, int ke, float
     return ke;
 }
 
+// The Q bucket's topic at t2 (a word's phi row ph and running sums qa over the
+// slab totals, qw within slabs): the first whose running sum exceeds it, else
+// the last of positive mass; -1 if there is none.
+__device__ __forceinline__ int fi_q_topic(float t2, const float *ph, const float *qa, const float *qw, int K, int NS,
+                                          float alpha) {
+    const int lo = first_above(qa, 0, NS, t2);
+    int js = lo < NS ? lo : -1;
+    if (js < 0)
+        for (int jj = NS - 1; jj >= 0; --jj)
+            if (qa[jj] > (jj > 0 ? qa[jj - 1] : 0.0f)) {
+                js = jj;
+                break;
+            }
+    if (js < 0) return -1;
+    const float t3 = t2 - (js > 0 ? qa[js - 1] : 0.0f);
+    const int k0 = js * 64, ke = min(k0 + 64, K);
+    const int kq = first_above(qw, k0, ke, t3);
+    if (kq < ke) return kq;
+    for (int k = ke - 1; k >= k0; --k)
+        if (alpha * ph[k] > 0.0f) return k;
+    return -1;
+}
+
 // One fold-in draw: token i of slot sl (its row of nz entries at pool
 // offset sl.y) for a word whose phi row (ph) and Q running sums (qa over
 // the slab totals, qw within slabs) are given, in LDS or in the tables.  S
@@ -1923,29 +1951,7 @@ __device__ __forceinline__ void fi_draw(const uint4 sl, uint32_t i, uint32_t nz,
             for (uint32_t g = 0; g < nz; ++g)
                 if ((row[g] >> 16) && ph[row[g] & 0xFFFFu] > 0.0f) zz = (int)(row[g] & 0xFFFFu);
     } else {
-        const float t2 = target - S;
-        const int lo = first_above(qa, 0, NS, t2);
-        int js = lo < NS ? lo : -1;
-        if (js < 0)
-            for (int jj = NS - 1; jj >= 0; --jj)
-                if (qa[jj] > (jj > 0 ? qa[jj - 1] : 0.0f)) {
-                    js = jj;
-                    break;
-                }
-        if (js >= 0) {
-            const float t3 = t2 - (js > 0 ? qa[js - 1] : 0.0f);
-            const int k0 = js * 64, ke = min(k0 + 64, K);
-            const int kq = first_above(qw, k0, ke, t3);
-            if (kq < ke) {
-                zz = kq;
-            } else {
-                for (int k = ke - 1; k >= k0; --k)
-                    if (alpha * ph[k] > 0.0f) {
-                        zz = k;
-                        break;
-                    }
-            }
-        }
+        zz = fi_q_topic(target - S, ph, qa, qw, K, NS, alpha);
     }
     zpool[sl.y + i] = (uint16_t)(zz < 0 ? 0 : zz);
 }
@@ -1995,67 +2001,301 @@ __global__ void __launch_bounds__(256) k_fi_sample(const uint4 *__restrict__ slo
     }
 }
 
-// The plain fold-in path: one launch runs every sweep of one document.  One
-// workgroup: the document's topics live in z (device memory, n values), its
-// 16-bit topic histogram and its row (topic | count << 16, ascending topic,
-// zero padded to a multiple of kFB) in LDS.  Each sweep rebuilds the row from
-// z, then every token is drawn against it (Jacobi: the row is complete before
-// any token of the sweep moves) with the draw the batched step uses, so the
-// topics are the server's and the oracle's.
-static size_t foldin_doc_lds(int K) {
-    const size_t kh4 = (((size_t)K + 1) / 2 + 3) & ~(size_t)3;  // 16-byte aligned row after the counts
-    return (kh4 + (((size_t)K + 7) & ~(size_t)7) + 8 + 4) * sizeof(uint32_t);
+// ---- few tokens: one wavefront draws T tokens of a document
+// One lane a token leaves most of the chip idle when there are few tokens,
+// and one document's gathers of phi all pass through one CU's L1 (64 lines an
+// instruction): 18.7 us a sweep for 217 tokens.  Here a wavefront gathers the
+// phi values of T tokens for a piece of the row (lane = entry, every load of
+// the piece in flight at once) into LDS, lane t then runs token t's FMA chain
+// over it in order, keeping the running sums in place, and bisects them; the
+// document's tokens are spread over workgroups of four wavefronts.
+static constexpr uint32_t kPiece = 256, kPieceRow = kPiece + 4;  // entries; LDS floats a token (padded)
+static constexpr uint32_t kMaxPieces = 64;                       // of a row (K <= 16383)
+
+// LDS floats of one wavefront: T rows of running sums, T lists of piece ends
+static constexpr uint32_t wave_draw_floats(int T) { return (uint32_t)T * (kPieceRow + kMaxPieces); }
+
+// What a wavefront's tokens [i0, i0 + T) of a document (those below n) need
+// besides the row, loaded before the row is there: lane t's word and uniform,
+// and (qv) the running sums of each token's slab totals, lane = slab (past the
+// 64th a token reads them itself).
+template <int T>
+struct WaveTokens {
+    uint32_t nt, w;
+    float u, qv[T];
+};
+template <int T>
+__device__ __forceinline__ WaveTokens<T> fi_wave_tokens(uint32_t i0, uint32_t n, const uint32_t *__restrict__ words,
+                                                        uint32_t rid, uint32_t sweep, const float *__restrict__ qacc,
+                                                        int NS, uint64_t seed) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t i = i0 + (uint32_t)lane;
+    WaveTokens<T> W;
+    W.nt = i0 < n ? min((uint32_t)T, n - i0) : 0u;
+    W.w = (uint32_t)lane < W.nt ? words[i] : 0u;
+#pragma unroll
+    for (int t = 0; t < T; ++t) W.qv[t] = qacc[(size_t)readlane_u(W.w, t) * NS + min(lane, NS - 1)];
+    W.u = ez_u24(ez_philox_x0(seed, ((uint64_t)rid << 32) | i, sweep, EZ_TAG_FOLDIN));
+    return W;
 }
 
-__global__ void __launch_bounds__(1024) k_fi_doc(const uint32_t *__restrict__ words, uint32_t n, uint32_t rid,
-                                                 int sweeps, int K, float alpha, const float *__restrict__ phi,
-                                                 const float *__restrict__ qs, const float *__restrict__ qacc,
-                                                 uint64_t seed, uint16_t *__restrict__ z) {
-    extern __shared__ uint32_t shd[];
-    const int NS = (K + 63) >> 6, tid = threadIdx.x, bd = blockDim.x, lane = tid & 63, wv = tid >> 6;
-    const int KH = (K + 1) >> 1, KH4 = (KH + 3) & ~3;
-    uint32_t *h = shd;                                   // KH words: 16-bit counts
-    uint32_t *row = shd + KH4;                           // the row, 16-byte aligned
-    uint32_t *s_nz = row + ((K + 7) & ~7) + 8;           // the row's entries
-    for (uint32_t i = tid; i < n; i += bd)
-        z[i] = (uint16_t)(ez_philox_x0(seed, ((uint64_t)rid << 32) | i, 0u, EZ_TAG_FOLDIN_INIT) % (uint32_t)K);
-    for (int k = tid; k < KH; k += bd) h[k] = 0;
-    __syncthreads();
-    for (int sw = 0; sw < sweeps; ++sw) {
-        for (uint32_t i = tid; i < n; i += bd) h16_add(h, z[i]);
-        __syncthreads();
-        if (wv == 0) {  // one wavefront compacts the row in ascending topic order and clears the counts
-            uint32_t nz = 0;
-            for (int c0 = 0; c0 < K; c0 += 64) {
-                const int k = c0 + lane;
-                const uint32_t c = k < K ? h16_get(h, (uint32_t)k) : 0u;
-                const uint64_t m = __ballot(c != 0);
-                if (c) row[nz + __popcll(m & lanemask_lt(lane))] = (uint32_t)k | (c << 16);
-                nz += (uint32_t)__popcll(m);
-                wave_lds_sync();
-                if (k < K && !(k & 1)) h[k >> 1] = 0;
-            }
-            // zero entries up to the next block: a count of 0 adds exactly nothing
-            if ((uint32_t)lane < ((kFB - (nz % kFB)) % kFB)) row[nz + lane] = 0u;
-            if (lane == 0) *s_nz = nz;
+// Draws them: row = the document's nz entries in LDS, 16-byte aligned and
+// zero padded to a multiple of 4; lane t writes its topic to z[t].
+template <int T>
+__device__ __forceinline__ void fi_draw_wave(const uint32_t *row, uint32_t nz, const WaveTokens<T> &W,
+                                             const float *__restrict__ phi, const float *__restrict__ qs,
+                                             const float *__restrict__ qacc, int K, int NS, float alpha,
+                                             float *pv, uint16_t *__restrict__ z) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t w = W.w;
+    const bool mine = (uint32_t)lane < W.nt;
+    float *pe = pv + T * kPieceRow + lane * kMaxPieces;  // this lane's piece ends
+    float *run = pv + lane * kPieceRow;                  // this lane's running sums
+    const uint32_t np = (nz + kPiece - 1u) / kPiece;
+    // phi of token t at piece c's entries, into its LDS row
+    auto gather = [&](const uint32_t (&e)[4], uint32_t c, int t, float (&v)[4]) {
+        const float *base = phi + (size_t)readlane_u(w, t) * K;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = c * kPiece + 64u * u < nz ? base[e[u] & 0xFFFFu] : 0.0f;
+    };
+    auto load_entries = [&](uint32_t c, uint32_t (&e)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t x = c * kPiece + (uint32_t)lane + 64u * u;
+            e[u] = x < nz ? row[x] : 0u;
         }
-        __syncthreads();
-        const uint32_t nz = *s_nz;
-        const uint4 sl = make_uint4(rid, 0u, n, (uint32_t)sw);
-        for (uint32_t i = tid; i < n; i += bd) {
-            const size_t w = words[i];
-            fi_draw(sl, i, nz, row, phi + w * K, qacc + w * NS, qs + w * K, K, NS, alpha, seed, z);
+    };
+    // this lane's chain over piece c from s, the running sums kept in place
+    auto chain = [&](uint32_t c, float s) {
+        const uint32_t ng = (min(kPiece, nz - c * kPiece) + 3u) >> 2;
+        const uint4 *r4 = reinterpret_cast<const uint4 *>(row + c * kPiece);
+        float4 *v4 = reinterpret_cast<float4 *>(run);
+#pragma unroll 4
+        for (uint32_t g = 0; g < ng; ++g) {
+            const uint4 e = r4[g];
+            float4 v = v4[g];
+            v.x = __builtin_fmaf((float)(e.x >> 16), v.x, s);
+            v.y = __builtin_fmaf((float)(e.y >> 16), v.y, v.x);
+            v.z = __builtin_fmaf((float)(e.z >> 16), v.z, v.y);
+            s = v.w = __builtin_fmaf((float)(e.w >> 16), v.w, v.z);
+            v4[g] = v;
         }
-        __syncthreads();  // every topic of the sweep is written before the next histogram
+        return s;
+    };
+    float S = 0.0f;
+    for (uint32_t c = 0; c < np; ++c) {
+        uint32_t e[4];
+        load_entries(c, e);
+        float v[T][4];
+#pragma unroll
+        for (int t = 0; t < T; ++t) gather(e, c, t, v[t]);
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) pv[t * kPieceRow + lane + 64 * u] = v[t][u];
+        wave_lds_sync();
+        if (mine) {
+            S = chain(c, S);
+            pe[c] = S;
+        }
+        wave_lds_sync();
     }
+    const float *qa = qacc + (size_t)w * NS;
+    float qlast = 0.0f;  // the Q mass: the running sum of the last slab
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const float x = readlane_f(W.qv[t], min(NS - 1, 63));
+        if (lane == t) qlast = x;
+    }
+    if (NS > 64 && mine) qlast = qa[NS - 1];
+    const float target = W.u * (S + qlast), t2 = target - S;
+    const bool in_q = mine && !(target < S);
+    int zz = -1;
+    uint32_t pc = 0xFFFFFFFFu;  // the piece that holds the target
+    if (mine && !in_q) {
+        uint32_t lo = 0, hi = np - 1u;  // the last piece's end is S
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (pe[mid] > target) hi = mid; else lo = mid + 1u;
+        }
+        pc = lo;
+    }
+    // Q: the whole wavefront looks for each token's slab, then its topic; what
+    // rounding leaves above every running sum goes the general way
+    uint64_t todo = __ballot(in_q);
+    if (NS <= 64) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            if (!((todo >> t) & 1ull)) continue;
+            const float x = readlane_f(t2, t);
+            const uint64_t ms = __ballot(lane < NS && W.qv[t] > x);
+            if (!ms) continue;
+            const int js = first_lane(ms), k0 = js * 64;
+            const float t3 = x - (js > 0 ? readlane_f(W.qv[t], js - 1) : 0.0f);
+            const bool in = k0 + lane < K;
+            const float q = in ? qs[(size_t)readlane_u(w, t) * K + k0 + lane] : 0.0f;
+            const uint64_t mk = __ballot(in && q > t3);
+            if (!mk) continue;
+            if (lane == t) zz = k0 + first_lane(mk);
+            todo &= ~(1ull << t);
+        }
+    }
+    if ((todo >> lane) & 1ull)
+        zz = fi_q_topic(t2, phi + (size_t)w * K, qa, qs + (size_t)w * K, K, NS, alpha);
+    if (np > 1) {  // the piece's running sums once more (LDS holds the last piece's)
+        for (int t = 0; t < T; ++t) {
+            const uint32_t c = readlane_u(pc, t);
+            if (c == 0xFFFFFFFFu) continue;
+            uint32_t e[4];
+            load_entries(c, e);
+            float v[4];
+            gather(e, c, t, v);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) pv[t * kPieceRow + lane + 64 * u] = v[u];
+        }
+        wave_lds_sync();
+        if (pc != 0xFFFFFFFFu) chain(pc, pc ? pe[pc - 1u] : 0.0f);
+    }
+    if (pc != 0xFFFFFFFFu) {
+        uint32_t lo = 0, hi = min(kPiece, nz - pc * kPiece) - 1u;  // the piece's last running sum exceeds the target
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (run[mid] > target) hi = mid; else lo = mid + 1u;
+        }
+        zz = (int)(row[pc * kPiece + lo] & 0xFFFFu);
+    }
+    if (mine) z[lane] = (uint16_t)(zz < 0 ? 0 : zz);
 }
+
+// One fold-in sweep of the resident documents when they have few tokens:
+// each workgroup takes 4 T tokens of a slot (groups: slot << 16 | part), copies
+// its row into LDS and draws T of them with each wavefront.  Measured for one document of 217 tokens at K = 1024: a
+// step of 18 us, against 48 us with its tokens bucketed by word (nine launches
+// of about 4 us, k_fi_sample 17).
+template <int T>
+__global__ void __launch_bounds__(256) k_fi_few(const uint4 *__restrict__ slots, int K, float alpha,
+                                                const float *__restrict__ phi, const float *__restrict__ qs,
+                                                const float *__restrict__ qacc, const uint32_t *__restrict__ wpool,
+                                                const uint32_t *__restrict__ rows, const uint32_t *__restrict__ row_nnz,
+                                                const uint32_t *__restrict__ groups, uint32_t row_cap,
+                                                uint16_t *__restrict__ zpool, uint64_t seed) {
+    extern __shared__ __align__(16) uint32_t shd[];
+    const int NS = (K + 63) >> 6, tid = threadIdx.x, wv = tid >> 6;
+    const uint32_t grp = groups[blockIdx.x], j = grp >> 16;
+    const uint4 sl = slots[j];
+    const uint32_t i0 = ((grp & 0xFFFFu) * 4u + (uint32_t)wv) * T;
+    uint32_t *row = shd;  // row_cap entries, padded to 4
+    float *pv = reinterpret_cast<float *>(row + ((row_cap + 3u) & ~3u)) + wv * wave_draw_floats(T);
+    const WaveTokens<T> W = fi_wave_tokens<T>(i0, sl.z, wpool + sl.y, sl.x, sl.w, qacc, NS, seed);
+    const uint32_t nz = row_nnz[j];
+    for (uint32_t x = tid; x < ((nz + 3u) & ~3u); x += 256) row[x] = rows[sl.y + x];  // rows are zero padded to 8
+    __syncthreads();
+    if (i0 < sl.z) fi_draw_wave<T>(row, nz, W, phi, qs, qacc, K, NS, alpha, pv, zpool + sl.y + i0);
+}
+
+// The plain fold-in path: one sweep of one document a launch (n tokens; the
+// topics go from zin to zout, so every workgroup may read them all).  Each
+// workgroup builds the document's row in LDS (a 16-bit histogram and a
+// bitmap of its topics, compacted by one wavefront in ascending topic order)
+// and draws 4 T tokens against it.  On sweep 0 with zin null the topics are
+// those of the init stream.  One launch of one workgroup for all sweeps took
+// 373 us for 217 tokens and 20 sweeps at K = 1024 and 29.4 ms for 4,098; this
+// takes 175 us (10 us a launch, a chain of latencies: topics, histogram, phi
+// gathers, sums, Q) and 0.66 ms.
+template <int T>
+__global__ void __launch_bounds__(256) k_fi_doc(const uint32_t *__restrict__ words, uint32_t n, uint32_t rid,
+                                                uint32_t sweep, int K, float alpha, const float *__restrict__ phi,
+                                                const float *__restrict__ qs, const float *__restrict__ qacc,
+                                                uint64_t seed, const uint16_t *__restrict__ zin,
+                                                uint16_t *__restrict__ zout) {
+    extern __shared__ __align__(16) uint32_t shd[];
+    const int NS = (K + 63) >> 6, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int KH4 = (((K + 1) >> 1) + 3) & ~3, NW4 = (((K + 31) >> 5) + 3) & ~3;
+    uint32_t *h = shd;                                 // KH4 words: 16-bit counts
+    uint32_t *bm = h + KH4;                            // NW4 words: bitmap of the topics
+    uint32_t *s_nz = bm + NW4;                         // 4 words: the row's entries
+    uint32_t *row = s_nz + 4;                          // min(n, K) entries, padded to 4
+    float *pv = reinterpret_cast<float *>(row + ((min(n, (uint32_t)K) + 3u) & ~3u)) + wv * wave_draw_floats(T);
+    const uint32_t i0 = (blockIdx.x * 4u + (uint32_t)wv) * T;
+    const WaveTokens<T> W = fi_wave_tokens<T>(i0, n, words, rid, sweep, qacc, NS, seed);
+    for (int k = tid; k < KH4 + NW4; k += 256) h[k] = 0;
+    __syncthreads();
+    auto add = [&](uint32_t t) {
+        h16_add(h, t);
+        atomicOr(&bm[t >> 5], 1u << (t & 31u));
+    };
+    if (zin)
+        for_doc_tokens(zin, n, [&](uint16_t t, uint32_t) { add(t); });
+    else
+        for (uint32_t i = tid; i < n; i += 256)
+            add(ez_philox_x0(seed, ((uint64_t)rid << 32) | i, 0u, EZ_TAG_FOLDIN_INIT) % (uint32_t)K);
+    __syncthreads();
+    if (wv == 0) {
+        uint32_t nz = 0;
+        for (int j = 0; j < NW4; j += 64) {
+            const int wi = j + lane;
+            const uint32_t word = wi < NW4 ? bm[wi] : 0u;
+            const uint32_t m = (uint32_t)__popc(word);
+            uint32_t incl = m;  // inclusive scan over lanes
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t v = __shfl_up(incl, d);
+                if (lane >= d) incl += v;
+            }
+            uint32_t pos = nz + incl - m;
+            for (uint32_t x = word; x; x &= x - 1u) {
+                const uint32_t k = ((uint32_t)wi << 5) + (uint32_t)__ffs(x) - 1u;
+                row[pos++] = k | (h16_get(h, k) << 16);
+            }
+            nz += __shfl(incl, 63);
+        }
+        if ((uint32_t)lane < ((4u - (nz & 3u)) & 3u)) row[nz + lane] = 0u;
+        if (lane == 0) *s_nz = nz;
+    }
+    __syncthreads();
+    if (i0 < n) fi_draw_wave<T>(row, *s_nz, W, phi, qs, qacc, K, NS, alpha, pv, zout + i0);
+}
+
+// Topics of the init stream (documents too long for every workgroup of
+// k_fi_doc to draw them itself).
+__global__ void __launch_bounds__(256) k_fi_init(uint32_t n, uint32_t rid, int K, uint64_t seed,
+                                                 uint16_t *__restrict__ z) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n) z[i] = (uint16_t)(ez_philox_x0(seed, ((uint64_t)rid << 32) | i, 0u, EZ_TAG_FOLDIN_INIT) % (uint32_t)K);
+}
+
+// LDS of k_fi_doc for a document of n tokens.
+static size_t foldin_doc_lds(int K, uint32_t n, int T) {
+    const size_t kh4 = (((size_t)K + 1) / 2 + 3) & ~(size_t)3, nw4 = (((size_t)K + 31) / 32 + 3) & ~(size_t)3;
+    return (kh4 + nw4 + 4 + ((std::min<size_t>(n, (size_t)K) + 3) & ~(size_t)3) + 4 * wave_draw_floats(T)) *
+           sizeof(uint32_t);
+}
+
+// Tokens a wavefront draws in k_fi_doc: one while the workgroups fit the
+// chip's CUs, more for longer documents (each workgroup builds the row).
+static int foldin_doc_t(uint32_t n) { return n <= 1024 ? 1 : n <= 2048 ? 2 : 4; }
 
 hipError_t launch_foldin_doc(const uint32_t *words, uint32_t n, uint32_t rid, int sweeps, int K, float alpha,
                              const float *phi, const float *qs, const float *qacc, uint64_t seed, uint16_t *z,
-                             hipStream_t st) {
+                             uint16_t *z2, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fi_doc, dim3(1), dim3(1024), foldin_doc_lds(K), st, words, n, rid, sweeps, K, alpha, phi, qs,
-                       qacc, seed, z);
+    uint16_t *buf[2] = {z, z2};  // the last sweep writes z
+    const int T = foldin_doc_t(n);
+    const unsigned grid = (n + 4u * (unsigned)T - 1u) / (4u * (unsigned)T);
+    const size_t lds = foldin_doc_lds(K, n, T);
+    const bool inline_init = n <= 1024;
+    if (!inline_init)
+        hipLaunchKernelGGL(k_fi_init, dim3((n + 255u) / 256u), dim3(256), 0, st, n, rid, K, seed, buf[sweeps & 1]);
+    for (int sw = 0; sw < sweeps; ++sw) {
+        const uint16_t *zin = sw == 0 && inline_init ? nullptr : buf[(sweeps - sw) & 1];
+        uint16_t *zout = buf[(sweeps - 1 - sw) & 1];
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, words, n, rid, (uint32_t)sw, K, alpha, phi, qs,
+                               qacc, seed, zin, zout);
+        };
+        if (T == 1) go(k_fi_doc<1>);
+        else if (T == 2) go(k_fi_doc<2>);
+        else go(k_fi_doc<4>);
+    }
     return hipGetLastError();
 }
 
@@ -2094,19 +2334,49 @@ hipError_t launch_foldin_admit(const uint4 *adm, int nadm, const uint32_t *src, 
     return hipGetLastError();
 }
 
-hipError_t launch_foldin_step(const FoldinBatch &fb, const uint4 *slots, const uint2 *fin, int nslots, uint32_t ntok,
-                              int V, int K, float alpha, const float *phi, const float *qs, const float *qacc,
+// Steps of few tokens are drawn by k_fi_few, straight from the tables: no
+// buckets by word, whose seven launches cost more than they save until big
+// words gather enough tokens to share a staged phi row.  Measured, ms to
+// drain a batch of documents (mean 300 tokens, 20 sweeps) bucketed / few, for
+// 39K, 161K, 315K and 609K tokens resident: K = 1024 2.49 / 1.16, 3.66 / 3.22,
+// 5.20 / 5.58, 7.66 / 9.32; K = 128 - / 0.58, 1.60 / 1.26, 2.39 / 2.27,
+// 3.42 / 3.86; K = 4096 (161K on) 4.18 / 4.42, 6.45 / 7.36, 9.80 / 10.64.
+static constexpr uint32_t kFewTokens = 196608;
+
+uint32_t foldin_few_group(uint32_t ntok) {
+    return ntok > kFewTokens ? 0u : ntok <= 4096 ? 4u : ntok <= 8192 ? 8u : 16u;
+}
+
+hipError_t launch_foldin_step(const FoldinBatch &fb, const uint4 *slots, const uint2 *fin, const uint32_t *goff,
+                              uint32_t ngroups, int nslots, uint32_t ntok, uint32_t max_n, bool any_fin, int V, int K,
+                              float alpha, const float *phi, const float *qs, const float *qacc,
                               const uint32_t *wpool, uint16_t *zpool, uint64_t seed, hipStream_t st) {
     if (nslots <= 0) return hipSuccess;
+    const unsigned gs = (unsigned)std::min(nslots, 1 << 16);
+    const size_t lds_rows = (size_t)((K + 1) >> 1) * sizeof(uint32_t);
+    const uint32_t group = foldin_few_group(ntok);
+    hipLaunchKernelGGL(k_fi_rows, dim3(gs), dim3(256), lds_rows, st, slots, nslots, K, seed, zpool, fb.rows,
+                       fb.row_nnz, group, goff, fb.tokw);
+    if (group) {
+        const uint32_t row_cap = std::min(max_n, (uint32_t)K);
+        const size_t lds = (((size_t)row_cap + 3) / 4 * 4 + 4 * wave_draw_floats((int)group / 4)) * sizeof(uint32_t);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(ngroups), dim3(256), lds, st, slots, K, alpha, phi, qs, qacc, wpool, fb.rows,
+                               fb.row_nnz, fb.tokw, row_cap, zpool, seed);
+        };
+        if (ngroups) {
+            if (group == 4) go(k_fi_few<1>);
+            else if (group == 8) go(k_fi_few<2>);
+            else go(k_fi_few<4>);
+        }
+        if (any_fin) hipLaunchKernelGGL(k_fi_final, dim3(gs), dim3(256), 0, st, slots, fin, nslots, zpool, fb.zout);
+        return hipGetLastError();
+    }
     // count and scatter: one workgroup per CU (fb.grid is 8 per CU), each
     // flushing its LDS table of the most frequent words once for many slots
-    const unsigned gs = (unsigned)std::min(nslots, 1 << 16);
     const unsigned gc = (unsigned)std::max(1, std::min(nslots, std::max(1, fb.grid / 8)));
     const unsigned nb = (unsigned)((V + 1023) / 1024);
-    const size_t lds_rows = (size_t)((K + 1) >> 1) * sizeof(uint32_t);
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for((size_t)V, 256, 4096)), dim3(256), 0, st, fb.wcount, (size_t)V, 0u);
-    hipLaunchKernelGGL(k_fi_rows, dim3(gs), dim3(256), lds_rows, st, slots, nslots, K, seed, zpool, fb.rows,
-                       fb.row_nnz);
     hipLaunchKernelGGL(k_fi_count, dim3(gc), dim3(256), 0, st, slots, nslots, wpool, fb.wcount);
     hipLaunchKernelGGL(k_fi_bsum, dim3(nb), dim3(1024), 0, st, V, fb.wcount, fb.bsum);
     hipLaunchKernelGGL(k_fi_btop, dim3(1), dim3(1024), 0, st, (int)nb, fb.bsum, fb.ctr);
@@ -2117,7 +2387,7 @@ hipError_t launch_foldin_step(const FoldinBatch &fb, const uint4 *slots, const u
     const unsigned gsmp = (unsigned)std::max<int64_t>(1, std::min<int64_t>(fb.grid, ((int64_t)ntok + 255) / 256));
     hipLaunchKernelGGL(k_fi_sample, dim3(gsmp), dim3(256), foldin_sample_lds(K), st, slots, K, alpha, phi, qs, qacc,
                        wpool, fb.rows, fb.row_nnz, fb.tokw, fb.items, fb.ctr, zpool, seed);
-    hipLaunchKernelGGL(k_fi_final, dim3(gs), dim3(256), 0, st, slots, fin, nslots, zpool, fb.zout);
+    if (any_fin) hipLaunchKernelGGL(k_fi_final, dim3(gs), dim3(256), 0, st, slots, fin, nslots, zpool, fb.zout);
     return hipGetLastError();
 }
 
@@ -2339,7 +2609,7 @@ size_t max_lds_bytes(int K, int bd) {
     m = std::max(m, (size_t)K * sizeof(double));                     // log-likelihood
     m = std::max(m, (size_t)K * sizeof(float) + 1024 * sizeof(float));  // fold-in tables
     m = std::max(m, foldin_lds_bytes(K));
-    m = std::max(m, foldin_doc_lds(K));
+    m = std::max(m, foldin_doc_lds(K, 65535, 4));
     return m;
 }
 

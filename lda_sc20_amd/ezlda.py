@@ -540,7 +540,7 @@ class Server:
         self._chk(self._L.ezlda_server_reset_stats(self._h))
 
     def plain(self, rid: int, words: np.ndarray):
-        """One document per kernel launch (all of its sweeps): (z, topic counts)."""
+        """One document alone, synchronously: (z, topic counts)."""
         w = np.ascontiguousarray(words, dtype=np.int32)
         z = np.zeros(max(len(w), 1), np.uint16)
         c = np.zeros(self.K, np.int32)

@@ -70,3 +70,50 @@ def test_sweeps_of_long_documents(K, D, lens, kw):
         assert np.array_equal(ctx.get_topics(), orc.get_topics()), s
     assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
     ctx.close()
+
+
+# fold-in: tokens a wavefront draws (1, 2, 4 by length), pieces of 256 row
+# entries, more than 64 slabs (K > 4096), empty documents
+@pytest.mark.parametrize("K", [7, 64, 300, 1024, 4096, 5000, 16383])
+def test_fold_in_at_the_edges_of_its_tiles(K):
+    lens = [0, 1, 3, 4, 5, 63, 255, 256, 257, 512, 513, 1023, 1024, 1025, 2048, 2049, 4500]
+    off, words = make_corpus(4, 200, 300, 60, zipf=1.2)
+    ctx, orc = _pair(off, words, 300, K)
+    ctx.sweep(2)
+    orc.sweep(2)
+    rng = np.random.default_rng(K)
+    doff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    dw = ((rng.zipf(1.2, int(doff[-1])) - 1) % 300).astype(np.int32)
+    rids = np.arange(50, 50 + len(lens), dtype=np.uint32)
+    zo, co = orc.foldin(doff, dw, rids, 3, 77)
+    srv = ezlda.Server(ctx, max_slots=len(lens), sweeps=3, hbm_budget_bytes=1 << 22, seed=77)
+    srv.submit_many(rids, doff, dw)
+    for r, rid in enumerate(rids.tolist()):
+        z, c, _ = srv.wait(rid, timeout_ms=60000)
+        assert np.array_equal(z, zo[doff[r]: doff[r + 1]]) and np.array_equal(c, co[r]), lens[r]
+        z, c = srv.plain(rid, dw[doff[r]: doff[r + 1]])
+        assert np.array_equal(z, zo[doff[r]: doff[r + 1]]) and np.array_equal(c, co[r]), lens[r]
+    srv.close()
+
+
+# steps of more and of fewer tokens than are drawn without buckets by word
+@pytest.mark.parametrize("K,D", [(128, 900), (1024, 700)])
+def test_fold_in_of_a_full_house(K, D):
+    off, words = make_corpus(4, 200, 300, 60, zipf=1.2)
+    ctx, orc = _pair(off, words, 300, K)
+    rng = np.random.default_rng(K)
+    lens = rng.integers(200, 600, D)
+    doff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    dw = ((rng.zipf(1.2, int(doff[-1])) - 1) % 300).astype(np.int32)
+    rids = np.arange(D, dtype=np.uint32)
+    ctx.build_wt()
+    orc.build_wt()
+    orc.topk()
+    zo, co = orc.foldin(doff, dw, rids, 2, 5)
+    srv = ezlda.Server(ctx, max_slots=D, sweeps=2, hbm_budget_bytes=1 << 24, seed=5)
+    srv.submit_many(rids, doff, dw)
+    for r in rids.tolist():
+        z, c, _ = srv.wait(r, timeout_ms=60000)
+        assert np.array_equal(z, zo[doff[r]: doff[r + 1]]) and np.array_equal(c, co[r]), r
+    assert srv.stats().max_active * 400 > 196608
+    srv.close()
