@@ -53,14 +53,16 @@ struct Slot {
     double t_submit = 0.0;
 };
 
+// A finished document's topics; the thread that claims it counts them (the
+// worker would otherwise spend a step's time on the K-sized counts of the
+// documents that finish with it).
 struct Result {
     std::vector<uint16_t> z;
-    std::vector<int32_t> counts;
     double latency_ms = 0.0;
 };
 
 // A document finishing with a step: where its topics land in the step's result
-// copy (the host counts them).
+// copy.
 struct Finishing {
     uint32_t rid = 0, n = 0, fidx = 0, zoff = 0;
     double t_submit = 0.0;
@@ -246,8 +248,6 @@ bool publish(ezlda_server *s, StepRec &R) {
     for (size_t f = 0; f < R.fins.size(); ++f) {
         const Finishing &x = R.fins[f];
         res[f].z.assign(R.z_h + x.zoff, R.z_h + x.zoff + x.n);
-        res[f].counts.assign(s->K, 0);
-        for (const uint16_t t : res[f].z) res[f].counts[t]++;
     }
     std::lock_guard<std::mutex> lk(s->mu);
     const double t = now_ms();
@@ -589,10 +589,15 @@ int ezlda_server_wait(ezlda_server *s, uint32_t request_id, uint16_t *z_out, int
         return sfail(s, EZLDA_ESTATE, "timed out waiting for fold-in request " + std::to_string(request_id));
     auto it = s->done.find(request_id);
     if (it == s->done.end()) return sfail(s, s->worker_rc, s->err);
-    if (z_out && !it->second.z.empty()) std::memcpy(z_out, it->second.z.data(), it->second.z.size() * sizeof(uint16_t));
-    if (counts_out) std::memcpy(counts_out, it->second.counts.data(), it->second.counts.size() * sizeof(int32_t));
-    if (latency_ms) *latency_ms = it->second.latency_ms;
+    const Result r = std::move(it->second);
     s->done.erase(it);
+    lk.unlock();
+    if (z_out && !r.z.empty()) std::memcpy(z_out, r.z.data(), r.z.size() * sizeof(uint16_t));
+    if (counts_out) {
+        std::memset(counts_out, 0, (size_t)s->K * sizeof(int32_t));
+        for (const uint16_t t : r.z) counts_out[t]++;
+    }
+    if (latency_ms) *latency_ms = r.latency_ms;
     return EZLDA_OK;
 } catch (...) {
     return ezc::server_exception_status(s);
