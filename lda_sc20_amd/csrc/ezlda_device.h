@@ -58,7 +58,8 @@ struct DevState {
                                     // a word's tokens in one doc
     int64_t n_runs = 0;
     int32_t n_queues = 1;           // persistent sampler: item queues (<= 8)
-    uint32_t *counters = nullptr;   // kCounterWords: [0] sweep, queue q's head at [kQueueStride * (q + 1)]
+    uint32_t *counters = nullptr;   // kCounterWords: [0] the next sweep, [1] the one launch_begin_sweep began,
+                                    // queue q's head at [kQueueStride * (q + 1)]
     unsigned long long *stats = nullptr;  // [0] full draws, [1] DT entries scanned
     double *ll_part = nullptr;      // n_smp_segs
     double *ll_out = nullptr;       // 1
@@ -70,6 +71,9 @@ struct DevState {
 
 hipError_t launch_zero_counts(const DevState &s, hipStream_t st);
 hipError_t launch_build_wt(const DevState &s, hipStream_t st);
+// The same for a whole sweep: also clears the sampler's queue heads and moves
+// the sweep counter on; launch_sample is then told that the sweep has begun.
+hipError_t launch_begin_sweep(const DevState &s, hipStream_t st);
 // Adds the counts of s.z (n_k, dense head rows, tail rows) without zeroing.
 hipError_t launch_accumulate_wt(const DevState &s, hipStream_t st);
 hipError_t launch_topk(const DevState &s, hipStream_t st);
@@ -88,7 +92,7 @@ hipError_t launch_topics_out(const DevState &s, uint32_t b, uint32_t n, uint16_t
 // any order.
 static constexpr uint32_t kSampleHead = 1u, kSampleTail = 2u, kShortcutOnly = 4u;
 hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st,
-                         uint32_t mode = kSampleHead | kSampleTail);
+                         uint32_t mode = kSampleHead | kSampleTail, bool begun = false);
 // Dense head rows of the current z (zeroed first) and n_k alone.
 hipError_t launch_head_rows(const DevState &s, hipStream_t st);
 hipError_t launch_topic_hist(const DevState &s, hipStream_t st);

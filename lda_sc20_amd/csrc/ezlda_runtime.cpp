@@ -1289,15 +1289,14 @@ int ezlda_wt_rowsum(ezlda_ctx *c) try {
 // events that bracket the stages.
 static int enqueue_sweep(ezlda_ctx *c, hipEvent_t *ev) {
     if (ev) EZ_TRY_HIP(c, hipEventRecord(ev[0], c->st));
-    EZ_TRY_HIP(c, ez::launch_build_wt(c->s, c->st));
+    EZ_TRY_HIP(c, ez::launch_begin_sweep(c->s, c->st));
     if (ev) EZ_TRY_HIP(c, hipEventRecord(ev[1], c->st));
     EZ_TRY_HIP(c, ez::launch_topk(c->s, c->st));
     if (ev) EZ_TRY_HIP(c, hipEventRecord(ev[2], c->st));
     EZ_TRY_HIP(c, ez::launch_build_dt(c->s, c->st));
     if (ev) EZ_TRY_HIP(c, hipEventRecord(ev[3], c->st));
-    EZ_TRY_HIP(c, ez::launch_sample(c->s, c->a.shortcut != 0, c->st));
+    EZ_TRY_HIP(c, ez::launch_sample(c->s, c->a.shortcut != 0, c->st, ez::kSampleHead | ez::kSampleTail, true));
     if (ev) EZ_TRY_HIP(c, hipEventRecord(ev[4], c->st));
-    EZ_TRY_HIP(c, ez::launch_advance_sweep(c->s, c->st));
     return EZLDA_OK;
 }
 
