@@ -47,6 +47,7 @@ struct DevState {
     uint32_t *tail_nnz = nullptr;   // V-VD
     int32_t *nk = nullptr;          // K
     float *inv = nullptr;           // K: 1/(n_k + V beta)
+    double *inv64 = nullptr;        // K: the same in FP64 (log-likelihood)
     ushort4 *wtop = nullptr;        // V: k1, k2, k3 (0xFFFF = none)
     uint32_t *zero_order = nullptr; // K: topics by beta * inv, largest first (tail words' zero counts)
     // work items

@@ -48,8 +48,9 @@ struct ezlda_ctx {
     std::vector<uint32_t> slot_tok;  // N: slot -> token id
     std::vector<uint32_t> row_off;   // D: DT row offset of doc q (the runs carry it)
     // readback of the topics (ezlda_get_topics): pinned slots, one a host
-    // thread, with the event of each slot's last kernel
-    uint16_t *read_buf = nullptr;
+    // thread, with the event of each slot's last kernel; one device buffer
+    // where the corpus is no longer than a slot
+    uint16_t *read_buf = nullptr, *read_dev = nullptr;
     std::vector<hipEvent_t> read_ev;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;

@@ -284,9 +284,13 @@ __global__ void __launch_bounds__(256) k_wt_all(int nb_hist, int nb_head, const 
 }
 
 // ----------------------------------------------------- inv and top-3
-__global__ void k_inv(const int32_t *__restrict__ nk, int K, float vbeta, float *__restrict__ inv) {
+// inv, and the same in FP64 (vbeta64) for the log-likelihood
+__global__ void k_inv(const int32_t *__restrict__ nk, int K, float vbeta, double vbeta64, float *__restrict__ inv,
+                      double *__restrict__ inv64) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < K) inv[k] = 1.0f / ((float)nk[k] + vbeta);
+    if (k >= K) return;
+    inv[k] = 1.0f / ((float)nk[k] + vbeta);
+    inv64[k] = 1.0 / ((double)nk[k] + vbeta64);
 }
 
 struct Top3 {
@@ -328,8 +332,9 @@ __device__ __forceinline__ void top3_insert(Top3 &t, float v, uint32_t k) {
 // only its own 64 need the tie test.  Bound by its K^2 compares: 20 -> 5.7 us at
 // K = 1024, 176 -> 19 us at K = 10000 (four wavefronts, a scalar read and the
 // tie test for each, inv from a launch before it).
-__global__ void __launch_bounds__(1024) k_inv_order(const int32_t *__restrict__ nk, int K, float vbeta, float beta,
-                                                    float *__restrict__ inv, uint32_t *__restrict__ zero_order) {
+__global__ void __launch_bounds__(1024) k_inv_order(const int32_t *__restrict__ nk, int K, float vbeta, double vbeta64,
+                                                    float beta, float *__restrict__ inv, double *__restrict__ inv64,
+                                                    uint32_t *__restrict__ zero_order) {
     extern __shared__ float sv[];  // K values padded to whole groups of 4, then 64 ranks
     const int KG = (K + 3) >> 2;
     uint32_t *rank = reinterpret_cast<uint32_t *>(sv + 4 * KG);
@@ -339,7 +344,10 @@ __global__ void __launch_bounds__(1024) k_inv_order(const int32_t *__restrict__ 
         if (k < K) {
             const float iv = 1.0f / ((float)nk[k] + vbeta);
             v = beta * iv;
-            if (k >= own && k < own + 64) inv[k] = iv;
+            if (k >= own && k < own + 64) {
+                inv[k] = iv;
+                inv64[k] = 1.0 / ((double)nk[k] + vbeta64);
+            }
         }
         sv[k] = v;
     }
@@ -1381,100 +1389,143 @@ __global__ void __launch_bounds__(1024) k_sample(const SampleArgs A) {
 // per token, the term of profilePerp/utility.cu:2398,2810 reduced in FP64
 // (profilePerp/utility.cu:2858-2928).  One workgroup per sampler item (phi_w
 // in FP64 in LDS), one lane per run; the per-item partials are summed in
-// fixed order by k_ll_final.
-__global__ void __launch_bounds__(1024) k_ll(const uint4 *__restrict__ segs, const uint4 *__restrict__ runs, int VD,
+// fixed order by k_ll_final.  Bound by the latencies of an item (most have
+// fewer than 64 runs: workgroups are as small as the LDS lets a CU hold 12
+// wavefronts of) and by the row scan: 9.9M tokens at K = 1024 1.40 -> 0.67 ms
+// (256 threads an item, an FP64 division a phi, one 16-byte load of the row in
+// flight).  Workgroups with further items keep beta * inv64 in phi between
+// tail words, so such a word stages only its nonzeros.
+template <bool COMPACT>
+__global__ void __launch_bounds__(1024) k_ll(uint32_t n_items, const uint4 *__restrict__ segs, const uint4 *__restrict__ runs, int VD,
                                              int K, double alpha, double beta,
-                                             double vbeta, const int32_t *__restrict__ wt_head,
+                                             const int32_t *__restrict__ wt_head,
                                              const uint32_t *__restrict__ tail_off,
                                              const uint32_t *__restrict__ wt_tail,
-                                             const uint32_t *__restrict__ tail_nnz, const int32_t *__restrict__ nk,
+                                             const uint32_t *__restrict__ tail_nnz, const double *__restrict__ inv64,
                                              const uint32_t *__restrict__ aux_doc, const uint32_t *__restrict__ dt,
-                                             int compact, uint32_t tb, double *__restrict__ part) {
+                                             uint32_t tb, double *__restrict__ part) {
     extern __shared__ double smd[];
     __shared__ double red[16];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
     double *phi = smd;
-    const uint4 sg = segs[blockIdx.x];
-    if (sg.x == 0xFFFFFFFFu) {  // padding item
-        if (tid == 0) part[blockIdx.x] = 0.0;
-        return;
-    }
-    const int w = (int)sg.x;
-    if (w < VD) {
-        const int32_t *row = wt_head + (size_t)w * K;
-        for (int k = tid; k < K; k += blockDim.x) phi[k] = ((double)row[k] + beta) / ((double)nk[k] + vbeta);
-    } else {
-        for (int k = tid; k < K; k += blockDim.x) phi[k] = beta / ((double)nk[k] + vbeta);
+    // sum over the workgroup, in wavefront order
+    auto block_total = [&](double v) {
+        for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
+        if (nwv == 1) return v;
+        __syncthreads();  // the previous total is read
+        if (lane == 0) red[wv] = v;
         __syncthreads();
-        const int tw = w - VD;
-        const uint32_t b = tail_off[tw], n = tail_nnz[tw];
-        for (uint32_t i = tid; i < n; i += blockDim.x) {
-            const uint32_t e = wt_tail[b + i];
-            const uint32_t k = e & 0xFFFFu;
-            phi[k] = ((double)(e >> 16) + beta) / ((double)nk[k] + vbeta);
+        v = 0.0;
+        for (int i = 0; i < nwv; ++i) v += red[i];
+        return v;
+    };
+    bool base = false;  // phi holds beta * inv64, their sum in qbase
+    double qbase = 0.0;
+    for (uint32_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+        const uint4 sg = segs[item];
+        if (sg.x == 0xFFFFFFFFu) {  // padding item
+            if (tid == 0) part[item] = 0.0;
+            continue;
         }
-    }
-    __syncthreads();
-    double q = 0.0;
-    for (int k = tid; k < K; k += blockDim.x) q += phi[k];
-    for (int off = 32; off >= 1; off >>= 1) q += __shfl_xor(q, off);
-    if (lane == 0) red[wv] = q;
-    __syncthreads();
-    q = 0.0;
-    for (int i = 0; i < nwv; ++i) q += red[i];
-    q *= alpha;
-    __syncthreads();
-    // one lane per run (a word's tokens in one doc share the term): its DT
-    // row in 16-byte loads (rows are 128-byte aligned and zero padded; a zero
-    // entry adds nothing)
-    double acc = 0.0;
-    const double kalpha = (double)K * alpha;
-    const uint32_t tmask = (1u << tb) - 1u;
-    for (uint32_t r = sg.y + (uint32_t)tid; r < sg.z; r += (uint32_t)blockDim.x) {
-        const uint4 rn = runs[r];
-        const uint2 di = make_uint2(rn.z, aux_doc[rn.y] >> 16);  // row offset, nnz
-        const uint32_t nnz = di.y & 0xFFFFu;
-        double s = 0.0;
-        if (compact) {
-            const uint4 *rp = reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(dt) + di.x);
-            for (uint32_t i = 0; i < (nnz + 7u) / 8u; ++i) {
-                const uint4 v = rp[i];
-                const uint32_t e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const uint32_t a = e[u] & 0xFFFFu, b = e[u] >> 16;
-                    s += (double)(a >> tb) * phi[a & tmask];
-                    s += (double)(b >> tb) * phi[b & tmask];
-                }
+        const int w = (int)sg.x;
+        uint32_t tb0 = 0, tn = 0;
+        double q = 0.0;
+        if (w < VD) {
+            const int32_t *row = wt_head + (size_t)w * K;
+            for (int k = tid; k < K; k += blockDim.x) {
+                const double v = ((double)row[k] + beta) * inv64[k];
+                phi[k] = v;
+                q += v;
             }
+            q = block_total(q);
+            base = false;
         } else {
-            const uint4 *rp = reinterpret_cast<const uint4 *>(dt + di.x);
-            for (uint32_t i = 0; i < (nnz + 3u) / 4u; ++i) {
-                const uint4 v = rp[i];
-                const uint32_t e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u) s += (double)(e[u] >> 16) * phi[dt_topic(e[u])];
+            if (!base) {
+                qbase = 0.0;
+                for (int k = tid; k < K; k += blockDim.x) {
+                    const double v = beta * inv64[k];
+                    phi[k] = v;
+                    qbase += v;
+                }
+                qbase = block_total(qbase);
+                base = true;
+                __syncthreads();
+            }
+            tb0 = tail_off[w - VD];
+            tn = tail_nnz[w - VD];
+            for (uint32_t i = tid; i < tn; i += blockDim.x) {
+                const uint32_t e = wt_tail[tb0 + i], k = e & 0xFFFFu;
+                const double c = (double)(e >> 16), iv = inv64[k];
+                phi[k] = (c + beta) * iv;
+                q += c * iv;
+            }
+            q = qbase + block_total(q);
+        }
+        q *= alpha;
+        __syncthreads();
+        // one lane per run (a word's tokens in one doc share the term): its DT
+        // row in blocks of kBlkU4 16-byte loads, the next one loaded while one is
+        // summed (rows are 128-byte aligned and zero padded; a zero entry adds
+        // nothing)
+        double acc = 0.0;
+        const double kalpha = (double)K * alpha;
+        const uint32_t tmask = (1u << tb) - 1u;
+        for (uint32_t r = sg.y + (uint32_t)tid; r < sg.z; r += (uint32_t)blockDim.x) {
+            const uint4 rn = runs[r];
+            const uint2 di = make_uint2(rn.z, aux_doc[rn.y] >> 16);  // row offset, nnz
+            const uint32_t nnz = di.y & 0xFFFFu;
+            const uint4 *rp = COMPACT ? reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(dt) + di.x)
+                                      : reinterpret_cast<const uint4 *>(dt + di.x);
+            constexpr uint32_t kEPB = (COMPACT ? 8u : 4u) * kBlkU4;  // entries per block
+            const uint32_t nb = (nnz + kEPB - 1u) / kEPB;
+            double s = 0.0;
+            RowBlock cur = load_block(rp);
+            for (uint32_t b = 0; b < nb; ++b) {
+                RowBlock nxt;
+                if (b + 1u < nb) nxt = load_block(rp + kBlkU4 * (b + 1u));
+    #pragma unroll
+                for (int i = 0; i < kBlkU4; ++i) {
+                    const uint4 v = cur.e[i];
+                    const uint32_t e[4] = {v.x, v.y, v.z, v.w};
+    #pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        if (COMPACT) {
+                            const uint32_t x = e[u] & 0xFFFFu, y = e[u] >> 16;
+                            s = __builtin_fma((double)(x >> tb), phi[x & tmask], s);
+                            s = __builtin_fma((double)(y >> tb), phi[y & tmask], s);
+                        } else {
+                            s = __builtin_fma((double)(e[u] >> 16), phi[dt_topic(e[u])], s);
+                        }
+                    }
+                }
+                cur = nxt;
+            }
+            acc += (double)(rn.w & 0xFFFFu) * log((s + q) / ((double)(rn.w >> 16) + kalpha));
+        }
+        acc = block_total(acc);
+        if (tid == 0) part[item] = acc;
+        if (w >= VD && item + gridDim.x < n_items) {  // the base again (every lane is past its reads of phi)
+            for (uint32_t i = tid; i < tn; i += blockDim.x) {
+                const uint32_t k = wt_tail[tb0 + i] & 0xFFFFu;
+                phi[k] = beta * inv64[k];
             }
         }
-        acc += (double)(rn.w & 0xFFFFu) * log((s + q) / ((double)(rn.w >> 16) + kalpha));
-    }
-    for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
-    if (lane == 0) red[wv] = acc;
-    __syncthreads();
-    if (tid == 0) {
-        double tot = 0.0;
-        for (int i = 0; i < nwv; ++i) tot += red[i];
-        part[blockIdx.x] = tot;
+        __syncthreads();  // the next item's phi
     }
 }
 
-__global__ void k_ll_final(const double *__restrict__ part, int n, double *__restrict__ out) {
-    __shared__ double red[256];
-    double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += part[i];
-    red[threadIdx.x] = s;
+// One workgroup of 1024 threads, eight partials in flight a thread (one by
+// one in 256 threads: 101 us for 140,000 partials, 16 now).
+__global__ void __launch_bounds__(1024) k_ll_final(const double *__restrict__ part, int n, double *__restrict__ out) {
+    __shared__ double red[1024];
+    double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int i = threadIdx.x; i < n; i += 8 * 1024) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s[u] += i + 1024 * u < n ? part[i + 1024 * u] : 0.0;
+    }
+    red[threadIdx.x] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     __syncthreads();
-    for (int h = blockDim.x / 2; h > 0; h >>= 1) {
+    for (int h = 512; h > 0; h >>= 1) {
         if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
         __syncthreads();
     }
@@ -2565,10 +2616,11 @@ hipError_t launch_topic_hist(const DevState &s, hipStream_t st) {
 hipError_t launch_topk(const DevState &s, hipStream_t st) {
     if (s.V > s.VD)
         hipLaunchKernelGGL(k_inv_order, dim3(grid_for(s.K, 64, 1 << 16)), dim3(1024),
-                           ((size_t)((s.K + 3) & ~3) + 64) * sizeof(float), st, s.nk, s.K, s.vbeta, s.beta, s.inv,
-                           s.zero_order);
+                           ((size_t)((s.K + 3) & ~3) + 64) * sizeof(float), st, s.nk, s.K, s.vbeta,
+                           (double)s.V * (double)s.beta, s.beta, s.inv, s.inv64, s.zero_order);
     else
-        hipLaunchKernelGGL(k_inv, dim3(grid_for(s.K, 256, 1 << 16)), dim3(256), 0, st, s.nk, s.K, s.vbeta, s.inv);
+        hipLaunchKernelGGL(k_inv, dim3(grid_for(s.K, 256, 1 << 16)), dim3(256), 0, st, s.nk, s.K, s.vbeta,
+                           (double)s.V * (double)s.beta, s.inv, s.inv64);
     if (s.V > 0) {
         const size_t lds = s.V > s.VD ? 4 * (size_t)((s.K + 31) >> 5) * sizeof(uint32_t) : 0;
         hipLaunchKernelGGL(k_word_top, dim3(grid_for((size_t)s.V, 4, 1 << 16)), dim3(256), lds, st, s.V, s.VD, s.K,
@@ -2708,16 +2760,28 @@ hipError_t launch_advance_sweep(const DevState &s, hipStream_t st) {
 }
 
 hipError_t launch_loglik(const DevState &s, hipStream_t st) {
-    if (s.n_smp_segs == 0) {
-        hipLaunchKernelGGL(k_ll_final, dim3(1), dim3(256), 0, st, s.ll_part, 0, s.ll_out);
-        return hipGetLastError();
+    if (s.n_smp_segs > 0) {
+        const size_t lds = (size_t)s.K * sizeof(double);
+        const int fit = std::max(1, (int)((size_t)s.lds_cu / (lds + 16 * sizeof(double))));
+        int bd = 64;
+        while (bd < 1024 && fit * (bd / 64) < 12) bd *= 2;
+        // K > 4096: as many workgroups as the CUs hold (at most 16 wavefronts
+        // each; a multiple of 8, so that an item stays on the XCD it was dealt
+        // to), so that most tail words find the base phi in LDS (K = 10000,
+        // 4.5M tokens: 1.30 -> 1.08 ms).  Below, a workgroup an item, which
+        // the dispatcher balances (K = 2048, heavy-tailed documents: 2.92
+        // against 3.65 ms; K = 1024: 0.81 against 0.88).
+        const int per_cu = std::max(1, std::min(fit, 16 / (bd / 64)));
+        const int grid = s.K > 4096 ? std::min(s.n_smp_segs, std::max(8, s.n_cu * per_cu / 8 * 8)) : s.n_smp_segs;
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(bd), lds, st, (uint32_t)s.n_smp_segs, s.smp_segs, s.runs, s.VD, s.K,
+                               (double)s.alpha, (double)s.beta, s.wt_head, s.tail_off, s.wt_tail, s.tail_nnz,
+                               s.inv64, s.aux_doc, s.dt, s.topic_bits, s.ll_part);
+        };
+        if (s.compact) go(k_ll<true>);
+        else go(k_ll<false>);
     }
-    const int bd = 256;
-    hipLaunchKernelGGL(k_ll, dim3(s.n_smp_segs), dim3(bd), (size_t)s.K * sizeof(double), st, s.smp_segs, s.runs, s.VD,
-                       s.K,
-                       (double)s.alpha, (double)s.beta, (double)s.V * (double)s.beta, s.wt_head, s.tail_off,
-                       s.wt_tail, s.tail_nnz, s.nk, s.aux_doc, s.dt, (int)s.compact, s.topic_bits, s.ll_part);
-    hipLaunchKernelGGL(k_ll_final, dim3(1), dim3(256), 0, st, s.ll_part, s.n_smp_segs, s.ll_out);
+    hipLaunchKernelGGL(k_ll_final, dim3(1), dim3(1024), 0, st, s.ll_part, std::max(s.n_smp_segs, 0), s.ll_out);
     return hipGetLastError();
 }
 

@@ -223,6 +223,7 @@ void free_device(ezlda_ctx *c) {
     c->s = ez::DevState{};
     if (c->read_buf) (void)hipHostFree(c->read_buf);
     c->read_buf = nullptr;
+    c->read_dev = nullptr;
     for (hipEvent_t e : c->read_ev) (void)hipEventDestroy(e);
     c->read_ev.clear();
     for (EzChunk &ch : c->chunks)
@@ -259,10 +260,10 @@ int lupload(ezlda_ctx *c, T **p, const std::vector<T> &v) {
 }
 
 int alloc_readback(ezlda_ctx *c, uint32_t N) {
-    const uint32_t slots = std::min<uint32_t>((uint32_t)std::min<int>(host_threads(), (int)kReadSlots),
-                                              (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens));
-    if (!slots) return EZLDA_OK;
-    EZ_TRY_HIP(c, hipHostMalloc((void **)&c->read_buf, (size_t)slots * std::min(N, kReadTokens) * sizeof(uint16_t),
+    const uint32_t pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
+    if (pieces <= 1) return dalloc(c, &c->read_dev, N);  // copied as it is: no pinned memory to set up
+    const uint32_t slots = std::min(pieces, std::min((uint32_t)host_threads(), kReadSlots));
+    EZ_TRY_HIP(c, hipHostMalloc((void **)&c->read_buf, (size_t)slots * kReadTokens * sizeof(uint16_t),
                                 hipHostMallocDefault));
     c->read_ev.reserve(slots);
     for (uint32_t i = 0; i < slots; ++i) {
@@ -716,6 +717,7 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
     if ((r = dalloc(c, &s.nk, K))) return r;
     if ((r = dalloc(c, &c->nk_next, K))) return r;
     if ((r = dalloc(c, &s.inv, K))) return r;
+    if ((r = dalloc(c, &s.inv64, K))) return r;
     if ((r = dalloc(c, &s.wtop, V))) return r;
     if ((r = dalloc(c, &s.zero_order, K))) return r;
     if ((r = dalloc(c, &s.tail_off, 1))) return r;
@@ -1144,6 +1146,7 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
     EZ_TRY_HIP(c, hipMemset(s.dt, 0, dt_words * sizeof(uint32_t)));
     if ((r = dalloc(c, &s.nk, K))) return r;
     if ((r = dalloc(c, &s.inv, K))) return r;
+    if ((r = dalloc(c, &s.inv64, K))) return r;
     if ((r = dalloc(c, &s.wtop, V))) return r;
     if ((r = dalloc(c, &s.zero_order, K))) return r;
     if ((r = dalloc(c, &s.counters, ez::kCounterWords))) return r;
@@ -1680,6 +1683,13 @@ namespace {
 // that could not be started leaves its pieces to the others).
 int read_topics(ezlda_ctx *c, uint16_t *zout) {
     const uint32_t N = c->s.N, n_pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
+    if (n_pieces <= 1) {
+        if (!N) return EZLDA_OK;
+        EZ_TRY_HIP(c, ez::launch_topics_out(c->s, 0, N, c->read_dev, c->st));
+        EZ_TRY_HIP(c, hipMemcpyAsync(zout, c->read_dev, (size_t)N * sizeof(uint16_t), hipMemcpyDeviceToHost, c->st));
+        EZ_TRY_HIP(c, hipStreamSynchronize(c->st));
+        return EZLDA_OK;
+    }
     int dev = 0;
     EZ_TRY_HIP(c, hipGetDevice(&dev));
     std::atomic<uint32_t> next{0};
@@ -1711,7 +1721,7 @@ int read_topics(ezlda_ctx *c, uint16_t *zout) {
         for (size_t k = 1; k < c->read_ev.size(); ++k) th.emplace_back(work, k);
     } catch (const std::system_error &) {
     }
-    if (N) work(0);
+    work(0);
     for (auto &x : th) x.join();
     if (failed != (int)hipSuccess)
         return fail(c, EZLDA_EHIP, std::string("reading the topics: ") + hipGetErrorString((hipError_t)failed.load()));
