@@ -1006,6 +1006,56 @@ struct SampleArgs {
     uint32_t mode;  // kSampleHead | kSampleTail: which words' items; | kShortcutOnly: no full draws
 };
 
+// phi (scaled by `up`) of a word's dense counts (COUNTS), or of no counts, into
+// LDS, zero past K up to whole slabs.  Every lane has four 16-byte loads of
+// each input in flight (eight scalar ones where K is no multiple of 4): one
+// load at a time was a chain of K / blockDim latencies an item.  Sampler ms a
+// sweep: 4.5M tokens K = 10000 1.36 -> 1.11, 9M K = 4096 0.84 -> 0.70, heavy-
+// tailed K = 2048 1.71 -> 1.57, 49.5M K = 1024 2.90 -> 2.87.
+template <bool COUNTS>
+__device__ __forceinline__ void stage_phi(float *phi, const int32_t *__restrict__ row, const float *__restrict__ inv,
+                                          int K, int NS, float beta, float up) {
+    const int tid = threadIdx.x, bd = blockDim.x;
+    auto value = [&](int32_t c, float iv) { return COUNTS ? ((float)c + beta) * iv * up : beta * iv * up; };
+    if ((K & 3) == 0) {
+        const int n4 = NS * 16, K4 = K >> 2;
+        const int4 *row4 = reinterpret_cast<const int4 *>(row);
+        const float4 *inv4 = reinterpret_cast<const float4 *>(inv);
+        float4 *phi4 = reinterpret_cast<float4 *>(phi);
+        for (int k0 = tid; k0 < n4; k0 += 4 * bd) {
+            int4 c[4];
+            float4 iv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = k0 + u * bd;
+                c[u] = COUNTS && k < K4 ? row4[k] : make_int4(0, 0, 0, 0);
+                iv[u] = k < K4 ? inv4[k] : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = k0 + u * bd;
+                if (k < n4)
+                    phi4[k] = make_float4(value(c[u].x, iv[u].x), value(c[u].y, iv[u].y), value(c[u].z, iv[u].z),
+                                          value(c[u].w, iv[u].w));
+            }
+        }
+    } else {
+        for (int k0 = tid; k0 < NS * 64; k0 += 8 * bd) {
+            int32_t c[8];
+            float iv[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int k = k0 + u * bd;
+                c[u] = COUNTS && k < K ? row[k] : 0;
+                iv[u] = k < K ? inv[k] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (k0 + u * bd < NS * 64) phi[k0 + u * bd] = value(c[u], iv[u]);
+        }
+    }
+}
+
 template <bool SHORTCUT, bool COMPACT, bool QTAB>
 __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, float *smf, float *f123,
                                             uint32_t sweep, uint32_t &n_full, uint32_t &n_scanned) {
@@ -1027,17 +1077,23 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
     const ushort4 tp = A.wtop[w];
 
     if (w < A.VD) {
-        const int32_t *row = A.wt_head + (size_t)w * K;
-        for (int k = tid; k < NS * 64; k += blockDim.x) phi[k] = k < K ? ((float)row[k] + beta) * A.inv[k] * up : 0.0f;
+        stage_phi<true>(phi, A.wt_head + (size_t)w * K, A.inv, K, NS, beta, up);
     } else {
-        for (int k = tid; k < NS * 64; k += blockDim.x) phi[k] = k < K ? beta * A.inv[k] * up : 0.0f;
-        __syncthreads();
+        // the word's row is on its way while the topics without a count are staged
         const int tw = w - A.VD;
         const uint32_t b = A.tail_off[tw], n = A.tail_nnz[tw];
-        for (uint32_t i = tid; i < n; i += blockDim.x) {
-            const uint32_t e = A.wt_tail[b + i];
-            const uint32_t k = e & 0xFFFFu;
-            phi[k] = ((float)(e >> 16) + beta) * A.inv[k] * up;
+        stage_phi<false>(phi, nullptr, A.inv, K, NS, beta, up);
+        __syncthreads();
+        for (uint32_t i0 = tid; i0 < n; i0 += 4u * blockDim.x) {
+            uint32_t e[4];
+            float iv[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) e[u] = i0 + u * blockDim.x < n ? A.wt_tail[b + i0 + u * blockDim.x] : 0u;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) iv[u] = A.inv[e[u] & 0xFFFFu];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+                if (i0 + u * blockDim.x < n) phi[e[u] & 0xFFFFu] = ((float)(e[u] >> 16) + beta) * iv[u] * up;
         }
     }
     __syncthreads();
@@ -1080,12 +1136,12 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
     __syncthreads();
     if (tid == 0) {
         float acc = 0.0f;
-        for (int j0 = 0; j0 < NS; j0 += 8) {
-            float v[8];
+        for (int j0 = 0; j0 < NS; j0 += 16) {
+            float v[16];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = j0 + i < NS ? qt[j0 + i] : 0.0f;
+            for (int i = 0; i < 16; ++i) v[i] = j0 + i < NS ? qt[j0 + i] : 0.0f;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
+            for (int i = 0; i < 16; ++i) {
                 if (j0 + i < NS) {
                     acc = acc + v[i];
                     qacc[j0 + i] = acc;
