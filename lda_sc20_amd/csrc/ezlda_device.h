@@ -16,6 +16,13 @@ static constexpr int kCounterWords = kQueueStride * 9;
 // sorting their topics (large K); longer ones use a K-sized histogram.
 static constexpr uint32_t kDtShort = 512;
 
+// A sampler item may be a group of up to kGroupMax consecutive words of few
+// tokens (K <= kGroupMaxK, one-wavefront workgroups): the first word in the
+// low bits of its record, the number of further words above them; a run then
+// carries its word's place in the group.
+static constexpr uint32_t kGroupShift = 26, kGroupWord = (1u << kGroupShift) - 1u, kGroupMax = 32;
+static constexpr int kGroupMaxK = 512;
+
 // Device image of one corpus + model.  Token ids are word-major positions;
 // N < 2^32.  Sizes: V words, VD head words, D docs, K topics.
 struct DevState {
@@ -53,9 +60,11 @@ struct DevState {
     // work items
     uint4 *wt_segs = nullptr;       // head-word histogram segments (w, beg, end)
     int32_t n_wt_segs = 0;
-    uint4 *smp_segs = nullptr;      // sampler items (w, first run, end run, draw-key offset)
+    uint4 *smp_segs = nullptr;      // sampler items (w | further words << kGroupShift, first run, end run,
+                                    // draw-key offset)
     int32_t n_smp_segs = 0;
-    uint4 *runs = nullptr;          // (first token, first slot, doc's DT row offset, tokens | doc length << 16):
+    int32_t group_words = 1;        // words of the largest group item
+    uint4 *runs = nullptr;          // (first token, first slot, doc's DT row offset, tokens | group place << 8 | doc length << 16):
                                     // a word's tokens in one doc
     int64_t n_runs = 0;
     int32_t n_queues = 1;           // persistent sampler: item queues (<= 8)
@@ -155,6 +164,8 @@ hipError_t launch_foldin_step(const FoldinBatch &fb, const uint4 *slots, const u
                               float alpha, const float *phi, const float *qs, const float *qacc,
                               const uint32_t *wpool, uint16_t *zpool, uint64_t seed, hipStream_t st);
 
+// LDS floats of one word of a group item at K topics.
+int group_stride(int K);
 // Bytes of dynamic LDS the sampler needs for K topics and block size bd.
 size_t sample_lds_bytes(int K, int bd);
 // Static LDS of the sampler kernels: must be 0 (phi is read at LDS address

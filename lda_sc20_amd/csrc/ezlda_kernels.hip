@@ -10,6 +10,8 @@
 // (wt_tail, word_top); in the sampler one lane owns a token.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "ezlda_device.h"
 #include "ezlda_philox.h"
 
@@ -829,10 +831,13 @@ __global__ void __launch_bounds__(256) k_dt_sort(int q0, int q1, int VD, uint32_
 // CP-th took most of the sampler on heavy-tailed documents (8.9M tokens of
 // up to 20,000 a document at K = 2048: 2.63 -> 1.67 ms a sweep with 8 + 8,
 // 1.72 with 9 + 6, 1.78 with 12 + 4; 49.5M tokens at K = 1024 2.92 -> 2.90
-// with 12 + 4, 2.92 with 9 + 6).  The counts are what fits 128 registers.
-template <bool COMPACT, bool QTAB>
+// with 12 + 4, 2.92 with 9 + 6).  The counts are what fits 128 registers
+// (MULTI, whose lanes each have their own word's values: 6 + 2, rows at most 512
+// topics).
+template <bool COMPACT, bool QTAB, bool MULTI>
 struct Checkpoints {
-    static constexpr int CP = !QTAB && COMPACT ? 8 : EZ_SAMPLE_CP, CF = !QTAB && COMPACT ? 8 : 4;
+    static constexpr int CP = MULTI ? 6 : !QTAB && COMPACT ? 8 : EZ_SAMPLE_CP;
+    static constexpr int CF = MULTI ? 2 : !QTAB && COMPACT ? 8 : 4;
 };
 static constexpr int kBlkU4 = EZ_SAMPLE_BLK;
 #ifndef EZ_SAMPLE_HALF_CP
@@ -886,10 +891,24 @@ __device__ __forceinline__ uint32_t lo16_times4(uint32_t t) {
         : "v"(2u), "v"(t));
     return r;
 }
-__device__ __forceinline__ C16x2 c16_x2(uint32_t w, uint32_t tb, uint32_t tm2) {
+// topic * 4 + base of the low / high half of t in one operation
+__device__ __forceinline__ uint32_t lo16_times4_plus(uint32_t t, uint32_t base) {
+    uint32_t r;
+    asm("v_mad_u32_u16 %0, %1, 4, %2" : "=v"(r) : "v"(t), "v"(base));
+    return r;
+}
+__device__ __forceinline__ uint32_t hi16_times4_plus(uint32_t t, uint32_t base) {
+    uint32_t r;
+    asm("v_mad_u32_u16 %0, %1, 4, %2 op_sel:[1,0,0,0]" : "=v"(r) : "v"(t), "v"(base));
+    return r;
+}
+// MULTI: the lane's phi table starts at LDS address lb (else at 0)
+template <bool MULTI>
+__device__ __forceinline__ C16x2 c16_x2(uint32_t w, uint32_t tb, uint32_t tm2, uint32_t lb) {
     const ez_us2 c = __builtin_bit_cast(ez_us2, w) >> (ez_us2)((unsigned short)tb);
     const ez_h2 h = __builtin_bit_cast(ez_h2, c);
     const uint32_t t = w & tm2;
+    if (MULTI) return C16x2{h.x, h.y, lo16_times4_plus(t, lb), hi16_times4_plus(t, lb)};
     return C16x2{h.x, h.y, lo16_times4(t), (t >> 16) << 2};
 }
 // s + count * phi in one rounding (v_fma_mix_f32)
@@ -897,14 +916,14 @@ __device__ __forceinline__ float fma_count(_Float16 c, float phi, float s) { ret
 __device__ __forceinline__ float phi_a(uint32_t a) { return *(lds_cfloat *)a; }
 
 // The entries of one 16-byte load, in order.
-template <bool COMPACT>
-__device__ __forceinline__ float sum_u4(const uint4 &e, float s, uint32_t tb) {
+template <bool COMPACT, bool MULTI>
+__device__ __forceinline__ float sum_u4(const uint4 &e, float s, uint32_t tb, uint32_t lb) {
     if (COMPACT) {  // two 16-bit entries per dword, low half first
         const uint32_t w[4] = {e.x, e.y, e.z, e.w};
         const uint32_t tm2 = ((1u << tb) - 1u) * 0x10001u;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const C16x2 d = c16_x2(w[q], tb, tm2);
+            const C16x2 d = c16_x2<MULTI>(w[q], tb, tm2, lb);
             s = fma_count(d.c0, phi_a(d.a0), s);
             s = fma_count(d.c1, phi_a(d.a1), s);
         }
@@ -919,11 +938,12 @@ __device__ __forceinline__ float sum_u4(const uint4 &e, float s, uint32_t tb) {
 
 // The block's entries in order; `half` gets the running sum after its
 // first kBlkU4 / 2 loads.
-template <bool COMPACT>
-__device__ __forceinline__ float sum_block(const RowBlock &r, float s, uint32_t tb, float &half) {
+template <bool COMPACT, bool MULTI>
+__device__ __forceinline__ float sum_block(const RowBlock &r, float s, uint32_t tb, uint32_t lb,
+                                           float &half) {
 #pragma unroll
     for (int i = 0; i < kBlkU4; ++i) {
-        s = sum_u4<COMPACT>(r.e[i], s, tb);
+        s = sum_u4<COMPACT, MULTI>(r.e[i], s, tb, lb);
         if (i == kBlkU4 / 2 - 1) half = s;
     }
     return s;
@@ -932,9 +952,9 @@ __device__ __forceinline__ float sum_block(const RowBlock &r, float s, uint32_t 
 // S-bucket search over n consecutive 16-byte pieces of a row from running
 // sum `run`: the first entry whose running sum exceeds t2 (running sums never
 // decrease).
-template <bool COMPACT, int N>
-__device__ __forceinline__ void search_u4(const uint4 (&blk)[N], float &run, float t2, uint32_t tb, uint32_t &newz,
-                                          bool &found) {
+template <bool COMPACT, bool MULTI, int N>
+__device__ __forceinline__ void search_u4(const uint4 (&blk)[N], float &run, float t2, uint32_t tb, uint32_t lb,
+                                          uint32_t &newz, bool &found) {
 #pragma unroll
     for (int gi = 0; gi < N; ++gi) {
         const uint4 e = blk[gi];
@@ -943,14 +963,14 @@ __device__ __forceinline__ void search_u4(const uint4 (&blk)[N], float &run, flo
             const uint32_t tm2 = ((1u << tb) - 1u) * 0x10001u;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const C16x2 d = c16_x2(w[q], tb, tm2);
+                const C16x2 d = c16_x2<MULTI>(w[q], tb, tm2, lb);
                 const float ra = fma_count(d.c0, phi_a(d.a0), run);
                 const float rb = fma_count(d.c1, phi_a(d.a1), ra);
                 if (!found && ra > t2) {
-                    newz = d.a0 >> 2;
+                    newz = (d.a0 - (MULTI ? lb : 0u)) >> 2;
                     found = true;
                 } else if (!found && rb > t2) {
-                    newz = d.a1 >> 2;
+                    newz = (d.a1 - (MULTI ? lb : 0u)) >> 2;
                     found = true;
                 }
                 run = rb;
@@ -1004,6 +1024,7 @@ struct SampleArgs {
     unsigned long long *stats;
     uint64_t seed;
     uint32_t mode;  // kSampleHead | kSampleTail: which words' items; | kShortcutOnly: no full draws
+    uint32_t word_stride;  // MULTI: LDS floats of one word's tables
 };
 
 // phi (scaled by `up`) of a word's dense counts (COUNTS), or of no counts, into
@@ -1056,103 +1077,228 @@ __device__ __forceinline__ void stage_phi(float *phi, const int32_t *__restrict_
     }
 }
 
-template <bool SHORTCUT, bool COMPACT, bool QTAB>
+// A group item's tables: G words of few tokens (all dense or all sparse),
+// word g's phi, Q running sums and totals at g * ST, after them f1, f2 and k1.
+// As for one word, but every phase works on all of them at once: small words
+// are a chain of latencies each, and fill few of a wavefront's lanes.
+template <bool COMPACT>
+__device__ __forceinline__ void stage_group(const SampleArgs &A, int w, int G, int ST, float *smf) {
+    const int K = A.K, NS = (K + 63) >> 6, tid = threadIdx.x, bd = blockDim.x;
+    const float alpha = A.alpha, beta = A.beta;
+    constexpr float up = COMPACT ? kPhiUp : 1.0f, down = COMPACT ? kPhiDown : 1.0f;
+    const bool head = w < A.VD;
+    const int32_t *rows = A.wt_head + (size_t)w * K;
+    auto value = [&](int32_t c, float iv) { return ((float)c + beta) * iv * up; };
+    if ((K & 3) == 0) {  // slab s of the group: 16 loads of 4 topics
+        const int n = G * NS * 16;
+        for (int i0 = tid; i0 < n; i0 += 4 * bd) {
+            int4 c[4];
+            float4 iv[4];
+            int at[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = i0 + u * bd, sl = i >> 4, g = sl / NS, k = (sl - g * NS) * 64 + (i & 15) * 4;
+                at[u] = i < n ? g * ST + k : -1;
+                const bool in = i < n && k < K;
+                c[u] = in && head ? *reinterpret_cast<const int4 *>(rows + (size_t)g * K + k) : make_int4(0, 0, 0, 0);
+                iv[u] = in ? *reinterpret_cast<const float4 *>(A.inv + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (at[u] >= 0)
+                    *reinterpret_cast<float4 *>(smf + at[u]) =
+                        make_float4(value(c[u].x, iv[u].x), value(c[u].y, iv[u].y), value(c[u].z, iv[u].z),
+                                    value(c[u].w, iv[u].w));
+        }
+    } else {
+        const int n = G * NS * 64;
+        for (int i0 = tid; i0 < n; i0 += 8 * bd) {
+            int32_t c[8];
+            float iv[8];
+            int at[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int i = i0 + u * bd, sl = i >> 6, g = sl / NS, k = (sl - g * NS) * 64 + (i & 63);
+                at[u] = i < n ? g * ST + k : -1;
+                const bool in = i < n && k < K;
+                c[u] = in && head ? rows[(size_t)g * K + k] : 0;
+                iv[u] = in ? A.inv[k] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (at[u] >= 0) smf[at[u]] = value(c[u], iv[u]);
+        }
+    }
+    __syncthreads();
+    if (!head) {  // four words' nonzeros at a time
+        for (int g0 = 0; g0 < G; g0 += 4) {
+            uint32_t b[4], n[4], most = 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                b[u] = g0 + u < G ? A.tail_off[w - A.VD + g0 + u] : 0u;
+                n[u] = g0 + u < G ? A.tail_nnz[w - A.VD + g0 + u] : 0u;
+                most = max(most, n[u]);
+            }
+            for (uint32_t i = tid; i < most; i += bd) {
+                uint32_t e[4];
+                float iv[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) e[u] = i < n[u] ? A.wt_tail[b[u] + i] : 0u;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) iv[u] = A.inv[e[u] & 0xFFFFu];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (i < n[u]) smf[(g0 + u) * ST + (int)(e[u] & 0xFFFFu)] = value((int32_t)(e[u] >> 16), iv[u]);
+            }
+        }
+        __syncthreads();
+    }
+    const int qo = NS * 64, to = 2 * NS * 64;  // a word's Q running sums, slab totals
+    for (int g = tid; g < G; g += bd) {
+        const ushort4 tp = A.wtop[w + g];
+        float *p = smf + g * ST, *wc = p + to + 2 * NS;
+        wc[0] = p[tp.x] * down;
+        wc[1] = tp.y != kNone ? p[tp.y] * down : 0.0f;
+        wc[2] = __uint_as_float((uint32_t)tp.x);
+        p[tp.x] = 0.0f;
+    }
+    __syncthreads();
+    for (int i = tid; i < G * NS; i += bd) {  // one slab a lane
+        const int g = i / NS, j = i - g * NS;
+        const float4 *p4 = reinterpret_cast<const float4 *>(smf + g * ST + j * 64);
+        float4 *q4 = reinterpret_cast<float4 *>(smf + g * ST + qo + j * 64);
+        float4 v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = p4[u];
+        float run = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            run = run + alpha * (v[u].x * down);
+            v[u].x = run;
+            run = run + alpha * (v[u].y * down);
+            v[u].y = run;
+            run = run + alpha * (v[u].z * down);
+            v[u].z = run;
+            run = run + alpha * (v[u].w * down);
+            v[u].w = run;
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) q4[u] = v[u];
+        smf[g * ST + to + j] = run;
+    }
+    __syncthreads();
+    for (int g = tid; g < G; g += bd) {
+        float acc = 0.0f;
+        float *qt = smf + g * ST + to;
+        for (int j = 0; j < NS; ++j) {
+            acc = acc + qt[j];
+            qt[NS + j] = acc;
+        }
+    }
+    __syncthreads();
+}
+
+template <bool SHORTCUT, bool COMPACT, bool QTAB, bool MULTI>
 __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, float *smf, float *f123,
                                             uint32_t sweep, uint32_t &n_full, uint32_t &n_scanned) {
     const int K = A.K, NS = (K + 63) >> 6;
     const float alpha = A.alpha, beta = A.beta;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
     constexpr bool qtab = QTAB;  // K <= EZ_Q_TABLE_MAX_K
-    constexpr int CP = Checkpoints<COMPACT, QTAB>::CP, CF = Checkpoints<COMPACT, QTAB>::CF;
+    constexpr int CP = Checkpoints<COMPACT, QTAB, MULTI>::CP, CF = Checkpoints<COMPACT, QTAB, MULTI>::CF;
     constexpr float up = COMPACT ? kPhiUp : 1.0f, down = COMPACT ? kPhiDown : 1.0f;
-    float *phi = smf;                         // NS*64
-    float *qs = phi + NS * 64;                // NS*64 when qtab: running sums inside each slab
-    float *qt = qs + (qtab ? NS * 64 : 0);    // NS: slab totals
-    float *qacc = qt + NS;                    // NS: running sum of the slab totals
+    float *phi0 = smf;                         // NS*64
+    float *qs0 = phi0 + NS * 64;                // NS*64 when qtab: running sums inside each slab
+    float *qt0 = qs0 + (qtab ? NS * 64 : 0);    // NS: slab totals
+    float *qacc0 = qt0 + NS;                    // NS: running sum of the slab totals
     const uint4 sg = A.segs[item];
     if (sg.x == 0xFFFFFFFFu) return;  // padding item (uniform over the block)
-    const int w = (int)sg.x;
+    // MULTI: the item's words are w .. w + G - 1, word g's tables at g * ST
+    const uint32_t gw = MULTI ? (uint32_t)__builtin_amdgcn_readfirstlane((int)sg.x) : sg.x;
+    const int w = MULTI ? (int)(gw & kGroupWord) : (int)gw, G = MULTI ? 1 + (int)(gw >> kGroupShift) : 1;
+    const int ST = MULTI ? (int)A.word_stride : 0;
     if (!(A.mode & (w < A.VD ? kSampleHead : kSampleTail))) return;  // the other words' stage
     const bool sc_only = (A.mode & kShortcutOnly) != 0;
-    const ushort4 tp = A.wtop[w];
-
-    if (w < A.VD) {
-        stage_phi<true>(phi, A.wt_head + (size_t)w * K, A.inv, K, NS, beta, up);
+    const ushort4 tp = MULTI ? make_ushort4(0, 0, 0, 0) : A.wtop[w];
+    if (MULTI) {
+        stage_group<COMPACT>(A, w, G, ST, smf);
     } else {
-        // the word's row is on its way while the topics without a count are staged
-        const int tw = w - A.VD;
-        const uint32_t b = A.tail_off[tw], n = A.tail_nnz[tw];
-        stage_phi<false>(phi, nullptr, A.inv, K, NS, beta, up);
+        if (w < A.VD) {
+            stage_phi<true>(phi0, A.wt_head + (size_t)w * K, A.inv, K, NS, beta, up);
+        } else {
+            // the word's row is on its way while the topics without a count are staged
+            const int tw = w - A.VD;
+            const uint32_t b = A.tail_off[tw], n = A.tail_nnz[tw];
+            stage_phi<false>(phi0, nullptr, A.inv, K, NS, beta, up);
+            __syncthreads();
+            for (uint32_t i0 = tid; i0 < n; i0 += 4u * blockDim.x) {
+                uint32_t e[4];
+                float iv[4];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) e[u] = i0 + u * blockDim.x < n ? A.wt_tail[b + i0 + u * blockDim.x] : 0u;
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) iv[u] = A.inv[e[u] & 0xFFFFu];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u)
+                    if (i0 + u * blockDim.x < n) phi0[e[u] & 0xFFFFu] = ((float)(e[u] >> 16) + beta) * iv[u] * up;
+            }
+        }
         __syncthreads();
-        for (uint32_t i0 = tid; i0 < n; i0 += 4u * blockDim.x) {
-            uint32_t e[4];
-            float iv[4];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) e[u] = i0 + u * blockDim.x < n ? A.wt_tail[b + i0 + u * blockDim.x] : 0u;
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) iv[u] = A.inv[e[u] & 0xFFFFu];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u)
-                if (i0 + u * blockDim.x < n) phi[e[u] & 0xFFFFu] = ((float)(e[u] >> 16) + beta) * iv[u] * up;
+        if (tid == 0) {
+            f123[0] = phi0[tp.x] * down;
+            f123[1] = tp.y != kNone ? phi0[tp.y] * down : 0.0f;
+            f123[2] = tp.z != kNone ? phi0[tp.z] * down : 0.0f;
+            phi0[tp.x] = 0.0f;
         }
-    }
-    __syncthreads();
-    if (tid == 0) {
-        f123[0] = phi[tp.x] * down;
-        f123[1] = tp.y != kNone ? phi[tp.y] * down : 0.0f;
-        f123[2] = tp.z != kNone ? phi[tp.z] * down : 0.0f;
-        phi[tp.x] = 0.0f;
-    }
-    __syncthreads();
-    // Q: the running sums inside each 64-topic slab, left to right (phi is 0
-    // past K, which leaves the sum unchanged); the slab's 64 values are
-    // loaded at once, then summed in order.  With qtab the running sums are
-    // kept; else only the slab total, and a Q draw recomputes its slab's
-    // running sums in the same order
-    for (int j = tid; j < NS; j += blockDim.x) {
-        const float4 *p4 = reinterpret_cast<const float4 *>(phi + j * 64);
-        float4 v[16];
+        __syncthreads();
+        // Q: the running sums inside each 64-topic slab, left to right (phi0 is 0
+        // past K, which leaves the sum unchanged); the slab's 64 values are
+        // loaded at once, then summed in order.  With qtab the running sums are
+        // kept; else only the slab total, and a Q draw recomputes its slab's
+        // running sums in the same order
+        for (int j = tid; j < NS; j += blockDim.x) {
+            const float4 *p4 = reinterpret_cast<const float4 *>(phi0 + j * 64);
+            float4 v[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = p4[i];
-        float run = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            run = run + alpha * (v[i].x * down);
-            v[i].x = run;
-            run = run + alpha * (v[i].y * down);
-            v[i].y = run;
-            run = run + alpha * (v[i].z * down);
-            v[i].z = run;
-            run = run + alpha * (v[i].w * down);
-            v[i].w = run;
-        }
-        if (qtab) {
-            float4 *q4 = reinterpret_cast<float4 *>(qs + j * 64);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) q4[i] = v[i];
-        }
-        qt[j] = run;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        float acc = 0.0f;
-        for (int j0 = 0; j0 < NS; j0 += 16) {
-            float v[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = j0 + i < NS ? qt[j0 + i] : 0.0f;
+            for (int i = 0; i < 16; ++i) v[i] = p4[i];
+            float run = 0.0f;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                if (j0 + i < NS) {
-                    acc = acc + v[i];
-                    qacc[j0 + i] = acc;
+                run = run + alpha * (v[i].x * down);
+                v[i].x = run;
+                run = run + alpha * (v[i].y * down);
+                v[i].y = run;
+                run = run + alpha * (v[i].z * down);
+                v[i].z = run;
+                run = run + alpha * (v[i].w * down);
+                v[i].w = run;
+            }
+            if (qtab) {
+                float4 *q4 = reinterpret_cast<float4 *>(qs0 + j * 64);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) q4[i] = v[i];
+            }
+            qt0[j] = run;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            float acc = 0.0f;
+            for (int j0 = 0; j0 < NS; j0 += 16) {
+                float v[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[i] = j0 + i < NS ? qt0[j0 + i] : 0.0f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    if (j0 + i < NS) {
+                        acc = acc + v[i];
+                        qacc0[j0 + i] = acc;
+                    }
                 }
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
-    const float Q = qacc[NS - 1];
-    const float f1 = f123[0], f2 = f123[1];
-    const uint32_t k1 = tp.x;
+    const float Q1 = MULTI ? 0.0f : qacc0[NS - 1], f11 = MULTI ? 0.0f : f123[0], f21 = MULTI ? 0.0f : f123[1];
     // head words also write the doc-slot copy of z (their items share a doc
     // tile, so the copy's lines fill in L2); tail tokens, in random docs,
     // are read back by token id in the DT rebuild instead
@@ -1164,7 +1310,13 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
         if (r >= sg.z) break;
         const uint4 rn = A.runs[r];
         const uint32_t t0 = rn.x, p0 = rn.y, nd = rn.w >> 16;
-        uint32_t len = rn.w & 0xFFFFu;
+        uint32_t len = rn.w & (MULTI ? 0xFFu : 0xFFFFu);
+        // the run's word: its tables and what the draws need of it
+        const uint32_t go = MULTI ? ((rn.w >> 8) & 0xFFu) * (uint32_t)ST : 0u, lb = 4u * go;
+        const float *phi = phi0 + go, *qs = qs0 + go, *qt = qt0 + go, *qacc = qacc0 + go;
+        const float *wc = qacc + NS;  // MULTI: f1, f2, k1
+        const float Q = MULTI ? qacc[NS - 1] : Q1, f1 = MULTI ? wc[0] : f11, f2 = MULTI ? wc[1] : f21;
+        const uint32_t k1 = MULTI ? __float_as_uint(wc[2]) : tp.x;
         // (the empty asm hides len's bound from the optimizer, whose
         // rewrites of the token loops from it otherwise cost a spill)
         asm volatile("" : "+v"(len));
@@ -1235,7 +1387,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
             RowBlock nxt;
             if ((uint32_t)b + 1u < nb) nxt = load_block(rp + kBlkU4 * (b + 1));
             ch[b] = S;
-            if ((uint32_t)b < nb) S = sum_block<COMPACT>(cur, S, tb, ch[b]);
+            if ((uint32_t)b < nb) S = sum_block<COMPACT, MULTI>(cur, S, tb, lb, ch[b]);
             cp[b] = S;
             cur = nxt;
         }
@@ -1250,7 +1402,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                 RowBlock nxt;
                 if (b + 1u < nb) nxt = load_block(rp + kBlkU4 * (b + 1u));
                 float unused;
-                if (b < nb) S = sum_block<COMPACT>(cur, S, tb, unused);
+                if (b < nb) S = sum_block<COMPACT, MULTI>(cur, S, tb, lb, unused);
                 cur = nxt;
             }
 #pragma unroll
@@ -1363,7 +1515,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
             if (in_s) {
                 bool found = false;
                 if (bs >= 0) {
-                    search_u4<COMPACT, NH>(blk, run, t2s, tb, newz, found);
+                    search_u4<COMPACT, MULTI, NH>(blk, run, t2s, tb, lb, newz, found);
                 } else if (nb > (uint32_t)CP) {
                     // past them: the blocks of the far checkpoint that holds
                     // the target, in order
@@ -1376,13 +1528,14 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                             run = cf[i];
                         }
                     for (uint32_t gb = g0; gb < nb && !found; ++gb)
-                        search_u4<COMPACT, kBlkU4>(load_block(rp + kBlkU4 * gb).e, run, t2s, tb, newz, found);
+                        search_u4<COMPACT, MULTI, kBlkU4>(load_block(rp + kBlkU4 * gb).e, run, t2s, tb, lb, newz,
+                                                            found);
                 }
                 if (!found) {  // rounding left every running sum at or below t2
                     if (COMPACT) {
                         const uint16_t *rr = reinterpret_cast<const uint16_t *>(A.dt) + di.x;
                         for (uint32_t i = 0; i < nnz; ++i)
-                            if (c16_count(rr[i], tb) > 0.0f && phi_c16(rr[i], tb) > 0.0f) newz = c16_topic(rr[i], tb);
+                            if (c16_count(rr[i], tb) > 0.0f && phi[c16_topic(rr[i], tb)] > 0.0f) newz = c16_topic(rr[i], tb);
                     } else {
                         const uint32_t *rr = A.dt + di.x;
                         for (uint32_t i = 0; i < nnz; ++i)
@@ -1396,27 +1549,30 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
     }
 }
 
-// One workgroup per item (grid = items), or persistent workgroups pulling
+// Workgroups that take items in turn (item = workgroup, then + grid: n_queues
+// 0), or persistent ones that pull
 // items from n_queues counters: queue q holds the items with index = q mod
 // n_queues (the items of one XCD when items are dealt round-robin to XCDs),
 // a workgroup drains its own queue (blockIdx mod n_queues) and then the
 // others.  Every workgroup leaves once every queue is past its last item.
-template <bool SHORTCUT, bool COMPACT, bool QTAB>
+template <bool SHORTCUT, bool COMPACT, bool QTAB, bool MULTI>
 __global__ void __launch_bounds__(1024) k_sample(const SampleArgs A) {
     // the only LDS of the kernel, so phi starts at address 0 and a DT entry's
     // low half is directly the LDS address of its phi value
     extern __shared__ float smf[];
     const int NS = (A.K + 63) >> 6;
     float *f123 = smf + (QTAB ? 2 : 1) * NS * 64 + 2 * NS;  // after phi, qs, qt, qacc
-    uint32_t &s_item = *reinterpret_cast<uint32_t *>(f123 + 3);
+    // MULTI: the item number before the words' tables end (the last word of
+    // the pad of its stride)
+    uint32_t &s_item = *reinterpret_cast<uint32_t *>(MULTI ? smf + A.word_stride - 1 : f123 + 3);
     const uint32_t sweep = A.counters[0];
     uint32_t n_full = 0, n_scanned = 0;
-    const bool own = A.n_queues == 0;  // one item a workgroup
+    const bool own = A.n_queues == 0;  // items dealt in turn
     const uint32_t nq = own ? 1u : A.n_queues, x0 = blockIdx.x % nq;
     for (uint32_t h = 0; h < nq; ++h) {
         const uint32_t q = (x0 + h) % nq;
-        while (true) {
-            uint64_t item = blockIdx.x;
+        for (uint32_t i = 0;; ++i) {
+            uint64_t item = (uint64_t)blockIdx.x + (uint64_t)i * gridDim.x;
             if (!own) {
                 __syncthreads();  // the previous item is done with s_item and LDS
                 if (threadIdx.x == 0) s_item = atomicAdd(&A.queue[q * kQueueStride], 1u);
@@ -1424,8 +1580,8 @@ __global__ void __launch_bounds__(1024) k_sample(const SampleArgs A) {
                 item = (uint64_t)q + (uint64_t)s_item * nq;
             }
             if (item >= A.n_items) break;
-            sample_item<SHORTCUT, COMPACT, QTAB>(A, (uint32_t)item, smf, f123, sweep, n_full, n_scanned);
-            if (own) break;
+            if (own && i) __syncthreads();
+            sample_item<SHORTCUT, COMPACT, QTAB, MULTI>(A, (uint32_t)item, smf, f123, sweep, n_full, n_scanned);
         }
     }
     // per-wavefront totals of the counters
@@ -1451,7 +1607,7 @@ __global__ void __launch_bounds__(1024) k_sample(const SampleArgs A) {
 // (256 threads an item, an FP64 division a phi, one 16-byte load of the row in
 // flight).  Workgroups with further items keep beta * inv64 in phi between
 // tail words, so such a word stages only its nonzeros.
-template <bool COMPACT>
+template <bool COMPACT, bool MULTI>
 __global__ void __launch_bounds__(1024) k_ll(uint32_t n_items, const uint4 *__restrict__ segs, const uint4 *__restrict__ runs, int VD,
                                              int K, double alpha, double beta,
                                              const int32_t *__restrict__ wt_head,
@@ -1464,6 +1620,7 @@ __global__ void __launch_bounds__(1024) k_ll(uint32_t n_items, const uint4 *__re
     __shared__ double red[16];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
     double *phi = smd;
+    __shared__ double qg[MULTI ? kGroupMax : 1];
     // sum over the workgroup, in wavefront order
     auto block_total = [&](double v) {
         for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
@@ -1483,10 +1640,32 @@ __global__ void __launch_bounds__(1024) k_ll(uint32_t n_items, const uint4 *__re
             if (tid == 0) part[item] = 0.0;
             continue;
         }
-        const int w = (int)sg.x;
+        const int w = MULTI ? (int)(sg.x & kGroupWord) : (int)sg.x;
         uint32_t tb0 = 0, tn = 0;
         double q = 0.0;
-        if (w < VD) {
+        if (MULTI) {  // word g's phi at g * K, its Q mass after the words' tables
+            const int G = 1 + (int)(sg.x >> kGroupShift);
+            for (int i = tid; i < G * K; i += blockDim.x) {
+                const int g = i / K, k = i - g * K;
+                phi[i] = ((w < VD ? (double)wt_head[(size_t)w * K + i] : 0.0) + beta) * inv64[k];
+            }
+            __syncthreads();
+            if (w >= VD)
+                for (int g = 0; g < G; ++g) {
+                    const uint32_t b = tail_off[w - VD + g], n = tail_nnz[w - VD + g];
+                    for (uint32_t i = tid; i < n; i += blockDim.x) {
+                        const uint32_t e = wt_tail[b + i], k = e & 0xFFFFu;
+                        phi[(uint32_t)(g * K) + k] = ((double)(e >> 16) + beta) * inv64[k];
+                    }
+                }
+            __syncthreads();
+            for (int g = wv; g < G; g += nwv) {
+                double x = 0.0;
+                for (int k = lane; k < K; k += 64) x += phi[g * K + k];
+                for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off);
+                if (lane == 0) qg[g] = x * alpha;
+            }
+        } else if (w < VD) {
             const int32_t *row = wt_head + (size_t)w * K;
             for (int k = tid; k < K; k += blockDim.x) {
                 const double v = ((double)row[k] + beta) * inv64[k];
@@ -1528,6 +1707,9 @@ __global__ void __launch_bounds__(1024) k_ll(uint32_t n_items, const uint4 *__re
         const uint32_t tmask = (1u << tb) - 1u;
         for (uint32_t r = sg.y + (uint32_t)tid; r < sg.z; r += (uint32_t)blockDim.x) {
             const uint4 rn = runs[r];
+            const uint32_t g = MULTI ? (rn.w >> 8) & 0xFFu : 0u;
+            const double *ph = phi + g * (uint32_t)K;
+            if (MULTI) q = qg[g];
             const uint2 di = make_uint2(rn.z, aux_doc[rn.y] >> 16);  // row offset, nnz
             const uint32_t nnz = di.y & 0xFFFFu;
             const uint4 *rp = COMPACT ? reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(dt) + di.x)
@@ -1547,20 +1729,20 @@ __global__ void __launch_bounds__(1024) k_ll(uint32_t n_items, const uint4 *__re
                     for (int u = 0; u < 4; ++u) {
                         if (COMPACT) {
                             const uint32_t x = e[u] & 0xFFFFu, y = e[u] >> 16;
-                            s = __builtin_fma((double)(x >> tb), phi[x & tmask], s);
-                            s = __builtin_fma((double)(y >> tb), phi[y & tmask], s);
+                            s = __builtin_fma((double)(x >> tb), ph[x & tmask], s);
+                            s = __builtin_fma((double)(y >> tb), ph[y & tmask], s);
                         } else {
-                            s = __builtin_fma((double)(e[u] >> 16), phi[dt_topic(e[u])], s);
+                            s = __builtin_fma((double)(e[u] >> 16), ph[dt_topic(e[u])], s);
                         }
                     }
                 }
                 cur = nxt;
             }
-            acc += (double)(rn.w & 0xFFFFu) * log((s + q) / ((double)(rn.w >> 16) + kalpha));
+            acc += (double)(rn.w & 0xFFu) * log((s + q) / ((double)(rn.w >> 16) + kalpha));
         }
         acc = block_total(acc);
         if (tid == 0) part[item] = acc;
-        if (w >= VD && item + gridDim.x < n_items) {  // the base again (every lane is past its reads of phi)
+        if (!MULTI && w >= VD && item + gridDim.x < n_items) {  // the base again (every lane is past its reads of phi)
             for (uint32_t i = tid; i < tn; i += blockDim.x) {
                 const uint32_t k = wt_tail[tb0 + i] & 0xFFFFu;
                 phi[k] = beta * inv64[k];
@@ -2718,6 +2900,17 @@ hipError_t launch_build_dt(const DevState &s, hipStream_t st, bool n_dk2) {
     return hipGetLastError();
 }
 
+// LDS floats of one word of a group item: phi and the Q running sums (whole
+// slabs), slab totals and their running sums, f1, f2, k1, the item number;
+// 4 more than a multiple of 8, so that lanes reading different words' slabs
+// start at different banks.
+int group_stride(int K) {
+    const int NS = (K + 63) >> 6;
+    int st = 2 * NS * 64 + 2 * NS + 4;
+    while ((st & 7) != 4) ++st;
+    return st;
+}
+
 size_t sample_lds_bytes(int K, int bd) {
     const int NS = (K + 63) >> 6;
     (void)bd;
@@ -2726,18 +2919,24 @@ size_t sample_lds_bytes(int K, int bd) {
 }
 
 size_t sampler_static_lds() {
-    const void *fs[6] = {reinterpret_cast<const void *>(&k_sample<true, true, true>),
-                         reinterpret_cast<const void *>(&k_sample<true, true, false>),
-                         reinterpret_cast<const void *>(&k_sample<true, false, false>),
-                         reinterpret_cast<const void *>(&k_sample<false, true, true>),
-                         reinterpret_cast<const void *>(&k_sample<false, true, false>),
-                         reinterpret_cast<const void *>(&k_sample<false, false, false>)};
+    // a property of the code: looked up until it is known, once a process
+    static std::atomic<size_t> known{(size_t)-1};
+    if (known != (size_t)-1) return known;
+    const void *fs[8] = {reinterpret_cast<const void *>(&k_sample<true, true, true, true>),
+                         reinterpret_cast<const void *>(&k_sample<true, true, true, false>),
+                         reinterpret_cast<const void *>(&k_sample<true, true, false, false>),
+                         reinterpret_cast<const void *>(&k_sample<true, false, false, false>),
+                         reinterpret_cast<const void *>(&k_sample<false, true, true, true>),
+                         reinterpret_cast<const void *>(&k_sample<false, true, true, false>),
+                         reinterpret_cast<const void *>(&k_sample<false, true, false, false>),
+                         reinterpret_cast<const void *>(&k_sample<false, false, false, false>)};
     size_t m = 0;
     for (const void *f : fs) {
         hipFuncAttributes a;
         if (hipFuncGetAttributes(&a, f) != hipSuccess) return (size_t)-1;
         m = std::max(m, a.sharedSizeBytes);
     }
+    known = m;
     return m;
 }
 
@@ -2754,8 +2953,9 @@ size_t max_lds_bytes(int K, int bd) {
 hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint32_t mode, bool begun) {
     if (s.n_smp_segs == 0) return hipSuccess;
     const int bd = s.block_dim;
-    const size_t lds = sample_lds_bytes(s.K, bd);
+    size_t lds = sample_lds_bytes(s.K, bd);
     SampleArgs A;
+    A.word_stride = 0;
     A.segs = s.smp_segs;
     A.runs = s.runs;
     A.n_items = (uint32_t)s.n_smp_segs;
@@ -2775,17 +2975,20 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
     A.z_doc = s.z_doc;
     A.counters = s.counters + (begun ? 1 : 0);
     A.queue = s.counters + kQueueStride;
-    // queues only where a workgroup has more than one item to take: with fewer
-    // items than workgroups, 18,000 tokens in 2,212 items spent 64 us a sweep
-    // on 4,096 workgroups' claims from eight queues, 20 us in 644 items of
-    // their own (one workgroup an item is the slower form already at 4 items
-    // a workgroup: 0.32 against 0.17 ms, 15,471 items at K = 64)
-    A.n_queues = s.grid_dim > 0 && s.n_smp_segs > s.grid_dim ? (uint32_t)s.n_queues : 0u;
+    // Queues only where a workgroup has many items to take: the claims, and
+    // the failed ones of all workgroups at every queue's end, cost more than
+    // the balance gains with a few.  Measured, sampler us a sweep in turn /
+    // from queues: 250 items 19 / 64 (as 2,212), 10,215 items (2.5 a
+    // workgroup) at K = 64 126 / 152, 10,113 at K = 300 159 / 169; 27,680
+    // items (13 a workgroup) at K = 4096 767 / 672, 98,189 (24) at K = 2048
+    // 2,277 / 1,564, 126,191 (31) at K = 1024 3,519 / 2,884.
+    unsigned grid = (unsigned)s.n_smp_segs;
+    A.n_queues = s.grid_dim > 0 && s.n_smp_segs / 4 >= s.grid_dim ? (uint32_t)s.n_queues : 0u;
+    if (s.grid_dim > 0 && A.n_queues == 0) grid = (unsigned)std::min(s.n_smp_segs, s.grid_dim);
     A.stats = s.stats;
     A.seed = s.seed;
     A.tb = s.topic_bits;
     A.mode = mode;
-    unsigned grid = (unsigned)s.n_smp_segs;
     if (A.n_queues) {
         // queue heads start at zero (a fill kernel, so a captured sweep
         // replays it)
@@ -2795,18 +2998,28 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
         grid = (unsigned)s.grid_dim;
     }
     const bool qtab = s.K <= EZ_Q_TABLE_MAX_K;  // implies compact rows
-    if (shortcut && qtab)
-        hipLaunchKernelGGL((k_sample<true, true, true>), dim3(grid), dim3(bd), lds, st, A);
+    const bool multi = s.group_words > 1;       // implies qtab
+    if (multi) {
+        A.word_stride = (uint32_t)group_stride(s.K);
+        lds = (size_t)s.group_words * A.word_stride * sizeof(float);
+    }
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(bd), lds, st, A); };
+    if (shortcut && multi)
+        go(k_sample<true, true, true, true>);
+    else if (shortcut && qtab)
+        go(k_sample<true, true, true, false>);
     else if (shortcut && s.compact)
-        hipLaunchKernelGGL((k_sample<true, true, false>), dim3(grid), dim3(bd), lds, st, A);
+        go(k_sample<true, true, false, false>);
     else if (shortcut)
-        hipLaunchKernelGGL((k_sample<true, false, false>), dim3(grid), dim3(bd), lds, st, A);
+        go(k_sample<true, false, false, false>);
+    else if (multi)
+        go(k_sample<false, true, true, true>);
     else if (qtab)
-        hipLaunchKernelGGL((k_sample<false, true, true>), dim3(grid), dim3(bd), lds, st, A);
+        go(k_sample<false, true, true, false>);
     else if (s.compact)
-        hipLaunchKernelGGL((k_sample<false, true, false>), dim3(grid), dim3(bd), lds, st, A);
+        go(k_sample<false, true, false, false>);
     else
-        hipLaunchKernelGGL((k_sample<false, false, false>), dim3(grid), dim3(bd), lds, st, A);
+        go(k_sample<false, false, false, false>);
     return hipGetLastError();
 }
 
@@ -2817,7 +3030,7 @@ hipError_t launch_advance_sweep(const DevState &s, hipStream_t st) {
 
 hipError_t launch_loglik(const DevState &s, hipStream_t st) {
     if (s.n_smp_segs > 0) {
-        const size_t lds = (size_t)s.K * sizeof(double);
+        const size_t lds = (size_t)s.K * (size_t)std::max(1, s.group_words) * sizeof(double);
         const int fit = std::max(1, (int)((size_t)s.lds_cu / (lds + 16 * sizeof(double))));
         int bd = 64;
         while (bd < 1024 && fit * (bd / 64) < 12) bd *= 2;
@@ -2834,8 +3047,9 @@ hipError_t launch_loglik(const DevState &s, hipStream_t st) {
                                (double)s.alpha, (double)s.beta, s.wt_head, s.tail_off, s.wt_tail, s.tail_nnz,
                                s.inv64, s.aux_doc, s.dt, s.topic_bits, s.ll_part);
         };
-        if (s.compact) go(k_ll<true>);
-        else go(k_ll<false>);
+        if (s.group_words > 1) go(k_ll<true, true>);
+        else if (s.compact) go(k_ll<true, false>);
+        else go(k_ll<false, false>);
     }
     hipLaunchKernelGGL(k_ll_final, dim3(1), dim3(1024), 0, st, s.ll_part, std::max(s.n_smp_segs, 0), s.ll_out);
     return hipGetLastError();

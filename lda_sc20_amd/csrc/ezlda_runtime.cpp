@@ -259,9 +259,17 @@ int lupload(ezlda_ctx *c, T **p, const std::vector<T> &v) {
     return EZLDA_OK;
 }
 
+// The readback's token order on the device and its buffers: a corpus of one
+// piece is copied as it is (no pinned memory to set up).
 int alloc_readback(ezlda_ctx *c, uint32_t N) {
     const uint32_t pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
-    if (pieces <= 1) return dalloc(c, &c->read_dev, N);  // copied as it is: no pinned memory to set up
+    const size_t order = ((size_t)N + 3) / 4 * 4;  // the buffer behind it is 16-byte aligned
+    if (int r = dalloc(c, &c->s.doc_tok, order + (pieces <= 1 ? order / 2 : 0))) return r;
+    if (N) EZ_TRY_HIP(c, hipMemcpy(c->s.doc_tok, c->doc_tok.data(), (size_t)N * sizeof(uint32_t), hipMemcpyHostToDevice));
+    if (pieces <= 1) {
+        c->read_dev = reinterpret_cast<uint16_t *>(c->s.doc_tok + order);
+        return EZLDA_OK;
+    }
     const uint32_t slots = std::min(pieces, std::min((uint32_t)host_threads(), kReadSlots));
     EZ_TRY_HIP(c, hipHostMalloc((void **)&c->read_buf, (size_t)slots * kReadTokens * sizeof(uint16_t),
                                 hipHostMallocDefault));
@@ -290,12 +298,15 @@ int need_loaded(ezlda_ctx *c) {
 // round-robin dispatch sends to XCD x, is XCD x's j-th item.  Short lists
 // are padded with empty items (word 0xFFFFFFFF).  Tail words follow, one
 // item per word.  Items of more than token_segment tokens, or of more than
-// `cap` cost (cost[q] a token of doc q), are split.  The order of
+// `cap` cost (cost[q] a token of doc q), are split.  Consecutive words of one
+// item each become one item (their number in its fourth field) while they are
+// at most `group` and have at most 64 tokens or `share` cost.  The order of
 // items changes which workgroup draws a token, never the draw.
 std::vector<uint4> cut_sample_items(const ezlda_args &a, const std::vector<uint32_t> &word_off,
                                     const std::vector<uint32_t> &tok_rank, const std::vector<uint32_t> &soff,
                                     const std::vector<uint32_t> &slot_wrd, int VD, int K, int n_xcd,
-                                    const std::vector<uint32_t> &cost, uint64_t cap, int *tiles_used) {
+                                    const std::vector<uint32_t> &cost, uint64_t cap, uint32_t group,
+                                    uint64_t share, int *tiles_used) {
     const uint32_t SEG = (uint32_t)a.token_segment;
     const int V = (int)word_off.size() - 1;
     const int D = (int)soff.size() - 1;
@@ -330,6 +341,7 @@ std::vector<uint4> cut_sample_items(const ezlda_args &a, const std::vector<uint3
     };
     int T = 0;
     uint64_t head_tokens = word_off[VD];
+    std::vector<char> whole(VD, true);  // head words that are not cut by doc tiles
     if (a.doc_tiles >= 0 && VD > 0 && D > 0 && n_xcd > 0 && head_tokens > 0) {
         // DT bytes of the whole corpus -> tiles of ~2 MiB
         uint64_t dt_bytes = 0;
@@ -359,7 +371,7 @@ std::vector<uint4> cut_sample_items(const ezlda_args &a, const std::vector<uint3
         tile_doc[T] = (uint32_t)D;
         const int per_xcd = T / n_xcd;
         const uint32_t kMinItemTokens = 512;
-        // per XCD: (tile, word, first, end)
+        // per XCD: (tile, word, first, end), of the words that are cut by tiles
         std::vector<std::vector<std::array<uint32_t, 4>>> lists(n_xcd);
         for (int w = 0; w < VD; ++w) {
             const uint32_t b = word_off[w], e = word_off[w + 1];
@@ -368,6 +380,8 @@ std::vector<uint4> cut_sample_items(const ezlda_args &a, const std::vector<uint3
             int g = per_xcd;  // tiles per item: the coarsest that still splits per XCD
             while (g > 1 && (uint64_t)n * (uint64_t)g / (uint64_t)T >= 2ull * kMinItemTokens) g /= 2;
             while (g < T && (uint64_t)n * (uint64_t)g / (uint64_t)T < kMinItemTokens) g = std::min(T, 2 * g);
+            if (g >= T) continue;
+            whole[w] = false;
             for (int t = 0; t < T; t += g) {
                 const uint32_t d0 = tile_doc[t], d1 = tile_doc[std::min(T, t + g)];
                 const uint32_t lo = (uint32_t)(std::lower_bound(tok_rank.begin() + b, tok_rank.begin() + e, d0) - tok_rank.begin());
@@ -387,10 +401,32 @@ std::vector<uint4> cut_sample_items(const ezlda_args &a, const std::vector<uint3
         for (size_t j = 0; j < longest; ++j)
             for (int x = 0; x < n_xcd; ++x)
                 out.push_back(j < split[x].size() ? split[x][j] : make_uint4(0xFFFFFFFFu, 0u, 0u, 0u));
-    } else {
-        for (int w = 0; w < VD; ++w) push_split(out, (uint32_t)w, word_off[w], word_off[w + 1]);
     }
-    for (int w = VD; w < V; ++w) push_split(out, (uint32_t)w, word_off[w], word_off[w + 1]);
+    uint64_t group_cost = 0;
+    bool open = false;  // the last item takes further words
+    for (int w = 0; w < V; ++w) {
+        if (w < VD && !whole[w]) continue;
+        const uint32_t b = word_off[w], e = word_off[w + 1];
+        if (b == e) continue;
+        const size_t at = out.size();
+        push_split(out, (uint32_t)w, b, e);
+        if (group <= 1) continue;
+        const uint64_t c = (uint64_t)(e - b) * cost[tok_rank[b]];  // at most
+        const bool one = out.size() == at + 1;
+        if (one && open && w != VD) {
+            uint4 &g = out[at - 1];
+            if (g.x + g.w == (uint32_t)w && g.w < group && (e - g.y <= 64u || group_cost + c <= share)) {
+                g.z = e;
+                ++g.w;
+                group_cost += c;
+                out.pop_back();
+                continue;
+            }
+        }
+        open = one;
+        if (open) out.back().w = 1u;
+        group_cost = c;
+    }
     if (tiles_used) *tiles_used = T;
     return out;
 }
@@ -409,7 +445,7 @@ std::vector<uint4> cut_sample_items(const ezlda_args &a, const std::vector<uint3
 // share: K = 300 0.231 / 0.254, heavy-tailed 2.82 / 3.21.
 std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uint32_t> &word_off,
                                       const std::vector<uint32_t> &tok_rank, const std::vector<uint32_t> &soff,
-                                      const std::vector<uint32_t> &slot_wrd, int VD, int K, int n_xcd,
+                                      const std::vector<uint32_t> &slot_wrd, int VD, int K, int n_xcd, bool groups,
                                       int *tiles_used) {
     const uint32_t kRunCost = 96;
     const int D = (int)soff.size() - 1;
@@ -422,11 +458,24 @@ std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uin
         total += (uint64_t)n * cost[q];
     }
     const uint64_t least = (uint64_t)a.block_dim * (256u + (uint64_t)K / 8u);
-    std::vector<uint4> out = cut_sample_items(a, word_off, tok_rank, soff, slot_wrd, VD, K, n_xcd, cost,
-                                              std::max(least, total / (2 * n_wg)), tiles_used);
-    // the cap never costs a corpus the allocation-free log-likelihood
-    if (out.size() > ez::kLLScratchItems)
-        out = cut_sample_items(a, word_off, tok_rank, soff, slot_wrd, VD, K, n_xcd, cost, UINT64_MAX, tiles_used);
+    // words of few tokens grouped where the tables of several fit the LDS that
+    // one of 16 wavefronts a CU has: 18,000 tokens at K = 20 (1,000 words) 22
+    // -> 19 us a sweep, 1M tokens at K = 64 164 -> 151, 1.7M at K = 300 191 ->
+    // 168 (with a whole or a quarter of a workgroup's share: 153, 161 and 174,
+    // 175)
+    uint32_t group = 1;
+    if (groups && K <= ez::kGroupMaxK && a.block_dim == 64 && word_off.size() <= (size_t)ez::kGroupWord)
+        group = std::min<uint32_t>(ez::kGroupMax, 10240u / (4u * (uint32_t)ez::group_stride(K)));
+    const uint64_t share = total / (2 * n_wg);
+    auto cut = [&](uint64_t cap, uint32_t g) {
+        return cut_sample_items(a, word_off, tok_rank, soff, slot_wrd, VD, K, n_xcd, cost, cap, g, share, tiles_used);
+    };
+    std::vector<uint4> out = cut(std::max(least, total / (2 * n_wg)), group);
+    // neither the cap nor the groups decide whether the allocation-free
+    // log-likelihood takes a corpus
+    size_t single = out.size();
+    for (const uint4 &it : out) single += it.w > 1 ? it.w - 1 : 0;
+    if (single > ez::kLLScratchItems) out = cut(UINT64_MAX, 1);
     return out;
 }
 
@@ -435,20 +484,25 @@ std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uin
 // doc, tokens); a run's slots are consecutive too (a doc's slots are grouped
 // by word, then position).  Inside an item the runs are ordered longest first
 // (then by token), so the lanes of a wavefront draw similar numbers of
-// tokens; the order does not affect any draw.  Items are rewritten as run
-// ranges (w, first run, end run, 0).
-std::vector<uint4> build_runs(std::vector<uint4> &items, const std::vector<uint32_t> &tok_doc,
-                              const std::vector<uint32_t> &tok_slot, uint32_t cap) {
+// tokens, then by doc (longest first); the order does not affect any draw.
+// In a group's item a run also carries its word's place (<< 8).  Items are
+// rewritten as run ranges (w, first run, end run, 0).
+std::vector<uint4> build_runs(std::vector<uint4> &items, const std::vector<uint32_t> &word_off,
+                              const std::vector<uint32_t> &tok_doc, const std::vector<uint32_t> &tok_slot,
+                              uint32_t cap) {
     const int64_t n = (int64_t)items.size();
     std::vector<uint64_t> cnt(n + 1, 0);
     auto for_runs = [&](const uint4 &it, auto &&emit) {
         uint32_t t = it.y;
-        while (t < it.z) {
-            uint32_t e = t + 1;
-            // same doc implies the next slot (the sampler writes z_doc[slot + j])
-            while (e < it.z && e - t < cap && tok_doc[e] == tok_doc[t] && tok_slot[e] == tok_slot[t] + (e - t)) ++e;
-            emit(t, e - t);
-            t = e;
+        for (uint32_t g = 0; g < std::max(1u, it.w); ++g) {  // a group's words: all of their tokens
+            const uint32_t end = it.w ? word_off[it.x + g + 1] : it.z;
+            while (t < end) {
+                uint32_t e = t + 1;
+                // same doc implies the next slot (the sampler writes z_doc[slot + j])
+                while (e < end && e - t < cap && tok_doc[e] == tok_doc[t] && tok_slot[e] == tok_slot[t] + (e - t)) ++e;
+                emit(t, (e - t) | g << 8);
+                t = e;
+            }
         }
     };
     parallel_for(n, [&](int64_t b, int64_t e, int) {
@@ -466,9 +520,12 @@ std::vector<uint4> build_runs(std::vector<uint4> &items, const std::vector<uint3
             if (it.x == 0xFFFFFFFFu) continue;
             uint64_t k = cnt[i];
             for_runs(it, [&](uint32_t t, uint32_t l) { runs[k++] = make_uint4(t, tok_slot[t], tok_doc[t], l); });
-            std::stable_sort(runs.begin() + cnt[i], runs.begin() + cnt[i + 1],
-                             [](const uint4 &x, const uint4 &y) { return x.w > y.w; });
-            it = make_uint4(it.x, (uint32_t)cnt[i], (uint32_t)cnt[i + 1], 0u);
+            std::stable_sort(runs.begin() + cnt[i], runs.begin() + cnt[i + 1], [](const uint4 &x, const uint4 &y) {
+                const uint32_t a = x.w & 0xFFu, b = y.w & 0xFFu;
+                return a > b || (a == b && x.z < y.z);
+            });
+            it = make_uint4(it.x | (it.w > 1 ? (it.w - 1u) << ez::kGroupShift : 0u), (uint32_t)cnt[i],
+                            (uint32_t)cnt[i + 1], 0u);
         }
     }, (int64_t)tok_doc.size());
     return runs;
@@ -522,8 +579,10 @@ int build_layout(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
             wt_segs.push_back(make_uint4((uint32_t)r, b, std::min(b + WT_SEG, c->word_off[r + 1]), 0u));
     (void)D;
     std::vector<uint4> smp_segs =
-        build_sample_items(c->a, c->word_off, tok_doc, c->soff, slot_wrd, VD, K, c->n_xcd, &c->doc_tiles);
-    std::vector<uint4> runs = build_runs(smp_segs, tok_doc, tok_slot, (uint32_t)c->a.run_cap);
+        build_sample_items(c->a, c->word_off, tok_doc, c->soff, slot_wrd, VD, K, c->n_xcd, true, &c->doc_tiles);
+    uint32_t group_words = 1;
+    for (const uint4 &it : smp_segs) group_words = std::max(group_words, it.w);
+    std::vector<uint4> runs = build_runs(smp_segs, c->word_off, tok_doc, tok_slot, (uint32_t)c->a.run_cap);
     for (uint4 &rn : runs) {  // doc q -> its DT row offset; the doc's length beside the run's
         rn.w |= (c->soff[rn.z + 1] - c->soff[rn.z]) << 16;
         rn.z = c->row_off[rn.z];
@@ -541,6 +600,7 @@ int build_layout(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
     s.n_wt_segs = (int32_t)wt_segs.size();
     s.n_smp_segs = (int32_t)smp_segs.size();
     s.n_runs = (int64_t)runs.size();
+    s.group_words = (int32_t)group_words;
     s.n_queues = c->doc_tiles > 0 ? std::min(c->n_xcd, 8) : 1;
     s.block_dim = c->a.block_dim;
     s.grid_dim = c->a.grid_dim;
@@ -637,8 +697,8 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
         if (dtc >= 0xFFFFFFF0ull) return fail(c, EZLDA_EINVAL, "DT capacity of a chunk exceeds 2^32 entries");
         ch.dt_entries = dtc;
         int tiles = 0;
-        std::vector<uint4> items = build_sample_items(c->a, woff, tdoc, soffc, swrd, VDi, K, c->n_xcd, &tiles);
-        std::vector<uint4> runs = build_runs(items, tdoc, tslot, (uint32_t)c->a.run_cap);
+        std::vector<uint4> items = build_sample_items(c->a, woff, tdoc, soffc, swrd, VDi, K, c->n_xcd, false, &tiles);
+        std::vector<uint4> runs = build_runs(items, woff, tdoc, tslot, (uint32_t)c->a.run_cap);
         for (uint4 &rn : runs) {  // doc q -> its DT row offset in the chunk; the doc's length
             rn.w |= (soffc[rn.z + 1] - soffc[rn.z]) << 16;
             rn.z = di[rn.z].x;
@@ -716,8 +776,8 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
     if ((r = dalloc(c, &c->wt_next, (size_t)V * K))) return r;
     if ((r = dalloc(c, &s.nk, K))) return r;
     if ((r = dalloc(c, &c->nk_next, K))) return r;
-    if ((r = dalloc(c, &s.inv, K))) return r;
-    if ((r = dalloc(c, &s.inv64, K))) return r;
+    if ((r = dalloc(c, &s.inv64, K + (K + 1) / 2))) return r;  // inv behind it
+    s.inv = reinterpret_cast<float *>(s.inv64 + K);
     if ((r = dalloc(c, &s.wtop, V))) return r;
     if ((r = dalloc(c, &s.zero_order, K))) return r;
     if ((r = dalloc(c, &s.tail_off, 1))) return r;
@@ -1132,7 +1192,6 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
     int r = 0;
     if ((r = upload(c, &s.word_off, c->word_off))) return r;
     if ((r = upload(c, &s.z, z))) return r;
-    if ((r = upload(c, &s.doc_tok, c->doc_tok))) return r;
     if ((r = alloc_readback(c, N))) return r;
     if ((r = upload(c, &s.soff, c->soff))) return r;
     if ((r = upload(c, &s.slot_wrd, slot_wrd))) return r;
@@ -1145,8 +1204,8 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
     if ((r = dalloc(c, &s.dt, dt_words))) return r;
     EZ_TRY_HIP(c, hipMemset(s.dt, 0, dt_words * sizeof(uint32_t)));
     if ((r = dalloc(c, &s.nk, K))) return r;
-    if ((r = dalloc(c, &s.inv, K))) return r;
-    if ((r = dalloc(c, &s.inv64, K))) return r;
+    if ((r = dalloc(c, &s.inv64, K + (K + 1) / 2))) return r;  // inv behind it
+    s.inv = reinterpret_cast<float *>(s.inv64 + K);
     if ((r = dalloc(c, &s.wtop, V))) return r;
     if ((r = dalloc(c, &s.zero_order, K))) return r;
     if ((r = dalloc(c, &s.counters, ez::kCounterWords))) return r;

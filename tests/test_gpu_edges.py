@@ -117,3 +117,37 @@ def test_fold_in_of_a_full_house(K, D):
         assert np.array_equal(z, zo[doff[r]: doff[r + 1]]) and np.array_equal(c, co[r]), r
     assert srv.stats().max_active * 400 > 196608
     srv.close()
+
+
+# words of few tokens drawn by groups (K <= 512): slabs and topics that fill no
+# whole load, groups of dense words, of sparse words and at the border of the
+# two, unused words, long words between; stages in any order
+@pytest.mark.parametrize("K", [1, 2, 5, 20, 63, 64, 65, 127, 130, 256, 300, 512, 513])
+@pytest.mark.parametrize("kw", [{"dense_words": 0}, {"dense_words": 37, "run_cap": 2}, {"dense_words": 10**6},
+                                {"grid_dim": 24, "shortcut": 0}])
+def test_groups_of_small_words(K, kw):
+    rng = np.random.default_rng(K)
+    n = rng.integers(1, 120, 90)
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int64)
+    words = np.where(rng.random(int(off[-1])) < 0.3, rng.integers(0, 3, int(off[-1])),
+                     rng.integers(0, 1500, int(off[-1]))).astype(np.int32)
+    ctx, orc = _pair(off, words, 1600, K, **kw)
+    for s in range(2):
+        ctx.sweep(1)
+        orc.sweep(1)
+        assert np.array_equal(ctx.get_topics(), orc.get_topics()), s
+        assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
+    for stages in (("sample_tail", "shortcut", "sample_head"), ("shortcut", "sample_head", "sample_tail")):
+        ctx.build_wt()
+        ctx.topk()
+        ctx.build_dt()
+        for name in stages:
+            getattr(ctx, name)()
+        ctx.commit_head()
+        orc.sweep(1)
+        assert np.array_equal(ctx.get_topics(), orc.get_topics()), stages
+    ctx.set_layout(block_dim=128)  # no groups there
+    ctx.sweep(1)
+    orc.sweep(1)
+    assert np.array_equal(ctx.get_topics(), orc.get_topics())
+    ctx.close()
