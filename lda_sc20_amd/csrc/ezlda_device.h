@@ -92,6 +92,17 @@ hipError_t launch_topk(const DevState &s, hipStream_t st);
 // per-token pair, which the sampler does not need).
 hipError_t launch_build_dt(const DevState &s, hipStream_t st, bool n_dk2 = false);
 hipError_t launch_z_to_doc(const DevState &s, hipStream_t st);
+// A chunk's layout in its short form: runs in token order, as first slot and
+// tokens, and the first token of every item.
+struct ChunkRuns {
+    const uint32_t *item_tok = nullptr, *run_slot = nullptr;
+    const uint8_t *run_len = nullptr;
+};
+// s.runs and s.slot_wrd of that form; begins sweep `sweep` (counters[1], the
+// queue heads) for launch_sample(begun).
+hipError_t launch_chunk_runs(const DevState &s, const ChunkRuns &r, uint32_t sweep, hipStream_t st);
+// s.z of s.z_doc.
+hipError_t launch_chunk_topics(const DevState &s, const ChunkRuns &r, hipStream_t st);
 // Topics of the doc-major positions [b, b + n) into out (device or pinned
 // host memory, 16-byte aligned); b is a multiple of 8.
 hipError_t launch_topics_out(const DevState &s, uint32_t b, uint32_t n, uint16_t *out, hipStream_t st);

@@ -18,10 +18,12 @@ struct EzChunk {
     uint32_t n_items = 0, n_wt_segs = 0, n_queues = 1;
     int32_t D_long = 0;             // docs of more than ez::kDtShort tokens (the chunk's first)
     uint64_t n_runs = 0, dt_entries = 0;
-    // image: z | z_doc | doc_info (copied back after each sweep), then
-    // soff, slot_wrd, slot_tok, items, runs, WT segments
-    size_t off_doc_info = 0, back_bytes = 0, off_soff = 0, off_slot_wrd = 0, off_slot_tok = 0, off_items = 0,
-           off_runs = 0, off_wt_segs = 0, bytes = 0;
+    // image: z_doc | doc_info (copied back after each sweep), then soff,
+    // items, their first tokens, the runs' slots and lengths in token order
+    // (5 bytes a run: launch_chunk_runs makes the rest of the layout of
+    // them), WT segments
+    size_t off_doc_info = 0, back_bytes = 0, off_soff = 0, off_items = 0, off_item_tok = 0, off_run_slot = 0,
+           off_run_len = 0, off_wt_segs = 0, bytes = 0;
     uint8_t *img = nullptr;  // pinned
 };
 
@@ -59,10 +61,13 @@ struct ezlda_ctx {
     // out-of-core execution
     std::vector<EzChunk> chunks;       // empty: the corpus is resident
     std::vector<uint32_t> chunk_slot0; // first slot of each chunk (lookup)
-    std::vector<uint32_t> tok_slot_g;  // token id -> corpus slot
+    std::vector<uint32_t> pos_slot;    // doc-major position -> corpus slot
     uint8_t *cimg[2] = {nullptr, nullptr};  // device image buffers
     uint32_t *cdt[2] = {nullptr, nullptr};  // DT rows of the chunk in flight
     uint32_t *caux[2] = {nullptr, nullptr};
+    uint16_t *cz[2] = {nullptr, nullptr};    // z by token, made of the image's z_doc or drawn
+    uint32_t *cwrd[2] = {nullptr, nullptr};  // slot_wrd and the sampler's runs, made of the image
+    uint4 *cruns[2] = {nullptr, nullptr};
     uint32_t *cctr[2] = {nullptr, nullptr};  // per-buffer sweep counter and item queues
     double *cll[2] = {nullptr, nullptr};     // per-item log-likelihood partials
     double *cllo[2] = {nullptr, nullptr};

@@ -515,6 +515,110 @@ hipError_t launch_topics_out(const DevState &s, uint32_t b, uint32_t n, uint16_t
     return hipGetLastError();
 }
 
+// A chunk's runs and slot words from the short form that its image carries
+// over the host link (run_slot and run_len, runs in token order), one
+// wavefront an item: a counting sort by length puts the runs in the order of
+// the sampler (longest first, then by token), a prefix sum of the lengths
+// numbers their tokens, and the doc of a run is searched by its first slot.
+// The link bounds a sweep over chunks, not the kernels: 5 bytes a run over it
+// instead of 16, and neither the word of each slot (4 bytes a token), nor its
+// token (4, not needed on the device), nor z beside z_doc (2, each way).
+// 6.6M tokens in 4 chunks, K = 1024: 31-50 us a chunk of 1.65M tokens beside
+// an upload of 160-225 us (was 480); a sweep 4.0 -> 1.95 ms with the first
+// uploads begun before the last sweep ends.
+// TOPICS: z of z_doc instead, which the first sweep counts.
+template <bool TOPICS>
+__global__ __launch_bounds__(256) void k_chunk_runs(const uint4 *__restrict__ items, uint32_t n_items, ChunkRuns R,
+                                                    uint32_t D, const uint32_t *__restrict__ soff,
+                                                    const uint2 *__restrict__ doc_info, uint4 *__restrict__ runs,
+                                                    uint32_t *__restrict__ slot_wrd,
+                                                    const uint16_t *__restrict__ z_doc, uint16_t *__restrict__ z,
+                                                    uint32_t *__restrict__ counters, uint32_t n_queues,
+                                                    uint32_t sweep) {
+    __shared__ uint32_t bins[TOPICS ? 1 : 4][64];  // run_cap is at most 32
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, gid = blockIdx.x * 256u + threadIdx.x;
+    if (!TOPICS) {
+        if (gid == 0) counters[1] = sweep;
+        if (gid < n_queues) counters[kQueueStride * (gid + 1)] = 0u;
+    }
+    uint32_t *bin = bins[TOPICS ? 0 : wv];
+    for (uint32_t i = blockIdx.x * 4u + wv; i < n_items; i += gridDim.x * 4u) {
+        const uint4 it = items[i];
+        if (it.x == 0xFFFFFFFFu) continue;
+        if (!TOPICS) {  // bin[n]: place of the next run of n tokens
+            bin[lane] = 0u;
+            wave_lds_sync();
+            for (uint32_t r = it.y + lane; r < it.z; r += 64) atomicAdd(&bin[R.run_len[r]], 1u);
+            wave_lds_sync();
+            const uint32_t c = bin[63u - lane];
+            uint32_t incl = c;
+            for (uint32_t d = 1; d < 64; d <<= 1) {
+                const uint32_t v = __shfl_up(incl, d);
+                if (lane >= d) incl += v;
+            }
+            wave_lds_sync();
+            bin[63u - lane] = it.y + incl - c;
+            wave_lds_sync();
+        }
+        uint32_t tok = R.item_tok[i];
+        for (uint32_t b = it.y; b < it.z; b += 64) {
+            const uint32_t r = b + lane;
+            const bool have = r < it.z;
+            const uint32_t n = have ? R.run_len[r] : 0u, slot = have ? R.run_slot[r] : 0u;
+            uint32_t incl = n;
+            for (uint32_t d = 1; d < 64; d <<= 1) {
+                const uint32_t v = __shfl_up(incl, d);
+                if (lane >= d) incl += v;
+            }
+            const uint32_t t0 = tok + incl - n;
+            tok += __shfl(incl, 63);
+            if (TOPICS) {
+                for (uint32_t j = 0; j < n; ++j) z[t0 + j] = z_doc[slot + j];
+                continue;
+            }
+            uint32_t q = 0;  // the last doc whose first slot is not after this one
+            for (uint32_t lo = 1, hi = D; lo < hi;) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (soff[mid] <= slot)
+                    q = mid, lo = mid + 1;
+                else
+                    hi = mid;
+            }
+            const uint32_t row = doc_info[q].x, len = soff[q + 1] - soff[q];
+            uint32_t at = 0;
+            for (uint64_t left = __ballot(have); left;) {
+                const uint32_t ln = __shfl(n, __ffsll((unsigned long long)left) - 1);
+                const uint64_t same = __ballot(have && n == ln);
+                const uint32_t first = bin[ln];
+                if (n == ln) at = first + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+                wave_lds_sync();
+                if (lane == 0) bin[ln] = first + (uint32_t)__popcll(same);
+                wave_lds_sync();
+                left &= ~same;
+            }
+            if (have) runs[at] = make_uint4(t0, slot, row, n | len << 16);
+            for (uint32_t j = 0; j < n; ++j) slot_wrd[slot + j] = it.x;
+        }
+    }
+}
+
+template <bool TOPICS>
+static hipError_t chunk_runs(const DevState &s, const ChunkRuns &r, uint32_t sweep, hipStream_t st) {
+    if (s.n_smp_segs == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_chunk_runs<TOPICS>), dim3(grid_for((size_t)s.n_smp_segs, 4, 1 << 14)), dim3(256), 0, st,
+                       s.smp_segs, (uint32_t)s.n_smp_segs, r, (uint32_t)s.D, s.soff, s.doc_info, s.runs, s.slot_wrd,
+                       s.z_doc, s.z, s.counters, (uint32_t)s.n_queues, sweep);
+    return hipGetLastError();
+}
+
+hipError_t launch_chunk_runs(const DevState &s, const ChunkRuns &r, uint32_t sweep, hipStream_t st) {
+    return chunk_runs<false>(s, r, sweep, st);
+}
+
+hipError_t launch_chunk_topics(const DevState &s, const ChunkRuns &r, hipStream_t st) {
+    return chunk_runs<true>(s, r, 0, st);
+}
+
 // --------------------------------------------------- DT rows and aux
 // DT_Update_Kernel (utility.cu:79-284), on the doc-major copy of z: doc q
 // (docs in descending length order) owns slots [soff[q], soff[q+1]), its

@@ -230,7 +230,7 @@ void free_device(ezlda_ctx *c) {
         if (ch.img) (void)hipHostFree(ch.img);
     c->chunks.clear();
     c->chunk_slot0.clear();
-    c->tok_slot_g.clear();
+    c->pos_slot.clear();
     for (int j = 0; j < 2; ++j) {
         c->cimg[j] = nullptr;
         c->cdt[j] = c->caux[j] = c->cctr[j] = nullptr;
@@ -479,56 +479,94 @@ std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uin
     return out;
 }
 
-// Runs: a word's consecutive tokens in one document (tokens of a word are
-// numbered in doc order), at most `cap` each, as (first token, first slot,
-// doc, tokens); a run's slots are consecutive too (a doc's slots are grouped
-// by word, then position).  Inside an item the runs are ordered longest first
-// (then by token), so the lanes of a wavefront draw similar numbers of
-// tokens, then by doc (longest first); the order does not affect any draw.
-// In a group's item a run also carries its word's place (<< 8).  Items are
-// rewritten as run ranges (w, first run, end run, 0).
-std::vector<uint4> build_runs(std::vector<uint4> &items, const std::vector<uint32_t> &word_off,
-                              const std::vector<uint32_t> &tok_doc, const std::vector<uint32_t> &tok_slot,
-                              uint32_t cap) {
+// Runs of an item's tokens, in token order: a word's consecutive tokens in
+// one document (tokens of a word are numbered in doc order), at most `cap`
+// each, as emit(first token, tokens | the word's place in a group << 8); a
+// run's slots are consecutive too (a doc's slots are grouped by word, then
+// position).
+template <typename Emit>
+void for_runs(const uint4 &it, const std::vector<uint32_t> &word_off, const std::vector<uint32_t> &tok_doc,
+              const std::vector<uint32_t> &tok_slot, uint32_t cap, Emit &&emit) {
+    if (it.x == 0xFFFFFFFFu) return;
+    uint32_t t = it.y;
+    for (uint32_t g = 0; g < std::max(1u, it.w); ++g) {  // a group's words: all of their tokens
+        const uint32_t end = it.w ? word_off[it.x + g + 1] : it.z;
+        while (t < end) {
+            uint32_t e = t + 1;
+            // same doc implies the next slot (the sampler writes z_doc[slot + j])
+            while (e < end && e - t < cap && tok_doc[e] == tok_doc[t] && tok_slot[e] == tok_slot[t] + (e - t)) ++e;
+            emit(t, (e - t) | g << 8);
+            t = e;
+        }
+    }
+}
+
+// The runs of all items: begin(their number), then per item i, on its thread,
+// put(i, first token, length, index) in token order and done(i, first run, end
+// run).  Items are rewritten as run ranges (w, first run, end run, 0).
+template <typename Begin, typename Put, typename Done>
+void number_runs(std::vector<uint4> &items, const std::vector<uint32_t> &word_off,
+                 const std::vector<uint32_t> &tok_doc, const std::vector<uint32_t> &tok_slot, uint32_t cap,
+                 Begin &&begin, Put &&put, Done &&done) {
     const int64_t n = (int64_t)items.size();
     std::vector<uint64_t> cnt(n + 1, 0);
-    auto for_runs = [&](const uint4 &it, auto &&emit) {
-        uint32_t t = it.y;
-        for (uint32_t g = 0; g < std::max(1u, it.w); ++g) {  // a group's words: all of their tokens
-            const uint32_t end = it.w ? word_off[it.x + g + 1] : it.z;
-            while (t < end) {
-                uint32_t e = t + 1;
-                // same doc implies the next slot (the sampler writes z_doc[slot + j])
-                while (e < end && e - t < cap && tok_doc[e] == tok_doc[t] && tok_slot[e] == tok_slot[t] + (e - t)) ++e;
-                emit(t, (e - t) | g << 8);
-                t = e;
-            }
-        }
-    };
     parallel_for(n, [&](int64_t b, int64_t e, int) {
         for (int64_t i = b; i < e; ++i) {
             uint64_t k = 0;
-            if (items[i].x != 0xFFFFFFFFu) for_runs(items[i], [&](uint32_t, uint32_t) { ++k; });
+            for_runs(items[i], word_off, tok_doc, tok_slot, cap, [&](uint32_t, uint32_t) { ++k; });
             cnt[i + 1] = k;
         }
     }, (int64_t)tok_doc.size());
     for (int64_t i = 0; i < n; ++i) cnt[i + 1] += cnt[i];
-    std::vector<uint4> runs(cnt[n]);
+    begin(cnt[n]);
     parallel_for(n, [&](int64_t b, int64_t e, int) {
         for (int64_t i = b; i < e; ++i) {
             uint4 &it = items[i];
             if (it.x == 0xFFFFFFFFu) continue;
             uint64_t k = cnt[i];
-            for_runs(it, [&](uint32_t t, uint32_t l) { runs[k++] = make_uint4(t, tok_slot[t], tok_doc[t], l); });
-            std::stable_sort(runs.begin() + cnt[i], runs.begin() + cnt[i + 1], [](const uint4 &x, const uint4 &y) {
-                const uint32_t a = x.w & 0xFFu, b = y.w & 0xFFu;
-                return a > b || (a == b && x.z < y.z);
-            });
+            for_runs(it, word_off, tok_doc, tok_slot, cap, [&](uint32_t t, uint32_t l) { put(t, l, k++); });
+            done(cnt[i], cnt[i + 1]);
             it = make_uint4(it.x | (it.w > 1 ? (it.w - 1u) << ez::kGroupShift : 0u), (uint32_t)cnt[i],
                             (uint32_t)cnt[i + 1], 0u);
         }
     }, (int64_t)tok_doc.size());
+}
+
+// The runs as (first token, first slot, doc, tokens).  Inside an item they are
+// ordered longest first (then by token), so the lanes of a wavefront draw
+// similar numbers of tokens, then by doc (longest first); the order does not
+// affect any draw.  In a group's item a run also carries its word's place
+// (<< 8).
+std::vector<uint4> build_runs(std::vector<uint4> &items, const std::vector<uint32_t> &word_off,
+                              const std::vector<uint32_t> &tok_doc, const std::vector<uint32_t> &tok_slot,
+                              uint32_t cap) {
+    std::vector<uint4> runs;
+    number_runs(items, word_off, tok_doc, tok_slot, cap, [&](uint64_t n) { runs.resize(n); },
+                [&](uint32_t t, uint32_t l, uint64_t k) { runs[k] = make_uint4(t, tok_slot[t], tok_doc[t], l); },
+                [&](uint64_t b, uint64_t e) {
+                    std::stable_sort(runs.begin() + b, runs.begin() + e, [](const uint4 &x, const uint4 &y) {
+                        const uint32_t p = x.w & 0xFFu, q = y.w & 0xFFu;
+                        return p > q || (p == q && x.z < y.z);
+                    });
+                });
     return runs;
+}
+
+// A chunk's runs in the short form of its image, in token order; the device
+// orders them as build_runs does (ez::launch_chunk_runs).
+void build_chunk_runs(std::vector<uint4> &items, const std::vector<uint32_t> &word_off,
+                      const std::vector<uint32_t> &tok_doc, const std::vector<uint32_t> &tok_slot, uint32_t cap,
+                      std::vector<uint32_t> &run_slot, std::vector<uint8_t> &run_len) {
+    number_runs(items, word_off, tok_doc, tok_slot, cap,
+                [&](uint64_t n) {
+                    run_slot.resize(n);
+                    run_len.resize(n);
+                },
+                [&](uint32_t t, uint32_t l, uint64_t k) {
+                    run_slot[k] = tok_slot[t];
+                    run_len[k] = (uint8_t)l;
+                },
+                [](uint64_t, uint64_t) {});
 }
 
 // Dense head words: the first dense_words ranks, else the ranks with at
@@ -633,8 +671,7 @@ int refuse_chunked(ezlda_ctx *c, const char *what) {
 size_t al16(size_t x) { return (x + 15u) & ~(size_t)15u; }
 
 int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::vector<uint32_t> &tok_slot,
-                 const std::vector<uint32_t> &slot_wrd, const std::vector<uint16_t> &z,
-                 const std::vector<uint16_t> &z_doc) {
+                 const std::vector<uint32_t> &slot_wrd, const std::vector<uint16_t> &z_doc) {
     ez::DevState &s = c->s;
     const int V = s.V, K = s.K, D = s.D;
     const uint32_t N = s.N;
@@ -659,7 +696,7 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
     c->chunks.assign(C, EzChunk{});
     c->chunk_slot0.assign(C, 0);
     size_t max_bytes = 0;
-    uint64_t max_dt = 0, dt_total = 0;
+    uint64_t max_dt = 0, dt_total = 0, max_runs = 1;
     uint32_t max_n = 1, max_items = 1;
     int64_t items_total = 0, runs_total = 0;
     for (int k = 0; k < C; ++k) {
@@ -670,17 +707,15 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
         ch.N = c->soff[qb[k + 1]] - ch.slot0;
         c->chunk_slot0[k] = ch.slot0;
         const uint32_t n = ch.N;
-        std::vector<uint32_t> woff(V + 1, 0), glob(n), tdoc(n), tslot(n), soffc(ch.D + 1), swrd(n), stok(n);
-        std::vector<uint16_t> zc(n), zd(n);
+        std::vector<uint32_t> woff(V + 1, 0), glob(n), tdoc(n), tslot(n), soffc(ch.D + 1), swrd(n);
+        std::vector<uint16_t> zd(n);
         for (uint32_t pp = 0; pp < n; ++pp) {
             const uint32_t p = ch.slot0 + pp, t = c->slot_tok[p], l = loc[t];
             glob[l] = t;
             tdoc[l] = tok_doc[t] - ch.q0;
             tslot[l] = tok_slot[t] - ch.slot0;
-            zc[l] = z[t];
             zd[pp] = z_doc[p];
             swrd[pp] = slot_wrd[p];
-            stok[pp] = l;
             woff[slot_wrd[p] + 1]++;
         }
         for (int r = 0; r < V; ++r) woff[r + 1] += woff[r];
@@ -698,11 +733,11 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
         ch.dt_entries = dtc;
         int tiles = 0;
         std::vector<uint4> items = build_sample_items(c->a, woff, tdoc, soffc, swrd, VDi, K, c->n_xcd, false, &tiles);
-        std::vector<uint4> runs = build_runs(items, woff, tdoc, tslot, (uint32_t)c->a.run_cap);
-        for (uint4 &rn : runs) {  // doc q -> its DT row offset in the chunk; the doc's length
-            rn.w |= (soffc[rn.z + 1] - soffc[rn.z]) << 16;
-            rn.z = di[rn.z].x;
-        }
+        std::vector<uint32_t> item_tok(items.size());
+        for (size_t i = 0; i < items.size(); ++i) item_tok[i] = items[i].y;
+        std::vector<uint32_t> run_slot;
+        std::vector<uint8_t> run_len;
+        build_chunk_runs(items, woff, tdoc, tslot, (uint32_t)c->a.run_cap, run_slot, run_len);
         for (uint4 &it : items)
             if (it.x != 0xFFFFFFFFu) it.w = glob[woff[it.x]] - woff[it.x];
         ch.n_queues = tiles > 0 ? (uint32_t)std::min(c->n_xcd, 8) : 1u;
@@ -711,54 +746,50 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
             for (uint32_t b = woff[r]; b < woff[r + 1]; b += 32768u)
                 wsegs.push_back(make_uint4((uint32_t)r, b, std::min(b + 32768u, woff[r + 1]), 0u));
         // image
-        size_t o = 4 * (size_t)n;  // z, z_doc
-        o = al16(o);
-        ch.off_doc_info = o;
-        o += sizeof(uint2) * ch.D;
+        size_t o = 2 * (size_t)n;  // z_doc
+        auto place = [&](size_t bytes) {
+            const size_t at = al16(o);
+            o = at + bytes;
+            return at;
+        };
+        ch.off_doc_info = place(sizeof(uint2) * ch.D);
         ch.back_bytes = o;
-        o = al16(o);
-        ch.off_soff = o;
-        o += 4 * ((size_t)ch.D + 1);
-        o = al16(o);
-        ch.off_slot_wrd = o;
-        o += 4 * (size_t)n;
-        o = al16(o);
-        ch.off_slot_tok = o;
-        o += 4 * (size_t)n;
-        o = al16(o);
-        ch.off_items = o;
-        o += sizeof(uint4) * items.size();
-        ch.off_runs = o;
-        o += sizeof(uint4) * runs.size();
-        ch.off_wt_segs = o;
-        o += sizeof(uint4) * wsegs.size();
+        ch.off_soff = place(4 * ((size_t)ch.D + 1));
+        ch.off_items = place(sizeof(uint4) * items.size());
+        ch.off_item_tok = place(4 * items.size());
+        ch.off_run_slot = place(4 * run_slot.size());
+        ch.off_run_len = place(run_len.size());
+        ch.off_wt_segs = place(sizeof(uint4) * wsegs.size());
         ch.bytes = al16(o);
         EZ_TRY_HIP(c, hipHostMalloc((void **)&ch.img, ch.bytes, hipHostMallocDefault));
         std::memset(ch.img, 0, ch.bytes);
         auto put = [&](size_t off, const void *src, size_t bytes) {
             if (bytes) std::memcpy(ch.img + off, src, bytes);
         };
-        put(0, zc.data(), 2 * (size_t)n);
-        put(2 * (size_t)n, zd.data(), 2 * (size_t)n);
+        put(0, zd.data(), 2 * (size_t)n);
         put(ch.off_doc_info, di.data(), sizeof(uint2) * ch.D);
         put(ch.off_soff, soffc.data(), 4 * ((size_t)ch.D + 1));
-        put(ch.off_slot_wrd, swrd.data(), 4 * (size_t)n);
-        put(ch.off_slot_tok, stok.data(), 4 * (size_t)n);
         put(ch.off_items, items.data(), sizeof(uint4) * items.size());
-        put(ch.off_runs, runs.data(), sizeof(uint4) * runs.size());
+        put(ch.off_item_tok, item_tok.data(), 4 * items.size());
+        put(ch.off_run_slot, run_slot.data(), 4 * run_slot.size());
+        put(ch.off_run_len, run_len.data(), run_len.size());
         put(ch.off_wt_segs, wsegs.data(), sizeof(uint4) * wsegs.size());
         ch.n_items = (uint32_t)items.size();
-        ch.n_runs = runs.size();
+        ch.n_runs = run_len.size();
         ch.n_wt_segs = (uint32_t)wsegs.size();
         max_bytes = std::max(max_bytes, ch.bytes);
         max_dt = std::max(max_dt, dtc);
         max_n = std::max(max_n, n);
+        max_runs = std::max(max_runs, ch.n_runs);
         max_items = std::max(max_items, ch.n_items);
         dt_total += dtc;
         items_total += ch.n_items;
         runs_total += (int64_t)ch.n_runs;
     }
-    c->tok_slot_g = tok_slot;
+    c->pos_slot.resize(N);
+    parallel_for((int64_t)N, [&](int64_t b, int64_t e, int) {
+        for (int64_t i = b; i < e; ++i) c->pos_slot[i] = tok_slot[c->doc_tok[i]];
+    });
     // device: two image buffers, the model and the next sweep's counts
     int r = 0;
     const size_t dt_words = compact ? (max_dt + 256 + 1) / 2 : max_dt + 256;
@@ -767,6 +798,9 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
         if ((r = dalloc(c, &c->cdt[j], dt_words))) return r;
         EZ_TRY_HIP(c, hipMemset(c->cdt[j], 0, dt_words * sizeof(uint32_t)));
         if ((r = dalloc(c, &c->caux[j], max_n))) return r;
+        if ((r = dalloc(c, &c->cz[j], max_n))) return r;
+        if ((r = dalloc(c, &c->cwrd[j], max_n))) return r;
+        if ((r = dalloc(c, &c->cruns[j], max_runs))) return r;
         if ((r = dalloc(c, &c->cctr[j], ez::kCounterWords))) return r;
         EZ_TRY_HIP(c, hipMemset(c->cctr[j], 0, ez::kCounterWords * sizeof(uint32_t)));
         if ((r = dalloc(c, &c->cll[j], max_items))) return r;
@@ -813,17 +847,17 @@ ez::DevState chunk_state(const ezlda_ctx *c, int k, int j) {
     cs.N = ch.N;
     cs.VD = c->s.V;
     cs.word_off = nullptr;
-    cs.z = reinterpret_cast<uint16_t *>(img);
-    cs.z_doc = reinterpret_cast<uint16_t *>(img + 2 * (size_t)ch.N);
+    cs.z = c->cz[j];
+    cs.z_doc = reinterpret_cast<uint16_t *>(img);
     cs.doc_info = reinterpret_cast<uint2 *>(img + ch.off_doc_info);
     cs.soff = reinterpret_cast<uint32_t *>(img + ch.off_soff);
-    cs.slot_wrd = reinterpret_cast<uint32_t *>(img + ch.off_slot_wrd);
-    cs.slot_tok = reinterpret_cast<uint32_t *>(img + ch.off_slot_tok);
+    cs.slot_wrd = c->cwrd[j];
+    cs.slot_tok = nullptr;  // read for tail words only
     cs.aux_doc = c->caux[j];
     cs.dt = c->cdt[j];
     cs.smp_segs = reinterpret_cast<uint4 *>(img + ch.off_items);
     cs.n_smp_segs = (int32_t)ch.n_items;
-    cs.runs = reinterpret_cast<uint4 *>(img + ch.off_runs);
+    cs.runs = c->cruns[j];
     cs.n_runs = (int64_t)ch.n_runs;
     cs.wt_segs = reinterpret_cast<uint4 *>(img + ch.off_wt_segs);
     cs.n_wt_segs = (int32_t)ch.n_wt_segs;
@@ -834,12 +868,22 @@ ez::DevState chunk_state(const ezlda_ctx *c, int k, int j) {
     return cs;
 }
 
+ez::ChunkRuns chunk_runs(const ezlda_ctx *c, int k, int j) {
+    const EzChunk &ch = c->chunks[k];
+    ez::ChunkRuns r;
+    r.item_tok = reinterpret_cast<const uint32_t *>(c->cimg[j] + ch.off_item_tok);
+    r.run_slot = reinterpret_cast<const uint32_t *>(c->cimg[j] + ch.off_run_slot);
+    r.run_len = c->cimg[j] + ch.off_run_len;
+    return r;
+}
+
 // Counts of the current topics: every chunk's histogram added up.
 int chunk_prime(ezlda_ctx *c) {
     EZ_TRY_HIP(c, ez::launch_zero_counts(c->s, c->st));
     for (int k = 0; k < (int)c->chunks.size(); ++k) {
         const EzChunk &ch = c->chunks[k];
         EZ_TRY_HIP(c, hipMemcpyAsync(c->cimg[0], ch.img, ch.bytes, hipMemcpyHostToDevice, c->st));
+        EZ_TRY_HIP(c, ez::launch_chunk_topics(chunk_state(c, k, 0), chunk_runs(c, k, 0), c->st));
         EZ_TRY_HIP(c, ez::launch_accumulate_wt(chunk_state(c, k, 0), c->st));
     }
     EZ_TRY_HIP(c, hipStreamSynchronize(c->st));
@@ -850,7 +894,7 @@ int chunk_prime(ezlda_ctx *c) {
 // n sweeps over the chunks; chunk k goes through image buffer k % 2 on its
 // own stream, so one chunk's copies overlap the other's kernels.  Each chunk
 // rebuilds its DT rows, samples against the sweep's model, adds its new
-// topics to the next counts and copies z, z_doc and its row lengths back.
+// topics to the next counts and copies z_doc and its row lengths back.
 int chunk_sweeps(ezlda_ctx *c, int n, hipEvent_t ev_begin, hipEvent_t ev_end) {
     if (!c->counts_fresh)
         if (int r = chunk_prime(c)) return r;
@@ -863,9 +907,21 @@ int chunk_sweeps(ezlda_ctx *c, int n, hipEvent_t ev_begin, hipEvent_t ev_end) {
     auto chk = [&](hipError_t e, const char *what) {
         if (rc == EZLDA_OK && e != hipSuccess) rc = fail(c, EZLDA_EHIP, std::string(what) + ": " + hipGetErrorString(e));
     };
-    if (rc == EZLDA_OK && ev_begin) chk(hipEventRecord(ev_begin, c->st), "hipEventRecord");
-    const size_t vk = (size_t)c->s.V * c->s.K;
+    if (rc == EZLDA_OK && ev_begin) {
+        chk(hipEventRecord(ev_begin, c->st), "hipEventRecord");
+        chk(hipStreamWaitEvent(c->st2, ev_begin, 0), "hipStreamWaitEvent");
+    }
+    auto bring = [&](int k) {
+        const int j = k & 1;
+        chk(hipMemcpyAsync(c->cimg[j], c->chunks[k].img, c->chunks[k].bytes, hipMemcpyHostToDevice, sts[j]),
+            "chunk upload");
+        chk(ez::launch_chunk_runs(chunk_state(c, k, j), chunk_runs(c, k, j), c->sweep, sts[j]), "chunk layout");
+    };
     for (int i = 0; i < n && rc == EZLDA_OK; ++i) {
+        // a stream's first chunk comes in while the other stream ends the
+        // sweep before: it needs nothing of the model
+        for (int k = 0; k < std::min<int>(2, (int)c->chunks.size()); ++k) bring(k);
+        if (i) chk(hipStreamWaitEvent(c->st, e_done, 0), "hipStreamWaitEvent");
         chk(ez::launch_topk(c->s, c->st), "top-3");
         ez::DevState nx = c->s;  // zero the next counts
         nx.wt_head = c->wt_next;
@@ -879,10 +935,9 @@ int chunk_sweeps(ezlda_ctx *c, int n, hipEvent_t ev_begin, hipEvent_t ev_end) {
             hipStream_t st = sts[j];
             const EzChunk &ch = c->chunks[k];
             const ez::DevState cs = chunk_state(c, k, j);
-            chk(hipMemcpyAsync(c->cimg[j], ch.img, ch.bytes, hipMemcpyHostToDevice, st), "chunk upload");
-            chk(ez::launch_set_u32(cs.counters, c->sweep, st), "sweep counter");
+            if (k >= 2) bring(k);
             chk(ez::launch_build_dt(cs, st), "DT rebuild");
-            chk(ez::launch_sample(cs, c->a.shortcut != 0, st), "sample");
+            chk(ez::launch_sample(cs, c->a.shortcut != 0, st, ez::kSampleHead | ez::kSampleTail, true), "sample");
             ez::DevState acc = cs;
             acc.wt_head = c->wt_next;
             acc.nk = c->nk_next;
@@ -890,12 +945,12 @@ int chunk_sweeps(ezlda_ctx *c, int n, hipEvent_t ev_begin, hipEvent_t ev_end) {
             chk(hipMemcpyAsync(ch.img, c->cimg[j], ch.back_bytes, hipMemcpyDeviceToHost, st), "chunk download");
         }
         chk(hipEventRecord(e_done, c->st2), "hipEventRecord");
-        chk(hipStreamWaitEvent(c->st, e_done, 0), "hipStreamWaitEvent");
         std::swap(c->s.wt_head, c->wt_next);
         std::swap(c->s.nk, c->nk_next);
         c->sweep++;
-        (void)vk;
     }
+    if (rc == EZLDA_OK && n > 0) chk(hipStreamWaitEvent(c->st, e_done, 0), "hipStreamWaitEvent");
+    if (rc != EZLDA_OK) (void)hipStreamSynchronize(c->st2);
     if (rc == EZLDA_OK && ev_end) chk(hipEventRecord(ev_end, c->st), "hipEventRecord");
     chk(hipStreamSynchronize(c->st), "chunked sweep");
     if (e_start) (void)hipEventDestroy(e_start);
@@ -1156,7 +1211,7 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
         s.seed = c->a.seed;
         c->dt_cap_canon = 0;
         for (int d = 0; d < D; ++d) c->dt_cap_canon += dt_cap(c->doc_off[d + 1] - c->doc_off[d], K);
-        if (int r = load_chunked(c, tok_doc, tok_slot, slot_wrd, z, z_doc)) return r;
+        if (int r = load_chunked(c, tok_doc, tok_slot, slot_wrd, z_doc)) return r;
         c->sweep = 0;
         c->counts_fresh = false;
         c->loaded = true;
@@ -1679,6 +1734,7 @@ int loglik_into(ezlda_ctx *c, double *ll, double *part, double *out) {
             }
             double v = 0.0;
             EZ_TRY_HIP(c, hipMemcpyAsync(c->cimg[0], ch.img, ch.bytes, hipMemcpyHostToDevice, c->st));
+            EZ_TRY_HIP(c, ez::launch_chunk_runs(cs, chunk_runs(c, k, 0), c->sweep, c->st));
             EZ_TRY_HIP(c, ez::launch_build_dt(cs, c->st));
             EZ_TRY_HIP(c, ez::launch_loglik(cs, c->st));
             EZ_TRY_HIP(c, hipMemcpyAsync(&v, cs.ll_out, sizeof(double), hipMemcpyDeviceToHost, c->st));
@@ -1793,10 +1849,17 @@ int ezlda_get_topics(ezlda_ctx *c, uint16_t *zout) try {
     if (int r = need_loaded(c)) return r;
     if (is_chunked(c)) {  // from the chunk images (z by doc slot)
         parallel_for((int64_t)c->doc_tok.size(), [&](int64_t b, int64_t e, int) {
+            const uint16_t *zd = nullptr;
+            uint32_t slot0 = 0, n = 0;
             for (int64_t i = b; i < e; ++i) {
-                const uint32_t p = c->tok_slot_g[c->doc_tok[i]];
-                const EzChunk &ch = c->chunks[chunk_of_slot(c, p)];
-                zout[i] = reinterpret_cast<const uint16_t *>(ch.img + 2 * (size_t)ch.N)[p - ch.slot0];
+                const uint32_t p = c->pos_slot[i];
+                if (p - slot0 >= n) {  // the next document, of another chunk
+                    const EzChunk &ch = c->chunks[chunk_of_slot(c, p)];
+                    zd = reinterpret_cast<const uint16_t *>(ch.img);
+                    slot0 = ch.slot0;
+                    n = ch.N;
+                }
+                zout[i] = zd[p - slot0];
             }
         });
         return EZLDA_OK;
@@ -1812,12 +1875,9 @@ int ezlda_set_topics(ezlda_ctx *c, const uint16_t *zin) try {
         for (size_t i = 0; i < c->doc_tok.size(); ++i)
             if (zin[i] >= c->s.K) return fail(c, EZLDA_EINVAL, "topic out of range");
         for (size_t i = 0; i < c->doc_tok.size(); ++i) {
-            const uint32_t p = c->tok_slot_g[c->doc_tok[i]];
+            const uint32_t p = c->pos_slot[i];
             EzChunk &ch = c->chunks[chunk_of_slot(c, p)];
-            const uint32_t pp = p - ch.slot0;
-            const uint32_t l = reinterpret_cast<const uint32_t *>(ch.img + ch.off_slot_tok)[pp];
-            reinterpret_cast<uint16_t *>(ch.img)[l] = zin[i];
-            reinterpret_cast<uint16_t *>(ch.img + 2 * (size_t)ch.N)[pp] = zin[i];
+            reinterpret_cast<uint16_t *>(ch.img)[p - ch.slot0] = zin[i];
         }
         c->counts_fresh = false;
         return EZLDA_OK;

@@ -151,3 +151,34 @@ def test_groups_of_small_words(K, kw):
     orc.sweep(1)
     assert np.array_equal(ctx.get_topics(), orc.get_topics())
     ctx.close()
+
+
+@pytest.mark.parametrize("D,V,mean,chunks,run_cap", [(3, 2, 300, 3, 32),      # runs of every length, chunks of one document
+                                                     (700, 1, 3, 2, 4),       # one word: items of many runs, empty documents
+                                                     (129, 4000, 40, 2, 1),   # runs of one token
+                                                     (2500, 30, 25, 2, 5)])   # items above and below 64 runs
+def test_chunk_layouts_made_on_the_device(D, V, mean, chunks, run_cap):
+    """A chunk's runs, ordered and numbered on the device from their slots and
+    lengths: topics, model and draw counts equal to the resident layout's and
+    the oracle's (exact)."""
+    rng = np.random.default_rng(D)
+    lens = rng.integers(0, 2 * mean + 1, D)
+    lens[0] = mean
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    words = np.minimum(rng.integers(0, V, off[-1]), rng.integers(0, V, off[-1])).astype(np.int32)
+    K = 48
+    res = ezlda.Context(K=K, alpha=50.0 / K, beta=0.01, seed=9, run_cap=run_cap)
+    chk = ezlda.Context(K=K, alpha=50.0 / K, beta=0.01, seed=9, run_cap=run_cap, num_chunks=chunks)
+    orc = ob.Oracle(K, float(np.float32(50.0 / K)), 0.01, 9, V, off, words)
+    for c in (res, chk):
+        c.load(ezlda.Corpus(V, off, words))
+        c.sweep(3)
+    orc.sweep(3)
+    assert np.array_equal(chk.get_topics(), orc.get_topics())
+    assert np.array_equal(res.get_topics(), orc.get_topics())
+    assert abs(chk.loglik() - res.loglik()) <= 1e-9 * abs(res.loglik())
+    chk.set_topics(orc.get_topics())
+    chk.sweep(1)
+    orc.sweep(1)
+    assert np.array_equal(chk.get_topics(), orc.get_topics())
+    assert chk.info().num_chunks == min(chunks, D)
