@@ -9,9 +9,10 @@ namespace ez {
 
 // Sweep counter and persistent-sampler queue heads: each head on its own
 // 128-byte line, so the workgroups claiming items from different queues do
-// not serialize on one line.
-static constexpr int kQueueStride = 32;
-static constexpr int kCounterWords = kQueueStride * 9;
+// not serialize on one line.  kQueues heads for workgroups, as many for the
+// wavefronts of k_sample_own.
+static constexpr int kQueueStride = 32, kQueues = 8;
+static constexpr int kCounterWords = kQueueStride * (1 + 2 * kQueues);
 // Documents of at most this many tokens can have their DT rows built by
 // sorting their topics (large K); longer ones use a K-sized histogram.
 static constexpr uint32_t kDtShort = 512;
@@ -22,6 +23,9 @@ static constexpr uint32_t kDtShort = 512;
 // carries its word's place in the group.
 static constexpr uint32_t kGroupShift = 26, kGroupWord = (1u << kGroupShift) - 1u, kGroupMax = 32;
 static constexpr int kGroupMaxK = 512;
+// Tail words of at most kOwnMax tokens are drawn by half a wavefront each
+// where DT rows are of 32-bit entries.
+static constexpr uint32_t kOwnMax = 128;
 
 // Device image of one corpus + model.  Token ids are word-major positions;
 // N < 2^32.  Sizes: V words, VD head words, D docs, K topics.
@@ -63,6 +67,7 @@ struct DevState {
     uint4 *smp_segs = nullptr;      // sampler items (w | further words << kGroupShift, first run, end run,
                                     // draw-key offset)
     int32_t n_smp_segs = 0;
+    int32_t first_own = INT32_MAX;  // items from here on: whole or cut tail words of at most kOwnMax tokens
     int32_t group_words = 1;        // words of the largest group item
     uint4 *runs = nullptr;          // (first token, first slot, doc's DT row offset, tokens | group place << 8 | doc length << 16):
                                     // a word's tokens in one doc

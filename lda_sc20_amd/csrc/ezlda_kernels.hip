@@ -1019,9 +1019,33 @@ __device__ __forceinline__ C16x2 c16_x2(uint32_t w, uint32_t tb, uint32_t tm2, u
 __device__ __forceinline__ float fma_count(_Float16 c, float phi, float s) { return __builtin_fmaf((float)c, phi, s); }
 __device__ __forceinline__ float phi_a(uint32_t a) { return *(lds_cfloat *)a; }
 
+// A word's phi as the topics without a count, which its workgroup's words
+// share (at LDS address 0), and the word's own values: by topic word (32
+// topics) the bits of the topics it has and the LDS float index of the first
+// one's value (uint2 at LDS address lb + 8 * (k / 32)).
+typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
+__device__ __forceinline__ float phi_own(uint32_t k, uint32_t lb) {
+    lds_cu32 *p = (lds_cu32 *)(lb + ((k >> 2) & ~7u));
+    const uint32_t bits = p[0], first = p[1];
+    const uint32_t i = first + (uint32_t)__popc(bits & ((1u << (k & 31u)) - 1u));
+    return phi_a(((bits >> (k & 31u)) & 1u ? i : k) << 2);
+}
+
+// Where a lane's phi is: one table at LDS address 0, its word's table at LDS
+// address lb, or the two of phi_own.
+enum PhiAt { kPhiOne, kPhiGroup, kPhiOwn };
+
 // The entries of one 16-byte load, in order.
-template <bool COMPACT, bool MULTI>
+template <bool COMPACT, PhiAt P>
 __device__ __forceinline__ float sum_u4(const uint4 &e, float s, uint32_t tb, uint32_t lb) {
+    constexpr bool MULTI = P == kPhiGroup;
+    static_assert(P != kPhiOwn || !COMPACT, "phi_own is for 32-bit rows");
+    if (P == kPhiOwn) {
+        s = __builtin_fmaf(dt_count(e.x), phi_own(dt_topic(e.x), lb), s);
+        s = __builtin_fmaf(dt_count(e.y), phi_own(dt_topic(e.y), lb), s);
+        s = __builtin_fmaf(dt_count(e.z), phi_own(dt_topic(e.z), lb), s);
+        return __builtin_fmaf(dt_count(e.w), phi_own(dt_topic(e.w), lb), s);
+    }
     if (COMPACT) {  // two 16-bit entries per dword, low half first
         const uint32_t w[4] = {e.x, e.y, e.z, e.w};
         const uint32_t tm2 = ((1u << tb) - 1u) * 0x10001u;
@@ -1042,12 +1066,12 @@ __device__ __forceinline__ float sum_u4(const uint4 &e, float s, uint32_t tb, ui
 
 // The block's entries in order; `half` gets the running sum after its
 // first kBlkU4 / 2 loads.
-template <bool COMPACT, bool MULTI>
+template <bool COMPACT, PhiAt P>
 __device__ __forceinline__ float sum_block(const RowBlock &r, float s, uint32_t tb, uint32_t lb,
                                            float &half) {
 #pragma unroll
     for (int i = 0; i < kBlkU4; ++i) {
-        s = sum_u4<COMPACT, MULTI>(r.e[i], s, tb, lb);
+        s = sum_u4<COMPACT, P>(r.e[i], s, tb, lb);
         if (i == kBlkU4 / 2 - 1) half = s;
     }
     return s;
@@ -1056,9 +1080,11 @@ __device__ __forceinline__ float sum_block(const RowBlock &r, float s, uint32_t 
 // S-bucket search over n consecutive 16-byte pieces of a row from running
 // sum `run`: the first entry whose running sum exceeds t2 (running sums never
 // decrease).
-template <bool COMPACT, bool MULTI, int N>
+template <bool COMPACT, PhiAt P, int N>
 __device__ __forceinline__ void search_u4(const uint4 (&blk)[N], float &run, float t2, uint32_t tb, uint32_t lb,
                                           uint32_t &newz, bool &found) {
+    constexpr bool MULTI = P == kPhiGroup;
+    auto at32 = [&](uint32_t e) { return P == kPhiOwn ? phi_own(dt_topic(e), lb) : phi_at0(e); };
 #pragma unroll
     for (int gi = 0; gi < N; ++gi) {
         const uint4 e = blk[gi];
@@ -1080,10 +1106,10 @@ __device__ __forceinline__ void search_u4(const uint4 (&blk)[N], float &run, flo
                 run = rb;
             }
         } else if (!found) {
-            const float r0 = __builtin_fmaf(dt_count(e.x), phi_at0(e.x), run);
-            const float r1 = __builtin_fmaf(dt_count(e.y), phi_at0(e.y), r0);
-            const float r2 = __builtin_fmaf(dt_count(e.z), phi_at0(e.z), r1);
-            const float r3 = __builtin_fmaf(dt_count(e.w), phi_at0(e.w), r2);
+            const float r0 = __builtin_fmaf(dt_count(e.x), at32(e.x), run);
+            const float r1 = __builtin_fmaf(dt_count(e.y), at32(e.y), r0);
+            const float r2 = __builtin_fmaf(dt_count(e.z), at32(e.z), r1);
+            const float r3 = __builtin_fmaf(dt_count(e.w), at32(e.w), r2);
             if (r3 > t2) {
                 newz = dt_topic(r0 > t2 ? e.x : r1 > t2 ? e.y : r2 > t2 ? e.z : e.w);
                 found = true;
@@ -1112,6 +1138,7 @@ struct SampleArgs {
     const uint4 *segs;
     const uint4 *runs;  // (first token, first doc slot, the doc's DT row offset, tokens | doc length << 16)
     uint32_t n_items;
+    uint32_t first_item;  // k_sample_own: its first
     int VD, K;
     float alpha, beta;
     const int32_t *wt_head;
@@ -1302,19 +1329,155 @@ __device__ __forceinline__ void stage_group(const SampleArgs &A, int w, int G, i
     __syncthreads();
 }
 
-template <bool SHORTCUT, bool COMPACT, bool QTAB, bool MULTI>
+// LDS floats of k_sample_own: of what all words of a workgroup share (phi of
+// the topics without a count, its slab totals), and of one word (its topics'
+// bits and first values, its values, its slabs' running sums, the list of the
+// slabs with topics of its own).
+__host__ __device__ __forceinline__ int own_shared(int NS) { return (NS * 65 + 3) & ~3; }
+__host__ __device__ __forceinline__ int own_stride(int NS) {
+    return NS * 4 + (int)kOwnMax + 4 + ((NS + 3) & ~3) + (int)kOwnMax / 4 + 4;
+}
+
+// The tables of a tail word of at most kOwnMax tokens, by half a wavefront:
+// see phi_own.  f1 and f2 as in sample_item.
+__device__ __forceinline__ void stage_own(const SampleArgs &A, int w, ushort4 tp, float *phi0, float *mine, float &f1,
+                                          float &f2) {
+    const int K = A.K, NS = (K + 63) >> 6, NW = NS * 2, l = threadIdx.x & 31;
+    const uint32_t half = threadIdx.x & 32u;
+    const float alpha = A.alpha, beta = A.beta;
+    constexpr int U = kOwnMax / 32;
+    const float *qt_shared = phi0 + NS * 64;
+    uint2 *bp = reinterpret_cast<uint2 *>(mine);
+    float *val = mine + 2 * NW, *qacc = val + kOwnMax + 4;
+    uint8_t *touched = reinterpret_cast<uint8_t *>(qacc + ((NS + 3) & ~3));
+    const uint32_t lb = 4u * (uint32_t)(mine - phi0), at0 = (uint32_t)(val - phi0);
+    wave_lds_sync();  // the words before are done with them
+    for (int i = l; i < NS; i += 32) reinterpret_cast<uint4 *>(bp)[i] = make_uint4(0u, 0u, 0u, 0u);
+    // the word's topics: four a lane
+    const uint32_t b = A.tail_off[w - A.VD], n = A.tail_nnz[w - A.VD];
+    uint32_t e[U];
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) e[u] = (uint32_t)(l + 32 * u) < n ? A.wt_tail[b + l + 32 * u] : 0u;
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = A.inv[e[u] & 0xFFFFu];
+    wave_lds_sync();
+    // bits of its topics and of its top one, then the index of each 32's first value
+    const uint32_t k1 = tp.x;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if ((uint32_t)(l + 32 * u) < n) atomicOr(&bp[(e[u] & 0xFFFFu) >> 5].x, 1u << (e[u] & 31u));
+    if (l == 0) atomicOr(&bp[k1 >> 5].x, 1u << (k1 & 31u));
+    wave_lds_sync();
+    {
+        const int per = (NW + 31) >> 5, i0 = l * per, i1 = min(NW, i0 + per);
+        uint32_t m = 0;
+        for (int i = i0; i < i1; ++i) m += (uint32_t)__popc(bp[i].x);
+        uint32_t incl = m;
+        for (int d = 1; d < 32; d <<= 1) {
+            const uint32_t x = __shfl_up(incl, d, 32);
+            if (l >= d) incl += x;
+        }
+        uint32_t at = at0 + incl - m;
+        for (int i = i0; i < i1; ++i) {
+            bp[i].y = at;
+            at += (uint32_t)__popc(bp[i].x);
+        }
+    }
+    wave_lds_sync();
+    auto index = [&](uint32_t k) {
+        const uint2 x = bp[k >> 5];
+        return x.y + (uint32_t)__popc(x.x & ((1u << (k & 31u)) - 1u));
+    };
+    if (l == 0) phi0[index(k1)] = phi0[k1];  // it may have no count
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if ((uint32_t)(l + 32 * u) < n) phi0[index(e[u] & 0xFFFFu)] = ((float)(e[u] >> 16) + beta) * v[u];
+    wave_lds_sync();
+    f1 = phi_own(k1, lb);
+    f2 = tp.y != kNone ? phi_own(tp.y, lb) : 0.0f;
+    wave_lds_sync();
+    if (l == 0) phi0[index(k1)] = 0.0f;
+    wave_lds_sync();
+    // slab totals: the shared ones, and those of the slabs with topics of the
+    // word's own, summed in the order of sample_item; then their running sums
+    uint32_t nt = 0;
+    for (int j0 = 0; j0 < ((NS + 3) & ~3); j0 += 32) {
+        const int j = j0 + l;
+        const bool t = j < NS && (bp[2 * j].x | bp[2 * j + 1].x) != 0u;
+        if (j < ((NS + 3) & ~3) && !t) qacc[j] = j < NS ? qt_shared[j] : 0.0f;
+        const uint32_t m = (uint32_t)(__ballot(t) >> half);
+        if (t) touched[nt + (uint32_t)__popc(m & ((1u << l) - 1u))] = (uint8_t)j;
+        nt += (uint32_t)__popc(m);
+    }
+    wave_lds_sync();
+    for (uint32_t i = l; i < nt; i += 32) {
+        const int j = (int)touched[i];
+        const float4 *p4 = reinterpret_cast<const float4 *>(phi0 + j * 64);
+        const uint4 b4 = reinterpret_cast<const uint4 *>(bp)[j];
+        const uint32_t bits[2] = {b4.x, b4.z};
+        uint32_t at = b4.y;
+        float run = 0.0f;
+#pragma unroll
+        for (int i4 = 0; i4 < 16; i4 += 4) {
+            float4 x4[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x4[u] = p4[i4 + u];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                float x[4] = {x4[u].x, x4[u].y, x4[u].z, x4[u].w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    if ((bits[i4 >> 3] >> (((4 * i4) & 31) + 4 * u + c)) & 1u) x[c] = phi0[at++];
+                    run = run + alpha * x[c];
+                }
+            }
+        }
+        qacc[j] = run;
+    }
+    wave_lds_sync();
+    float acc = 0.0f;
+    float4 *q4 = reinterpret_cast<float4 *>(qacc);
+    for (int j0 = 0; j0 < ((NS + 3) >> 2); j0 += 4) {  // by every lane, the half's first one writes
+        float4 x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = j0 + i < ((NS + 3) >> 2) ? q4[j0 + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[i].x = acc = acc + x[i].x;
+            x[i].y = acc = acc + x[i].y;
+            x[i].z = acc = acc + x[i].z;
+            x[i].w = acc = acc + x[i].w;
+        }
+        if (l == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (j0 + i < ((NS + 3) >> 2)) q4[j0 + i] = x[i];
+        }
+    }
+    wave_lds_sync();
+}
+
+// (kPhiOwn: the item and its tables f123 are those of the lane's half
+// wavefront; without `any`, it draws nothing)
+template <bool SHORTCUT, bool COMPACT, bool QTAB, PhiAt P>
 __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, float *smf, float *f123,
-                                            uint32_t sweep, uint32_t &n_full, uint32_t &n_scanned) {
+                                            uint32_t sweep, uint32_t &n_full, uint32_t &n_scanned, bool any = true) {
     const int K = A.K, NS = (K + 63) >> 6;
     const float alpha = A.alpha, beta = A.beta;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
+    const int tid = threadIdx.x, lane = P == kPhiOwn ? tid & 31 : tid & 63, wv = P == kPhiOwn ? 0 : tid >> 6,
+              nwv = P == kPhiOwn ? 1 : blockDim.x >> 6;
     constexpr bool qtab = QTAB;  // K <= EZ_Q_TABLE_MAX_K
+    constexpr bool MULTI = P == kPhiGroup;
+    constexpr bool OWN = P == kPhiOwn;
+    const uint32_t own = OWN ? 4u * (uint32_t)(f123 - smf) : 0u;
     constexpr int CP = Checkpoints<COMPACT, QTAB, MULTI>::CP, CF = Checkpoints<COMPACT, QTAB, MULTI>::CF;
     constexpr float up = COMPACT ? kPhiUp : 1.0f, down = COMPACT ? kPhiDown : 1.0f;
     float *phi0 = smf;                         // NS*64
     float *qs0 = phi0 + NS * 64;                // NS*64 when qtab: running sums inside each slab
     float *qt0 = qs0 + (qtab ? NS * 64 : 0);    // NS: slab totals
-    float *qacc0 = qt0 + NS;                    // NS: running sum of the slab totals
+    float *qacc0 = OWN ? f123 + NS * 4 + kOwnMax + 4 : qt0 + NS;                    // NS: running sum of the slab totals
     const uint4 sg = A.segs[item];
     if (sg.x == 0xFFFFFFFFu) return;  // padding item (uniform over the block)
     // MULTI: the item's words are w .. w + G - 1, word g's tables at g * ST
@@ -1324,8 +1487,11 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
     if (!(A.mode & (w < A.VD ? kSampleHead : kSampleTail))) return;  // the other words' stage
     const bool sc_only = (A.mode & kShortcutOnly) != 0;
     const ushort4 tp = MULTI ? make_ushort4(0, 0, 0, 0) : A.wtop[w];
+    float fo1 = 0.0f, fo2 = 0.0f;
     if (MULTI) {
         stage_group<COMPACT>(A, w, G, ST, smf);
+    } else if (OWN) {
+        stage_own(A, w, tp, smf, f123, fo1, fo2);
     } else {
         if (w < A.VD) {
             stage_phi<true>(phi0, A.wt_head + (size_t)w * K, A.inv, K, NS, beta, up);
@@ -1402,21 +1568,23 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
         }
         __syncthreads();
     }
-    const float Q1 = MULTI ? 0.0f : qacc0[NS - 1], f11 = MULTI ? 0.0f : f123[0], f21 = MULTI ? 0.0f : f123[1];
+    const float Q1 = MULTI ? 0.0f : qacc0[NS - 1], f11 = MULTI ? 0.0f : OWN ? fo1 : f123[0],
+                f21 = MULTI ? 0.0f : OWN ? fo2 : f123[1];
     // head words also write the doc-slot copy of z (their items share a doc
     // tile, so the copy's lines fill in L2); tail tokens, in random docs,
     // are read back by token id in the DT rebuild instead
     const bool head = w < A.VD;
     const uint32_t tb = A.tb;
 
-    for (uint32_t base = sg.y + (uint32_t)wv * 64u; base < sg.z; base += (uint32_t)nwv * 64u) {
+    if (OWN && !any) return;
+    for (uint32_t base = sg.y + (uint32_t)wv * 64u; base < sg.z; base += OWN ? 32u : (uint32_t)nwv * 64u) {
         const uint32_t r = base + (uint32_t)lane;
         if (r >= sg.z) break;
         const uint4 rn = A.runs[r];
         const uint32_t t0 = rn.x, p0 = rn.y, nd = rn.w >> 16;
         uint32_t len = rn.w & (MULTI ? 0xFFu : 0xFFFFu);
         // the run's word: its tables and what the draws need of it
-        const uint32_t go = MULTI ? ((rn.w >> 8) & 0xFFu) * (uint32_t)ST : 0u, lb = 4u * go;
+        const uint32_t go = MULTI ? ((rn.w >> 8) & 0xFFu) * (uint32_t)ST : 0u, lb = MULTI ? 4u * go : own;
         const float *phi = phi0 + go, *qs = qs0 + go, *qt = qt0 + go, *qacc = qacc0 + go;
         const float *wc = qacc + NS;  // MULTI: f1, f2, k1
         const float Q = MULTI ? qacc[NS - 1] : Q1, f1 = MULTI ? wc[0] : f11, f2 = MULTI ? wc[1] : f21;
@@ -1491,7 +1659,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
             RowBlock nxt;
             if ((uint32_t)b + 1u < nb) nxt = load_block(rp + kBlkU4 * (b + 1));
             ch[b] = S;
-            if ((uint32_t)b < nb) S = sum_block<COMPACT, MULTI>(cur, S, tb, lb, ch[b]);
+            if ((uint32_t)b < nb) S = sum_block<COMPACT, P>(cur, S, tb, lb, ch[b]);
             cp[b] = S;
             cur = nxt;
         }
@@ -1506,7 +1674,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                 RowBlock nxt;
                 if (b + 1u < nb) nxt = load_block(rp + kBlkU4 * (b + 1u));
                 float unused;
-                if (b < nb) S = sum_block<COMPACT, MULTI>(cur, S, tb, lb, unused);
+                if (b < nb) S = sum_block<COMPACT, P>(cur, S, tb, lb, unused);
                 cur = nxt;
             }
 #pragma unroll
@@ -1568,7 +1736,13 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                     if (qacc[mid] > t2) hi = mid; else lo = mid + 1;
                 }
                 int js = lo < NS ? lo : -1;
-                if (js < 0)
+                if (js < 0 && OWN)  // the last slab with mass
+                    for (int k = K - 1; k >= 0; --k)
+                        if (alpha * (phi_own((uint32_t)k, lb) * down) > 0.0f) {
+                            js = k >> 6;
+                            break;
+                        }
+                if (js < 0 && !OWN)
                     for (int jj = NS - 1; jj >= 0; --jj)
                         if (qt[jj] > 0.0f) {
                             js = jj;
@@ -1590,16 +1764,25 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                     // its total was summed: the first above t3
                     const float4 *p4 = reinterpret_cast<const float4 *>(phi + k0);
                     float run = 0.0f;
+                    uint32_t bits[2] = {0u, 0u}, own_at = 0;  // the word's own topics of the slab, their next value
+                    if (P == kPhiOwn) {
+                        lds_cu32 *p = (lds_cu32 *)(lb + 16u * (uint32_t)js);
+                        bits[0] = p[0], bits[1] = p[2], own_at = 4u * p[1];
+                    }
                     for (int i4 = 0; i4 < 16 && !qtab && lo == ke; i4 += 4) {
                         float4 v[4];
 #pragma unroll
                         for (int u = 0; u < 4; ++u) v[u] = p4[i4 + u];
 #pragma unroll
                         for (int u = 0; u < 4; ++u) {
-                            const float x[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+                            float x[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
 #pragma unroll
                             for (int c = 0; c < 4; ++c) {
                                 const int k = k0 + 4 * (i4 + u) + c;
+                                if (P == kPhiOwn && ((bits[i4 >> 3] >> (((4 * i4) & 31) + 4 * u + c)) & 1u)) {
+                                    x[c] = phi_a(own_at);
+                                    own_at += 4u;
+                                }
                                 run = run + alpha * (x[c] * down);
                                 if (lo == ke && k < ke && run > t3) lo = k;
                             }
@@ -1609,7 +1792,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                         newz = (uint32_t)lo;
                     } else {
                         for (int k = ke - 1; k >= k0; --k)
-                            if (alpha * (phi[k] * down) > 0.0f) {
+                            if (alpha * ((P == kPhiOwn ? phi_own((uint32_t)k, lb) : phi[k]) * down) > 0.0f) {
                                 newz = (uint32_t)k;
                                 break;
                             }
@@ -1619,7 +1802,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
             if (in_s) {
                 bool found = false;
                 if (bs >= 0) {
-                    search_u4<COMPACT, MULTI, NH>(blk, run, t2s, tb, lb, newz, found);
+                    search_u4<COMPACT, P, NH>(blk, run, t2s, tb, lb, newz, found);
                 } else if (nb > (uint32_t)CP) {
                     // past them: the blocks of the far checkpoint that holds
                     // the target, in order
@@ -1632,7 +1815,7 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                             run = cf[i];
                         }
                     for (uint32_t gb = g0; gb < nb && !found; ++gb)
-                        search_u4<COMPACT, MULTI, kBlkU4>(load_block(rp + kBlkU4 * gb).e, run, t2s, tb, lb, newz,
+                        search_u4<COMPACT, P, kBlkU4>(load_block(rp + kBlkU4 * gb).e, run, t2s, tb, lb, newz,
                                                             found);
                 }
                 if (!found) {  // rounding left every running sum at or below t2
@@ -1643,7 +1826,9 @@ __device__ __forceinline__ void sample_item(const SampleArgs &A, uint32_t item, 
                     } else {
                         const uint32_t *rr = A.dt + di.x;
                         for (uint32_t i = 0; i < nnz; ++i)
-                            if (dt_count(rr[i]) > 0.0f && phi_at0(rr[i]) > 0.0f) newz = dt_topic(rr[i]);
+                            if (dt_count(rr[i]) > 0.0f &&
+                                (P == kPhiOwn ? phi_own(dt_topic(rr[i]), lb) : phi_at0(rr[i])) > 0.0f)
+                                newz = dt_topic(rr[i]);
                     }
                 }
             }
@@ -1685,10 +1870,70 @@ __global__ void __launch_bounds__(1024) k_sample(const SampleArgs A) {
             }
             if (item >= A.n_items) break;
             if (own && i) __syncthreads();
-            sample_item<SHORTCUT, COMPACT, QTAB, MULTI>(A, (uint32_t)item, smf, f123, sweep, n_full, n_scanned);
+            sample_item<SHORTCUT, COMPACT, QTAB, MULTI ? kPhiGroup : kPhiOne>(A, (uint32_t)item, smf, f123, sweep, n_full, n_scanned);
         }
     }
     // per-wavefront totals of the counters
+    const int lane = threadIdx.x & 63;
+    for (int off = 32; off >= 1; off >>= 1) {
+        n_full += __shfl_xor(n_full, off);
+        n_scanned += __shfl_xor(n_scanned, off);
+    }
+    if (lane == 0 && n_full) {
+        atomicAdd(&A.stats[0], (unsigned long long)n_full);
+        atomicAdd(&A.stats[1], (unsigned long long)n_scanned);
+    }
+}
+
+// Tail words of at most kOwnMax tokens (32-bit rows), two a wavefront: what
+// their phi has in common is staged once for the whole launch and a word adds
+// its own few values (phi_own), so a CU works on 32 words at a time, without
+// barriers, where three workgroups with a table each fit (K = 10000) and wait
+// for memory in 78% of their cycles.  Bound by the VALU (a lookup is 11
+// operations where one table takes one) and by lanes without a run: a word a
+// wavefront took 412 us where two take 312.  Sampler ms a sweep, with a table
+// a word / with this: 4.5M tokens in short documents at K = 10000 1.11 / 0.74,
+// 16383 1.84 / 0.90; 3.2M heavy-tailed at K = 10000 7.57 / 3.80; 3M tokens of
+// 60,000 equally frequent words at K = 8200 2.42 / 1.14, 10000 3.06 / 1.16.
+// In 16-bit rows (K <= 8192) an entry takes 3.5 operations and 4 to 16 tables
+// fit: there it lost (a word a wavefront at K = 4096: 0.96 / 1.63 and, heavy-
+// tailed, 1.76 / 4.84; K = 7000 0.80 / 0.72).  Items from first_item on, in
+// pairs from a queue an XCD (dealt in turn, 320 us and 4.29 ms heavy-tailed).
+template <bool SHORTCUT>
+__global__ void __launch_bounds__(1024) k_sample_own(const SampleArgs A) {
+    extern __shared__ float smf[];  // the only LDS: phi at address 0
+    const int NS = (A.K + 63) >> 6, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+    const uint32_t sweep = A.counters[0];
+    uint32_t n_full = 0, n_scanned = 0;
+    stage_phi<false>(smf, nullptr, A.inv, A.K, NS, A.beta, 1.0f);
+    __syncthreads();
+    for (int j = threadIdx.x; j < NS; j += blockDim.x) {
+        const float *p = smf + j * 64;
+        float run = 0.0f;
+        for (int i = 0; i < 64; ++i) run = run + A.alpha * p[i];
+        smf[NS * 64 + j] = run;
+    }
+    __syncthreads();
+    const uint32_t h = (threadIdx.x >> 5) & 1u;
+    float *mine = smf + own_shared(NS) + (2 * wv + (int)h) * own_stride(NS);
+    // queue q: the pairs of items with index = q mod kQueues, of which a
+    // wavefront claims its next one while it draws the last
+    const uint32_t q = blockIdx.x % kQueues, n_pairs = (A.n_items - A.first_item + 1u) / 2u;
+    uint32_t *head = A.queue + kQueueStride * (kQueues + q);
+    auto claim = [&]() {
+        uint32_t c = 0;
+        if ((threadIdx.x & 63u) == 0) c = atomicAdd(head, 1u);
+        return c;
+    };
+    uint32_t next = claim();
+    for (;;) {
+        const uint32_t pair = q + kQueues * (uint32_t)__builtin_amdgcn_readfirstlane((int)next);
+        if (pair >= n_pairs) break;
+        next = claim();
+        const uint32_t at = A.first_item + 2u * pair;
+        const bool any = at + h < A.n_items;
+        sample_item<SHORTCUT, false, false, kPhiOwn>(A, at + (any ? h : 0u), smf, mine, sweep, n_full, n_scanned, any);
+    }
     const int lane = threadIdx.x & 63;
     for (int off = 32; off >= 1; off >>= 1) {
         n_full += __shfl_xor(n_full, off);
@@ -2873,14 +3118,14 @@ hipError_t launch_set_u32(uint32_t *p, uint32_t v, hipStream_t st) {
 // of every sweep, nearly all of it the launches: 43.2 -> 38.7 us a sweep on 18,000
 // tokens.
 __global__ void __launch_bounds__(256) k_begin(uint32_t *__restrict__ wt, size_t n, uint32_t *__restrict__ nk, int K,
-                                               uint32_t *__restrict__ counters, uint32_t n_queues) {
+                                               uint32_t *__restrict__ counters) {
     const size_t gid = (size_t)blockIdx.x * 256u + threadIdx.x, stride = (size_t)gridDim.x * 256u;
     uint4 *w4 = reinterpret_cast<uint4 *>(wt);
     for (size_t i = gid; i < n / 4; i += stride) w4[i] = make_uint4(0u, 0u, 0u, 0u);
     if (gid < (n & 3u)) wt[(n & ~(size_t)3u) + gid] = 0u;
     for (size_t i = gid; i < (size_t)K; i += stride) nk[i] = 0u;
     if (counters) {
-        if (gid < n_queues) counters[kQueueStride * (gid + 1)] = 0u;
+        if (gid < 2 * kQueues) counters[kQueueStride * (gid + 1)] = 0u;
         if (gid == 0) {
             const uint32_t sweep = counters[0];
             counters[1] = sweep;
@@ -2892,8 +3137,7 @@ __global__ void __launch_bounds__(256) k_begin(uint32_t *__restrict__ wt, size_t
 static hipError_t begin(const DevState &s, uint32_t *counters, hipStream_t st) {
     const size_t nh = (size_t)s.VD * s.K;
     hipLaunchKernelGGL(k_begin, dim3(grid_for(std::max(nh / 4, (size_t)s.K), 256, 4096)), dim3(256), 0, st,
-                       reinterpret_cast<uint32_t *>(s.wt_head), nh, reinterpret_cast<uint32_t *>(s.nk), s.K, counters,
-                       (uint32_t)s.n_queues);
+                       reinterpret_cast<uint32_t *>(s.wt_head), nh, reinterpret_cast<uint32_t *>(s.nk), s.K, counters);
     return hipGetLastError();
 }
 
@@ -3026,14 +3270,16 @@ size_t sampler_static_lds() {
     // a property of the code: looked up until it is known, once a process
     static std::atomic<size_t> known{(size_t)-1};
     if (known != (size_t)-1) return known;
-    const void *fs[8] = {reinterpret_cast<const void *>(&k_sample<true, true, true, true>),
+    const void *fs[] = {reinterpret_cast<const void *>(&k_sample<true, true, true, true>),
                          reinterpret_cast<const void *>(&k_sample<true, true, true, false>),
                          reinterpret_cast<const void *>(&k_sample<true, true, false, false>),
                          reinterpret_cast<const void *>(&k_sample<true, false, false, false>),
                          reinterpret_cast<const void *>(&k_sample<false, true, true, true>),
                          reinterpret_cast<const void *>(&k_sample<false, true, true, false>),
                          reinterpret_cast<const void *>(&k_sample<false, true, false, false>),
-                         reinterpret_cast<const void *>(&k_sample<false, false, false, false>)};
+                         reinterpret_cast<const void *>(&k_sample<false, false, false, false>),
+                         reinterpret_cast<const void *>(&k_sample_own<true>),
+                         reinterpret_cast<const void *>(&k_sample_own<false>)};
     size_t m = 0;
     for (const void *f : fs) {
         hipFuncAttributes a;
@@ -3062,7 +3308,14 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
     A.word_stride = 0;
     A.segs = s.smp_segs;
     A.runs = s.runs;
-    A.n_items = (uint32_t)s.n_smp_segs;
+    // the items from first_own on by k_sample_own, where enough wavefronts' tables fit
+    const int NS = (s.K + 63) >> 6;
+    const long room = (long)s.lds_cu / 4 - own_shared(NS);
+    const int own_wv = room > 0 ? (int)std::min<long>(16, room / (2 * own_stride(NS))) : 0;
+    const bool own = s.first_own < s.n_smp_segs && own_wv >= 4;
+    const int32_t n_first = own ? s.first_own : s.n_smp_segs;
+    A.first_item = (uint32_t)n_first;
+    A.n_items = (uint32_t)n_first;
     A.VD = s.VD;
     A.K = s.K;
     A.alpha = s.alpha;
@@ -3086,19 +3339,17 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
     // workgroup) at K = 64 126 / 152, 10,113 at K = 300 159 / 169; 27,680
     // items (13 a workgroup) at K = 4096 767 / 672, 98,189 (24) at K = 2048
     // 2,277 / 1,564, 126,191 (31) at K = 1024 3,519 / 2,884.
-    unsigned grid = (unsigned)s.n_smp_segs;
-    A.n_queues = s.grid_dim > 0 && s.n_smp_segs / 4 >= s.grid_dim ? (uint32_t)s.n_queues : 0u;
-    if (s.grid_dim > 0 && A.n_queues == 0) grid = (unsigned)std::min(s.n_smp_segs, s.grid_dim);
+    unsigned grid = (unsigned)n_first;
+    A.n_queues = s.grid_dim > 0 && n_first / 4 >= s.grid_dim ? (uint32_t)s.n_queues : 0u;
+    if (s.grid_dim > 0 && A.n_queues == 0) grid = (unsigned)std::min(n_first, s.grid_dim);
     A.stats = s.stats;
     A.seed = s.seed;
     A.tb = s.topic_bits;
     A.mode = mode;
+    // queue heads start at zero (a fill kernel, so a captured sweep replays it)
+    if (!begun && (A.n_queues || own))
+        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, st, A.queue, (size_t)kQueueStride * 2 * kQueues, 0u);
     if (A.n_queues) {
-        // queue heads start at zero (a fill kernel, so a captured sweep
-        // replays it)
-        if (!begun)
-            hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, st, s.counters + kQueueStride,
-                               (size_t)kQueueStride * A.n_queues, 0u);
         grid = (unsigned)s.grid_dim;
     }
     const bool qtab = s.K <= EZ_Q_TABLE_MAX_K;  // implies compact rows
@@ -3107,7 +3358,9 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
         A.word_stride = (uint32_t)group_stride(s.K);
         lds = (size_t)s.group_words * A.word_stride * sizeof(float);
     }
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(bd), lds, st, A); };
+    auto go = [&](auto kernel) {
+        if (n_first) hipLaunchKernelGGL(kernel, dim3(grid), dim3(bd), lds, st, A);
+    };
     if (shortcut && multi)
         go(k_sample<true, true, true, true>);
     else if (shortcut && qtab)
@@ -3124,6 +3377,12 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
         go(k_sample<false, true, false, false>);
     else
         go(k_sample<false, false, false, false>);
+    if (own && (mode & kSampleTail)) {
+        A.n_items = (uint32_t)s.n_smp_segs;
+        lds = (size_t)(own_shared(NS) + 2 * own_wv * own_stride(NS)) * sizeof(float);
+        auto go_own = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(s.n_cu), dim3(64 * own_wv), lds, st, A); };
+        shortcut ? go_own(k_sample_own<true>) : go_own(k_sample_own<false>);
+    }
     return hipGetLastError();
 }
 

@@ -639,6 +639,13 @@ int build_layout(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
     s.n_smp_segs = (int32_t)smp_segs.size();
     s.n_runs = (int64_t)runs.size();
     s.group_words = (int32_t)group_words;
+    s.first_own = s.n_smp_segs;
+    if (!s.compact)  // the last items, of the least frequent words
+        while (s.first_own > 0) {
+            const uint32_t w = smp_segs[s.first_own - 1].x;
+            if (w == 0xFFFFFFFFu || w < (uint32_t)VD || c->word_off[w + 1] - c->word_off[w] > ez::kOwnMax) break;
+            --s.first_own;
+        }
     s.n_queues = c->doc_tiles > 0 ? std::min(c->n_xcd, 8) : 1;
     s.block_dim = c->a.block_dim;
     s.grid_dim = c->a.grid_dim;

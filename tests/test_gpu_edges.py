@@ -182,3 +182,27 @@ def test_chunk_layouts_made_on_the_device(D, V, mean, chunks, run_cap):
     orc.sweep(1)
     assert np.array_equal(chk.get_topics(), orc.get_topics())
     assert chk.info().num_chunks == min(chunks, D)
+
+
+# half wavefronts of words of up to 128 tokens beside workgroups of larger
+# ones (32-bit rows): 31 to 33 and 127 to 129 tokens, an odd and an even number
+# of words, words cut by block_dim, rows past the checkpoints
+@pytest.mark.parametrize("K,kw", [(8192, {}), (8193, {}), (8256, {"shortcut": 0}), (10000, {"grid_dim": 0}),
+                                  (16383, {}), (16383, {"block_dim": 64, "run_cap": 1})])
+@pytest.mark.parametrize("odd", [0, 1])
+def test_words_of_few_tokens_at_large_k(K, kw, odd):
+    rng = np.random.default_rng(K + odd)
+    counts = np.array([700, 300, 257, 256, 130, 129, 128, 128, 127, 65, 64, 63, 33, 32, 31] + [5] * 20 + [1] * (30 + odd))
+    bag = np.repeat(rng.permutation(len(counts)), counts)  # the words' order of frequency is not that of their numbers
+    rng.shuffle(bag)
+    lens = np.concatenate([[len(bag) // 2], rng.multinomial(len(bag) - len(bag) // 2, np.ones(90) / 90)])
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    for z0 in (None, (np.arange(len(bag)) % 7).astype(np.uint16)):
+        ctx, orc = _pair(off, bag.astype(np.int32), len(counts), K, z0=z0, dense_words=2, **kw)
+        for n in (1, 2):
+            ctx.sweep(n)
+            orc.sweep(n)
+            assert np.array_equal(ctx.get_topics(), orc.get_topics()), n
+        ctx.sweep_graph(2)
+        orc.sweep(2)
+        assert np.array_equal(ctx.get_topics(), orc.get_topics())
