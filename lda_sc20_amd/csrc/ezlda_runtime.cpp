@@ -509,27 +509,38 @@ void number_runs(std::vector<uint4> &items, const std::vector<uint32_t> &word_of
                  const std::vector<uint32_t> &tok_doc, const std::vector<uint32_t> &tok_slot, uint32_t cap,
                  Begin &&begin, Put &&put, Done &&done) {
     const int64_t n = (int64_t)items.size();
-    std::vector<uint64_t> cnt(n + 1, 0);
-    parallel_for(n, [&](int64_t b, int64_t e, int) {
-        for (int64_t i = b; i < e; ++i) {
-            uint64_t k = 0;
-            for_runs(items[i], word_off, tok_doc, tok_slot, cap, [&](uint32_t, uint32_t) { ++k; });
-            cnt[i + 1] = k;
-        }
-    }, (int64_t)tok_doc.size());
+    // threads take items of equal numbers of tokens: most are in few items
+    std::vector<uint64_t> cnt(n + 1, 0), tokens(n + 1, 0);
+    for (int64_t i = 0; i < n; ++i) {
+        const uint4 &it = items[i];
+        tokens[i + 1] = tokens[i] + (it.x == 0xFFFFFFFFu ? 0u : it.w ? word_off[it.x + it.w] - it.y : it.z - it.y);
+    }
+    auto each_item = [&](auto &&work) {
+        const uint64_t N = tokens[n], parts = 64;
+        auto first = [&](int64_t p) {
+            return std::lower_bound(tokens.begin(), tokens.end() - 1, N * (uint64_t)p / parts) - tokens.begin();
+        };
+        parallel_for((int64_t)parts, [&](int64_t b, int64_t e, int) {
+            const int64_t end = e == (int64_t)parts ? n : first(e);
+            for (int64_t i = b ? first(b) : 0; i < end; ++i) work(i);
+        }, (int64_t)N);
+    };
+    each_item([&](int64_t i) {
+        uint64_t k = 0;
+        for_runs(items[i], word_off, tok_doc, tok_slot, cap, [&](uint32_t, uint32_t) { ++k; });
+        cnt[i + 1] = k;
+    });
     for (int64_t i = 0; i < n; ++i) cnt[i + 1] += cnt[i];
     begin(cnt[n]);
-    parallel_for(n, [&](int64_t b, int64_t e, int) {
-        for (int64_t i = b; i < e; ++i) {
-            uint4 &it = items[i];
-            if (it.x == 0xFFFFFFFFu) continue;
-            uint64_t k = cnt[i];
-            for_runs(it, word_off, tok_doc, tok_slot, cap, [&](uint32_t t, uint32_t l) { put(t, l, k++); });
-            done(cnt[i], cnt[i + 1]);
-            it = make_uint4(it.x | (it.w > 1 ? (it.w - 1u) << ez::kGroupShift : 0u), (uint32_t)cnt[i],
-                            (uint32_t)cnt[i + 1], 0u);
-        }
-    }, (int64_t)tok_doc.size());
+    each_item([&](int64_t i) {
+        uint4 &it = items[i];
+        if (it.x == 0xFFFFFFFFu) return;
+        uint64_t k = cnt[i];
+        for_runs(it, word_off, tok_doc, tok_slot, cap, [&](uint32_t t, uint32_t l) { put(t, l, k++); });
+        done(cnt[i], cnt[i + 1]);
+        it = make_uint4(it.x | (it.w > 1 ? (it.w - 1u) << ez::kGroupShift : 0u), (uint32_t)cnt[i],
+                        (uint32_t)cnt[i + 1], 0u);
+    });
 }
 
 // The runs as (first token, first slot, doc, tokens).  Inside an item they are
