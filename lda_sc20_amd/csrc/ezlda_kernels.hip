@@ -179,25 +179,35 @@ __global__ void k_topic_hist(const uint16_t *__restrict__ z, uint32_t N, int K, 
 // ------------------------------------------------------------- head WT
 // Dense head rows (WTDen_Update_Kernel, utility.cu:1067-1102): one workgroup
 // per segment of a head word's tokens, LDS histogram, atomic flush into the
-// (pre-zeroed) row.
+// (pre-zeroed) row; with `fresh`, the only segment of a word writes its whole
+// row, which then needs no zeroing: 20,011 words at K = 4096 (328 MB) 125 ->
+// 57 us, the time of one pass of writes.
 __device__ __forceinline__ void wt_head_block(uint32_t *sh, const uint16_t *__restrict__ z,
                                               const uint4 *__restrict__ segs, int K, int32_t *__restrict__ wt_head,
-                                              uint32_t seg) {
+                                              bool fresh, uint32_t seg) {
     const uint4 sg = segs[seg];
     for (int k = threadIdx.x; k < K; k += blockDim.x) sh[k] = 0;
     __syncthreads();
     hist_add_tokens(sh, z + sg.y, sg.z - sg.y, threadIdx.x, blockDim.x);
     __syncthreads();
     int32_t *row = wt_head + (size_t)sg.x * K;
+    if (fresh && sg.w) {
+        if ((K & 3) == 0)
+            for (int k = threadIdx.x; k < K >> 2; k += blockDim.x)
+                reinterpret_cast<uint4 *>(row)[k] = reinterpret_cast<const uint4 *>(sh)[k];
+        else
+            for (int k = threadIdx.x; k < K; k += blockDim.x) row[k] = (int32_t)sh[k];
+        return;
+    }
     for (int k = threadIdx.x; k < K; k += blockDim.x) {
         uint32_t c = sh[k];
         if (c) atomicAdd(&row[k], (int32_t)c);
     }
 }
 __global__ void k_wt_head(const uint16_t *__restrict__ z, const uint4 *__restrict__ segs, int K,
-                          int32_t *__restrict__ wt_head) {
+                          int32_t *__restrict__ wt_head, bool fresh) {
     extern __shared__ uint32_t sh[];
-    wt_head_block(sh, z, segs, K, wt_head, blockIdx.x);
+    wt_head_block(sh, z, segs, K, wt_head, fresh, blockIdx.x);
 }
 
 // ------------------------------------------------------------- tail WT
@@ -271,7 +281,7 @@ __global__ void k_wt_tail(const uint16_t *__restrict__ z, const uint32_t *__rest
 __global__ void __launch_bounds__(256) k_wt_all(int nb_hist, int nb_head, const uint16_t *__restrict__ z,
                                                 uint32_t N, int K, int32_t *__restrict__ nk,
                                                 const uint4 *__restrict__ segs, int32_t *__restrict__ wt_head,
-                                                const uint32_t *__restrict__ word_off, int VD, int V,
+                                                bool fresh, const uint32_t *__restrict__ word_off, int VD, int V,
                                                 const uint32_t *__restrict__ tail_off, uint32_t *__restrict__ wt_tail,
                                                 uint32_t *__restrict__ tail_nnz) {
     extern __shared__ uint32_t sh[];
@@ -279,7 +289,7 @@ __global__ void __launch_bounds__(256) k_wt_all(int nb_hist, int nb_head, const 
     if (b < nb_hist)
         topic_hist_block(sh, z, N, K, nk, (uint32_t)b, (uint32_t)nb_hist);
     else if (b < nb_hist + nb_head)
-        wt_head_block(sh, z, segs, K, wt_head, (uint32_t)(b - nb_hist));
+        wt_head_block(sh, z, segs, K, wt_head, fresh, (uint32_t)(b - nb_hist));
     else
         wt_tail_block(sh, z, word_off, VD, V, K, tail_off, wt_tail, tail_nnz, b - nb_hist - nb_head,
                       (int)gridDim.x - nb_hist - nb_head);
@@ -388,7 +398,8 @@ __global__ void __launch_bounds__(1024) k_inv_order(const int32_t *__restrict__ 
 // wavefront per word; a tail word's topics are marked in a bitmap in LDS (K
 // bits, so it leaves the occupancy alone at every K: with a table of 16-bit
 // counts, 20 KB a wavefront at K = 10000, 30,000 words took 104 us, in two
-// launches, 59 with the bitmap).  The order is total, so the order in which
+// launches, 59 with the bitmap).  A dense row is read by 16-byte loads where K
+// is a multiple of 4 (20,011 rows at K = 4096 136 -> 98 us).  The order is total, so the order in which
 // the lanes' lists are merged does not matter.
 __global__ void k_word_top(int V, int VD, int K, float beta, const int32_t *__restrict__ wt_head,
                            const uint32_t *__restrict__ tail_off, const uint32_t *__restrict__ wt_tail,
@@ -407,7 +418,31 @@ __global__ void k_word_top(int V, int VD, int K, float beta, const int32_t *__re
         if (w < VD) {
             // four loads of the row and of inv in flight per lane
             const int32_t *row = wt_head + (size_t)w * K;
-            for (int k0 = lane; k0 < K; k0 += 256) {
+            if ((K & 3) == 0) {
+                const int4 *row4 = reinterpret_cast<const int4 *>(row);
+                const float4 *inv4 = reinterpret_cast<const float4 *>(inv);
+                const int K4 = K >> 2;
+                for (int k0 = lane; k0 < K4; k0 += 256) {
+                    int4 c[4];
+                    float4 iv[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int k = k0 + 64 * u;
+                        c[u] = k < K4 ? row4[k] : make_int4(0, 0, 0, 0);
+                        iv[u] = k < K4 ? inv4[k] : make_float4(0.f, 0.f, 0.f, 0.f);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (k0 + 64 * u < K4) {
+                            const uint32_t k = 4u * (uint32_t)(k0 + 64 * u);
+                            top3_insert(t, ((float)c[u].x + beta) * iv[u].x, k);
+                            top3_insert(t, ((float)c[u].y + beta) * iv[u].y, k + 1u);
+                            top3_insert(t, ((float)c[u].z + beta) * iv[u].z, k + 2u);
+                            top3_insert(t, ((float)c[u].w + beta) * iv[u].w, k + 3u);
+                        }
+                }
+            }
+            for (int k0 = lane; (K & 3) != 0 && k0 < K; k0 += 256) {
                 int32_t c[4];
                 float iv[4];
 #pragma unroll
@@ -782,7 +817,8 @@ __global__ void k_dt_build(int q0, int q1, int K, int VD, uint32_t tb, const uin
 // The same DT rows and aux for short documents (n <= kDtShort slots) at
 // large K, where a K-sized LDS histogram per wavefront limits a CU to a few
 // wavefronts: one wavefront per doc sorts its topics in 2 KB of LDS (a
-// bitonic network over the next power of two >= n, 64..512 keys), reads the
+// bitonic network over the next power of two >= n, 64..512 keys, in
+// registers), reads the
 // runs of equal topics off the sorted keys (ascending topic, as the
 // histogram's compaction writes them) and finds each slot's (n_dk1, n_dk2)
 // by bisection.  Rows, pieces, padding and aux are those of k_dt_build.
@@ -3134,44 +3170,59 @@ __global__ void __launch_bounds__(256) k_begin(uint32_t *__restrict__ wt, size_t
     }
 }
 
-static hipError_t begin(const DevState &s, uint32_t *counters, hipStream_t st) {
-    const size_t nh = (size_t)s.VD * s.K;
+// (fresh: head rows of one segment are about to be written whole)
+static hipError_t begin(const DevState &s, bool fresh, uint32_t *counters, hipStream_t st) {
+    const size_t nh = (size_t)(fresh ? s.n_cut_rows : s.VD) * s.K;
     hipLaunchKernelGGL(k_begin, dim3(grid_for(std::max(nh / 4, (size_t)s.K), 256, 4096)), dim3(256), 0, st,
                        reinterpret_cast<uint32_t *>(s.wt_head), nh, reinterpret_cast<uint32_t *>(s.nk), s.K, counters);
     return hipGetLastError();
 }
 
-hipError_t launch_zero_counts(const DevState &s, hipStream_t st) { return begin(s, nullptr, st); }
+hipError_t launch_zero_counts(const DevState &s, hipStream_t st) { return begin(s, false, nullptr, st); }
+
+static hipError_t count_topics(const DevState &s, bool fresh, hipStream_t st);
 
 hipError_t launch_begin_sweep(const DevState &s, hipStream_t st) {
-    hipError_t e = begin(s, s.counters, st);
+    hipError_t e = begin(s, true, s.counters, st);
     if (e != hipSuccess) return e;
-    return launch_accumulate_wt(s, st);
+    return count_topics(s, true, st);
 }
 
 hipError_t launch_build_wt(const DevState &s, hipStream_t st) {
-    hipError_t e = launch_zero_counts(s, st);
+    hipError_t e = begin(s, true, nullptr, st);
     if (e != hipSuccess) return e;
-    return launch_accumulate_wt(s, st);
+    return count_topics(s, true, st);
 }
 
-hipError_t launch_accumulate_wt(const DevState &s, hipStream_t st) {
+hipError_t launch_accumulate_wt(const DevState &s, hipStream_t st) { return count_topics(s, false, st); }
+
+// n_k: about a workgroup a CU, as each adds up to K counts to the same K
+// addresses in memory (2,048 of them before: 9M tokens at K = 4096 55 -> 10
+// us, 4.5M at K = 10000 53 -> 9, and as a role of k_wt_all, which then took
+// 49.5M at K = 1024 111 -> 81 us, 8.9M at K = 2048 90 -> 49).
+static void topic_hist(const DevState &s, hipStream_t st) {
+    const size_t least = std::max<size_t>(4096, 4 * (size_t)s.K);
+    hipLaunchKernelGGL(k_topic_hist, dim3(grid_for(s.N, (int)least, s.n_cu)), dim3(1024), (size_t)s.K * sizeof(uint32_t),
+                       st, s.z, s.N, s.K, s.nk);
+}
+
+static hipError_t count_topics(const DevState &s, bool fresh, hipStream_t st) {
     const size_t ldsK = (size_t)s.K * sizeof(uint32_t);
     const int ntail = s.V - s.VD;
     if (s.N && s.n_wt_segs && ntail > 0 && (size_t)s.lds_cu / dt_wave_bytes(s.K) >= 16) {
         // one launch of 256-thread blocks (the tail rows' four wavefronts a
         // block, as their own launch takes when 16 wavefronts' tables fit a CU)
-        const int nb_hist = (int)grid_for(s.N, 256 * 16, 2048);
+        const int nb_hist = (int)grid_for(s.N, 256 * 16, std::max(s.n_cu, (int)(s.N >> 18)));
         const int nb_tail = (int)grid_for((size_t)ntail, 4, 1 << 16);
         const size_t lds = std::max(ldsK, 4 * dt_wave_bytes(s.K));
         hipLaunchKernelGGL(k_wt_all, dim3(nb_hist + s.n_wt_segs + nb_tail), dim3(256), lds, st, nb_hist, s.n_wt_segs,
-                           s.z, s.N, s.K, s.nk, s.wt_segs, s.wt_head, s.word_off, s.VD, s.V, s.tail_off, s.wt_tail,
+                           s.z, s.N, s.K, s.nk, s.wt_segs, s.wt_head, fresh, s.word_off, s.VD, s.V, s.tail_off, s.wt_tail,
                            s.tail_nnz);
         return hipGetLastError();
     }
-    if (s.N) hipLaunchKernelGGL(k_topic_hist, dim3(grid_for(s.N, 256 * 16, 2048)), dim3(256), ldsK, st, s.z, s.N, s.K, s.nk);
+    if (s.N) topic_hist(s, st);
     if (s.n_wt_segs)
-        hipLaunchKernelGGL(k_wt_head, dim3(s.n_wt_segs), dim3(256), ldsK, st, s.z, s.wt_segs, s.K, s.wt_head);
+        hipLaunchKernelGGL(k_wt_head, dim3(s.n_wt_segs), dim3(256), ldsK, st, s.z, s.wt_segs, s.K, s.wt_head, fresh);
     if (ntail > 0) {
         const WaveGrid g = wave_grid(s, (size_t)ntail, dt_wave_bytes(s.K), 1 << 16);
         hipLaunchKernelGGL(k_wt_tail, dim3(g.grid), dim3(64 * g.nwv), g.nwv * dt_wave_bytes(s.K), st,
@@ -3181,21 +3232,19 @@ hipError_t launch_accumulate_wt(const DevState &s, hipStream_t st) {
 }
 
 hipError_t launch_head_rows(const DevState &s, hipStream_t st) {
-    const size_t nh = (size_t)s.VD * s.K;
+    const size_t nh = (size_t)s.n_cut_rows * s.K;
     if (nh) hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(nh, 256, 4096)), dim3(256), 0, st,
                                reinterpret_cast<uint32_t *>(s.wt_head), nh, 0u);
     if (s.n_wt_segs)
         hipLaunchKernelGGL(k_wt_head, dim3(s.n_wt_segs), dim3(256), (size_t)s.K * sizeof(uint32_t), st, s.z, s.wt_segs,
-                           s.K, s.wt_head);
+                           s.K, s.wt_head, true);
     return hipGetLastError();
 }
 
 hipError_t launch_topic_hist(const DevState &s, hipStream_t st) {
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(s.K, 256, 64)), dim3(256), 0, st, reinterpret_cast<uint32_t *>(s.nk),
                        (size_t)s.K, 0u);
-    if (s.N)
-        hipLaunchKernelGGL(k_topic_hist, dim3(grid_for(s.N, 256 * 16, 2048)), dim3(256), (size_t)s.K * sizeof(uint32_t),
-                           st, s.z, s.N, s.K, s.nk);
+    if (s.N) topic_hist(s, st);
     return hipGetLastError();
 }
 

@@ -623,9 +623,16 @@ int build_layout(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
     // work items
     const uint32_t WT_SEG = 32768;
     std::vector<uint4> wt_segs;
-    for (int r = 0; r < VD; ++r)
-        for (uint32_t b = c->word_off[r]; b < c->word_off[r + 1]; b += WT_SEG)
-            wt_segs.push_back(make_uint4((uint32_t)r, b, std::min(b + WT_SEG, c->word_off[r + 1]), 0u));
+    int32_t n_cut_rows = 0;
+    for (int r = 0; r < VD; ++r) {  // a word without a token has one, too: it writes the zeros
+        uint32_t b = c->word_off[r];
+        const uint32_t e = c->word_off[r + 1], one = e - b <= WT_SEG ? 1u : 0u;
+        if (!one) n_cut_rows = r + 1;
+        do {
+            wt_segs.push_back(make_uint4((uint32_t)r, b, std::min(b + WT_SEG, e), one));
+            b = std::min(b + WT_SEG, e);
+        } while (b < e);
+    }
     (void)D;
     std::vector<uint4> smp_segs =
         build_sample_items(c->a, c->word_off, tok_doc, c->soff, slot_wrd, VD, K, c->n_xcd, true, &c->doc_tiles);
@@ -647,6 +654,7 @@ int build_layout(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
     if ((r = ldalloc(c, &s.ll_part, smp_segs.size()))) return r;
     s.VD = VD;
     s.n_wt_segs = (int32_t)wt_segs.size();
+    s.n_cut_rows = n_cut_rows;
     s.n_smp_segs = (int32_t)smp_segs.size();
     s.n_runs = (int64_t)runs.size();
     s.group_words = (int32_t)group_words;

@@ -206,3 +206,24 @@ def test_words_of_few_tokens_at_large_k(K, kw, odd):
         ctx.sweep_graph(2)
         orc.sweep(2)
         assert np.array_equal(ctx.get_topics(), orc.get_topics())
+
+
+# dense rows of one segment (32,768 tokens) are written whole, of several added
+# up; words without a token; K with and without 16-byte rows
+@pytest.mark.parametrize("K", [64, 65, 1026, 2600])
+def test_dense_rows_with_and_without_tokens(K):
+    rng = np.random.default_rng(K)
+    counts = [65537, 32769, 32768, 700, 3, 1, 1]
+    bag = rng.permutation(np.repeat(rng.permutation(len(counts)), counts)).astype(np.int32)
+    off = np.linspace(0, len(bag), 41).astype(np.int64)
+    V = len(counts) + 5  # five words of the vocabulary do not occur
+    for dense in (V, 4):
+        ctx, orc = _pair(off, bag, V, K, dense_words=dense)
+        for _ in range(2):
+            for c in (ctx, orc):
+                c.sweep(1)
+                c.build_wt()
+                c.topk()
+            assert np.array_equal(ctx.get_topics(), orc.get_topics())
+            assert np.array_equal(ctx.get_wt_dense(), orc.get_wt_dense())
+            assert np.array_equal(ctx.get_nk(), orc.get_nk()) and np.array_equal(ctx.get_top(), orc.get_top())
