@@ -63,6 +63,7 @@ struct DevState {
     uint32_t *zero_order = nullptr; // K: topics by beta * inv, largest first (tail words' zero counts)
     // work items
     uint4 *wt_segs = nullptr;       // head-word histogram segments (w, beg, end, 1 if the word's only one)
+    int32_t w_short = 0;            // words from here on have at most kDtShort tokens
     int32_t n_cut_rows = 0;         // head words of several segments (the first ones)
     int32_t n_wt_segs = 0;
     uint4 *smp_segs = nullptr;      // sampler items (w | further words << kGroupShift, first run, end run,

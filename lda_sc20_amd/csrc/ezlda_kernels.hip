@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "ezlda_device.h"
 #include "ezlda_philox.h"
@@ -210,6 +211,88 @@ __global__ void k_wt_head(const uint16_t *__restrict__ z, const uint4 *__restric
     wt_head_block(sh, z, segs, K, wt_head, fresh, blockIdx.x);
 }
 
+// ------------------------------------------------------ sorted topics
+// Bitonic sort, ascending, of 64 NU topics of a wavefront in registers
+// (element 64 u + lane in x[u]): partners 64 or more apart are in the same
+// lane, the others are fetched by a lane swizzle.
+template <int NU>
+__device__ __forceinline__ void sort_topics(uint32_t (&x)[NU], uint32_t lane) {
+#pragma unroll
+    for (uint32_t k = 2; k <= 64u * NU; k <<= 1) {
+#pragma unroll
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+#pragma unroll
+            for (uint32_t u = 0; u < (uint32_t)NU; ++u) {
+                if (j >= 64) {
+                    const uint32_t v = u ^ (j >> 6);
+                    if (v > u) {
+                        const bool up = ((64u * u) & k) == 0;
+                        const uint32_t lo = min(x[u], x[v]), hi = max(x[u], x[v]);
+                        x[u] = up ? lo : hi;
+                        x[v] = up ? hi : lo;
+                    }
+                } else {
+                    const uint32_t o = __shfl_xor(x[u], (int)j);
+                    const bool up = ((64u * u + lane) & k) == 0, first = (lane & j) == 0;
+                    x[u] = up == first ? min(x[u], o) : max(x[u], o);
+                }
+            }
+        }
+    }
+}
+
+// Sorts the n <= 64 NU topics that load(i) gives into key[0, 64 NU) (LDS),
+// 0xFFFF past them; NU the power of two that n needs.
+template <typename Load>
+__device__ __forceinline__ void sort_into(uint16_t *key, uint32_t n, uint32_t lane, Load &&load) {
+    auto go = [&](auto nu) {
+        constexpr int NU = decltype(nu)::value;
+        uint32_t x[NU];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) x[u] = lane + 64u * u < n ? load(u) : 0xFFFFu;
+        sort_topics<NU>(x, lane);
+#pragma unroll
+        for (int u = 0; u < NU; ++u) key[lane + 64 * u] = (uint16_t)x[u];
+    };
+    if (n <= 64)
+        go(std::integral_constant<int, 1>{});
+    else if (n <= 128)
+        go(std::integral_constant<int, 2>{});
+    else if (n <= 256)
+        go(std::integral_constant<int, 4>{});
+    else
+        go(std::integral_constant<int, 8>{});
+    static_assert(kDtShort == 512, "at most eight topics a lane");
+}
+
+// Lengths of the runs of equal topics of key[0, n): len(u) of the run that
+// starts at 64 u + lane (0: none starts there), hm the heads by 64.
+struct TopicRuns {
+    uint64_t hm[kDtShort / 64];
+    int nu;
+    __device__ __forceinline__ TopicRuns(const uint16_t *key, uint32_t n, uint32_t lane) {
+        nu = (int)((n + 63u) >> 6);
+#pragma unroll
+        for (int u = 0; u < (int)(kDtShort / 64); ++u) {
+            const uint32_t i = lane + 64u * u;
+            hm[u] = __ballot(u < nu && i < n && (i == 0 || key[i - 1] != key[i]));
+        }
+    }
+    __device__ __forceinline__ uint32_t len(int u, uint32_t n, uint32_t lane) const {
+        if (!((hm[u] >> lane) & 1ull)) return 0u;
+        const uint64_t above = hm[u] & ~((2ull << lane) - 1ull);
+        uint32_t nxt = n;  // the first head after it
+        if (above) {
+            nxt = 64u * u + (uint32_t)first_lane(above);
+        } else {
+#pragma unroll
+            for (int v = (int)(kDtShort / 64) - 1; v >= 0; --v)
+                if (v > u && v < nu && hm[v]) nxt = 64u * v + (uint32_t)first_lane(hm[v]);
+        }
+        return nxt - (64u * u + lane);
+    }
+};
+
 // ------------------------------------------------------------- tail WT
 // Sorted sparse tail rows (WT_Update_Kernel, utility.cu:10-76): one
 // wavefront per tail word; a 16-bit LDS histogram and a bitmap of the
@@ -272,6 +355,35 @@ __global__ void k_wt_tail(const uint16_t *__restrict__ z, const uint32_t *__rest
                           uint32_t *__restrict__ tail_nnz) {
     extern __shared__ uint32_t sh[];
     wt_tail_block(sh, z, word_off, VD, V, K, tail_off, wt_tail, tail_nnz, blockIdx.x, gridDim.x);
+}
+
+// The rows of tail words of at most kDtShort tokens at large K, where a
+// K-sized histogram leaves a CU few wavefronts (seven at K = 10000, 95 us for
+// 29,600 words, of which 29,200 take 22 us here): a wavefront sorts its word's
+// topics.
+__global__ void __launch_bounds__(256) k_wt_sort(const uint16_t *__restrict__ z, const uint32_t *__restrict__ word_off,
+                                                 int w0, int VD, int V, const uint32_t *__restrict__ tail_off,
+                                                 uint32_t *__restrict__ wt_tail, uint32_t *__restrict__ tail_nnz) {
+    __shared__ uint16_t keys[4][kDtShort];
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    uint16_t *key = keys[wv];
+    for (int w = w0 + (int)(blockIdx.x * 4u + wv); w < V; w += (int)gridDim.x * 4) {
+        const uint32_t b = word_off[w], n = word_off[w + 1] - b, base = tail_off[w - VD];
+        sort_into(key, n, lane, [&](int u) { return (uint32_t)z[b + lane + 64 * u]; });
+        wave_lds_sync();
+        const TopicRuns r(key, n, lane);
+        uint32_t nz = 0;
+#pragma unroll
+        for (int u = 0; u < (int)(kDtShort / 64); ++u) {
+            if (u >= r.nu) break;
+            const uint32_t len = r.len(u, n, lane);
+            const uint32_t pos = nz + (uint32_t)__popcll(r.hm[u] & lanemask_lt((int)lane));
+            if (len) wt_tail[base + pos] = (uint32_t)key[lane + 64 * u] | len << 16;
+            nz += (uint32_t)__popcll(r.hm[u]);
+        }
+        if (lane == 0) tail_nnz[w - VD] = nz;
+        wave_lds_sync();
+    }
 }
 
 // The three count builds of a sweep in one launch (they touch disjoint
@@ -816,13 +928,12 @@ __global__ void k_dt_build(int q0, int q1, int K, int VD, uint32_t tb, const uin
 
 // The same DT rows and aux for short documents (n <= kDtShort slots) at
 // large K, where a K-sized LDS histogram per wavefront limits a CU to a few
-// wavefronts: one wavefront per doc sorts its topics in 2 KB of LDS (a
-// bitonic network over the next power of two >= n, 64..512 keys, in
-// registers), reads the
-// runs of equal topics off the sorted keys (ascending topic, as the
+// wavefronts: one wavefront per doc sorts its topics in registers, reads the
+// runs of equal topics off the sorted keys in LDS (ascending topic, as the
 // histogram's compaction writes them) and finds each slot's (n_dk1, n_dk2)
 // by bisection.  Rows, pieces, padding and aux are those of k_dt_build.
-
+// 50,000 documents of 90 tokens at K = 10000: 120 -> 86 us (sorted in LDS
+// before, two reads and a barrier a pass).
 template <bool COMPACT, bool N_DK2>
 __global__ void __launch_bounds__(256) k_dt_sort(int q0, int q1, int VD, uint32_t tb,
                                                  const uint32_t *__restrict__ soff, const uint32_t *__restrict__ slot_wrd,
@@ -838,9 +949,7 @@ __global__ void __launch_bounds__(256) k_dt_sort(int q0, int q1, int VD, uint32_
     constexpr int kU = kDtShort / 64;
     for (int q = q0 + blockIdx.x * nwv + wv; q < q1; q += gridDim.x * nwv) {
         const uint32_t b = soff[q], e = soff[q + 1], n = e - b;  // n <= kDtShort
-        uint32_t P = 64;
-        while (P < n) P <<= 1;
-        const int nu = (int)(P >> 6);
+        const int nu = (int)((n + 63u) >> 6);
         uint32_t wrd[kU];
         // topics (the doc-slot copy for head words, z by token id for tail
         // words), padded with 0xFFFF, which sorts last
@@ -849,60 +958,21 @@ __global__ void __launch_bounds__(256) k_dt_sort(int q0, int q1, int VD, uint32_
             const uint32_t i = (uint32_t)lane + 64u * u;
             wrd[u] = i < n ? slot_wrd[b + i] : 0u;
         }
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const uint32_t i = (uint32_t)lane + 64u * u;
-            if (u < nu) {
-                uint32_t t = 0xFFFFu;
-                if (i < n) t = wrd[u] < (uint32_t)VD ? z_doc[b + i] : z[slot_tok[b + i]];
-                key[i] = (uint16_t)t;
-            }
-        }
+        sort_into(key, n, (uint32_t)lane, [&](int u) {
+            const uint32_t i = b + lane + 64u * u;
+            return (uint32_t)(wrd[u] < (uint32_t)VD ? z_doc[i] : z[slot_tok[i]]);
+        });
         wave_lds_sync();
-        // bitonic sort, ascending: P / 2 compare-exchanges per pass
-        for (uint32_t k = 2; k <= P; k <<= 1)
-            for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-                for (uint32_t p = (uint32_t)lane; p < (P >> 1); p += 64) {
-                    const uint32_t i = (p / j) * (j << 1) + (p % j), l = i + j;
-                    const uint16_t a = key[i], c = key[l];
-                    const bool up = (i & k) == 0;
-                    if ((a > c) == up && a != c) {
-                        key[i] = c;
-                        key[l] = a;
-                    }
-                }
-                wave_lds_sync();
-            }
-        // run heads and their lengths: the next head (or n) minus the head
-        uint64_t hm[kU];
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const uint32_t i = (uint32_t)lane + 64u * u;
-            const bool head = u < nu && i < n && (i == 0 || key[i - 1] != key[i]);
-            hm[u] = __ballot(head);
-        }
+        const TopicRuns runs(key, n, (uint32_t)lane);
         const uint32_t base = doc_info[q].x;
         uint32_t nz = 0;
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
             if (u >= nu) break;
             const uint32_t i = (uint32_t)lane + 64u * u;
-            const bool head = (hm[u] >> lane) & 1ull;
-            uint32_t len = 0, m = 0;
-            if (head) {
-                uint32_t nxt = n;  // the first head after i
-                const uint64_t above = hm[u] & ~((2ull << lane) - 1ull);
-                if (above) {
-                    nxt = 64u * u + (uint32_t)first_lane(above);
-                } else {
-#pragma unroll
-                    for (int v = kU - 1; v > u; --v)
-                        if (v < nu && hm[v]) nxt = 64u * v + (uint32_t)first_lane(hm[v]);
-                }
-                len = nxt - i;
-                m = COMPACT ? (len + piece - 1u) / piece : 1u;
-                run[i] = (uint16_t)len;
-            }
+            const uint32_t len = runs.len(u, n, (uint32_t)lane), m = COMPACT ? (len + piece - 1u) / piece : len ? 1u : 0u;
+            const bool head = len != 0u;
+            if (head) run[i] = (uint16_t)len;
             uint32_t incl = m;  // inclusive scan over lanes
             for (int d = 1; d < 64; d <<= 1) {
                 const uint32_t v = __shfl_up(incl, d);
@@ -3223,11 +3293,17 @@ static hipError_t count_topics(const DevState &s, bool fresh, hipStream_t st) {
     if (s.N) topic_hist(s, st);
     if (s.n_wt_segs)
         hipLaunchKernelGGL(k_wt_head, dim3(s.n_wt_segs), dim3(256), ldsK, st, s.z, s.wt_segs, s.K, s.wt_head, fresh);
-    if (ntail > 0) {
-        const WaveGrid g = wave_grid(s, (size_t)ntail, dt_wave_bytes(s.K), 1 << 16);
+    // (at small K there is no head word or no tail word; the rows are then
+    // built by histograms at every length)
+    const int w1 = (size_t)s.lds_cu / dt_wave_bytes(s.K) < 16 ? std::max(s.VD, std::min(s.V, s.w_short)) : s.V;
+    if (w1 > s.VD) {
+        const WaveGrid g = wave_grid(s, (size_t)(w1 - s.VD), dt_wave_bytes(s.K), 1 << 16);
         hipLaunchKernelGGL(k_wt_tail, dim3(g.grid), dim3(64 * g.nwv), g.nwv * dt_wave_bytes(s.K), st,
-                           s.z, s.word_off, s.VD, s.V, s.K, s.tail_off, s.wt_tail, s.tail_nnz);
+                           s.z, s.word_off, s.VD, w1, s.K, s.tail_off, s.wt_tail, s.tail_nnz);
     }
+    if (s.V > w1)
+        hipLaunchKernelGGL(k_wt_sort, dim3(grid_for((size_t)(s.V - w1), 4, 1 << 16)), dim3(256), 0, st, s.z, s.word_off,
+                           w1, s.VD, s.V, s.tail_off, s.wt_tail, s.tail_nnz);
     return hipGetLastError();
 }
 

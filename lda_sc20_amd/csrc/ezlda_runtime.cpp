@@ -655,6 +655,8 @@ int build_layout(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
     s.VD = VD;
     s.n_wt_segs = (int32_t)wt_segs.size();
     s.n_cut_rows = n_cut_rows;
+    s.w_short = V;
+    while (s.w_short > 0 && count(s.w_short - 1) <= (int64_t)ez::kDtShort) --s.w_short;
     s.n_smp_segs = (int32_t)smp_segs.size();
     s.n_runs = (int64_t)runs.size();
     s.group_words = (int32_t)group_words;

@@ -227,3 +227,26 @@ def test_dense_rows_with_and_without_tokens(K):
             assert np.array_equal(ctx.get_topics(), orc.get_topics())
             assert np.array_equal(ctx.get_wt_dense(), orc.get_wt_dense())
             assert np.array_equal(ctx.get_nk(), orc.get_nk()) and np.array_equal(ctx.get_top(), orc.get_top())
+
+
+# where rows are sorted instead of counted (K > 4819): tail words and documents
+# of 0, 1 and 64, 128, 256, 512 topics and one more or less, equal and distinct
+@pytest.mark.parametrize("K", [4800, 4900, 8193, 16383])
+def test_rows_of_sorted_topics(K):
+    sizes = [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 600]
+    rng = np.random.default_rng(K)
+    words = rng.permutation(np.repeat(np.arange(len(sizes)), sizes)).astype(np.int32)
+    rest = len(words) - sum(sizes[:-2])
+    off = np.concatenate([[0, 0], np.cumsum(sizes[:-2] + [rest // 2, rest - rest // 2])]).astype(np.int64)
+    for z0 in (None, np.full(len(words), K - 1, np.uint16), (np.arange(len(words)) % 5).astype(np.uint16)):
+        ctx, orc = _pair(off, words, len(sizes) + 1, K, z0=z0, dense_words=0)
+        for c in (ctx, orc):
+            c.build_wt()
+            c.topk()
+        assert np.array_equal(ctx.get_wt_dense(), orc.get_wt_dense())
+        assert np.array_equal(ctx.get_top(), orc.get_top())
+        for n in (1, 2):
+            ctx.sweep(n)
+            orc.sweep(n)
+            assert np.array_equal(ctx.get_topics(), orc.get_topics())
+        assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
