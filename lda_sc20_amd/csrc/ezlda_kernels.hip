@@ -67,6 +67,9 @@ static size_t wave_hist_bytes(int K) { return (size_t)((K + 1) >> 1) * sizeof(ui
 // DT rebuild: 16-bit counts plus a topic bitmap per wavefront
 static size_t dt_wave_bytes(int K) { return wave_hist_bytes(K) + (size_t)((K + 31) >> 5) * sizeof(uint32_t); }
 
+// the same without the bitmap, whole 16-byte words
+__host__ __device__ static inline size_t scan_wave_bytes(int K) { return ((size_t)((K + 1) >> 1) + 3) / 4 * 16; }
+
 // Launch of a kernel whose wavefronts each own wb bytes of LDS (cleared
 // when the wavefront starts) and stride over n units (words, docs).  When
 // at least 16 wavefronts' LDS fits on a CU: workgroups of four wavefronts,
@@ -776,9 +779,16 @@ hipError_t launch_chunk_topics(const DevState &s, const ChunkRuns &r, hipStream_
 // with the row's length (the sampler's), or with n_dk2 = n_dk at its word's
 // second topic (the re-pack of :125-161, for the getter).  A row starts on a
 // 128-byte boundary and is zero-padded to a multiple of 32 entries.
+// Up to this K the row is compacted from the counts themselves, two topics a
+// lane and 128 a step, and no bitmap is kept: that costs K / 128 short steps,
+// the bitmap three loops over the topics of the fullest 32 (and, before, a
+// division a topic).  us a sweep: 1M tokens at K = 64 29 -> 14, 1.7M at K = 300
+// 34 -> 27, 18,000 at K = 20 11.5 -> 7, 49.5M at K = 1024 338 -> 331; equal at K
+// = 2048 (161), at K = 4096 160 -> 250.
+static constexpr int kScanMaxK = 1024;
 static constexpr int kDtU = 8;  // slots per lane per chunk in k_dt_build
 
-template <bool COMPACT, bool N_DK2>
+template <bool COMPACT, bool N_DK2, bool SCAN>
 __global__ void k_dt_build(int q0, int q1, int K, int VD, uint32_t tb, const uint32_t *__restrict__ soff,
                            const uint32_t *__restrict__ slot_wrd, const uint32_t *__restrict__ slot_tok,
                            const uint16_t *__restrict__ z, const uint16_t *__restrict__ z_doc,
@@ -786,7 +796,7 @@ __global__ void k_dt_build(int q0, int q1, int K, int VD, uint32_t tb, const uin
                            uint32_t *__restrict__ aux_doc, uint2 *__restrict__ doc_info, uint32_t *__restrict__ dt) {
     extern __shared__ uint32_t sh[];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-    const int KH = (K + 1) >> 1, NW = (K + 31) >> 5;
+    const int KH = SCAN ? (int)(scan_wave_bytes(K) / 4) : (K + 1) >> 1, NW = SCAN ? 0 : (K + 31) >> 5;
     const uint32_t piece = (1u << (16u - tb)) - 1u;  // compact rows: largest count of one entry
     uint32_t *h = sh + wv * (KH + NW);  // 16-bit counts
     uint32_t *bm = h + KH;              // bitmap of the doc's topics
@@ -823,7 +833,7 @@ __global__ void k_dt_build(int q0, int q1, int K, int VD, uint32_t tb, const uin
             for (int u = 0; u < kDtU; ++u) {
                 if (c + lane + 64u * u < e) {
                     h16_add(h, t[u]);
-                    atomicOr(&bm[t[u] >> 5], 1u << (t[u] & 31u));
+                    if (!SCAN) atomicOr(&bm[t[u] >> 5], 1u << (t[u] & 31u));
                 }
             }
         }
@@ -834,6 +844,35 @@ __global__ void k_dt_build(int q0, int q1, int K, int VD, uint32_t tb, const uin
         // follows the doc's topics, not K.
         const uint32_t base = doc_info[q].x;
         uint32_t nz = 0;
+        auto put = [&](uint32_t at, uint32_t k, uint32_t c) {
+            if (COMPACT)
+                (reinterpret_cast<uint16_t *>(dt) + base)[at] = (uint16_t)(k | (c << tb));
+            else
+                dt[base + at] = (k << 2) | (c << 16);
+        };
+        // SCAN: the counts themselves, two topics a lane
+        for (int j = 0; SCAN && j < KH; j += 64) {
+            const uint32_t k = 2u * (uint32_t)(j + lane), cc = j + lane < KH ? h[j + lane] : 0u;
+            const uint32_t c0 = cc & 0xFFFFu, c1 = cc >> 16;
+            if (COMPACT && __ballot(max(c0, c1) > piece)) {  // entries of several pieces
+                const uint32_t m = (c0 + piece - 1u) / piece + (c1 + piece - 1u) / piece;
+                uint32_t incl = m;
+                for (int d = 1; d < 64; d <<= 1) {
+                    const uint32_t v = __shfl_up(incl, d);
+                    if (lane >= d) incl += v;
+                }
+                uint32_t pos = nz + incl - m;
+                for (uint32_t c = c0; c; c -= min(c, piece)) put(pos++, k, min(c, piece));
+                for (uint32_t c = c1; c; c -= min(c, piece)) put(pos++, k + 1u, min(c, piece));
+                nz += __shfl(incl, 63);
+            } else {
+                const uint64_t m0 = __ballot(c0 != 0u), m1 = __ballot(c1 != 0u), lt = lanemask_lt(lane);
+                const uint32_t pos = nz + (uint32_t)(__popcll(m0 & lt) + __popcll(m1 & lt));
+                if (c0) put(pos, k, c0);
+                if (c1) put(pos + (c0 ? 1u : 0u), k + 1u, c1);
+                nz += (uint32_t)(__popcll(m0) + __popcll(m1));
+            }
+        }
         for (int j = 0; j < NW; j += 64) {
             const int wi = j + lane;
             const uint32_t word = wi < NW ? bm[wi] : 0u;
@@ -841,7 +880,8 @@ __global__ void k_dt_build(int q0, int q1, int K, int VD, uint32_t tb, const uin
             if (COMPACT) {
                 for (uint32_t x = word; x; x &= x - 1u) {
                     const uint32_t k = ((uint32_t)wi << 5) + (uint32_t)__ffs(x) - 1u;
-                    m += (h16_get(h, k) + piece - 1u) / piece;
+                    const uint32_t c = h16_get(h, k);
+                    m += c <= piece ? 1u : (c + piece - 1u) / piece;
                 }
             } else {
                 m = (uint32_t)__popc(word);
@@ -914,6 +954,8 @@ __global__ void k_dt_build(int q0, int q1, int K, int VD, uint32_t tb, const uin
             }
         }
         wave_lds_sync();
+        if (SCAN)
+            for (int k = lane; k < KH >> 2; k += 64) reinterpret_cast<uint4 *>(h)[k] = make_uint4(0u, 0u, 0u, 0u);
         // each lane clears its own count words and bitmap words
         for (int wi = lane; wi < NW; wi += 64) {
             for (uint32_t x = bm[wi]; x; x &= x - 1u) {
@@ -3348,10 +3390,13 @@ static void build_dt_kernels(const DevState &s, hipStream_t st) {
     const bool sort_short = (size_t)s.lds_cu / dt_wave_bytes(s.K) < 16;
     const int q1 = sort_short ? s.D_long : s.D;
     if (q1 > 0) {
-        const WaveGrid g = wave_grid(s, (size_t)q1, dt_wave_bytes(s.K), 1 << 18);
-        hipLaunchKernelGGL((k_dt_build<COMPACT, N_DK2>), dim3(g.grid), dim3(64 * g.nwv), g.nwv * dt_wave_bytes(s.K), st,
-                           0, q1, s.K, s.VD, s.topic_bits, s.soff, s.slot_wrd, s.slot_tok, s.z, s.z_doc, s.wtop,
-                           s.aux_doc, s.doc_info, s.dt);
+        const size_t wb = s.K <= kScanMaxK ? scan_wave_bytes(s.K) : dt_wave_bytes(s.K);
+        const WaveGrid g = wave_grid(s, (size_t)q1, wb, 1 << 18);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(g.grid), dim3(64 * g.nwv), g.nwv * wb, st, 0, q1, s.K, s.VD, s.topic_bits,
+                               s.soff, s.slot_wrd, s.slot_tok, s.z, s.z_doc, s.wtop, s.aux_doc, s.doc_info, s.dt);
+        };
+        s.K <= kScanMaxK ? go(k_dt_build<COMPACT, N_DK2, true>) : go(k_dt_build<COMPACT, N_DK2, false>);
     }
     if (q1 < s.D) {
         const size_t lds = 4 * kDtShort * sizeof(uint32_t);  // four wavefronts, 2 KB each

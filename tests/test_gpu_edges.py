@@ -250,3 +250,30 @@ def test_rows_of_sorted_topics(K):
             orc.sweep(n)
             assert np.array_equal(ctx.get_topics(), orc.get_topics())
         assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
+
+
+# DT rows compacted 128 topics a step (K <= 1024), from a bitmap above it;
+# counts below, at and above one entry's 63 (K <= 1024), 31 and 15
+@pytest.mark.parametrize("K", [1, 2, 3, 64, 127, 128, 129, 255, 257, 1023, 1024, 1025, 2049])
+def test_rows_of_many_counts(K):
+    n = np.array([0, 1, 63, 64, 65, 126, 127, 300, 513, 700])
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int64)
+    words = (np.arange(off[-1]) * 7 % 50).astype(np.int32)
+    last = np.full(off[-1], K - 1, np.uint16)
+    pair = (np.arange(off[-1]) % 130 < 65) * (K - 1)  # two topics, next to each other's counts in turn
+    spread = np.arange(off[-1]) * 5 % K
+    for z0 in (last, pair.astype(np.uint16), spread.astype(np.uint16)):
+        ctx, orc = _pair(off, words, 50, K, z0=z0)
+        for c in (1, 2):
+            ctx.sweep(c)
+            orc.sweep(c)
+            assert np.array_equal(ctx.get_topics(), orc.get_topics()), c
+        for c in (ctx, orc):
+            c.build_wt()
+            c.topk()
+            c.build_dt()
+        (ge, gn), (oe, on) = ctx.get_dt_raw(), orc.get_dt_raw()
+        assert np.array_equal(gn, on)
+        for d, b in enumerate(ezlda.dt_offsets(off, K)[: len(gn)]):
+            assert np.array_equal(ge[b: b + gn[d]], oe[b: b + gn[d]]), d
+        assert np.array_equal(ctx.get_aux(), orc.get_aux())
