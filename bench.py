@@ -212,7 +212,7 @@ def foldin_perplexity(wt, nk, beta: float, alpha: float, docs, counts) -> float:
 def serving_bench(ctx, ezlda, wl: dict, args) -> dict:
     """Fold-in serving against the trained model frozen: an open-loop burst
     measures batched capacity, then Poisson arrivals at fractions of it give
-    p50/p99 latency; the plain one-document-per-launch path runs beside it."""
+    p50/p99 latency; the plain path, a document at a time, runs beside it."""
     fr = [float(x) for x in args.serve_levels.split(",") if x]
     n_burst, secs = args.serve_docs, args.serve_seconds
     K = ctx.args.K

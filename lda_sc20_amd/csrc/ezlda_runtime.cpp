@@ -234,6 +234,9 @@ void free_device(ezlda_ctx *c) {
     for (int j = 0; j < 2; ++j) {
         c->cimg[j] = nullptr;
         c->cdt[j] = c->caux[j] = c->cctr[j] = nullptr;
+        c->cz[j] = nullptr;
+        c->cwrd[j] = nullptr;
+        c->cruns[j] = nullptr;
         c->cll[j] = c->cllo[j] = nullptr;
     }
     c->wt_next = c->nk_next = nullptr;
