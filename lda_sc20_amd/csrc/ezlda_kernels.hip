@@ -514,8 +514,10 @@ __global__ void __launch_bounds__(1024) k_inv_order(const int32_t *__restrict__ 
 // bits, so it leaves the occupancy alone at every K: with a table of 16-bit
 // counts, 20 KB a wavefront at K = 10000, 30,000 words took 104 us, in two
 // launches, 59 with the bitmap).  A dense row is read by 16-byte loads where K
-// is a multiple of 4 (20,011 rows at K = 4096 136 -> 98 us).  The order is total, so the order in which
-// the lanes' lists are merged does not matter.
+// is a multiple of 4, two in flight (20,011 rows at K = 4096 136 -> 100 us; four
+// took 74 registers and the tail words of 49.5M tokens at K = 1024 65 -> 74).
+// The order is total, so the order in which the lanes' lists are merged does
+// not matter.
 __global__ void k_word_top(int V, int VD, int K, float beta, const int32_t *__restrict__ wt_head,
                            const uint32_t *__restrict__ tail_off, const uint32_t *__restrict__ wt_tail,
                            const uint32_t *__restrict__ tail_nnz, const float *__restrict__ inv,
@@ -537,17 +539,17 @@ __global__ void k_word_top(int V, int VD, int K, float beta, const int32_t *__re
                 const int4 *row4 = reinterpret_cast<const int4 *>(row);
                 const float4 *inv4 = reinterpret_cast<const float4 *>(inv);
                 const int K4 = K >> 2;
-                for (int k0 = lane; k0 < K4; k0 += 256) {
-                    int4 c[4];
-                    float4 iv[4];
+                for (int k0 = lane; k0 < K4; k0 += 128) {
+                    int4 c[2];
+                    float4 iv[2];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
+                    for (int u = 0; u < 2; ++u) {
                         const int k = k0 + 64 * u;
                         c[u] = k < K4 ? row4[k] : make_int4(0, 0, 0, 0);
                         iv[u] = k < K4 ? inv4[k] : make_float4(0.f, 0.f, 0.f, 0.f);
                     }
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
+                    for (int u = 0; u < 2; ++u)
                         if (k0 + 64 * u < K4) {
                             const uint32_t k = 4u * (uint32_t)(k0 + 64 * u);
                             top3_insert(t, ((float)c[u].x + beta) * iv[u].x, k);
