@@ -84,6 +84,7 @@ struct StepRec {
 
 struct ezlda_server {
     int K = 0, V = 0, NS = 0, sweeps = 20, max_slots = 0;
+    int n_cu = 1, lds_cu = 0;
     float alpha = 0.f;
     uint64_t seed = 0;
     std::vector<int32_t> rank_of;
@@ -286,7 +287,8 @@ void worker_main(ezlda_server *s) {
         StepRec &R = s->rec[cur], &P = s->rec[cur ^ 1];
         adm.clear();
         adm_rec.clear();
-        uint32_t up_words = 0, ns = 0, nfin = 0, zsum = 0, ntok = 0, max_n = 0, ngroups = 0;
+        uint32_t up_words = 0, ns = 0, nfin = 0, zsum = 0, ntok = 0, max_n = 0;
+        ez::FoldinFew few;
         UpLayout L{};
         {
             std::unique_lock<std::mutex> lk(s->mu);
@@ -353,11 +355,22 @@ void worker_main(ezlda_server *s) {
                     }
                 }
                 // places of the slots' workgroups where the step needs no buckets
-                if (const uint32_t group = ez::foldin_few_group(ntok)) {
+                few.group = ez::foldin_few_group(ntok);
+                if (const uint32_t group = few.group) {
                     uint32_t *hg = (uint32_t *)(R.up_h + L.goff);
-                    for (uint32_t j = 0; j < ns; ++j) {
-                        hg[j] = ngroups;
-                        ngroups += (hs[j].z + group - 1) / group;
+                    uint32_t ngroups = 0;
+                    for (uint32_t j = 0; j < ns; ++j) ngroups += (hs[j].z + group - 1) / group;
+                    const bool split = ez::foldin_few_split(ngroups, group, max_n, s->K, s->n_cu, s->lds_cu);
+                    ngroups = 0;
+                    for (uint32_t h = 0; h < (split ? 2u : 1u); ++h) {
+                        for (uint32_t j = 0; j < ns; ++j) {
+                            const uint32_t n = hs[j].z, row = std::min(n, (uint32_t)s->K);
+                            if ((split && row > ez::kFewShortRow ? 1u : 0u) != h) continue;
+                            hg[j] = ngroups + few.groups[h];
+                            few.groups[h] += (n + group - 1) / group;
+                            few.row_cap[h] = std::max(few.row_cap[h], row);
+                        }
+                        ngroups += few.groups[h];
                     }
                 }
                 if (nfin) {
@@ -383,8 +396,8 @@ void worker_main(ezlda_server *s) {
                                             (const uint32_t *)(s->up_d + L.words), s->wpool, s->st);
             if (e == hipSuccess)
                 e = ez::launch_foldin_step(s->fb, (const uint4 *)s->up_d, (const uint2 *)(s->up_d + L.fin),
-                                           (const uint32_t *)(s->up_d + L.goff), ngroups, (int)ns,
-                                           ntok, max_n, nfin > 0, s->V, s->K, s->alpha, s->phi, s->qs, s->qacc, s->wpool, s->zpool,
+                                           (const uint32_t *)(s->up_d + L.goff), few, (int)ns,
+                                           ntok, nfin > 0, s->V, s->K, s->alpha, s->phi, s->qs, s->qacc, s->wpool, s->zpool,
                                            s->seed, s->st);
             if (e == hipSuccess && zsum)
                 e = hipMemcpyAsync(R.z_h, s->fb.zout, (size_t)zsum * sizeof(uint16_t), hipMemcpyDeviceToHost, s->st);
@@ -433,6 +446,8 @@ ezlda_server *ezlda_server_create(ezlda_ctx *ctx, const ezlda_server_args *a) tr
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess || cus < 1)
         cus = 1;
+    s->n_cu = cus;
+    s->lds_cu = ctx->s.lds_cu;
     s->K = ctx->s.K;
     s->V = ctx->s.V;
     s->NS = (s->K + 63) / 64;

@@ -3135,27 +3135,45 @@ uint32_t foldin_few_group(uint32_t ntok) {
     return ntok > kFewTokens ? 0u : ntok <= 4096 ? 4u : ntok <= 8192 ? 8u : 16u;
 }
 
+static size_t foldin_few_lds(uint32_t row_cap, uint32_t group) {
+    return (((size_t)row_cap + 3) / 4 * 4 + 4 * wave_draw_floats((int)group / 4)) * sizeof(uint32_t);
+}
+
+// A step's longest row sizes the LDS of every workgroup of a launch.  Where
+// that leaves a CU one or two of them, and there are many, the documents of
+// long rows get a launch of their own.  K = 16,383, ms to drain 83K tokens in
+// short documents (alone 3.0) and one long document, in one launch / two /
+// bucketed: 16,000 tokens 10.3 / 7.2 / 9.8, 9,000 5.3 / 4.8 / 7.3; 5,000 in one
+// launch 2.3 of 5.2.  Few workgroups are better off in one: 34K short tokens and
+// one document of 9,000 3.4 / 3.7, 4K and one of 16,000 5.0 / 5.2.
+bool foldin_few_split(uint32_t ngroups, uint32_t group, uint32_t max_n, int K, int n_cu, int lds_cu) {
+    const uint32_t cap = std::min(max_n, (uint32_t)K);
+    const size_t fit = std::max<size_t>(1, (size_t)lds_cu / foldin_few_lds(cap, group));
+    return cap > kFewShortRow && fit < 3 && ngroups > 8u * (uint32_t)(n_cu * fit);
+}
+
 hipError_t launch_foldin_step(const FoldinBatch &fb, const uint4 *slots, const uint2 *fin, const uint32_t *goff,
-                              uint32_t ngroups, int nslots, uint32_t ntok, uint32_t max_n, bool any_fin, int V, int K,
+                              const FoldinFew &few, int nslots, uint32_t ntok, bool any_fin, int V, int K,
                               float alpha, const float *phi, const float *qs, const float *qacc,
                               const uint32_t *wpool, uint16_t *zpool, uint64_t seed, hipStream_t st) {
     if (nslots <= 0) return hipSuccess;
     const unsigned gs = (unsigned)std::min(nslots, 1 << 16);
     const size_t lds_rows = (size_t)((K + 1) >> 1) * sizeof(uint32_t);
-    const uint32_t group = foldin_few_group(ntok);
     hipLaunchKernelGGL(k_fi_rows, dim3(gs), dim3(256), lds_rows, st, slots, nslots, K, seed, zpool, fb.rows,
-                       fb.row_nnz, group, goff, fb.tokw);
-    if (group) {
-        const uint32_t row_cap = std::min(max_n, (uint32_t)K);
-        const size_t lds = (((size_t)row_cap + 3) / 4 * 4 + 4 * wave_draw_floats((int)group / 4)) * sizeof(uint32_t);
-        auto go = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3(ngroups), dim3(256), lds, st, slots, K, alpha, phi, qs, qacc, wpool, fb.rows,
-                               fb.row_nnz, fb.tokw, row_cap, zpool, seed);
-        };
-        if (ngroups) {
-            if (group == 4) go(k_fi_few<1>);
-            else if (group == 8) go(k_fi_few<2>);
+                       fb.row_nnz, few.group, goff, fb.tokw);
+    if (few.group) {
+        const uint32_t *groups = fb.tokw;
+        for (int h = 0; h < 2; ++h) {
+            if (!few.groups[h]) continue;
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(few.groups[h]), dim3(256), foldin_few_lds(few.row_cap[h], few.group), st,
+                                   slots, K, alpha, phi, qs, qacc, wpool, fb.rows, fb.row_nnz, groups, few.row_cap[h],
+                                   zpool, seed);
+            };
+            if (few.group == 4) go(k_fi_few<1>);
+            else if (few.group == 8) go(k_fi_few<2>);
             else go(k_fi_few<4>);
+            groups += few.groups[h];
         }
         if (any_fin) hipLaunchKernelGGL(k_fi_final, dim3(gs), dim3(256), 0, st, slots, fin, nslots, zpool, fb.zout);
         return hipGetLastError();

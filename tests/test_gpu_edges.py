@@ -119,6 +119,41 @@ def test_fold_in_of_a_full_house(K, D):
     srv.close()
 
 
+def _fold_in_case(K, lens, sweeps, V=300):
+    """A frozen model and documents of these lengths, with the oracle's topics and counts."""
+    off, words = make_corpus(4, 200, V, 60, zipf=1.2)
+    ctx, orc = _pair(off, words, V, K)
+    rng = np.random.default_rng(K + len(lens))
+    doff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    dw = ((rng.zipf(1.2, int(doff[-1])) - 1) % V).astype(np.int32)
+    rids = np.arange(len(lens), dtype=np.uint32)
+    ctx.build_wt()
+    orc.build_wt()
+    orc.topk()
+    return ctx, doff, dw, rids, orc.foldin(doff, dw, rids, sweeps, 5)
+
+
+def _serve(ctx, doff, dw, rids, want, sweeps, slots):
+    srv = ezlda.Server(ctx, max_slots=slots, sweeps=sweeps, hbm_budget_bytes=1 << 24, seed=5)
+    srv.submit_many(rids, doff, dw)
+    for r in rids.tolist():
+        z, c, _ = srv.wait(r, timeout_ms=60000)
+        assert np.array_equal(z, want[0][doff[r]: doff[r + 1]]) and np.array_equal(c, want[1][r]), r
+    st = srv.stats()
+    srv.close()
+    return st
+
+
+# a long row among short documents: a launch of its own (16,383 topics, more workgroups than the CUs hold), and
+# steps of few workgroups or of rows that leave room, in one
+@pytest.mark.parametrize("K,short,long", [(16383, 60, 20000), (16383, 5, 20000), (16383, 60, 4097), (9000, 130, 16500)])
+def test_fold_in_of_a_long_row_among_short_ones(K, short, long):
+    lens = np.random.default_rng(K).integers(200, 400, short)
+    lens = np.concatenate([lens[: short // 2], [long], lens[short // 2:], [0]])
+    ctx, doff, dw, rids, want = _fold_in_case(K, lens, 2)
+    _serve(ctx, doff, dw, rids, want, 2, len(lens))
+
+
 # words of few tokens drawn by groups (K <= 512): slabs and topics that fill no
 # whole load, groups of dense words, of sparse words and at the border of the
 # two, unused words, long words between; stages in any order
