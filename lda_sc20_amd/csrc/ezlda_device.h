@@ -172,18 +172,19 @@ hipError_t launch_foldin_doc(const uint32_t *words, uint32_t n, uint32_t rid, in
 // tokens, sweep); fin[j] = (output index or ~0, topic offset) for the
 // documents that finish with this sweep (any_fin: there are some); ntok = the
 // slots' tokens.  nslots <= 65535 documents of <= 65535 tokens.
-// A step of ntok tokens that is drawn without bucketing them by word runs in
-// workgroups of foldin_few_group(ntok) tokens of a slot (0: it is bucketed).
-// goff[j] is then the first of slot j's workgroups; groups[0] of them (rows
-// of at most row_cap[0] entries) are one launch, the groups[1] after them
-// (row_cap[1]) another: with foldin_few_split, those of the documents that may
-// have more than kFewShortRow topics.
+// A step of ntok tokens, of documents of `cost` in all, is drawn without
+// bucketing them by word in workgroups of foldin_few_group tokens of a slot
+// (0: it is bucketed).  goff[j] is then the first of slot j's workgroups;
+// groups[0] of them (rows of at most row_cap[0] entries) are one launch, the
+// groups[1] after them (row_cap[1]) another: with foldin_few_split, those of
+// the documents that may have more than kFewShortRow topics.
 static constexpr uint32_t kFewShortRow = 4096;
 struct FoldinFew {
     uint32_t group = 0;
     uint32_t groups[2] = {0, 0}, row_cap[2] = {0, 0};
 };
-uint32_t foldin_few_group(uint32_t ntok);
+uint64_t foldin_few_cost(uint32_t n, int K);
+uint32_t foldin_few_group(uint32_t ntok, uint64_t cost, int V);
 bool foldin_few_split(uint32_t ngroups, uint32_t group, uint32_t max_n, int K, int n_cu, int lds_cu);
 hipError_t launch_foldin_step(const FoldinBatch &fb, const uint4 *slots, const uint2 *fin, const uint32_t *goff,
                               const FoldinFew &few, int nslots, uint32_t ntok, bool any_fin, int V, int K,

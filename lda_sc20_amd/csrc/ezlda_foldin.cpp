@@ -50,6 +50,7 @@ struct Request {
 struct Slot {
     bool active = false;
     uint32_t rid = 0, off = 0, n = 0, sweep = 0;
+    uint64_t cost = 0;  // ez::foldin_few_cost
     double t_submit = 0.0;
 };
 
@@ -288,6 +289,7 @@ void worker_main(ezlda_server *s) {
         adm.clear();
         adm_rec.clear();
         uint32_t up_words = 0, ns = 0, nfin = 0, zsum = 0, ntok = 0, max_n = 0;
+        uint64_t cost = 0;
         ez::FoldinFew few;
         UpLayout L{};
         {
@@ -312,6 +314,7 @@ void worker_main(ezlda_server *s) {
                 x.off = off;
                 x.n = n;
                 x.sweep = 0;
+                x.cost = ez::foldin_few_cost(n, s->K);
                 x.t_submit = adm.back().t_submit;
                 s->active.push_back(j);
                 adm_rec.push_back(make_uint4(up_words, off, n, 0u));
@@ -337,6 +340,7 @@ void worker_main(ezlda_server *s) {
                     hs[j] = make_uint4(x.rid, x.off, x.n, x.sweep);
                     ntok += x.n;
                     max_n = std::max(max_n, x.n);
+                    cost += x.cost;
                     if (++x.sweep == (uint32_t)s->sweeps) {
                         Finishing f;
                         f.rid = x.rid;
@@ -355,7 +359,7 @@ void worker_main(ezlda_server *s) {
                     }
                 }
                 // places of the slots' workgroups where the step needs no buckets
-                few.group = ez::foldin_few_group(ntok);
+                few.group = ez::foldin_few_group(ntok, cost, s->V);
                 if (const uint32_t group = few.group) {
                     uint32_t *hg = (uint32_t *)(R.up_h + L.goff);
                     uint32_t ngroups = 0;

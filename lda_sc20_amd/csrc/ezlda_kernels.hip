@@ -3124,15 +3124,35 @@ hipError_t launch_foldin_admit(const uint4 *adm, int nadm, const uint32_t *src, 
 
 // Steps of few tokens are drawn by k_fi_few, straight from the tables: no
 // buckets by word, whose seven launches cost more than they save until big
-// words gather enough tokens to share a staged phi row.  Measured, ms to
-// drain a batch of documents (mean 300 tokens, 20 sweeps) bucketed / few, for
-// 39K, 161K, 315K and 609K tokens resident: K = 1024 2.49 / 1.16, 3.66 / 3.22,
-// 5.20 / 5.58, 7.66 / 9.32; K = 128 - / 0.58, 1.60 / 1.26, 2.39 / 2.27,
-// 3.42 / 3.86; K = 4096 (161K on) 4.18 / 4.42, 6.45 / 7.36, 9.80 / 10.64.
-static constexpr uint32_t kFewTokens = 196608;
+// words gather enough tokens to share a staged phi row.  What a token costs
+// there follows its document's row, about min(n / 3, K) entries of which the
+// first few hundred count; what buckets save follows V, whose few frequent
+// words hold more of the tokens where it is small.  Measured, ms to drain a
+// batch of documents (20 sweeps) bucketed / few, on both sides of the line:
+//   K = 1024, mean 300, V = 1,000: 120K tokens 2.70 / 2.29, 160K 2.83 / 2.76,
+//     200K 3.15 / 3.61; V = 102,660: 150K 3.12 / 2.65, 260K 4.43 / 4.36
+//   K = 1024, mean 600: 80K 2.50 / 2.26, 118K 2.65 / 2.94 (V = 2,000),
+//     3.13 / 2.91 (V = 102,660)
+//   K = 1024, mean 2,000: 59K 3.76 / 3.12, 78K 3.65 / 3.73 (V = 2,000), 77K
+//     4.01 / 3.42, 115K 4.15 / 4.67 (V = 102,660)
+//   K = 300, mean 2,000: 78K 1.80 / 1.61, 116K 2.15 / 2.31 (V = 2,000)
+//   K = 64 to 16,383, mean 60: few up to 150K-200K and more
+//   K = 16,383, V = 2,000: mean 300 80K 3.61 / 2.99, 120K 4.16 / 4.16; mean
+//     2,000 59K 7.66 / 6.68, 78K 7.43 / 7.75
+// Rows of thousands of topics cost more again (K = 16,383, 34K tokens in short
+// documents and one, two, three of 16,000: 9.6 / 6.1, 10.0 / 9.6, 10.1 / 13.2).
+static constexpr uint32_t kFewTokens = 196608, kFewRow = 430;
+static constexpr uint64_t kFewCost = 45000000, kFewCostLargeV = 56000000;
 
-uint32_t foldin_few_group(uint32_t ntok) {
-    return ntok > kFewTokens ? 0u : ntok <= 4096 ? 4u : ntok <= 8192 ? 8u : 16u;
+uint64_t foldin_few_cost(uint32_t n, int K) {
+    const uint32_t row = std::min(n, (uint32_t)K);
+    return (uint64_t)n * (160u + std::min(std::min(n / 3u, kFewRow), (uint32_t)K) +
+                          (row > kFewShortRow ? (row - kFewShortRow) / 16u : 0u));
+}
+
+uint32_t foldin_few_group(uint32_t ntok, uint64_t cost, int V) {
+    if (ntok > kFewTokens || cost > (V >= 16384 ? kFewCostLargeV : kFewCost)) return 0u;
+    return ntok <= 4096 ? 4u : ntok <= 8192 ? 8u : 16u;
 }
 
 static size_t foldin_few_lds(uint32_t row_cap, uint32_t group) {
@@ -3143,9 +3163,9 @@ static size_t foldin_few_lds(uint32_t row_cap, uint32_t group) {
 // that leaves a CU one or two of them, and there are many, the documents of
 // long rows get a launch of their own.  K = 16,383, ms to drain 83K tokens in
 // short documents (alone 3.0) and one long document, in one launch / two /
-// bucketed: 16,000 tokens 10.3 / 7.2 / 9.8, 9,000 5.3 / 4.8 / 7.3; 5,000 in one
-// launch 2.3 of 5.2.  Few workgroups are better off in one: 34K short tokens and
-// one document of 9,000 3.4 / 3.7, 4K and one of 16,000 5.0 / 5.2.
+// bucketed: 16,000 tokens 10.3 / 7.2 / 9.8, 9,000 5.3 / 4.8 / 7.3.  Few
+// workgroups are better off in one: 34K short tokens and one document of 9,000
+// 3.4 / 3.7, 4K and one of 16,000 5.0 / 5.2.
 bool foldin_few_split(uint32_t ngroups, uint32_t group, uint32_t max_n, int K, int n_cu, int lds_cu) {
     const uint32_t cap = std::min(max_n, (uint32_t)K);
     const size_t fit = std::max<size_t>(1, (size_t)lds_cu / foldin_few_lds(cap, group));

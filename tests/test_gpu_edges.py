@@ -144,6 +144,15 @@ def _serve(ctx, doff, dw, rids, want, sweeps, slots):
     return st
 
 
+# documents in flight while the steps go from unbucketed to bucketed and back: half of them are admitted at a time
+@pytest.mark.parametrize("K", [128, 1024])
+def test_fold_in_steps_change_their_path(K):
+    lens = np.random.default_rng(K).integers(120, 360, 840)
+    ctx, doff, dw, rids, want = _fold_in_case(K, lens, 4)
+    st = _serve(ctx, doff, dw, rids, want, 4, len(lens))
+    assert st.max_active == len(lens) and int(doff[-1]) > 196608 > int(doff[430])
+
+
 # a long row among short documents: a launch of its own (16,383 topics, more workgroups than the CUs hold), and
 # steps of few workgroups or of rows that leave room, in one
 @pytest.mark.parametrize("K,short,long", [(16383, 60, 20000), (16383, 5, 20000), (16383, 60, 4097), (9000, 130, 16500)])
