@@ -144,6 +144,16 @@ def _serve(ctx, doff, dw, rids, want, sweeps, slots):
     return st
 
 
+# a step's tokens decide how many a wavefront draws (1, 2, 4: lines at 4,096 and 8,192)
+@pytest.mark.parametrize("total", [4096, 4097, 6000, 8192, 8193])
+@pytest.mark.parametrize("K", [64, 1024])
+def test_fold_in_steps_by_their_tokens(K, total):
+    lens = [300] * (total // 300) + [total % 300]
+    ctx, doff, dw, rids, want = _fold_in_case(K, lens, 2)
+    st = _serve(ctx, doff, dw, rids, want, 2, len(lens))
+    assert st.max_active == len(lens)  # all in one step
+
+
 # documents in flight while the steps go from unbucketed to bucketed and back: half of them are admitted at a time
 @pytest.mark.parametrize("K", [128, 1024])
 def test_fold_in_steps_change_their_path(K):
