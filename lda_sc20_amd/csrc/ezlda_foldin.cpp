@@ -22,6 +22,7 @@
 #include <cstring>
 #include <deque>
 #include <map>
+#include <memory_resource>
 #include <mutex>
 #include <new>
 #include <stdexcept>
@@ -40,6 +41,10 @@ namespace {
 double now_ms() {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
+
+// Least bytes of a buffer that one thread allocates and another frees: above
+// the heap's small blocks (128 bytes with their headers).
+constexpr size_t kLeastBuffer = 192;
 
 struct Request {
     uint32_t rid = 0;
@@ -110,8 +115,15 @@ struct ezlda_server {
     std::vector<Slot> slots;
     std::vector<int> free_slots, active;
     std::deque<Request> pending;
-    std::unordered_map<uint32_t, Result> done;
-    std::unordered_set<uint32_t> inflight;  // queued or resident request ids
+    // Results are made by the worker and freed by the threads that claim them.
+    // As small blocks of the heap they would wait there, by the thousand, to be
+    // merged in one go inside one of the worker's own calls: 240,000 documents/s
+    // after 120,000 claims had 8 to 9 ms of latency over their first 5 ms (5 to
+    // 6 with this).  So the tables' nodes stay in a pool (guarded by mu, as the
+    // tables; given back with the server), and buffers are no small blocks.
+    std::pmr::unsynchronized_pool_resource nodes;
+    std::pmr::unordered_map<uint32_t, Result> done{&nodes};
+    std::pmr::unordered_set<uint32_t> inflight{&nodes};  // queued or resident request ids
     std::mutex mu;
     std::condition_variable cv_work, cv_done;
     std::thread worker;
@@ -249,6 +261,7 @@ bool publish(ezlda_server *s, StepRec &R) {
     std::vector<Result> res(R.fins.size());
     for (size_t f = 0; f < R.fins.size(); ++f) {
         const Finishing &x = R.fins[f];
+        res[f].z.reserve(std::max<size_t>(x.n, kLeastBuffer / sizeof(uint16_t)));
         res[f].z.assign(R.z_h + x.zoff, R.z_h + x.zoff + x.n);
     }
     std::lock_guard<std::mutex> lk(s->mu);
@@ -527,6 +540,7 @@ int ezlda_server_submit(ezlda_server *s, uint32_t request_id, const int32_t *wor
     if (n > 65535) return sfail(s, EZLDA_EINVAL, "a fold-in document has more than 65535 tokens");
     Request rq;
     rq.rid = request_id;
+    rq.words.reserve(std::max<size_t>((size_t)n, kLeastBuffer / sizeof(uint32_t)));
     rq.words.resize(n);
     for (int32_t i = 0; i < n; ++i) {
         if (words[i] < 0 || words[i] >= s->V) return sfail(s, EZLDA_EINVAL, "word id out of range in fold-in request");
@@ -562,6 +576,7 @@ int ezlda_server_submit_many(ezlda_server *s, int32_t n_docs, const uint32_t *re
         if (n > 65535) return sfail(s, EZLDA_EINVAL, "a fold-in document has more than 65535 tokens");
         if (n > 0 && !words) return sfail(s, EZLDA_EINVAL, "bad fold-in batch");
         rq[d].rid = request_ids[d];
+        rq[d].words.reserve(std::max<size_t>((size_t)n, kLeastBuffer / sizeof(uint32_t)));
         rq[d].words.resize((size_t)n);
         const int32_t *w = words + doc_off[d];
         for (int64_t i = 0; i < n; ++i) {
@@ -571,7 +586,8 @@ int ezlda_server_submit_many(ezlda_server *s, int32_t n_docs, const uint32_t *re
     }
     std::lock_guard<std::mutex> lk(s->mu);
     if (s->worker_rc != EZLDA_OK) return sfail(s, s->worker_rc, s->err);
-    std::unordered_set<uint32_t> ids;
+    std::pmr::monotonic_buffer_resource ids_mem;
+    std::pmr::unordered_set<uint32_t> ids(&ids_mem);
     for (const Request &r : rq) {
         if (r.words.size() > s->budget_tokens) {
             s->rejected++;

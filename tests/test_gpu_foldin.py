@@ -4,6 +4,7 @@ Bit-exact topics and counts per request, whatever the batch a request shares
 a launch with, its arrival order, the slot count or the HBM token budget, and
 on the one-document-per-launch plain path.
 """
+import ctypes
 import threading
 
 import numpy as np
@@ -192,3 +193,29 @@ def test_wait_buffer_comes_from_the_submitted_length():
     z, c, _ = srv.wait(5, 1, timeout_ms=30000)
     assert len(z) == 150 and np.array_equal(z, zo) and np.array_equal(c, co[0])
     srv.close()
+
+
+class _MallInfo2(ctypes.Structure):
+    _fields_ = [(k, ctypes.c_size_t) for k in ("arena", "ordblks", "smblks", "hblks", "hblkhd", "usmblks", "fsmblks",
+                                               "uordblks", "fordblks", "keepcost")]
+
+
+def test_claimed_results_leave_no_small_blocks_to_merge():
+    # the heap's freed small blocks (of all threads) are merged by whichever call comes along, the worker's included
+    try:
+        info = ctypes.CDLL(None).mallinfo2
+    except AttributeError:
+        pytest.skip("no mallinfo2")
+    info.restype = _MallInfo2
+    n = 6000
+    ctx, _ = _model(16)
+    off, words = _docs(300, [40] * n)
+    srv = ezlda.Server(ctx, max_slots=1024, sweeps=2, hbm_budget_bytes=1 << 24, seed=5)
+    srv.submit_many(np.arange(n, dtype=np.uint32), off, words)
+    srv.drain()
+    before = info().fsmblks
+    for r in range(n):
+        srv.wait(r)
+    grown = int(info().fsmblks) - int(before)
+    srv.close()
+    assert grown < 16 * n, grown  # a block is at least 32 bytes
