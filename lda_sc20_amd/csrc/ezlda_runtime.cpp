@@ -1448,11 +1448,21 @@ static int enqueue_sweep(ezlda_ctx *c, hipEvent_t *ev) {
     return EZLDA_OK;
 }
 
+// After a sweep of which only a part could be launched: the device's sweep
+// counter moved on with its first kernel, and the counts may be of older
+// topics.  Sweep c->sweep is still to be done.
+static int sweep_failed(ezlda_ctx *c, int r) {
+    (void)ez::launch_set_u32(c->s.counters, c->sweep, c->st);
+    (void)hipStreamSynchronize(c->st);
+    c->counts_fresh = false;
+    return r;
+}
+
 int ezlda_sweep(ezlda_ctx *c, int32_t n) try {
     if (int r = need_loaded(c)) return r;
     if (is_chunked(c)) return chunk_sweeps(c, n, nullptr, nullptr);
     for (int i = 0; i < n; ++i) {
-        if (int r = enqueue_sweep(c, nullptr)) return r;
+        if (int r = enqueue_sweep(c, nullptr)) return sweep_failed(c, r);
         c->sweep++;
     }
     EZ_TRY_HIP(c, hipStreamSynchronize(c->st));
@@ -1666,14 +1676,15 @@ int ezlda_time_sweeps(ezlda_ctx *c, int32_t n, int32_t use_graph, double *total_
             if (hipEventRecord(ev[0], c->st) != hipSuccess) rc = fail(c, EZLDA_EHIP, "hipEventRecord failed");
             for (int i = 0; i < n && rc == EZLDA_OK; ++i) {
                 if (hipGraphLaunch(c->graph_exec, c->st) != hipSuccess) rc = fail(c, EZLDA_EHIP, "hipGraphLaunch failed");
-                c->sweep++;
+                else c->sweep++;
             }
             if (rc == EZLDA_OK && hipEventRecord(ev[1], c->st) != hipSuccess)
                 rc = fail(c, EZLDA_EHIP, "hipEventRecord failed");
         } else {
             for (int i = 0; i < n && rc == EZLDA_OK; ++i) {
                 rc = enqueue_sweep(c, &ev[(size_t)i * per]);
-                c->sweep++;
+                if (rc) (void)sweep_failed(c, rc);
+                else c->sweep++;
             }
         }
     }

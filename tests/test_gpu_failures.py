@@ -1,0 +1,89 @@
+"""GPU: calls of the runtime that fail on the host (a launch, an allocation, a
+thread), and devices of few CUs, forced by a shim between the library and the
+HIP runtime.  The library must then stand as before the call, and go on."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+pytestmark = pytest.mark.gpu
+
+HEADER = """
+import ctypes, os, sys
+sys.path[:0] = [{root!r}, os.path.join({root!r}, "tests")]
+shim = ctypes.CDLL({shim!r}, mode=ctypes.RTLD_GLOBAL)
+shim.shim_fail_launch.argtypes = [ctypes.c_long]
+shim.shim_launches_left.restype = ctypes.c_long
+shim.shim_fail_malloc.argtypes = [ctypes.c_size_t]
+import numpy as np
+from conftest import make_corpus
+from lda_sc20_amd import ezlda
+from oracle import binding as ob
+
+def context(off, words, V, K, seed=21, **kw):
+    ctx = ezlda.Context(K=K, alpha=50.0 / K, beta=0.01, seed=seed, **kw)
+    ctx.load(ezlda.Corpus(V, off, words))
+    return ctx
+
+def failing(call):
+    try:
+        call()
+    except ezlda.EzldaError:
+        return True
+    return False
+"""
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    cc = shutil.which("gcc")
+    if cc is None:
+        pytest.skip("no C compiler")
+    so = tmp_path_factory.mktemp("shim") / "libshim.so"
+    subprocess.run([cc, "-O1", "-shared", "-fPIC", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "hip_shim.c"),
+                    "-o", str(so), "-ldl", "-lpthread"], check=True)
+    return str(so)
+
+
+def _run(shim, body):
+    """The body in a process of its own, with the shim between the library and the runtime."""
+    r = subprocess.run([sys.executable, "-c", HEADER.format(root=ROOT, shim=shim) + body], stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout[-3000:]
+    return r.stdout
+
+
+# every launch of a sweep fails once: the sweep is as if it had not been asked
+# for (the sampler's launch is the last), its number included
+@pytest.mark.parametrize("call", ["ctx.sweep(1)", "ctx.time_sweeps(1, use_graph=False)"])
+def test_a_failed_launch_leaves_the_sweep_undone(shim, call):
+    out = _run(shim, f"""
+off, words = make_corpus(3, 120, 200, 60)
+orc = ob.Oracle(64, float(np.float32(50.0 / 64)), 0.01, 21, 200, off, words)
+want = []
+for s in range(3):
+    orc.sweep(1)
+    want.append((orc.get_topics(), orc.loglik()))
+j = 0
+while True:
+    ctx = context(off, words, 200, 64)
+    ctx.loglik()
+    ctx.sweep(1)
+    shim.shim_fail_launch(j)
+    if not failing(lambda: {call}):
+        assert shim.shim_launches_left() == 0, "no launch failed"
+        break
+    assert ctx.info().sweep == 1, j
+    assert np.array_equal(ctx.get_topics(), want[0][0]), j
+    assert abs(ctx.loglik() - want[0][1]) <= 1e-9 * abs(want[0][1]), j
+    for s in (1, 2):
+        ctx.sweep(1)
+        assert ctx.info().sweep == s + 1 and np.array_equal(ctx.get_topics(), want[s][0]), (j, s)
+    j += 1
+print("launches", j)
+""")
+    assert int(out.split("launches")[1]) >= 4
