@@ -2049,6 +2049,8 @@ __global__ void __launch_bounds__(1024) k_sample(const SampleArgs A) {
 // fit: there it lost (a word a wavefront at K = 4096: 0.96 / 1.63 and, heavy-
 // tailed, 1.76 / 4.84; K = 7000 0.80 / 0.72).  Items from first_item on, in
 // pairs from a queue an XCD (dealt in turn, 320 us and 4.29 ms heavy-tailed).
+// A workgroup drains the queue of its number modulo kQueues and no other, so
+// the grid is at least kQueues workgroups.
 template <bool SHORTCUT>
 __global__ void __launch_bounds__(1024) k_sample_own(const SampleArgs A) {
     extern __shared__ float smf[];  // the only LDS: phi at address 0
@@ -3590,7 +3592,9 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
     if (own && (mode & kSampleTail)) {
         A.n_items = (uint32_t)s.n_smp_segs;
         lds = (size_t)(own_shared(NS) + 2 * own_wv * own_stride(NS)) * sizeof(float);
-        auto go_own = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(s.n_cu), dim3(64 * own_wv), lds, st, A); };
+        // a workgroup drains one queue: each of the kQueues needs one
+        const unsigned g = (unsigned)std::max(s.n_cu, kQueues);
+        auto go_own = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(g), dim3(64 * own_wv), lds, st, A); };
         shortcut ? go_own(k_sample_own<true>) : go_own(k_sample_own<false>);
     }
     return hipGetLastError();

@@ -87,3 +87,19 @@ while True:
 print("launches", j)
 """)
     assert int(out.split("launches")[1]) >= 4
+
+
+# a device of 4 CUs (a partition): every queue of the samplers is still drained
+@pytest.mark.parametrize("K", [10000, 2000, 64])
+def test_a_device_of_few_cus(shim, K):
+    _run(shim, f"""
+shim.shim_cus(4)
+off, words = make_corpus(5, 150, 400, 60, zipf=1.15)
+ctx = context(off, words, 400, {K})
+orc = ob.Oracle({K}, float(np.float32(50.0 / {K})), 0.01, 21, 400, off, words)
+for s in range(2):
+    ctx.sweep(1)
+    orc.sweep(1)
+    assert np.array_equal(ctx.get_topics(), orc.get_topics()), s
+assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
+""")
