@@ -13,7 +13,6 @@
 #include <new>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -34,6 +33,22 @@ int host_threads() {
     return (int)n;
 }
 
+// f(0) .. f(T - 1), each on a thread of its own, the first on the caller's,
+// which also takes over what threads that could not be started leave.
+template <class F>
+void run_threads(int T, const F &f) {
+    std::vector<std::thread> th;
+    th.reserve(T);
+    int t = 1;
+    try {
+        for (; t < T; ++t) th.emplace_back([&f, t] { f(t); });
+    } catch (const std::exception &) {  // no thread, or no memory for one
+    }
+    f(0);
+    for (; t < T; ++t) f(t);
+    for (auto &x : th) x.join();
+}
+
 // f(begin, end, thread) over parts of [0, n); `work` is what n stands for
 // where it isn't n itself (items of many tokens).
 template <class F>
@@ -43,12 +58,7 @@ void parallel_for(int64_t n, F f, int64_t work = 0) {
         f(0, n, 0);
         return;
     }
-    std::vector<std::thread> th;
-    for (int t = 0; t < T; ++t) {
-        const int64_t b = n * t / T, e = n * (t + 1) / T;
-        th.emplace_back([=] { f(b, e, t); });
-    }
-    for (auto &x : th) x.join();
+    run_threads(T, [&](int t) { f(n * t / T, n * (t + 1) / T, t); });
 }
 
 // Topics of one readback slot (a multiple of 8), and slots at most: the copy
@@ -1169,15 +1179,10 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
     dsplit[0] = 0;
     dsplit[T] = D;
     std::vector<std::vector<uint32_t>> tcnt(T, std::vector<uint32_t>(V, 0));
-    {
-        std::vector<std::thread> th;
-        for (int t = 0; t < T; ++t)
-            th.emplace_back([&, t] {
-                for (int q = dsplit[t]; q < dsplit[t + 1]; ++q)
-                    for (int64_t i = doc_off[dord[q]]; i < doc_off[dord[q] + 1]; ++i) tcnt[t][c->rank_of[words[i]]]++;
-            });
-        for (auto &x : th) x.join();
-    }
+    run_threads(T, [&](int t) {
+        for (int q = dsplit[t]; q < dsplit[t + 1]; ++q)
+            for (int64_t i = doc_off[dord[q]]; i < doc_off[dord[q] + 1]; ++i) tcnt[t][c->rank_of[words[i]]]++;
+    });
     for (int r = 0; r < V; ++r) {
         uint32_t cur = c->word_off[r];
         for (int t = 0; t < T; ++t) {
@@ -1192,34 +1197,29 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
     std::vector<uint16_t> z(N);
     c->doc_tok.assign(N, 0);
     c->slot_tok.assign(N, 0);
-    {
-        std::vector<std::thread> th;
-        for (int t = 0; t < T; ++t)
-            th.emplace_back([&, t] {
-                std::vector<uint32_t> &cur = tcnt[t];
-                std::vector<uint64_t> key;
-                for (int q = dsplit[t]; q < dsplit[t + 1]; ++q) {
-                    const int d = dord[q];
-                    const int64_t b = doc_off[d], n = doc_off[d + 1] - b;
-                    key.resize((size_t)n);
-                    for (int64_t i = 0; i < n; ++i) key[i] = ((uint64_t)c->rank_of[words[b + i]] << 16) | (uint64_t)i;
-                    std::sort(key.begin(), key.end());
-                    uint32_t p = c->soff[q];
-                    for (int64_t j = 0; j < n; ++j, ++p) {
-                        const uint32_t r = (uint32_t)(key[j] >> 16);
-                        const int64_t i = b + (int64_t)(key[j] & 0xFFFFu);
-                        const uint32_t tk = cur[r]++;
-                        tok_doc[tk] = (uint32_t)q;
-                        tok_slot[tk] = p;
-                        c->slot_tok[p] = tk;
-                        slot_wrd[p] = r;
-                        c->doc_tok[i] = tk;
-                        if (z0) z[tk] = z0[i];
-                    }
-                }
-            });
-        for (auto &x : th) x.join();
-    }
+    run_threads(T, [&](int t) {
+        std::vector<uint32_t> &cur = tcnt[t];
+        std::vector<uint64_t> key;
+        for (int q = dsplit[t]; q < dsplit[t + 1]; ++q) {
+            const int d = dord[q];
+            const int64_t b = doc_off[d], n = doc_off[d + 1] - b;
+            key.resize((size_t)n);
+            for (int64_t i = 0; i < n; ++i) key[i] = ((uint64_t)c->rank_of[words[b + i]] << 16) | (uint64_t)i;
+            std::sort(key.begin(), key.end());
+            uint32_t p = c->soff[q];
+            for (int64_t j = 0; j < n; ++j, ++p) {
+                const uint32_t r = (uint32_t)(key[j] >> 16);
+                const int64_t i = b + (int64_t)(key[j] & 0xFFFFu);
+                const uint32_t tk = cur[r]++;
+                tok_doc[tk] = (uint32_t)q;
+                tok_slot[tk] = p;
+                c->slot_tok[p] = tk;
+                slot_wrd[p] = r;
+                c->doc_tok[i] = tk;
+                if (z0) z[tk] = z0[i];
+            }
+        }
+    });
     tcnt.clear();
     if (!z0) {
         const uint64_t seed = c->a.seed;
@@ -1872,14 +1872,7 @@ int read_topics(ezlda_ctx *c, uint16_t *zout) {
             std::memcpy(zout + b, buf, (size_t)n * sizeof(uint16_t));
         }
     };
-    std::vector<std::thread> th;
-    th.reserve(c->read_ev.size());
-    try {
-        for (size_t k = 1; k < c->read_ev.size(); ++k) th.emplace_back(work, k);
-    } catch (const std::system_error &) {
-    }
-    work(0);
-    for (auto &x : th) x.join();
+    run_threads((int)c->read_ev.size(), work);
     if (failed != (int)hipSuccess)
         return fail(c, EZLDA_EHIP, std::string("reading the topics: ") + hipGetErrorString((hipError_t)failed.load()));
     return EZLDA_OK;

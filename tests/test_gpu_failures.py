@@ -18,7 +18,7 @@ sys.path[:0] = [{root!r}, os.path.join({root!r}, "tests")]
 shim = ctypes.CDLL({shim!r}, mode=ctypes.RTLD_GLOBAL)
 shim.shim_fail_launch.argtypes = [ctypes.c_long]
 shim.shim_launches_left.restype = ctypes.c_long
-shim.shim_fail_malloc.argtypes = [ctypes.c_size_t]
+shim.shim_fail_malloc.argtypes = [ctypes.c_size_t, ctypes.c_long]
 import numpy as np
 from conftest import make_corpus
 from lda_sc20_amd import ezlda
@@ -40,11 +40,11 @@ def failing(call):
 
 @pytest.fixture(scope="module")
 def shim(tmp_path_factory):
-    cc = shutil.which("gcc")
+    cc = shutil.which("g++")
     if cc is None:
-        pytest.skip("no C compiler")
+        pytest.skip("no C++ compiler")
     so = tmp_path_factory.mktemp("shim") / "libshim.so"
-    subprocess.run([cc, "-O1", "-shared", "-fPIC", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "hip_shim.c"),
+    subprocess.run([cc, "-std=c++17", "-O1", "-shared", "-fPIC", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "hip_shim.cpp"),
                     "-o", str(so), "-ldl", "-lpthread"], check=True)
     return str(so)
 
@@ -102,4 +102,25 @@ for s in range(2):
     orc.sweep(1)
     assert np.array_equal(ctx.get_topics(), orc.get_topics()), s
 assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
+""")
+
+
+# threads that cannot be started: the caller does their part (the readback of a resident and of a chunked corpus, and
+# the layout)
+@pytest.mark.parametrize("kw", ["{}", "{'num_chunks': 3}"])
+def test_threads_that_cannot_be_started(shim, kw):
+    _run(shim, f"""
+rng = np.random.default_rng(7)
+n = 1100000
+off = np.arange(0, n + 1, 100, dtype=np.int64)
+words = rng.integers(0, 500, n).astype(np.int32)
+z = rng.integers(0, 9, n).astype(np.uint16)
+for failing_load in (0, 1):
+    shim.shim_fail_threads(failing_load)
+    ctx = ezlda.Context(K=9, alpha=0.5, beta=0.01, seed=1, **{kw})
+    ctx.load(ezlda.Corpus(500, off, words), z0=z)
+    for on in (1, 0):
+        shim.shim_fail_threads(on)
+        assert np.array_equal(ctx.get_topics(), z), on
+    ctx.close()
 """)
