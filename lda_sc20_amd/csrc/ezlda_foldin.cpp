@@ -91,6 +91,7 @@ struct StepRec {
 struct ezlda_server {
     int K = 0, V = 0, NS = 0, sweeps = 20, max_slots = 0;
     int n_cu = 1, lds_cu = 0;
+    ezlda_ctx *ctx = nullptr;  // while the server is created
     float alpha = 0.f;
     uint64_t seed = 0;
     std::vector<int32_t> rank_of;
@@ -172,7 +173,7 @@ namespace {
 
 template <class T>
 int salloc(ezlda_server *s, T **p, size_t n) {
-    hipError_t e = hipMalloc((void **)p, std::max<size_t>(n, 1) * sizeof(T));
+    hipError_t e = ezc::device_alloc(s->ctx, (void **)p, std::max<size_t>(n, 1) * sizeof(T));
     if (e != hipSuccess) return sfail(s, EZLDA_EHIP, std::string("hipMalloc: ") + hipGetErrorString(e));
     s->allocs.push_back((void *)*p);
     return EZLDA_OK;
@@ -459,6 +460,7 @@ ezlda_server *ezlda_server_create(ezlda_ctx *ctx, const ezlda_server_args *a) tr
     }
     if (ezc::refresh_counts(ctx) != EZLDA_OK) return nullptr;
     auto *s = new ezlda_server();
+    s->ctx = ctx;
     if (hipGetDevice(&s->device) != hipSuccess) s->device = 0;
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess || cus < 1)
@@ -498,6 +500,7 @@ ezlda_server *ezlda_server_create(ezlda_ctx *ctx, const ezlda_server_args *a) tr
         ezlda_server_destroy(s);
         return nullptr;
     }
+    s->ctx = nullptr;
     s->slots.resize(s->max_slots);
     for (int j = s->max_slots - 1; j >= 0; --j) s->free_slots.push_back(j);
     s->free_ranges[0] = s->pool_tokens;

@@ -54,6 +54,7 @@ struct ezlda_ctx {
     // where the corpus is no longer than a slot
     uint16_t *read_buf = nullptr, *read_dev = nullptr;
     std::vector<hipEvent_t> read_ev;
+    int64_t read_bytes = 0;  // device bytes of s.doc_tok and read_dev
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     int n_xcd = 1;      // XCDs of the device (round-robin workgroup dispatch)
@@ -87,6 +88,10 @@ void set_error(const std::string &m);
 // exception leaves an extern "C" entry point.
 int exception_status(ezlda_ctx *c);
 int server_exception_status(ezlda_server *s);
+// hipMalloc that gives back the context's readback buffers (s.doc_tok, read_*:
+// needed by no call) and tries again where memory is short; c may be null.
+hipError_t device_alloc(ezlda_ctx *c, void **p, size_t bytes);
+void drop_readback(ezlda_ctx *c);
 // Rebuilds ctx's counts from its current z and 1/(n_k + V beta), synchronously.
 int refresh_counts(ezlda_ctx *c);
 // The chunked folder at root (ezlda_corpus.cpp): per doc-major token,

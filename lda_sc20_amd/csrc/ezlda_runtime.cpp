@@ -199,11 +199,36 @@ namespace {
             return fail((ctx), EZLDA_EHIP, std::string(#call) + ": " + hipGetErrorString(e_));   \
     } while (0)
 
+}  // namespace
+
+void ezc::drop_readback(ezlda_ctx *c) {
+    if (c->st) (void)hipStreamSynchronize(c->st);
+    if (c->s.doc_tok) (void)hipFree(c->s.doc_tok);
+    if (c->read_buf) (void)hipHostFree(c->read_buf);
+    for (hipEvent_t e : c->read_ev) (void)hipEventDestroy(e);
+    c->read_ev.clear();
+    c->s.doc_tok = nullptr;
+    c->read_buf = c->read_dev = nullptr;
+    c->read_bytes = 0;
+}
+
+hipError_t ezc::device_alloc(ezlda_ctx *c, void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && c && c->s.doc_tok) {
+        (void)hipGetLastError();
+        drop_readback(c);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+namespace {
+
 template <class T>
 int dalloc(ezlda_ctx *c, T **p, size_t n) {
     *p = nullptr;
     const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-    hipError_t e = hipMalloc((void **)p, bytes);
+    hipError_t e = ezc::device_alloc(c, (void **)p, bytes);
     if (e != hipSuccess) return fail(c, EZLDA_EHIP, std::string("hipMalloc: ") + hipGetErrorString(e));
     c->allocs.push_back((void *)*p);
     c->dev_bytes += (int64_t)bytes;
@@ -230,12 +255,8 @@ void free_device(ezlda_ctx *c) {
     c->layout_allocs.clear();
     c->dev_bytes = 0;
     c->layout_bytes = 0;
+    ezc::drop_readback(c);
     c->s = ez::DevState{};
-    if (c->read_buf) (void)hipHostFree(c->read_buf);
-    c->read_buf = nullptr;
-    c->read_dev = nullptr;
-    for (hipEvent_t e : c->read_ev) (void)hipEventDestroy(e);
-    c->read_ev.clear();
     for (EzChunk &ch : c->chunks)
         if (ch.img) (void)hipHostFree(ch.img);
     c->chunks.clear();
@@ -257,7 +278,7 @@ template <class T>
 int ldalloc(ezlda_ctx *c, T **p, size_t n) {
     *p = nullptr;
     const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-    hipError_t e = hipMalloc((void **)p, bytes);
+    hipError_t e = ezc::device_alloc(c, (void **)p, bytes);
     if (e != hipSuccess) return fail(c, EZLDA_EHIP, std::string("hipMalloc: ") + hipGetErrorString(e));
     c->layout_allocs.push_back((void *)*p);
     c->layout_bytes += (int64_t)bytes;
@@ -273,26 +294,38 @@ int lupload(ezlda_ctx *c, T **p, const std::vector<T> &v) {
 }
 
 // The readback's token order on the device and its buffers: a corpus of one
-// piece is copied as it is (no pinned memory to set up).
-int alloc_readback(ezlda_ctx *c, uint32_t N) {
-    const uint32_t pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
+// piece is copied as it is (no pinned memory to set up).  4 bytes a token that
+// no call needs: where they cannot be had, the topics are read back through
+// the host, and a later allocation that fails has them back (device_alloc).
+void alloc_readback(ezlda_ctx *c) {
+    const uint32_t N = c->s.N, pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
+    if (pieces == 0) return;
     const size_t order = ((size_t)N + 3) / 4 * 4;  // the buffer behind it is 16-byte aligned
-    if (int r = dalloc(c, &c->s.doc_tok, order + (pieces <= 1 ? order / 2 : 0))) return r;
-    if (N) EZ_TRY_HIP(c, hipMemcpy(c->s.doc_tok, c->doc_tok.data(), (size_t)N * sizeof(uint32_t), hipMemcpyHostToDevice));
-    if (pieces <= 1) {
+    const size_t bytes = order * sizeof(uint32_t) + (pieces == 1 ? order * sizeof(uint16_t) : 0);
+    bool ok = hipMalloc((void **)&c->s.doc_tok, bytes) == hipSuccess;
+    if (!ok) c->s.doc_tok = nullptr;
+    ok = ok && hipMemcpy(c->s.doc_tok, c->doc_tok.data(), (size_t)N * sizeof(uint32_t), hipMemcpyHostToDevice) ==
+                   hipSuccess;
+    if (ok && pieces == 1) {
         c->read_dev = reinterpret_cast<uint16_t *>(c->s.doc_tok + order);
-        return EZLDA_OK;
+    } else if (ok) {
+        const uint32_t slots = std::min(pieces, std::min((uint32_t)host_threads(), kReadSlots));
+        c->read_ev.reserve(slots);
+        ok = hipHostMalloc((void **)&c->read_buf, (size_t)slots * kReadTokens * sizeof(uint16_t),
+                           hipHostMallocDefault) == hipSuccess;
+        if (!ok) c->read_buf = nullptr;
+        for (uint32_t i = 0; ok && i < slots; ++i) {
+            hipEvent_t e = nullptr;
+            ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+            if (ok) c->read_ev.push_back(e);
+        }
     }
-    const uint32_t slots = std::min(pieces, std::min((uint32_t)host_threads(), kReadSlots));
-    EZ_TRY_HIP(c, hipHostMalloc((void **)&c->read_buf, (size_t)slots * kReadTokens * sizeof(uint16_t),
-                                hipHostMallocDefault));
-    c->read_ev.reserve(slots);
-    for (uint32_t i = 0; i < slots; ++i) {
-        hipEvent_t e = nullptr;
-        EZ_TRY_HIP(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        c->read_ev.push_back(e);
+    if (ok) {
+        c->read_bytes = (int64_t)bytes;
+    } else {
+        (void)hipGetLastError();
+        ezc::drop_readback(c);
     }
-    return EZLDA_OK;
 }
 
 int need_loaded(ezlda_ctx *c) {
@@ -1278,7 +1311,6 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
     int r = 0;
     if ((r = upload(c, &s.word_off, c->word_off))) return r;
     if ((r = upload(c, &s.z, z))) return r;
-    if ((r = alloc_readback(c, N))) return r;
     if ((r = upload(c, &s.soff, c->soff))) return r;
     if ((r = upload(c, &s.slot_wrd, slot_wrd))) return r;
     if ((r = upload(c, &s.slot_tok, c->slot_tok))) return r;
@@ -1302,6 +1334,7 @@ int ezlda_load_docs(ezlda_ctx *c, int32_t V, int32_t D, const int64_t *doc_off, 
     EZ_TRY_HIP(c, hipMemsetAsync(s.stats, 0, 2 * sizeof(unsigned long long), c->st));
     EZ_TRY_HIP(c, hipStreamSynchronize(c->st));
     EZ_TRY_HIP(c, hipDeviceSynchronize());
+    alloc_readback(c);
     c->sweep = 0;
     c->counts_fresh = false;
     c->loaded = true;
@@ -1333,7 +1366,7 @@ int ezlda_get_info(ezlda_ctx *c, ezlda_info *info) try {
     info->wt_tail_capacity = c->tail_cap;
     info->num_sample_items = c->s.n_smp_segs;
     info->sweep = c->sweep;
-    info->device_bytes = c->dev_bytes + c->layout_bytes;
+    info->device_bytes = c->dev_bytes + c->layout_bytes + c->read_bytes;
     info->doc_tiles = c->doc_tiles;
     info->num_xcd = c->n_xcd;
     info->run_cap = c->a.run_cap;
@@ -1840,8 +1873,17 @@ namespace {
 // that could not be started leaves its pieces to the others).
 int read_topics(ezlda_ctx *c, uint16_t *zout) {
     const uint32_t N = c->s.N, n_pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
-    if (n_pieces <= 1) {
-        if (!N) return EZLDA_OK;
+    if (!N) return EZLDA_OK;
+    if (!c->s.doc_tok) {  // no device memory for their order: through the host
+        std::vector<uint16_t> z(N);
+        EZ_TRY_HIP(c, hipMemcpyAsync(z.data(), c->s.z, z.size() * sizeof(uint16_t), hipMemcpyDeviceToHost, c->st));
+        EZ_TRY_HIP(c, hipStreamSynchronize(c->st));
+        parallel_for((int64_t)N, [&](int64_t b, int64_t e, int) {
+            for (int64_t i = b; i < e; ++i) zout[i] = z[c->doc_tok[i]];
+        });
+        return EZLDA_OK;
+    }
+    if (n_pieces == 1) {
         EZ_TRY_HIP(c, ez::launch_topics_out(c->s, 0, N, c->read_dev, c->st));
         EZ_TRY_HIP(c, hipMemcpyAsync(zout, c->read_dev, (size_t)N * sizeof(uint16_t), hipMemcpyDeviceToHost, c->st));
         EZ_TRY_HIP(c, hipStreamSynchronize(c->st));
@@ -2102,9 +2144,9 @@ int ezlda_get_aux(ezlda_ctx *c, uint32_t *aux) try {
     auto chk = [&](hipError_t e, const char *what) {
         if (rc == EZLDA_OK && e != hipSuccess) rc = fail(c, EZLDA_EHIP, std::string(what) + ": " + hipGetErrorString(e));
     };
-    chk(hipMalloc((void **)&t.aux_doc, std::max<size_t>(s.N, 1) * sizeof(uint32_t)), "hipMalloc");
-    chk(hipMalloc((void **)&t.dt, dt_words * sizeof(uint32_t)), "hipMalloc");
-    chk(hipMalloc((void **)&t.doc_info, std::max<size_t>(s.D, 1) * sizeof(uint2)), "hipMalloc");
+    chk(ezc::device_alloc(c, (void **)&t.aux_doc, std::max<size_t>(s.N, 1) * sizeof(uint32_t)), "hipMalloc");
+    chk(ezc::device_alloc(c, (void **)&t.dt, dt_words * sizeof(uint32_t)), "hipMalloc");
+    chk(ezc::device_alloc(c, (void **)&t.doc_info, std::max<size_t>(s.D, 1) * sizeof(uint2)), "hipMalloc");
     if (rc == EZLDA_OK && s.D)
         chk(hipMemcpyAsync(t.doc_info, s.doc_info, (size_t)s.D * sizeof(uint2), hipMemcpyDeviceToDevice, c->st),
             "hipMemcpyAsync");

@@ -124,3 +124,49 @@ for failing_load in (0, 1):
         assert np.array_equal(ctx.get_topics(), z), on
     ctx.close()
 """)
+
+
+# the readback's own buffers (4 bytes a token, pinned pieces) are no condition: without them, when loading or given
+# back to a later allocation, the topics come through the host
+@pytest.mark.parametrize("n", [70001, (1 << 19) + 70001])
+@pytest.mark.parametrize("when", ["order", "pinned", "later", "server"])
+def test_readback_without_its_buffers(shim, n, when):
+    _run(shim, f"""
+n, when = {n}, {when!r}
+rng = np.random.default_rng(n)
+off = np.append(np.arange(0, n, 97, dtype=np.int64), n)
+words = rng.integers(0, 300, n).astype(np.int32)
+one = n <= 1 << 19
+order = (n + 3) // 4 * 4 * (6 if one else 4)  # its allocation, no other of this size
+ref = context(off, words, 300, 16)
+if when == "order":
+    shim.shim_fail_malloc(order, 1)
+elif when == "pinned":
+    shim.shim_fail_pinned(1)
+ctx = context(off, words, 300, 16)
+shim.shim_fail_pinned(0)
+gone = when == "order" or (when == "pinned" and not one)
+assert ref.info().device_bytes - ctx.info().device_bytes == (order if gone else 0)
+ctx.sweep(1)
+ref.sweep(1)
+z, aux = ref.get_topics(), ref.get_aux()
+if when == "later":  # the records of get_aux
+    shim.shim_fail_malloc(4 * n, 1)
+elif when == "server":  # its pool
+    shim.shim_fail_malloc(300 * 16 * 4, 1)
+    srv = ezlda.Server(ctx, max_slots=4, sweeps=2, hbm_budget_bytes=1 << 20, seed=3)
+    srv.submit(1, words[:50])
+    srv.wait(1)
+    srv.close()
+if when == "server":  # its creation renews the top topics that the records are of
+    ref.loglik()
+    aux = ref.get_aux()
+assert np.array_equal(ctx.get_aux(), aux)
+if when in ("later", "server"):
+    assert ref.info().device_bytes - ctx.info().device_bytes == order
+assert np.array_equal(ctx.get_topics(), z)
+ctx.sweep(1)
+ref.sweep(1)
+assert np.array_equal(ctx.get_topics(), ref.get_topics())
+assert ctx.loglik() == ref.loglik()
+""")
