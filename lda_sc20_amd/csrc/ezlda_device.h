@@ -17,11 +17,13 @@ static constexpr int kCounterWords = kQueueStride * (1 + 2 * kQueues);
 // sorting their topics (large K); longer ones use a K-sized histogram.
 static constexpr uint32_t kDtShort = 512;
 
-// A sampler item may be a group of up to kGroupMax consecutive words of few
-// tokens (K <= kGroupMaxK, one-wavefront workgroups): the first word in the
-// low bits of its record, the number of further words above them; a run then
-// carries its word's place in the group.
-static constexpr uint32_t kGroupShift = 26, kGroupWord = (1u << kGroupShift) - 1u, kGroupMax = 32;
+// A sampler item may be a group of consecutive words of few tokens (K <=
+// kGroupMaxK, one-wavefront workgroups): the first word in the low bits of its
+// record, the number of further words above them; a run then carries its
+// word's place in the group.  As many words as have room for their tables in
+// kGroupLds bytes: at most kGroupMax (K <= 64), 9 at K = 128, 3 at K = 300.
+static constexpr uint32_t kGroupShift = 26, kGroupWord = (1u << kGroupShift) - 1u, kGroupMax = 18;
+static constexpr uint32_t kGroupLds = 10240;
 static constexpr int kGroupMaxK = 512;
 // Tail words of at most kOwnMax tokens are drawn by half a wavefront each
 // where DT rows are of 32-bit entries.

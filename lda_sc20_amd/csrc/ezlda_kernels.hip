@@ -1,9 +1,10 @@
 // gfx950 kernels of one EZLDA Gibbs sweep.
 //
 // Stage order per sweep (reference EZLDA/mainKernel.cu:158-380):
-//   zero_counts -> topic_hist (n_k) -> wt_head / wt_tail (WT from z)
-//   -> inv + word_top (phi top-3) -> dt_build (DT rows + per-token aux)
-//   -> sample (three-bucket draw, writes z) -> advance_sweep.
+//   begin (clears what the counts add to, moves the sweep counter on)
+//   -> topic_hist (n_k), wt_head, wt_tail (WT from z) -> inv_order + word_top
+//   (phi top-3) -> dt_build (DT rows + per-token aux) -> sample (three-bucket
+//   draw, writes z).
 // Every float operation follows the canonical order of the CPU oracle
 // (oracle/ezlda_oracle.c); builds use -ffp-contract=off, so the topics agree
 // bit for bit.  Wave64: one wavefront owns a doc (dt_build) or a tail word
@@ -46,7 +47,6 @@ __device__ __forceinline__ uint32_t readlane_u(uint32_t v, int l) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
 }
 __device__ __forceinline__ int first_lane(uint64_t m) { return __ffsll((unsigned long long)m) - 1; }
-__device__ __forceinline__ int last_lane(uint64_t m) { return 63 - __clzll((long long)m); }
 __device__ __forceinline__ uint64_t lanemask_lt(int lane) { return (1ull << lane) - 1ull; }
 
 // Orders LDS traffic between the phases of one wavefront.
@@ -89,9 +89,6 @@ static WaveGrid wave_grid(const DevState &s, size_t n, size_t wb, int cap) {
 // offset of phi[topic] in a float array, so a gather needs one AND.
 __device__ __forceinline__ uint32_t dt_topic(uint32_t e) { return (e & 0xFFFFu) >> 2; }
 __device__ __forceinline__ float dt_count(uint32_t e) { return (float)(e >> 16); }
-__device__ __forceinline__ float phi_of(const float *phi, uint32_t e) {
-    return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(phi) + (e & 0xFFFCu));
-}
 
 // Compact DT rows (K <= 8192): 16-bit entries topic | piece << tb, tb =
 // max(10, ceil(log2 K)) topic bits; a count stored in pieces of at most
@@ -99,13 +96,11 @@ __device__ __forceinline__ float phi_of(const float *phi, uint32_t e) {
 __device__ __forceinline__ float c16_count(uint32_t e, uint32_t tb) { return (float)((e & 0xFFFFu) >> tb); }
 __device__ __forceinline__ uint32_t c16_topic(uint32_t e, uint32_t tb) { return e & ((1u << tb) - 1u); }
 
-// The same read for a phi table at LDS address 0 (the sampler's dynamic LDS
+// phi of a DT entry, its table at LDS address 0 (the sampler's dynamic LDS
 // when the kernel has no static LDS, which sampler_static_lds() lets the host
 // check): the entry's low half is the address itself, no base to add.
 typedef __attribute__((address_space(3))) const float lds_cfloat;
 __device__ __forceinline__ float phi_at0(uint32_t e) { return *(lds_cfloat *)(e & 0xFFFCu); }
-// phi of a compact entry (the 16-bit entry in the low half of e)
-__device__ __forceinline__ float phi_c16(uint32_t e, uint32_t tb) { return *(lds_cfloat *)(c16_topic(e, tb) << 2); }
 
 // 16-bit counters, two per LDS word (counts < 65536 by construction).
 __device__ __forceinline__ void h16_add(uint32_t *h, uint32_t k) {
@@ -533,7 +528,7 @@ __global__ void k_word_top(int V, int VD, int K, float beta, const int32_t *__re
     for (int w = blockIdx.x * nwv + wv; w < V; w += gridDim.x * nwv) {
         Top3 t{-1.f, -1.f, -1.f, kNone, kNone, kNone};
         if (w < VD) {
-            // four loads of the row and of inv in flight per lane
+            // two 16-byte (else four 4-byte) loads of the row and of inv in flight a lane
             const int32_t *row = wt_head + (size_t)w * K;
             if ((K & 3) == 0) {
                 const int4 *row4 = reinterpret_cast<const int4 *>(row);
@@ -675,8 +670,9 @@ hipError_t launch_topics_out(const DevState &s, uint32_t b, uint32_t n, uint16_t
 // The link bounds a sweep over chunks, not the kernels: 5 bytes a run over it
 // instead of 16, and neither the word of each slot (4 bytes a token), nor its
 // token (4, not needed on the device), nor z beside z_doc (2, each way).
-// 6.6M tokens in 4 chunks, K = 1024: 31-50 us a chunk of 1.65M tokens beside
-// an upload of 160-225 us (was 480); a sweep 4.0 -> 1.95 ms with the first
+// 6.6M tokens in 4 chunks, K = 1024: 29 us a chunk of 1.65M tokens alone, 75
+// on average beside the other stream's kernels and an upload of 160-225 us (was
+// 480); a sweep 4.0 -> 1.95 ms with the first
 // uploads begun before the last sweep ends.
 // TOPICS: z of z_doc instead, which the first sweep counts.
 template <bool TOPICS>
@@ -1298,7 +1294,7 @@ struct SampleArgs {
     const uint32_t *aux_doc;  // by doc slot: n_dk1 | the doc's row length (nnz) << 16
     const uint32_t *dt;
     uint16_t *z, *z_doc;      // by token (word-major) and by doc slot
-    const uint32_t *counters;  // [0]: the sweep
+    const uint32_t *counters;  // [0]: the sweep drawn (DevState's counters, or from their [1] on where it was begun)
     uint32_t *queue;  // persistent mode: queue q's item counter at queue[q * kQueueStride]
     uint32_t n_queues;
     uint32_t tb;  // compact rows: topic bits
@@ -2336,8 +2332,9 @@ static constexpr uint32_t kFoldStageQ = 64;   // tokens of a word in a step that
 // by word (k_fi_count, the three-pass scan, k_fi_scatter), and persistent
 // workgroups take one (word, segment) item at a time, stage the frozen phi
 // row and Q running sums in LDS and draw its tokens (k_fi_sample); documents
-// finishing their last sweep get their topic counts and topics packed for
-// one copy to the host (k_fi_final).  The order tokens are drawn in never
+// finishing their last sweep get their topics packed for one copy to the host
+// (k_fi_final), where they are counted.  Steps of few tokens are drawn
+// without buckets (k_fi_few).  The order tokens are drawn in never
 // changes a draw, which is keyed by (seed, request id, position, sweep).
 // Slots are (request id, pool offset, tokens, sweep); pool offsets are
 // multiples of 8, and a document's row lives in the row pool at its offset
@@ -2959,9 +2956,10 @@ __device__ __forceinline__ void fi_draw_wave(const uint32_t *row, uint32_t nz, c
 
 // One fold-in sweep of the resident documents when they have few tokens:
 // each workgroup takes 4 T tokens of a slot (groups: slot << 16 | part), copies
-// its row into LDS and draws T of them with each wavefront.  Measured for one document of 217 tokens at K = 1024: a
-// step of 18 us, against 48 us with its tokens bucketed by word (nine launches
-// of about 4 us, k_fi_sample 17).
+// its row into LDS and draws T of them with each wavefront.  Measured for one
+// document of 217 tokens at K = 1024: a step of 18 us, against 48 us with its
+// tokens bucketed by word (nine launches, k_fi_sample of 17 us and the others
+// of about 4).
 template <int T>
 __global__ void __launch_bounds__(256) k_fi_few(const uint4 *__restrict__ slots, int K, float alpha,
                                                 const float *__restrict__ phi, const float *__restrict__ qs,
@@ -3125,7 +3123,7 @@ hipError_t launch_foldin_admit(const uint4 *adm, int nadm, const uint32_t *src, 
 }
 
 // Steps of few tokens are drawn by k_fi_few, straight from the tables: no
-// buckets by word, whose seven launches cost more than they save until big
+// buckets by word, whose six more launches cost more than they save until big
 // words gather enough tokens to share a staged phi row.  What a token costs
 // there follows its document's row, about min(n / 3, K) entries of which the
 // first few hundred count; what buckets save follows V, whose few frequent

@@ -511,7 +511,7 @@ std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uin
     // 175)
     uint32_t group = 1;
     if (groups && K <= ez::kGroupMaxK && a.block_dim == 64 && word_off.size() <= (size_t)ez::kGroupWord)
-        group = std::min<uint32_t>(ez::kGroupMax, 10240u / (4u * (uint32_t)ez::group_stride(K)));
+        group = std::min(ez::kGroupMax, ez::kGroupLds / (4u * (uint32_t)ez::group_stride(K)));
     const uint64_t share = total / (2 * n_wg);
     auto cut = [&](uint64_t cap, uint32_t g) {
         return cut_sample_items(a, word_off, tok_rank, soff, slot_wrd, VD, K, n_xcd, cost, cap, g, share, tiles_used);
