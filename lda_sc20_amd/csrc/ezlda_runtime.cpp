@@ -49,12 +49,13 @@ void run_threads(int T, const F &f) {
     for (auto &x : th) x.join();
 }
 
-// f(begin, end, thread) over parts of [0, n); `work` is what n stands for
-// where it isn't n itself (items of many tokens).
+// f(begin, end, thread) over parts of [0, n), on the caller's thread below
+// `least`; `work` is what n stands for where it isn't n itself (items of many
+// tokens).  Starting the threads takes about 0.25 ms.
 template <class F>
-void parallel_for(int64_t n, F f, int64_t work = 0) {
-    const int T = host_threads();
-    if (std::max(n, work) < 65536 || T == 1) {
+void parallel_for(int64_t n, F f, int64_t work = 0, int64_t least = 65536) {
+    const int T = std::max(n, work) < least ? 1 : host_threads();
+    if (T == 1) {
         f(0, n, 0);
         return;
     }
@@ -66,6 +67,10 @@ void parallel_for(int64_t n, F f, int64_t work = 0) {
 // the link that fills it, so several threads share it.
 constexpr uint32_t kReadTokens = 1u << 19;
 constexpr uint32_t kReadSlots = 8;
+// Corpora of at most this many tokens are read back through the host, one
+// copy and a loop, and need no buffers for it: 300 tokens 15 us (26 by a kernel
+// and a copy), 20,000 17 (27), 40,000 23 (29), 65,000 31 (31), 100,000 42 (35).
+constexpr uint32_t kHostReadTokens = 65536;
 
 // DT rows: 16-bit entries for K <= kCompactK (the oracle's ORC_COMPACT_K),
 // tb = max(10, ceil(log2 K)) topic bits, counts in pieces of at most
@@ -202,8 +207,9 @@ namespace {
 }  // namespace
 
 void ezc::drop_readback(ezlda_ctx *c) {
-    if (c->st) (void)hipStreamSynchronize(c->st);
-    if (c->s.doc_tok) (void)hipFree(c->s.doc_tok);
+    if (!c->s.doc_tok) return;
+    (void)hipStreamSynchronize(c->st);
+    (void)hipFree(c->s.doc_tok);
     if (c->read_buf) (void)hipHostFree(c->read_buf);
     for (hipEvent_t e : c->read_ev) (void)hipEventDestroy(e);
     c->read_ev.clear();
@@ -299,7 +305,7 @@ int lupload(ezlda_ctx *c, T **p, const std::vector<T> &v) {
 // the host, and a later allocation that fails has them back (device_alloc).
 void alloc_readback(ezlda_ctx *c) {
     const uint32_t N = c->s.N, pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
-    if (pieces == 0) return;
+    if (N <= kHostReadTokens) return;
     const size_t order = ((size_t)N + 3) / 4 * 4;  // the buffer behind it is 16-byte aligned
     const size_t bytes = order * sizeof(uint32_t) + (pieces == 1 ? order * sizeof(uint16_t) : 0);
     bool ok = hipMalloc((void **)&c->s.doc_tok, bytes) == hipSuccess;
@@ -871,10 +877,12 @@ int load_chunked(ezlda_ctx *c, const std::vector<uint32_t> &tok_doc, const std::
         if ((r = dalloc(c, &c->cimg[j], max_bytes))) return r;
         if ((r = dalloc(c, &c->cdt[j], dt_words))) return r;
         EZ_TRY_HIP(c, hipMemset(c->cdt[j], 0, dt_words * sizeof(uint32_t)));
-        if ((r = dalloc(c, &c->caux[j], max_n))) return r;
-        if ((r = dalloc(c, &c->cz[j], max_n))) return r;
-        if ((r = dalloc(c, &c->cwrd[j], max_n))) return r;
-        if ((r = dalloc(c, &c->cruns[j], max_runs))) return r;
+        // runs, then slot_wrd, the slots' records and z (16-byte aligned), in one allocation
+        const size_t n8 = ((size_t)max_n + 7) & ~(size_t)7;
+        if ((r = dalloc(c, &c->cruns[j], max_runs + n8 * 10 / sizeof(uint4)))) return r;
+        c->cwrd[j] = reinterpret_cast<uint32_t *>(c->cruns[j] + max_runs);
+        c->caux[j] = c->cwrd[j] + n8;
+        c->cz[j] = reinterpret_cast<uint16_t *>(c->caux[j] + n8);
         if ((r = dalloc(c, &c->cctr[j], ez::kCounterWords))) return r;
         EZ_TRY_HIP(c, hipMemset(c->cctr[j], 0, ez::kCounterWords * sizeof(uint32_t)));
         if ((r = dalloc(c, &c->cll[j], max_items))) return r;
@@ -1874,10 +1882,9 @@ namespace {
 int read_topics(ezlda_ctx *c, uint16_t *zout) {
     const uint32_t N = c->s.N, n_pieces = (uint32_t)(((uint64_t)N + kReadTokens - 1) / kReadTokens);
     if (!N) return EZLDA_OK;
-    if (!c->s.doc_tok) {  // no device memory for their order: through the host
+    if (!c->s.doc_tok) {  // few tokens, or no device memory for their order
         std::vector<uint16_t> z(N);
-        EZ_TRY_HIP(c, hipMemcpyAsync(z.data(), c->s.z, z.size() * sizeof(uint16_t), hipMemcpyDeviceToHost, c->st));
-        EZ_TRY_HIP(c, hipStreamSynchronize(c->st));
+        EZ_TRY_HIP(c, hipMemcpy(z.data(), c->s.z, z.size() * sizeof(uint16_t), hipMemcpyDeviceToHost));
         parallel_for((int64_t)N, [&](int64_t b, int64_t e, int) {
             for (int64_t i = b; i < e; ++i) zout[i] = z[c->doc_tok[i]];
         });
@@ -1938,7 +1945,7 @@ int ezlda_get_topics(ezlda_ctx *c, uint16_t *zout) try {
                 }
                 zout[i] = zd[p - slot0];
             }
-        });
+        }, 0, kReadTokens);  // 0.5 ns a token on one thread
         return EZLDA_OK;
     }
     return read_topics(c, zout);

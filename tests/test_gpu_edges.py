@@ -47,6 +47,22 @@ def test_topics_are_read_back_in_the_corpus_order(n):
     ctx.close()
 
 
+# where the topics stop coming through the host's loop, and a lane's eight behind it
+@pytest.mark.parametrize("n", [65535, 65536, 65537, 65543, 65544, 65545])
+@pytest.mark.parametrize("chunks", [1, 3])
+def test_topics_of_corpora_around_the_host_readback(n, chunks):
+    rng = np.random.default_rng(n)
+    off = np.append(np.arange(0, n, 61, dtype=np.int64), n)
+    words = rng.integers(0, 300, n).astype(np.int32)
+    z = rng.integers(0, 9, n).astype(np.uint16)
+    ctx = ezlda.Context(K=9, alpha=0.5, beta=BETA, seed=1, num_chunks=chunks)
+    ctx.load(ezlda.Corpus(300, off, words), z0=z)
+    assert np.array_equal(ctx.get_topics(), z)
+    ctx.set_topics(z[::-1].copy())
+    assert np.array_equal(ctx.get_topics(), z[::-1])
+    ctx.close()
+
+
 # items cut by cost: documents of up to 5,000 tokens holding a word hundreds of
 # times, rows of more than a block per checkpoint (16- and 32-bit), and
 # corpora of fewer items than workgroups; the run cap does not change a draw
