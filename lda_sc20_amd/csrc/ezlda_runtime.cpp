@@ -522,7 +522,17 @@ std::vector<uint4> build_sample_items(const ezlda_args &a, const std::vector<uin
     auto cut = [&](uint64_t cap, uint32_t g) {
         return cut_sample_items(a, word_off, tok_rank, soff, slot_wrd, VD, K, n_xcd, cost, cap, g, share, tiles_used);
     };
-    std::vector<uint4> out = cut(std::max(least, total / (2 * n_wg)), group);
+    uint64_t cap = std::max(least, total / (2 * n_wg));
+    if (K > (int)kCompactK) {
+        // an item stages 33 to 65 KB, so the CUs hold a quarter to half of the
+        // workgroups: one such share an item, not a quarter of it (sampler ms a
+        // sweep, first sweeps / topical state: 3.7M tokens of 1,478 words at K =
+        // 13523 3.87 -> 2.55 / 0.87 -> 0.56; 2.6M of 25,000 words at K = 12013
+        // 4.35 -> 2.98 / 0.82 -> 0.57; two shares: 2.47 / 0.58 and 3.01 / 0.55)
+        const uint64_t fit = std::max<uint64_t>(1, (uint64_t)device_lds_per_cu() / ez::sample_lds_bytes(K, a.block_dim));
+        cap = std::max(least, total / std::min(n_wg, fit * (uint64_t)device_cus()));
+    }
+    std::vector<uint4> out = cut(cap, group);
     // neither the cap nor the groups decide whether the allocation-free
     // log-likelihood takes a corpus
     size_t single = out.size();
