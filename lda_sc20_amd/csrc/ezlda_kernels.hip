@@ -3522,7 +3522,16 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
     const int NS = (s.K + 63) >> 6;
     const long room = (long)s.lds_cu / 4 - own_shared(NS);
     const int own_wv = room > 0 ? (int)std::min<long>(16, room / (2 * own_stride(NS))) : 0;
-    const bool own = s.first_own < s.n_smp_segs && own_wv >= 4;
+    // and where there are enough of these items: the launch takes 80 to 110 us
+    // however few, as many items a CU as 32 take in k_sample where four of its
+    // tables fit a CU, 14 where three do, 10 where two do (without it / with it: 0
+    // to 2,500 items at K > 8192 0.36 to 1.0; 6,500 at K = 8348 0.76, 11,000 at K =
+    // 8661 0.9 to 1.1, 15,000 at K = 8867 1.4; 2,784 at K = 11709 0.83, 3,151 at K =
+    // 11287 0.8 to 0.9, 3,600 to 7,700 at K > 9,950 1.0 to 2.7; 2,568 at K = 13463
+    // 1.0, 3,458 at K = 13358 1.4, 2,627 at K = 15552 1.1 to 1.2)
+    const int fit = (int)((size_t)s.lds_cu / lds);
+    const int line = fit >= 4 ? 32 : fit == 3 ? 14 : 10;
+    const bool own = s.n_smp_segs - s.first_own >= s.n_cu * line && own_wv >= 4;
     const int32_t n_first = own ? s.first_own : s.n_smp_segs;
     A.first_item = (uint32_t)n_first;
     A.n_items = (uint32_t)n_first;
@@ -3550,7 +3559,17 @@ hipError_t launch_sample(const DevState &s, bool shortcut, hipStream_t st, uint3
     // items (13 a workgroup) at K = 4096 767 / 672, 98,189 (24) at K = 2048
     // 2,277 / 1,564, 126,191 (31) at K = 1024 3,519 / 2,884.
     unsigned grid = (unsigned)n_first;
-    A.n_queues = s.grid_dim > 0 && n_first / 4 >= s.grid_dim ? (uint32_t)s.n_queues : 0u;
+    // At K > 8192 fewer workgroups fit the CUs than the grid has and an item's
+    // tables take long: a resident corpus takes from queues as soon as there are
+    // more items than fit (in turn / from queues: 5,392 items at K = 12368 700 /
+    // 586, 4,948 at K = 10383 763 / 730, 5,292 at K = 8924 371 / 335).  A chunk,
+    // whose first_own is past its items, does not: its many words of few tokens go
+    // faster in turn (a sweep of 14,552 items in 4 chunks at K = 15063 2,810 /
+    // 3,177, of 17,582 in 5 at K = 15854 3,076 / 3,442, of 13,970 in 3 at K = 9061
+    // 2,153 / 1,910 first and 1,336 / 1,369 later).
+    const bool resident = s.first_own <= s.n_smp_segs;
+    const int32_t many = s.compact || !resident ? 4 * s.grid_dim : std::min(s.grid_dim, s.n_cu * std::max(1, fit) + 1);
+    A.n_queues = s.grid_dim > 0 && n_first >= many ? (uint32_t)s.n_queues : 0u;
     if (s.grid_dim > 0 && A.n_queues == 0) grid = (unsigned)std::min(n_first, s.grid_dim);
     A.stats = s.stats;
     A.seed = s.seed;

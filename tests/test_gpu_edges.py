@@ -278,6 +278,22 @@ def test_words_of_few_tokens_at_large_k(K, kw, odd):
         assert np.array_equal(ctx.get_topics(), orc.get_topics())
 
 
+# enough of them for the launch of half wavefronts (32, 14 or 10 a CU of 256, as
+# four, three or two of the sampler's tables fit a CU), and one less
+@pytest.mark.parametrize("K,n", [(8200, 8191), (8200, 8192), (10000, 3583), (10000, 3584), (16383, 2559), (16383, 2560)])
+def test_many_words_of_few_tokens_at_large_k(K, n):
+    rng = np.random.default_rng(K + n)
+    counts = np.concatenate([[900, 400, 200, 129], np.full(9, 128), rng.integers(1, 7, n - 9)])
+    bag = rng.permutation(np.repeat(rng.permutation(len(counts)), counts)).astype(np.int32)
+    off = np.linspace(0, len(bag), 301).astype(np.int64)
+    ctx, orc = _pair(off, bag, len(counts), K, dense_words=2)
+    for n in (1, 2):
+        ctx.sweep(n)
+        orc.sweep(n)
+        assert np.array_equal(ctx.get_topics(), orc.get_topics()), n
+    ctx.close()
+
+
 # dense rows of one segment (32,768 tokens) are written whole, of several added
 # up; words without a token; K with and without 16-byte rows
 @pytest.mark.parametrize("K", [64, 65, 1026, 2600])

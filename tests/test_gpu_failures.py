@@ -170,3 +170,15 @@ ref.sweep(1)
 assert np.array_equal(ctx.get_topics(), ref.get_topics())
 assert ctx.loglik() == ref.loglik()
 """)
+
+
+# half wavefronts of words of few tokens on one CU, where a handful of such words is enough for them
+@pytest.mark.parametrize("K", [8192, 8193, 10000, 16383])
+def test_words_of_few_tokens_on_one_cu(shim, K):
+    _run(shim, f"""
+shim.shim_cus(1)
+from test_gpu_edges import test_words_of_few_tokens_at_large_k as test
+for odd in (0, 1):
+    for kw in (dict(), dict(shortcut=0), dict(block_dim=64, run_cap=1)):
+        test({K}, kw, odd)
+""")
