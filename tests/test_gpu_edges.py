@@ -338,6 +338,27 @@ def test_rows_of_sorted_topics(K):
         assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
 
 
+# tail words none of which is longer than those sorted; and beside longer words as
+# many short ones as are counted with them (2^18 counts a CU of 256), and one more
+@pytest.mark.parametrize("K,longer,short", [(4900, 0, 0), (16383, 0, 0), (4900, 2, 13695), (4900, 2, 13696), (16383, 2, 4096), (16383, 2, 4097)])
+def test_rows_sorted_beside_rows_counted(K, longer, short):
+    sizes = [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512]
+    counts = [700, 513][:longer] + sizes + [1] * (short - len(sizes))
+    rng = np.random.default_rng(K + short)
+    words = rng.permutation(np.repeat(rng.permutation(len(counts)), counts)).astype(np.int32)
+    off = np.linspace(0, len(words), 101).astype(np.int64)
+    ctx, orc = _pair(off, words, len(counts) + 1 if short == 0 else len(counts), K, dense_words=0)
+    for n in (1, 2):
+        for c in (ctx, orc):
+            c.sweep(n)
+            c.build_wt()
+            c.topk()
+        assert np.array_equal(ctx.get_topics(), orc.get_topics())
+        assert np.array_equal(ctx.get_top(), orc.get_top())
+    assert abs(ctx.loglik() - orc.loglik()) <= 1e-9 * abs(orc.loglik())
+    ctx.close()
+
+
 # DT rows compacted 128 topics a step (K <= 1024), from a bitmap above it;
 # counts below, at and above one entry's 63 (K <= 1024), 31 and 15
 @pytest.mark.parametrize("K", [1, 2, 3, 64, 127, 128, 129, 255, 257, 1023, 1024, 1025, 2049])
