@@ -3378,12 +3378,14 @@ static hipError_t count_topics(const DevState &s, bool fresh, hipStream_t st) {
     // (at small K there is no head word or no tail word; the rows are then
     // built by histograms at every length)
     int w1 = (size_t)s.lds_cu / dt_wave_bytes(s.K) < 16 ? std::max(s.VD, std::min(s.V, s.w_short)) : s.V;
-    // Where longer words are counted in any case, short ones of at most 2^18
-    // counts a CU are too: a second launch costs 10 us (sorted / counted: 2,938
-    // words at K = 4900 59.7 / 45.4, 1,936 at K = 8000 72.8 / 59.0, 3,938 at K =
-    // 8200 68.0 / 63.5; beyond it 9,942 at K = 8200 75.0 / 76.7, 19,943 at K =
-    // 12000 92.1 / 101.5).
-    if (w1 > s.VD && (size_t)(s.V - w1) * (size_t)s.K <= (size_t)s.n_cu << 18) w1 = s.V;
+    // Where longer words are counted in any case, few short ones are too: a
+    // second launch costs 10 us.  The counts take a time like K a word on a number
+    // of wavefronts like 1 / K, hence the square (sorted / counted: 2,938 words at
+    // K = 4900 59.7 / 45.4, 19,943 56.4 / 53.8, 5,939 at K = 8000 65.8 / 59.1, 3,649
+    // at K = 12000 97.4 / 91.9, 1,936 at K = 16383 94.7 / 84.8; beyond the line 9,942
+    // at K = 8000 72.3 / 72.8, 9,942 at K = 12000 88.2 / 88.5, 5,939 at K = 16383
+    // 101.9 / 105.7, some 3,800 at K = 15099 60.0 / 68.7).
+    if (w1 > s.VD && (uint64_t)(s.V - w1) * (uint64_t)s.K * (uint64_t)s.K <= (uint64_t)s.n_cu << 31) w1 = s.V;
     if (w1 > s.VD) {
         const WaveGrid g = wave_grid(s, (size_t)(w1 - s.VD), dt_wave_bytes(s.K), 1 << 16);
         hipLaunchKernelGGL(k_wt_tail, dim3(g.grid), dim3(64 * g.nwv), g.nwv * dt_wave_bytes(s.K), st,

@@ -339,8 +339,8 @@ def test_rows_of_sorted_topics(K):
 
 
 # tail words none of which is longer than those sorted; and beside longer words as
-# many short ones as are counted with them (2^18 counts a CU of 256), and one more
-@pytest.mark.parametrize("K,longer,short", [(4900, 0, 0), (16383, 0, 0), (4900, 2, 13695), (4900, 2, 13696), (16383, 2, 4096), (16383, 2, 4097)])
+# many short ones as are counted with them (2^31 / K^2 a CU of 256), and one more
+@pytest.mark.parametrize("K,longer,short", [(4900, 0, 0), (16383, 0, 0), (8000, 2, 8589), (8000, 2, 8590), (16383, 2, 2048), (16383, 2, 2049)])
 def test_rows_sorted_beside_rows_counted(K, longer, short):
     sizes = [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512]
     counts = [700, 513][:longer] + sizes + [1] * (short - len(sizes))
